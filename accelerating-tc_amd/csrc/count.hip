@@ -984,6 +984,7 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   const uint32_t* col = g->col.as<uint32_t>();
   Timer prep(c);
   LaunchMarks lm(c);
+  bool on16 = false;  // AUTO over the 16-bit list layer
   TCX_TRY(prep.begin());
   // schedule (cached per graph)
   switch (s.kernel) {
@@ -1011,8 +1012,17 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
       if (s.auto_thresholds[3] > kLaneMaxDeg)
         return fail(TC_ERR_ARG, "auto_thresholds[3] must be <= %u", kLaneMaxDeg);
       const uint32_t lmax = s.auto_thresholds[3] ? s.auto_thresholds[3] : kLaneMaxDeg;
-      if (s.auto_thresholds[2] == TC_AUTO_PUSH) TCX_TRY(auto_schedule(c, g, wmax, hmin));
-      else TCX_TRY(wl_schedule(c, g, wmax, hmin, lmax));
+      if (s.auto_thresholds[2] == TC_AUTO_PUSH) {
+        TCX_TRY(auto_schedule(c, g, wmax, hmin));
+        break;
+      }
+      // the default schedule counts over 16-bit lists where they suit the
+      // graph; a caller's thresholds select the 32-bit work-list tasks
+      if (!s.auto_thresholds[0] && !s.auto_thresholds[1] && !s.auto_thresholds[3]) {
+        TCX_TRY(lists16(c, g));
+        on16 = g->sc.l16.usable;
+      }
+      if (!on16) TCX_TRY(wl_schedule(c, g, wmax, hmin, lmax));
       break;
     }
     default:
@@ -1104,6 +1114,15 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     }
     case TC_KERNEL_AUTO: {
       const SchedCache& sc = g->sc;
+      if (on16) {
+        TCX_TRY(c->scratch.reserve(64 + kAccBytes16));
+        uint32_t* cur = c->scratch.as<uint32_t>();
+        unsigned long long* acc16 = c->scratch.as<unsigned long long>() + 8;
+        TCX_HIP(hipMemsetAsync(cur, 0, 64 + kAccBytes16, c->stream));
+        TCX_TRY(lm.mark());
+        TCX_TRY(count16(c, g, s.grid_size, cur, acc16, &tm.launches));
+        break;
+      }
       TCX_TRY(c->scratch.reserve(64));
       uint32_t* cursor = c->scratch.as<uint32_t>();
       TCX_HIP(hipMemsetAsync(cursor, 0, 8 * sizeof(uint32_t), c->stream));
@@ -1164,8 +1183,16 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   TCX_HIP(hipGetLastError());
   TCX_TRY(lm.finish(&tm));
   unsigned long long h = 0;
-  TCX_HIP(hipMemcpyAsync(&h, acc, 8, hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
+  if (on16) {
+    unsigned long long part[kAccBytes16 / 8];
+    TCX_HIP(hipMemcpyAsync(part, c->scratch.as<unsigned long long>() + 8, kAccBytes16,
+                           hipMemcpyDeviceToHost, c->stream));
+    TCX_HIP(hipStreamSynchronize(c->stream));
+    h = sum16(part);
+  } else {
+    TCX_HIP(hipMemcpyAsync(&h, acc, 8, hipMemcpyDeviceToHost, c->stream));
+    TCX_HIP(hipStreamSynchronize(c->stream));
+  }
   *count = h;
   tm.ms_prep = prep.ms;
   if (timing) *timing = tm;

@@ -574,7 +574,7 @@ static int csr_from_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint
 }
 
 int compute_csr_stats(tc_ctx* c, tc_graph* g) {
-  DevBuf indeg;
+  DevBuf& indeg = g->indeg;
   TCX_TRY(indeg.reserve(sizeof(uint32_t) * ((size_t)g->n + 1)));
   TCX_TRY(c->accum.reserve(64));
   unsigned long long* acc = c->accum.as<unsigned long long>();

@@ -75,6 +75,24 @@ struct tc_ctx {
 };
 
 namespace tcx {
+// Out-list rows in 16-byte units and the work lists and tasks over them
+// (lists16.h).
+struct Rows16 {
+  DevBuf row;                      // uint2[n]: first unit of the row, units
+  DevBuf col;                      // entries, rows padded to whole units
+  DevBuf se;                       // uint2[entries]: row of each work-list entry's list
+  DevBuf who;                      // uint32[tasks]: owner
+  DevBuf act;                      // uint4[tasks + 1]: entry range, owner's row
+  DevBuf slice;                    // uint2[nslice + 1]: first (task, entry) of each slice
+  uint64_t units = 0, entries = 0, tasks = 0;
+  uint32_t nslice = 0;
+};
+struct Lists16 {
+  uint64_t version = ~0ull;        // the CSR it was built (or found unsuitable) for
+  bool usable = false;
+  Rows16 hub, tail;                // entries with 16-bit ids, the others (32-bit)
+};
+
 // Per-graph schedules, rebuilt when the oriented CSR changes.
 struct SchedCache {
   uint64_t version = ~0ull;
@@ -95,6 +113,7 @@ struct SchedCache {
   DevBuf wl_ell;                   // uint32[8 n]: out-lists of <= 8 entries, kEmpty-padded rows
   uint64_t nw_small = 0, nw_large = 0, nw_huge = 0, nw_lane = 0;
   uint64_t wl_entries = 0;         // edges kept in the work lists
+  Lists16 l16;
   double wl_bytes = 0;             // bytes one count streams (see count.hip)
   bool rows_ok = false;
   DevBuf rows;                     // rows with d+ >= 2
@@ -134,6 +153,7 @@ struct tc_graph {
   tcx::DevBuf rowptr;       // uint32[n+1]
   tcx::DevBuf col;          // uint32[m_or]
   tcx::DevBuf esrc;         // uint32[m_or]  source of each CSR edge
+  tcx::DevBuf indeg;        // uint32[n]  in-degrees of the oriented CSR
   tcx::DevBuf vkey;         // int32[n] ADIR priority / KCORE core number
   uint64_t sum_out_sq = 0, sum_in_out = 0;
   // cached schedules (valid for the current CSR)
@@ -144,8 +164,9 @@ struct tc_graph {
 namespace tcx {
 
 // ---- primitives (prims.hip) ---------------------------------------------
+// Ascending by bits [begin_bit, end_bit), stable.
 int sort_u64(tc_ctx* c, uint64_t* keys, uint64_t* tmp, uint64_t n, int end_bit,
-             uint64_t** sorted);
+             uint64_t** sorted, int begin_bit = 0);
 int sort_pairs_u64_u32(tc_ctx* c, uint64_t* keys, uint64_t* ktmp, uint32_t* vals,
                        uint32_t* vtmp, uint64_t n, int end_bit, uint64_t** skeys,
                        uint32_t** svals);
@@ -181,6 +202,16 @@ int graph_clone_records(tc_ctx* c, const tc_graph* g, tc_graph** out);
 // Builds (or keeps) the default work-list schedule of g: sc.wl_rp / wl_col
 // and the fixed rule's task lists.
 int worklists(tc_ctx* c, tc_graph* g);
+
+// ---- the 16-bit list layer (lists16.hip) -----------------------------------
+// Builds (or keeps) g's layer when its lists suit it (g->sc.l16.usable).
+int lists16(tc_ctx* c, tc_graph* g);
+// Enqueues the count over a usable layer; acc: kAccBytes16 bytes, cleared, as
+// are cursor[0] and [1]; sum16 adds the copied-back accumulators.
+constexpr size_t kAccBytes16 = 8 * 64 * 16;
+int count16(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor, unsigned long long* acc,
+            uint32_t* launches);
+unsigned long long sum16(const unsigned long long* acc);
 
 // ---- cost model and per-vertex counts (mlp.hip, count.hip) ---------------
 // Predicted log2 costs Y[n][2] for device features X[n][8]; fails when the

@@ -1,0 +1,452 @@
+// Builds and counts over the 16-bit list layer (lists16.h).
+#include "lists16.h"
+
+#include <algorithm>
+#include <vector>
+
+#include "internal.h"
+
+namespace tcx {
+namespace {
+
+using namespace dev;
+
+constexpr uint32_t kHistBins = 4096;  // in-degree histogram, the last bin open
+// A graph takes the layer when its average pushed list (sum d- d+ / m) has at
+// least this many entries and at least this share of its entries gets a
+// 16-bit id.  Below 20 entries a list is one step of a group with most lanes
+// idle (ER of 65,536 vertices and 2^20 edges, 16 entries, stays with the
+// 32-bit tasks); below the share, the tail's work lists and tasks come on top
+// of the layer's.  R-MAT graphs are at 0.88-1.0.
+constexpr uint64_t kMinList = 20;
+constexpr double kMinShare = 0.7;
+constexpr uint64_t kTaskCost = 48;  // a task's own row and map, in group steps
+
+unsigned grid_for(uint64_t n, int tb = TB) {
+  uint64_t b = (n + tb - 1) / tb;
+  return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(b, 1u << 20));
+}
+
+__global__ void k_fill16(uint32_t* p, uint32_t v, uint64_t n) {
+  for (uint64_t i = gtid(); i < n; i += gstride()) p[i] = v;
+}
+
+// hist[min(indeg, bins - 1)] += 1, and the in-degree sum of the open bin
+__global__ __launch_bounds__(TB) void k_indeg_hist(const uint32_t* __restrict__ indeg, uint32_t n,
+                                                   uint32_t* __restrict__ hist,
+                                                   unsigned long long* open_sum) {
+  __shared__ uint32_t h[kHistBins];
+  for (uint32_t i = threadIdx.x; i < kHistBins; i += TB) h[i] = 0;
+  __syncthreads();
+  unsigned long long s = 0;
+  for (uint64_t v = gtid(); v < n; v += gstride()) {
+    const uint32_t d = indeg[v];
+    if (d >= kHistBins - 1) s += d;
+    atomicAdd(h + min(d, kHistBins - 1), 1u);
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < kHistBins; i += TB)
+    if (h[i]) atomicAdd(hist + i, h[i]);
+  flush_count(s, open_sum);
+}
+
+__global__ void k_hub_flags(const uint32_t* __restrict__ indeg, uint32_t n, uint32_t t,
+                            uint32_t* __restrict__ f) {
+  for (uint64_t v = gtid(); v < n; v += gstride()) f[v] = indeg[v] >= t ? 1u : 0u;
+}
+
+__global__ void k_hub_ids(const uint32_t* __restrict__ indeg, const uint32_t* __restrict__ pos,
+                          uint32_t n, uint32_t t, uint16_t* __restrict__ id) {
+  for (uint64_t v = gtid(); v < n; v += gstride())
+    id[v] = indeg[v] >= t ? (uint16_t)pos[v] : (uint16_t)kPad16;
+}
+
+// f[e] = 1 where the entry has a 16-bit id; f[m] = 0
+__global__ void k_entry_flags(const uint32_t* __restrict__ col, uint64_t m,
+                              const uint16_t* __restrict__ id, uint32_t* __restrict__ f) {
+  for (uint64_t e = gtid(); e <= m; e += gstride())
+    f[e] = e < m && id[col[e]] != kPad16 ? 1u : 0u;
+}
+
+// Rows are laid out so that none touches a cache line more than its length
+// needs: rows above four units start on a 128-byte line, shorter ones are
+// grouped by their size rounded up to 1, 2 or 4 units (lists average a few
+// lines: with rows packed one after the other R-MAT-22, A-ordered, moved 28.0
+// instead of 25.5 GB a count, in 3.80 instead of 3.57 ms).  A row's place is the number of
+// rows, or of 8-unit lines, before it in its class; the four counters ride
+// in two 64-bit scans.
+struct Place16 {
+  uint64_t a, b;  // (lines of the 8-unit class, rows of 4), (rows of 2, rows of 1)
+};
+
+__device__ inline Place16 place16(uint32_t units) {
+  if (units > 4) return {(uint64_t)((units + 7) / 8) << 32, 0ull};
+  if (units > 2) return {1ull, 0ull};
+  return units == 2 ? Place16{0ull, 1ull << 32} : Place16{0ull, units ? 1ull : 0ull};
+}
+
+// First unit of a row from its place and the classes' totals t.
+__device__ inline uint32_t start16(uint32_t units, Place16 p, Place16 t) {
+  const uint32_t base4 = (uint32_t)(t.a >> 32) * 8u, base2 = base4 + (uint32_t)t.a * 4u,
+                 base1 = base2 + (uint32_t)(t.b >> 32) * 2u;
+  if (units > 4) return (uint32_t)(p.a >> 32) * 8u;
+  if (units > 2) return base4 + (uint32_t)p.a * 4u;
+  return units == 2 ? base2 + (uint32_t)(p.b >> 32) * 2u : base1 + (uint32_t)p.b;
+}
+
+// Entries of each row with (cnt) and without (tcnt) a 16-bit id, from the
+// prefix `pre` of k_entry_flags (null: all of them have one).
+__global__ void k_counts16(const uint32_t* __restrict__ rp, const uint32_t* __restrict__ pre,
+                           uint32_t n, uint32_t* __restrict__ cnt, uint32_t* __restrict__ tcnt) {
+  for (uint64_t u = gtid(); u < n; u += gstride()) {
+    const uint32_t b = rp[u], e = rp[u + 1], c = pre ? pre[e] - pre[b] : e - b;
+    cnt[u] = c;
+    if (tcnt) tcnt[u] = e - b - c;
+  }
+}
+
+// The rows' class counters (n + 1 entries), per entries to a unit.
+__global__ void k_places16(const uint32_t* __restrict__ cnt, uint32_t n, uint32_t per,
+                           uint64_t* __restrict__ pa, uint64_t* __restrict__ pb) {
+  for (uint64_t u = gtid(); u <= n; u += gstride()) {
+    const Place16 p = place16(u < n ? (cnt[u] + per - 1) / per : 0u);
+    pa[u] = p.a;
+    pb[u] = p.b;
+  }
+}
+
+__global__ void k_row_pairs(const uint32_t* __restrict__ cnt, const uint64_t* __restrict__ pa,
+                            const uint64_t* __restrict__ pb, uint32_t n, uint32_t per,
+                            uint2* __restrict__ row) {
+  const Place16 t{pa[n], pb[n]};
+  for (uint64_t u = gtid(); u < n; u += gstride()) {
+    const uint32_t units = (cnt[u] + per - 1) / per;
+    row[u] = make_uint2(start16(units, Place16{pa[u], pb[u]}, t), units);
+  }
+}
+
+__global__ void k_scatter16(const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
+                            const uint32_t* __restrict__ esrc, uint64_t m,
+                            const uint16_t* __restrict__ id, const uint32_t* __restrict__ pre,
+                            const uint2* __restrict__ row, uint16_t* __restrict__ col16,
+                            const uint2* __restrict__ trow, uint32_t* __restrict__ tcol) {
+  for (uint64_t e = gtid(); e < m; e += gstride()) {
+    const uint32_t u = esrc[e], v = col[e], b = rp[u];
+    const uint32_t h = id ? id[v] : v;
+    const uint32_t p = pre ? pre[e] : (uint32_t)e, pb = pre ? pre[b] : b;
+    if (h != kPad16) col16[8ull * row[u].x + (p - pb)] = (uint16_t)h;
+    else tcol[4ull * trow[u].x + ((uint32_t)e - b - (p - pb))] = v;
+  }
+}
+
+// Work-list key (owner << 32 | streamed) of every edge u -> v: the end with
+// the longer row (cnt entries) owns it, u on a tie; no key ((n << 32), sorted
+// last) when either row is empty, or the owner u's only entry is v itself.
+// id: the 16-bit ids (null: every vertex has one); tail: rows of the entries
+// without one.
+__global__ void k_keys16(const uint32_t* __restrict__ esrc, const uint32_t* __restrict__ col,
+                         uint64_t m, uint32_t n, const uint32_t* __restrict__ cnt,
+                         const uint16_t* __restrict__ id, bool tail, uint64_t* __restrict__ key) {
+  for (uint64_t e = gtid(); e < m; e += gstride()) {
+    const uint32_t u = esrc[e], v = col[e], cu = cnt[u], cv = cnt[v];
+    uint64_t k = (uint64_t)n << 32;
+    if (cu && cv) {
+      if (cv > cu) k = ((uint64_t)v << 32) | u;
+      else if (cu > 1 || (id && id[v] == kPad16) != tail) k = ((uint64_t)u << 32) | v;
+    }
+    key[e] = k;
+  }
+}
+
+// se[i] = row of the streamed list of sorted key i; cost[owner] += its group
+// steps, summed over each wave's runs of one owner before the atomic.
+__global__ __launch_bounds__(TB) void k_entries16(const uint64_t* __restrict__ key, uint64_t E,
+                                                  const uint2* __restrict__ row,
+                                                  uint2* __restrict__ se,
+                                                  unsigned long long* __restrict__ cost) {
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint64_t b = gtid() & ~63ull; b < E; b += gstride()) {
+    const uint64_t i = b + lane;
+    uint32_t o = 0xFFFFFFFFu, st = 0;
+    if (i < E) {
+      const uint64_t k = key[i];
+      const uint2 r = row[(uint32_t)k];
+      se[i] = r;
+      o = (uint32_t)(k >> 32);
+      st = (r.y + kGroup16 - 1) / kGroup16;
+    }
+    const uint32_t incl = wave_incl_scan_dpp(st);
+    const uint32_t prev = (uint32_t)__shfl_up((int)o, 1, 64), next = (uint32_t)__shfl_down((int)o, 1, 64);
+    const uint64_t heads = lanes(lane == 0 || o != prev);
+    const uint32_t h = 63u - (uint32_t)__builtin_clzll(heads & (~0ull >> (63 - lane)));
+    const uint32_t before = (uint32_t)__shfl((int)(incl - st), (int)h, 64);
+    if (i < E && (lane == 63 || o != next))
+      atomicAdd(cost + o, (unsigned long long)(incl - before));
+  }
+}
+
+__global__ void k_nonempty(const uint32_t* __restrict__ wrp, uint32_t n, uint8_t* __restrict__ f) {
+  for (uint64_t x = gtid(); x < n; x += gstride()) f[x] = wrp[x + 1] > wrp[x] ? 1 : 0;
+}
+
+// act[i] of k_count16 for the owners ids[0, nt), one closing entry after them
+__global__ void k_tasks16(const uint32_t* __restrict__ ids, uint32_t nt,
+                          const uint32_t* __restrict__ wrp, const uint2* __restrict__ row,
+                          const unsigned long long* __restrict__ cost, uint4* __restrict__ act,
+                          uint64_t* __restrict__ work) {
+  for (uint64_t i = gtid(); i <= nt; i += gstride()) {
+    if (i == nt) {
+      const uint32_t end = wrp[ids[nt - 1] + 1];
+      act[i] = make_uint4(end, end, 0u, 0u);
+      work[i] = 0;
+      continue;
+    }
+    const uint32_t x = ids[i];
+    const uint2 r = row[x];
+    act[i] = make_uint4(wrp[x], wrp[x + 1], r.x, r.y);
+    work[i] = cost[x] + kTaskCost;
+  }
+}
+
+// slice[s] = the (task, entry) at s / ns of the total work; a task's work is
+// taken as spread evenly over its entries.
+__global__ void k_slices16(const uint64_t* __restrict__ pre, const uint4* __restrict__ act,
+                           uint32_t nt, uint64_t E, uint32_t ns, uint2* __restrict__ slice) {
+  const uint64_t total = pre[nt];
+  for (uint64_t s = gtid(); s <= ns; s += gstride()) {
+    if (s == ns) {
+      slice[s] = make_uint2(nt, (uint32_t)E);
+      continue;
+    }
+    const uint64_t t = (uint64_t)((double)total * (double)s / (double)ns);
+    uint32_t lo = 0, hi = nt - 1;  // last task with pre[task] <= t
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi + 1) >> 1;
+      if (pre[mid] <= t) lo = mid;
+      else hi = mid - 1;
+    }
+    const uint4 a = act[lo];
+    const double f = (double)(t - pre[lo]) / (double)(pre[lo + 1] - pre[lo]);
+    const uint32_t off = min(a.y - a.x - 1, (uint32_t)((double)(a.y - a.x) * f));
+    slice[s] = make_uint2(lo, a.x + off);
+  }
+}
+
+template <class T>
+int read_back(tc_ctx* c, const void* src, T* out) {
+  TCX_HIP(hipMemcpyAsync(out, src, sizeof(T), hipMemcpyDeviceToHost, c->stream));
+  TCX_HIP(hipStreamSynchronize(c->stream));
+  return TC_OK;
+}
+
+// 16-bit ids by in-degree: the vertices of in-degree t and above for the
+// smallest t that leaves at most kMax16 of them.  *share = the part of the
+// CSR's entries that get one.
+int hub_ids(tc_ctx* c, tc_graph* g, DevBuf& id, double* share) {
+  const uint32_t n = g->n;
+  DevBuf hist;
+  TCX_TRY(hist.reserve(4 * kHistBins + 8));
+  TCX_HIP(hipMemsetAsync(hist.p, 0, 4 * kHistBins + 8, c->stream));
+  hipLaunchKernelGGL(k_indeg_hist, dim3(std::min<unsigned>(grid_for(n), c->num_cus * 2u)), dim3(TB),
+                     0, c->stream, g->indeg.as<uint32_t>(), n, hist.as<uint32_t>(),
+                     reinterpret_cast<unsigned long long*>(hist.as<uint32_t>() + kHistBins));
+  TCX_HIP(hipGetLastError());
+  struct { uint32_t bin[kHistBins]; unsigned long long open; } h;
+  TCX_TRY(read_back(c, hist.p, &h));
+  *share = 0;
+  uint64_t have = 0, sum = 0;
+  uint32_t t = kHistBins;
+  while (t > 1 && have + h.bin[t - 1] <= kMax16) {
+    --t;
+    have += h.bin[t];
+    sum += t == kHistBins - 1 ? h.open : (uint64_t)t * h.bin[t];
+  }
+  if (t == kHistBins) return TC_OK;  // too many in the open bin
+  *share = (double)sum / (double)g->m_or;
+  if (*share < kMinShare) return TC_OK;
+  DevBuf flag, pos;
+  TCX_TRY(flag.reserve(4 * ((size_t)n + 1)));
+  TCX_TRY(pos.reserve(4 * ((size_t)n + 1)));
+  TCX_TRY(id.reserve(2 * ((size_t)n + 1)));
+  hipLaunchKernelGGL(k_hub_flags, dim3(grid_for(n)), dim3(TB), 0, c->stream, g->indeg.as<uint32_t>(),
+                     n, t, flag.as<uint32_t>());
+  TCX_TRY(exclusive_scan_u32(c, flag.as<uint32_t>(), pos.as<uint32_t>(), n));
+  hipLaunchKernelGGL(k_hub_ids, dim3(grid_for(n)), dim3(TB), 0, c->stream, g->indeg.as<uint32_t>(),
+                     pos.as<uint32_t>(), n, t, id.as<uint16_t>());
+  TCX_HIP(hipGetLastError());
+  return TC_OK;
+}
+
+// Row places for cnt entries a row, `per` to a unit; the entries are padding.
+int place_rows(tc_ctx* c, uint32_t n, const uint32_t* cnt, uint32_t per, Rows16& R) {
+  DevBuf pa, pb, sa, sb;
+  for (DevBuf* b : {&pa, &pb, &sa, &sb}) TCX_TRY(b->reserve(8 * ((size_t)n + 1)));
+  hipLaunchKernelGGL(k_places16, dim3(grid_for((uint64_t)n + 1)), dim3(TB), 0, c->stream, cnt, n,
+                     per, pa.as<uint64_t>(), pb.as<uint64_t>());
+  TCX_TRY(exclusive_scan_u64(c, pa.as<uint64_t>(), sa.as<uint64_t>(), (uint64_t)n + 1));
+  TCX_TRY(exclusive_scan_u64(c, pb.as<uint64_t>(), sb.as<uint64_t>(), (uint64_t)n + 1));
+  uint64_t ta = 0, tb = 0;
+  TCX_TRY(read_back(c, sa.as<uint64_t>() + n, &ta));
+  TCX_TRY(read_back(c, sb.as<uint64_t>() + n, &tb));
+  R.units = 8 * (ta >> 32) + 4 * (ta & 0xFFFFFFFFu) + 2 * (tb >> 32) + (tb & 0xFFFFFFFFu);
+  if (R.units > 0xFFFFFFFFull) return fail(TC_ERR_RANGE, "list rows exceed 2^32 16-byte units");
+  TCX_TRY(R.row.reserve(8 * ((size_t)n + 1)));
+  TCX_TRY(R.col.reserve(16 * std::max<uint64_t>(R.units, 1)));
+  hipLaunchKernelGGL(k_row_pairs, dim3(grid_for(n)), dim3(TB), 0, c->stream, cnt,
+                     sa.as<uint64_t>(), sb.as<uint64_t>(), n, per, R.row.as<uint2>());
+  hipLaunchKernelGGL(k_fill16, dim3(std::min<unsigned>(grid_for(4 * R.units), 16384)), dim3(TB), 0,
+                     c->stream, R.col.as<uint32_t>(), 0xFFFFFFFFu, 4 * R.units);
+  TCX_HIP(hipGetLastError());
+  return TC_OK;
+}
+
+// Work lists over the rows R (cnt entries each), grouped by owner, and
+// slices of equal work.
+int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, bool tail,
+               Rows16& R) {
+  const uint32_t n = g->n;
+  const uint64_t m = g->m_or;
+  DevBuf keys, tmp, wrp, cost, flags, work, prew;
+  DevBuf& ids = R.who;
+  TCX_TRY(keys.reserve(8 * m));
+  TCX_TRY(tmp.reserve(8 * m));
+  TCX_TRY(wrp.reserve(4 * ((size_t)n + 1)));
+  hipLaunchKernelGGL(k_keys16, dim3(grid_for(m)), dim3(TB), 0, c->stream, g->esrc.as<uint32_t>(),
+                     g->col.as<uint32_t>(), m, n, cnt, id, tail, keys.as<uint64_t>());
+  TCX_HIP(hipGetLastError());
+  // only the owner's bits are sorted: the order within a list is free
+  uint64_t* sorted;
+  TCX_TRY(sort_u64(c, keys.as<uint64_t>(), tmp.as<uint64_t>(), m, 32 + bit_width_u32(n), &sorted,
+                   32));
+  hipLaunchKernelGGL(k_rowptr_search<uint64_t>, dim3(grid_for((uint64_t)n + 1)), dim3(TB), 0,
+                     c->stream, sorted, m, n, wrp.as<uint32_t>());
+  TCX_HIP(hipGetLastError());
+  uint32_t kept = 0;
+  TCX_TRY(read_back(c, wrp.as<uint32_t>() + n, &kept));
+  R.entries = kept;
+  R.tasks = 0;
+  R.nslice = 0;
+  if (!kept) return TC_OK;
+  TCX_TRY(R.se.reserve(8ull * kept));
+  TCX_TRY(cost.reserve(8 * ((size_t)n + 1)));
+  TCX_TRY(flags.reserve((size_t)n + 1));
+  TCX_TRY(ids.reserve(4 * ((size_t)n + 1)));
+  TCX_HIP(hipMemsetAsync(cost.p, 0, 8 * (size_t)n, c->stream));
+  hipLaunchKernelGGL(k_entries16, dim3(grid_for(kept)), dim3(TB), 0, c->stream, sorted,
+                     (uint64_t)kept, R.row.as<uint2>(), R.se.as<uint2>(),
+                     cost.as<unsigned long long>());
+  hipLaunchKernelGGL(k_nonempty, dim3(grid_for(n)), dim3(TB), 0, c->stream, wrp.as<uint32_t>(), n,
+                     flags.as<uint8_t>());
+  TCX_HIP(hipGetLastError());
+  TCX_TRY(select_indices(c, flags.as<uint8_t>(), n, ids.as<uint32_t>(), &R.tasks));
+  const uint64_t nt = R.tasks;
+  TCX_TRY(R.act.reserve(16 * (nt + 1)));
+  TCX_TRY(work.reserve(8 * (nt + 1)));
+  TCX_TRY(prew.reserve(8 * (nt + 1)));
+  hipLaunchKernelGGL(k_tasks16, dim3(grid_for(nt + 1)), dim3(TB), 0, c->stream, ids.as<uint32_t>(),
+                     (uint32_t)nt, wrp.as<uint32_t>(), R.row.as<uint2>(),
+                     cost.as<unsigned long long>(), R.act.as<uint4>(), work.as<uint64_t>());
+  TCX_TRY(exclusive_scan_u64(c, work.as<uint64_t>(), prew.as<uint64_t>(), nt + 1));
+  uint64_t total = 0;
+  TCX_TRY(read_back(c, prew.as<uint64_t>() + nt, &total));
+  // at least 256 group steps a slice; one slice per wave of the default grid,
+  // or eight where that still leaves them long
+  const uint64_t nw = (uint64_t)c->num_cus * 16u;
+  uint64_t ns = std::min<uint64_t>(std::max<uint64_t>(total / 256, 1), 8 * nw);
+  if (ns > nw && ns < 4 * nw) ns = nw;
+  R.nslice = (uint32_t)ns;
+  TCX_TRY(R.slice.reserve(8 * (ns + 1)));
+  hipLaunchKernelGGL(k_slices16, dim3(grid_for(ns + 1)), dim3(TB), 0, c->stream,
+                     prew.as<uint64_t>(), R.act.as<uint4>(), (uint32_t)nt, R.entries, (uint32_t)ns,
+                     R.slice.as<uint2>());
+  TCX_HIP(hipGetLastError());
+  TCX_HIP(hipStreamSynchronize(c->stream));  // before the scratch buffers go
+  return TC_OK;
+}
+
+// Rows, work lists and slices for the ids `id` (null: every vertex id is its
+// own 16-bit id, and there is no tail).
+int build(tc_ctx* c, tc_graph* g, const uint16_t* id, Lists16& L) {
+  const uint32_t n = g->n;
+  const uint64_t m = g->m_or;
+  const uint32_t* rp = g->rowptr.as<uint32_t>();
+  const uint32_t* col = g->col.as<uint32_t>();
+  const uint32_t* esrc = g->esrc.as<uint32_t>();
+  DevBuf pre_b, cnt, tcnt;
+  const uint32_t* pre = nullptr;
+  uint32_t with_id = (uint32_t)m;
+  if (id) {
+    DevBuf flag;
+    TCX_TRY(flag.reserve(4 * (m + 1)));
+    TCX_TRY(pre_b.reserve(4 * (m + 1)));
+    hipLaunchKernelGGL(k_entry_flags, dim3(grid_for(m + 1)), dim3(TB), 0, c->stream, col, m, id,
+                       flag.as<uint32_t>());
+    TCX_TRY(exclusive_scan_u32(c, flag.as<uint32_t>(), pre_b.as<uint32_t>(), m + 1));
+    pre = pre_b.as<uint32_t>();
+    TCX_TRY(read_back(c, pre + m, &with_id));
+  }
+  const bool tail = with_id < m;
+  TCX_TRY(cnt.reserve(4 * ((size_t)n + 1)));
+  if (tail) TCX_TRY(tcnt.reserve(4 * ((size_t)n + 1)));
+  hipLaunchKernelGGL(k_counts16, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp, pre, n,
+                     cnt.as<uint32_t>(), tail ? tcnt.as<uint32_t>() : nullptr);
+  TCX_TRY(place_rows(c, n, cnt.as<uint32_t>(), 8, L.hub));
+  if (tail) TCX_TRY(place_rows(c, n, tcnt.as<uint32_t>(), 4, L.tail));
+  hipLaunchKernelGGL(k_scatter16, dim3(grid_for(m)), dim3(TB), 0, c->stream, rp, col, esrc, m, id,
+                     pre, L.hub.row.as<uint2>(), L.hub.col.as<uint16_t>(),
+                     L.tail.row.as<uint2>(), L.tail.col.as<uint32_t>());
+  TCX_HIP(hipGetLastError());
+  TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), id, false, L.hub));
+  L.tail.tasks = 0;
+  if (tail) TCX_TRY(work_lists(c, g, tcnt.as<uint32_t>(), id, true, L.tail));
+  return TC_OK;
+}
+
+}  // namespace
+
+int lists16(tc_ctx* c, tc_graph* g) {
+  Lists16& L = g->sc.l16;
+  if (L.version == g->sched_version) return TC_OK;
+  L.usable = false;
+  if (g->n && g->m_or && g->sum_in_out >= kMinList * g->m_or) {
+    if (g->n <= kMax16) {
+      TCX_TRY(build(c, g, nullptr, L));
+      L.usable = true;
+    } else {
+      DevBuf id;
+      double share = 0;
+      TCX_TRY(hub_ids(c, g, id, &share));
+      if (share >= kMinShare) {
+        TCX_TRY(build(c, g, id.as<uint16_t>(), L));
+        L.usable = true;
+      }
+    }
+  }
+  L.version = g->sched_version;
+  return TC_OK;
+}
+
+int count16(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor, unsigned long long* acc,
+            uint32_t* launches) {
+  const Lists16& L = g->sc.l16;
+  const uint32_t G = grid ? grid : (uint32_t)c->num_cus * 4u;
+  auto launch = [&](auto kernel, const Rows16& R, uint32_t* cur) {
+    if (!R.tasks) return;
+    hipLaunchKernelGGL(kernel, dim3(G), dim3(TB), 0, c->stream, R.col.as<uint4>(),
+                       R.se.as<uint2>(), R.act.as<uint4>(), R.who.as<uint32_t>(),
+                       R.slice.as<uint2>(), R.nslice, cur, acc);
+    ++*launches;
+  };
+  launch(k_count16<true, kOutTotal, 4>, L.hub, cursor);
+  launch(k_count16<false, kOutTotal, 4>, L.tail, cursor + 1);
+  TCX_HIP(hipGetLastError());
+  return TC_OK;
+}
+
+unsigned long long sum16(const unsigned long long* acc) {
+  unsigned long long s = 0;
+  for (uint32_t i = 0; i < kAcc16; ++i) s += acc[i * kAccStride16];
+  return s;
+}
+
+}  // namespace tcx

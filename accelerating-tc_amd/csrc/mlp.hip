@@ -1321,6 +1321,15 @@ int tc_count_learned(tc_ctx* c, tc_graph* g, tc_model* md, uint64_t* count, tc_t
     return TC_OK;
   }
   const SchedCache& S = g->sc;
+  // graphs that the 16-bit list layer suits are counted there, by equal
+  // slices of work; the model schedules the 32-bit tasks of the others
+  if (S.l16.version != g->sched_version) TCX_TRY(lists16(c, g));
+  if (S.l16.usable) {
+    tc_sched s;
+    memset(&s, 0, sizeof(s));
+    s.kernel = TC_KERNEL_AUTO;
+    return tc_count(c, g, &s, count, timing);
+  }
   // the schedule is built once per (graph, model) and timed then; a count
   // that reuses it enqueues nothing before the kernel and waits once
   if (S.learned_version != g->sched_version || S.learned_model != md->id) {

@@ -20,12 +20,13 @@ int run_prim(tc_ctx* c, F&& f) {
 }  // namespace
 
 int sort_u64(tc_ctx* c, uint64_t* keys, uint64_t* tmp, uint64_t n, int end_bit,
-             uint64_t** sorted) {
+             uint64_t** sorted, int begin_bit) {
   *sorted = keys;
   if (n <= 1) return TC_OK;
   rocprim::double_buffer<uint64_t> db(keys, tmp);
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
-    return rocprim::radix_sort_keys(t, b, db, (size_t)n, 0u, (unsigned)end_bit, c->stream);
+    return rocprim::radix_sort_keys(t, b, db, (size_t)n, (unsigned)begin_bit, (unsigned)end_bit,
+                                    c->stream);
   }));
   *sorted = db.current();
   return TC_OK;
