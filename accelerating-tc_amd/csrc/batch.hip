@@ -224,6 +224,7 @@ struct tc_batch {
   tc_graph* g = nullptr;
   uint32_t ngraphs = 0;
   std::vector<uint32_t> voff;
+  bool ids16 = false;  // every graph has at most 65,535 vertices
   DevBuf d_voff, gid, counts, cursors;
   // schedule for one (wave_max_deg, form)
   uint32_t sched_deg = 0, sched_form = 0;
@@ -232,7 +233,7 @@ struct tc_batch {
   DevBuf blk_off, wav_off;  // per-graph ranges of blk_id / wav
   std::vector<uint32_t> h_blk_off, h_wav_off;
   // captured replay
-  bool captured = false;
+  bool captured = false, cap_on16 = false;
   uint32_t cap_deg = 0, cap_chunk = 0, cap_grid = 0, cap_fmin = 0, cap_form = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -351,10 +352,15 @@ int schedule(tc_ctx* c, tc_batch* b, uint32_t wave_max_deg, uint32_t form) {
   return TC_OK;
 }
 
-int enqueue_batched(tc_ctx* c, tc_batch* b, const tc_batch_sched& s) {
+int enqueue_batched(tc_ctx* c, tc_batch* b, const tc_batch_sched& s, bool on16) {
   tc_graph* g = b->g;
-  hipLaunchKernelGGL(k_batch_reset, dim3(grid_for(2ull + b->ngraphs)), dim3(256), 0, c->stream,
-                     b->cursors.as<uint32_t>(), 2u, b->counts.as<unsigned long long>(), b->ngraphs);
+  const uint32_t ncur = on16 ? (uint32_t)(kCurBytes16 / 4) : 2u;
+  hipLaunchKernelGGL(k_batch_reset, dim3(grid_for((uint64_t)ncur + b->ngraphs)), dim3(256), 0,
+                     c->stream, b->cursors.as<uint32_t>(), ncur,
+                     b->counts.as<unsigned long long>(), b->ngraphs);
+  if (on16)
+    return count16_graphs(c, g, s.grid, b->cursors.as<uint32_t>(),
+                          b->counts.as<unsigned long long>());
   launch_batch(s, dim3(s.grid), c->stream, g->rowptr.as<uint32_t>(), g->col.as<uint32_t>(),
                g->sc.wl_rp.as<uint32_t>(), g->sc.wl_se.as<uint2>(),
                b->gid.as<uint32_t>(), b->blk_lpt.as<uint32_t>(), (uint32_t)b->nblk,
@@ -400,12 +406,13 @@ int tc_batch_create(tc_ctx* c, uint32_t ngraphs, const uint64_t* eoff, const uin
   b->ctx = c;
   b->ngraphs = ngraphs;
   b->voff = voff;
+  b->ids16 = *std::max_element(nverts, nverts + ngraphs) <= 65535u;
   int st = tc_graph_create(c, gs.data(), gd.data(), M, (uint32_t)total, &b->g);
   if (!st) st = tc_graph_orient(c, b->g, TC_ORIENT_DEGREE, 0);
   if (!st) st = b->gid.reserve(4 * std::max<uint64_t>(total, 1));
   if (!st) st = b->d_voff.reserve(4 * ((size_t)ngraphs + 1));
   if (!st) st = b->counts.reserve(8 * (size_t)ngraphs);
-  if (!st) st = b->cursors.reserve(8 * ((size_t)ngraphs + 2));
+  if (!st) st = b->cursors.reserve(std::max(kCurBytes16, 8 * ((size_t)ngraphs + 2)));
   if (!st && total &&
       hipMemcpyAsync(b->gid.p, gidh.data(), 4 * total, hipMemcpyHostToDevice, c->stream) != hipSuccess)
     st = fail(TC_ERR_HIP, "gid upload failed");
@@ -451,12 +458,19 @@ int tc_batch_count(tc_ctx* c, tc_batch* b, const tc_batch_sched* sched, uint64_t
   memset(&tm, 0, sizeof(tm));
   TCX_HIP(hipEventRecord(c->ev0, c->stream));
   TCX_TRY(check_sched(sched));
-  TCX_TRY(schedule(c, b, s.wave_max_deg, s.form));
-  if (!b->captured || b->cap_chunk != s.wave_chunk || b->cap_grid != s.grid ||
+  // the work-list form counts over 16-bit lists where they suit the batch
+  // (one split of the work: the task parameters are the 32-bit tasks')
+  bool on16 = false;
+  if (s.form == TC_BATCH_WORKLIST && b->ids16) {
+    TCX_TRY(lists16_batch(c, b->g, b->gid.as<uint32_t>(), b->d_voff.as<uint32_t>()));
+    on16 = b->g->sc.l16.usable;
+  }
+  if (!on16) TCX_TRY(schedule(c, b, s.wave_max_deg, s.form));
+  if (!b->captured || b->cap_on16 != on16 || b->cap_chunk != s.wave_chunk || b->cap_grid != s.grid ||
       b->cap_deg != s.wave_max_deg || b->cap_fmin != s.filter_min || b->cap_form != s.form) {
     release_capture(b);
     TCX_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int st = enqueue_batched(c, b, s);
+    int st = enqueue_batched(c, b, s, on16);
     hipGraph_t gr = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &gr);
     if (st) {
@@ -467,6 +481,7 @@ int tc_batch_count(tc_ctx* c, tc_batch* b, const tc_batch_sched* sched, uint64_t
     b->graph = gr;
     TCX_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
     b->captured = true;
+    b->cap_on16 = on16;
     b->cap_chunk = s.wave_chunk;
     b->cap_grid = s.grid;
     b->cap_deg = s.wave_max_deg;

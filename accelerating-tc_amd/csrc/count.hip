@@ -1115,12 +1115,10 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     case TC_KERNEL_AUTO: {
       const SchedCache& sc = g->sc;
       if (on16) {
-        TCX_TRY(c->scratch.reserve(64 + kAccBytes16));
-        uint32_t* cur = c->scratch.as<uint32_t>();
-        unsigned long long* acc16 = c->scratch.as<unsigned long long>() + 8;
-        TCX_HIP(hipMemsetAsync(cur, 0, 64 + kAccBytes16, c->stream));
+        TCX_TRY(c->scratch.reserve(kAccBytes16));
+        TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kAccBytes16, c->stream));
         TCX_TRY(lm.mark());
-        TCX_TRY(count16(c, g, s.grid_size, cur, acc16, &tm.launches));
+        TCX_TRY(count16(c, g, s.grid_size, c->scratch.as<unsigned long long>(), &tm.launches));
         break;
       }
       TCX_TRY(c->scratch.reserve(64));
@@ -1185,8 +1183,7 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   unsigned long long h = 0;
   if (on16) {
     unsigned long long part[kAccBytes16 / 8];
-    TCX_HIP(hipMemcpyAsync(part, c->scratch.as<unsigned long long>() + 8, kAccBytes16,
-                           hipMemcpyDeviceToHost, c->stream));
+    TCX_HIP(hipMemcpyAsync(part, c->scratch.p, kAccBytes16, hipMemcpyDeviceToHost, c->stream));
     TCX_HIP(hipStreamSynchronize(c->stream));
     h = sum16(part);
   } else {

@@ -206,12 +206,19 @@ int worklists(tc_ctx* c, tc_graph* g);
 // ---- the 16-bit list layer (lists16.hip) -----------------------------------
 // Builds (or keeps) g's layer when its lists suit it (g->sc.l16.usable).
 int lists16(tc_ctx* c, tc_graph* g);
-// Enqueues the count over a usable layer; acc: kAccBytes16 bytes, cleared, as
-// are cursor[0] and [1]; sum16 adds the copied-back accumulators.
+// Enqueues the count over a usable layer; acc: kAccBytes16 bytes, cleared;
+// sum16 adds the copied-back accumulators.
 constexpr size_t kAccBytes16 = 8 * 64 * 16;
-int count16(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor, unsigned long long* acc,
-            uint32_t* launches);
+int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches);
 unsigned long long sum16(const unsigned long long* acc);
+// The same for a batch's union graph: 16-bit ids are the ids within each
+// graph (vertex v of graph gid[v], which starts at voff[gid[v]]; device
+// arrays), so every graph must have at most 65,535 vertices.  Counts go to
+// counts[graph]; cursor: kCurBytes16 bytes, cleared.
+constexpr size_t kCurBytes16 = 64 * 128;
+int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* voff);
+int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
+                   unsigned long long* counts);
 
 // ---- cost model and per-vertex counts (mlp.hip, count.hip) ---------------
 // Predicted log2 costs Y[n][2] for device features X[n][8]; fails when the

@@ -24,7 +24,7 @@ namespace dev {
 constexpr uint32_t kPad16 = 0xFFFFu;    // padding entry: its bit is never set
 constexpr uint32_t kMax16 = 65535u;     // 16-bit ids are below this
 constexpr uint32_t kMap16Words = 2048;  // bit map: id c is bit c >> 13 of byte c & 8191
-constexpr uint32_t kGroup16 = 8;        // lanes that read one list together (128 bytes a step)
+constexpr uint32_t kGroup16 = 4;        // lanes that read one list together (64 bytes a step)
 constexpr uint32_t kRing16 = 128;       // list bounds held in LDS per wave
 
 // LDS of one wave.
@@ -138,8 +138,8 @@ __device__ inline uint32_t map32_count4(const uint8_t* map, const uint4& q, Prob
 }
 
 // Streams the lists (start, 16-byte units) se[0, total) against the wave's
-// map; returns this lane's members.  Each group of eight lanes reads one
-// list, 128 bytes a step, and takes the next list not yet taken when its own
+// map; returns this lane's members.  Each group of four lanes reads one list,
+// 64 bytes a step, and takes the next list not yet taken when its own
 // is used up, so lists of unequal length keep all groups busy; U steps of
 // every group are in flight together.  The bounds pass through a ring in
 // LDS, 64 per refill, the next 64 already loaded (nb: this lane's of the
@@ -150,6 +150,8 @@ __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
                                               uint2 nb, uint32_t lane, Wave16& W, Probe32& P) {
   const uint8_t* map = reinterpret_cast<const uint8_t*>(W.map);
   const uint32_t j = lane & (kGroup16 - 1);
+  constexpr uint64_t kLastLanes = 0x8888888888888888ull;
+  static_assert(kGroup16 == 4, "kLastLanes has the last lane of each group");
   unsigned long long sum = 0;
   uint32_t acc = 0;
   uint32_t cur = 0;            // next unit of this group's list
@@ -162,9 +164,9 @@ __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
     for (int s = 0; s < U; ++s) {
       // one bit per group that needs a list, at its last lane, so that every
       // lane of a group has the same number of bits below it
-      const uint64_t m = lanes(rem <= 0) & 0x8080808080808080ull;
+      const uint64_t m = lanes(rem <= 0) & kLastLanes;
       if (m && cnt < total) {
-        if (held - cnt < 8 && held < total) {
+        if (held - cnt < 64 / kGroup16 && held < total) {
           W.ring[(held + lane) & (kRing16 - 1)] = nb;
           held = uniform(total - held < 64 ? total : held + 64);
           nb = held + lane < total ? se[held + lane] : make_uint2(0u, 0u);
@@ -232,22 +234,26 @@ enum Out16 { kOutTotal = 0, kOutVertex = 1, kOutGraph = 2 };
 
 // Counts over the rows.  act[i] = (first and end entry of the task's work list
 // in se, first unit and units of the owner's row); slice s runs from (task,
-// entry) slice[s] to slice[s + 1], slices of equal work, a wave each: the
-// first gridDim * 4 in order, the rest claimed from the cursor.  A task cut by
-// a slice border is counted in parts.  While a task is streamed, the next
+// entry) slice[s] to slice[s + 1], slices of equal work, a wave each.  The
+// workgroups form up to kAcc16 groups, group q with every kAcc16-th slice from
+// q on and a cursor of its own (kCurStride16 words apart): its waves take one
+// slice each, then claim the rest.  (One cursor for all serialised the claims
+// at about 14 ns: R-MAT-18 took 0.40 ms, and takes 0.145.)  A task cut by a slice
+// border is counted in parts.  While a task is streamed, the next
 // one's own row and first 64 list bounds and the description of the one after
 // it are on their way: with a few lists per task (the tail, most of an R-MAT
 // graph's owners) those three dependent reads took longer than the lists.
 // `total` holds kAcc16 accumulators kAccStride16 words apart (kOutTotal), or
 // one word per vertex or graph.
-// Bound by the fabric between memory and L2: R-MAT-23 (A-order, A-direction)
-// reads 61 GB in 8.57 ms, 7.2 TB/s, with vector-ALU issue near 0.68 and LDS
-// near 0.65 of their rates; the whole count takes 9.75 ms where the 32-bit
-// rank tables took 19.7, R-MAT-24 22.5 where they took 43.6.  36 KB of LDS a
-// workgroup, four workgroups a CU.  Eight lanes a list and U = 4 steps in
-// flight: R-MAT-22 4.75 ms against 4.93 with 16 lanes, 4.78 with 4, and 4.91
-// with U = 2.
-constexpr uint32_t kAcc16 = 64, kAccStride16 = 16;
+// Bound by the fabric between memory and L2 on large graphs: R-MAT-23 (A-order,
+// A-direction) reads 61 GB in 8.57 ms, 7.2 TB/s, with vector-ALU issue near
+// 0.68 and LDS near 0.65 of their rates; the whole count takes 9.8 ms where
+// the 32-bit rank tables took 19.7, R-MAT-24 22.5 where they took 43.6.  36 KB
+// of LDS a workgroup, four workgroups a CU.  Four lanes a list and U = 4 steps
+// in flight: R-MAT-23 9.65 ms against 9.75 with 8 lanes and 10.37 with 2, a
+// batch of 384 small graphs 1.67 against 1.90 ms with 8; R-MAT-22 with U = 2
+// 4.91 against 4.75 ms.
+constexpr uint32_t kAcc16 = 64, kAccStride16 = 16, kCurStride16 = 32;
 
 template <bool B16, int OUT, int U>
 __global__ __launch_bounds__(TB) void k_count16(const uint4* __restrict__ col,
@@ -267,63 +273,68 @@ __global__ __launch_bounds__(TB) void k_count16(const uint4* __restrict__ col,
   wave_sync();
   unsigned long long cnt = 0;
   uint32_t graph = 0xFFFFFFFFu;
-  const uint32_t nw = gridDim.x * (TB / 64);
-  for (uint32_t s = uniform(blockIdx.x * (TB / 64) + wv); s < nslice;) {
+  const uint32_t ng = min(kAcc16, gridDim.x), q = blockIdx.x % ng;
+  const uint32_t nw = (gridDim.x - q + ng - 1) / ng * (TB / 64);  // the group's waves
+  for (uint32_t s = uniform(q + ng * (blockIdx.x / ng * (TB / 64) + wv)); s < nslice;) {
     const uint2 b = slice[s], e = slice[s + 1];
     // tasks [i, last], entries [at, stop) of the work lists
     uint32_t i = b.x, at = b.y;
     const uint32_t stop = e.y, last = stop > at ? e.x - (e.y == act[e.x].x ? 1u : 0u) : 0u;
     if (stop > at) {
       uint4 a = act[i], an = act[min(i + 1, last)];
-      uint4 q = lane < a.w ? col[(uint64_t)a.z + lane] : pad;
+      uint32_t w = 0, wn = 0;
+      if (OUT != kOutTotal) {
+        w = who[i];
+        wn = who[min(i + 1, last)];
+      }
+      uint4 own = lane < a.w ? col[(uint64_t)a.z + lane] : pad;
       uint32_t end = min(a.y, stop);
       uint2 nb = at + lane < end ? se[at + lane] : make_uint2(0u, 0u);
       for (;;) {
         const bool more = i < last;
         const uint32_t nend = min(an.y, stop);
-        uint4 qn = pad;
+        uint4 ownn = pad;
         uint2 nbn = make_uint2(0u, 0u);
         uint4 an2 = an;
+        uint32_t wn2 = wn;
         if (more) {
-          if (lane < an.w) qn = col[(uint64_t)an.z + lane];
+          if (lane < an.w) ownn = col[(uint64_t)an.z + lane];
           if (an.x + lane < nend) nbn = se[an.x + lane];
           an2 = act[min(i + 2, last)];
+          if (OUT != kOutTotal) wn2 = who[min(i + 2, last)];
         }
-        if (OUT == kOutGraph) {
-          const uint32_t g = who[i];
-          if (g != graph) {
-            if (graph != 0xFFFFFFFFu) {
-              const unsigned long long t = wave_sum(cnt);
-              if (lane == 0 && t) atomicAdd(total + graph, t);
-              cnt = 0;
-            }
-            graph = g;
+        if (OUT == kOutGraph && w != graph) {
+          if (graph != 0xFFFFFFFFu) {
+            const unsigned long long t = wave_sum(cnt);
+            if (lane == 0 && t) atomicAdd(total + graph, t);
+            cnt = 0;
           }
+          graph = w;
         }
         const unsigned long long c =
-            task16<B16, U>(col, make_uint2(a.z, a.w), q, se + at, end - at, nb, lane, W, Q[wv]);
+            task16<B16, U>(col, make_uint2(a.z, a.w), own, se + at, end - at, nb, lane, W, Q[wv]);
         if (OUT == kOutVertex) {
           const unsigned long long t = wave_sum(c);
-          if (lane == 0 && t) atomicAdd(total + who[i], t);
+          if (lane == 0 && t) atomicAdd(total + w, t);
         } else {
           cnt += c;
         }
         if (!more) break;
         ++i;
         a = an;
+        w = wn;
+        wn = wn2;
         at = an.x;
         end = nend;
-        q = qn;
+        own = ownn;
         nb = nbn;
         an = an2;
       }
     }
+    if ((uint64_t)nw * ng + q >= nslice) break;  // one slice a wave at most
     uint32_t nx = 0;
-    if (nslice > nw) {
-      if (lane == 0) nx = atomicAdd(cursor, 1u);
-      nx = (uint32_t)__shfl((int)nx, 0, 64);
-    }
-    s = nslice > nw ? nw + uniform(nx) : nslice;
+    if (lane == 0) nx = atomicAdd(cursor + q * kCurStride16, 1u);
+    s = q + ng * (nw + uniform((uint32_t)__shfl((int)nx, 0, 64)));
   }
   if (OUT == kOutTotal) flush_block(cnt, total + (blockIdx.x % kAcc16) * kAccStride16, red);
   if (OUT == kOutGraph && graph != 0xFFFFFFFFu) {

@@ -12,13 +12,13 @@ namespace {
 using namespace dev;
 
 constexpr uint32_t kHistBins = 4096;  // in-degree histogram, the last bin open
-// A graph takes the layer when its average pushed list (sum d- d+ / m) has at
-// least this many entries and at least this share of its entries gets a
-// 16-bit id.  Below 20 entries a list is one step of a group with most lanes
-// idle (ER of 65,536 vertices and 2^20 edges, 16 entries, stays with the
-// 32-bit tasks); below the share, the tail's work lists and tasks come on top
-// of the layer's.  R-MAT graphs are at 0.88-1.0.
-constexpr uint64_t kMinList = 20;
+// A graph of more than 65,535 vertices takes the layer when at least this
+// share of its entries gets a 16-bit id; below it, the tail's work lists and
+// tasks cost as much as the layer saves (Barabasi-Albert, 90,000 vertices, 16
+// edges each, share 0.73: 75 us either way; ER of 100,000 vertices and 1.5 M
+// edges, share 0.7: 86 against 106 us; R-MAT graphs are at 0.88-1.0).  Smaller
+// graphs always take it: 14 against 60-120 us at 3,001 vertices, 41 against 90
+// us on ER of 65,536 vertices and 2^20 edges.
 constexpr double kMinShare = 0.7;
 constexpr uint64_t kTaskCost = 48;  // a task's own row and map, in group steps
 
@@ -232,6 +232,16 @@ __global__ void k_slices16(const uint64_t* __restrict__ pre, const uint4* __rest
   }
 }
 
+__global__ void k_local_ids(const uint32_t* __restrict__ gid, const uint32_t* __restrict__ voff,
+                            uint32_t n, uint16_t* __restrict__ id) {
+  for (uint64_t v = gtid(); v < n; v += gstride()) id[v] = (uint16_t)(v - voff[gid[v]]);
+}
+
+__global__ void k_graph_of(uint32_t* __restrict__ who, uint64_t nt,
+                           const uint32_t* __restrict__ gid) {
+  for (uint64_t i = gtid(); i < nt; i += gstride()) who[i] = gid[who[i]];
+}
+
 template <class T>
 int read_back(tc_ctx* c, const void* src, T* out) {
   TCX_HIP(hipMemcpyAsync(out, src, sizeof(T), hipMemcpyDeviceToHost, c->stream));
@@ -349,11 +359,14 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
   TCX_TRY(exclusive_scan_u64(c, work.as<uint64_t>(), prew.as<uint64_t>(), nt + 1));
   uint64_t total = 0;
   TCX_TRY(read_back(c, prew.as<uint64_t>() + nt, &total));
-  // at least 256 group steps a slice; one slice per wave of the default grid,
-  // or eight where that still leaves them long
+  // One slice per wave of the default grid, at least 256 group steps long; up
+  // to 32 a wave where they still have 2,048.  A slice begins with a claim and
+  // a chain of reads: with 1,024-step slices a batch of 128 small ER graphs
+  // took 0.67 instead of 0.48 ms, and with eight slices a wave instead of 32
+  // the last ones left R-MAT-23 waiting (10.15 instead of 9.85 ms).
   const uint64_t nw = (uint64_t)c->num_cus * 16u;
-  uint64_t ns = std::min<uint64_t>(std::max<uint64_t>(total / 256, 1), 8 * nw);
-  if (ns > nw && ns < 4 * nw) ns = nw;
+  uint64_t ns = std::min<uint64_t>(std::max<uint64_t>(total / 256, 1), nw);
+  if (total / 2048 > 2 * nw) ns = std::min<uint64_t>(total / 2048, 32 * nw);
   R.nslice = (uint32_t)ns;
   TCX_TRY(R.slice.reserve(8 * (ns + 1)));
   hipLaunchKernelGGL(k_slices16, dim3(grid_for(ns + 1)), dim3(TB), 0, c->stream,
@@ -365,8 +378,8 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
 }
 
 // Rows, work lists and slices for the ids `id` (null: every vertex id is its
-// own 16-bit id, and there is no tail).
-int build(tc_ctx* c, tc_graph* g, const uint16_t* id, Lists16& L) {
+// own 16-bit id; id_all: every vertex has one, and there is no tail).
+int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, Lists16& L) {
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
@@ -375,7 +388,7 @@ int build(tc_ctx* c, tc_graph* g, const uint16_t* id, Lists16& L) {
   DevBuf pre_b, cnt, tcnt;
   const uint32_t* pre = nullptr;
   uint32_t with_id = (uint32_t)m;
-  if (id) {
+  if (!id_all) {
     DevBuf flag;
     TCX_TRY(flag.reserve(4 * (m + 1)));
     TCX_TRY(pre_b.reserve(4 * (m + 1)));
@@ -408,16 +421,16 @@ int lists16(tc_ctx* c, tc_graph* g) {
   Lists16& L = g->sc.l16;
   if (L.version == g->sched_version) return TC_OK;
   L.usable = false;
-  if (g->n && g->m_or && g->sum_in_out >= kMinList * g->m_or) {
+  if (g->n && g->m_or) {
     if (g->n <= kMax16) {
-      TCX_TRY(build(c, g, nullptr, L));
+      TCX_TRY(build(c, g, nullptr, true, L));
       L.usable = true;
     } else {
       DevBuf id;
       double share = 0;
       TCX_TRY(hub_ids(c, g, id, &share));
       if (share >= kMinShare) {
-        TCX_TRY(build(c, g, id.as<uint16_t>(), L));
+        TCX_TRY(build(c, g, id.as<uint16_t>(), false, L));
         L.usable = true;
       }
     }
@@ -426,10 +439,44 @@ int lists16(tc_ctx* c, tc_graph* g) {
   return TC_OK;
 }
 
-int count16(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor, unsigned long long* acc,
-            uint32_t* launches) {
+int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* voff) {
+  Lists16& L = g->sc.l16;
+  if (L.version == g->sched_version) return TC_OK;
+  L.usable = false;
+  if (g->n && g->m_or) {
+    DevBuf id;
+    TCX_TRY(id.reserve(2 * (size_t)g->n));
+    hipLaunchKernelGGL(k_local_ids, dim3(grid_for(g->n)), dim3(TB), 0, c->stream, gid, voff, g->n,
+                       id.as<uint16_t>());
+    TCX_HIP(hipGetLastError());
+    TCX_TRY(build(c, g, id.as<uint16_t>(), true, L));
+    if (L.hub.tasks)
+      hipLaunchKernelGGL(k_graph_of, dim3(grid_for(L.hub.tasks)), dim3(TB), 0, c->stream,
+                         L.hub.who.as<uint32_t>(), L.hub.tasks, gid);
+    TCX_HIP(hipGetLastError());
+    L.usable = true;
+  }
+  L.version = g->sched_version;
+  return TC_OK;
+}
+
+int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
+                   unsigned long long* counts) {
+  const Rows16& R = g->sc.l16.hub;
+  if (R.tasks)
+    hipLaunchKernelGGL((k_count16<true, kOutGraph, 4>),
+                       dim3(std::min<uint32_t>(grid, (uint32_t)c->num_cus * 4u)), dim3(TB), 0,
+                       c->stream, R.col.as<uint4>(), R.se.as<uint2>(), R.act.as<uint4>(),
+                       R.who.as<uint32_t>(), R.slice.as<uint2>(), R.nslice, cursor, counts);
+  TCX_HIP(hipGetLastError());
+  return TC_OK;
+}
+
+int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches) {
   const Lists16& L = g->sc.l16;
   const uint32_t G = grid ? grid : (uint32_t)c->num_cus * 4u;
+  // the cursors ride between the accumulators, one line each
+  static_assert(kCurStride16 * 4 == kAccStride16 * 8, "one line per accumulator");
   auto launch = [&](auto kernel, const Rows16& R, uint32_t* cur) {
     if (!R.tasks) return;
     hipLaunchKernelGGL(kernel, dim3(G), dim3(TB), 0, c->stream, R.col.as<uint4>(),
@@ -437,8 +484,8 @@ int count16(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor, unsigned lo
                        R.slice.as<uint2>(), R.nslice, cur, acc);
     ++*launches;
   };
-  launch(k_count16<true, kOutTotal, 4>, L.hub, cursor);
-  launch(k_count16<false, kOutTotal, 4>, L.tail, cursor + 1);
+  launch(k_count16<true, kOutTotal, 4>, L.hub, reinterpret_cast<uint32_t*>(acc + 8));
+  launch(k_count16<false, kOutTotal, 4>, L.tail, reinterpret_cast<uint32_t*>(acc + 9));
   TCX_HIP(hipGetLastError());
   return TC_OK;
 }

@@ -1307,10 +1307,11 @@ int tc_learned_assignment(tc_ctx* c, tc_graph* g, tc_model* md, uint8_t* variant
 int tc_count_learned(tc_ctx* c, tc_graph* g, tc_model* md, uint64_t* count, tc_timing* timing) {
   TCX_TRY(check_graph(c, g, md));
   if (!count) return fail(TC_ERR_ARG, "NULL argument");
-  if (!md) {  // the fixed rule: AUTO's work-list schedule
+  if (!md) {  // the fixed rule: AUTO's 32-bit work-list tasks
     tc_sched s;
     memset(&s, 0, sizeof(s));
     s.kernel = TC_KERNEL_AUTO;
+    s.auto_thresholds[0] = 64u;
     return tc_count(c, g, &s, count, timing);
   }
   tc_timing tm;

@@ -113,7 +113,11 @@ typedef struct tc_sched {
   uint32_t fox_max_lanes;   /* Fox: widest lanes-per-edge bin, 1..64 (64)        */
   uint32_t tricore_parts;   /* TriCore: node-range partitions (1)                */
   uint32_t auto_bins;       /* reserved                                          */
-  uint32_t auto_thresholds[4]; /* AUTO: [0] largest d+ run as a wave task (64,
+  uint32_t auto_thresholds[4]; /* AUTO: with [0], [1] and [3] all 0 the WORKLIST
+                               schedule counts over 16-bit list rows in equal
+                               slices of work where they suit the graph (at most
+                               65,535 vertices, or most entries in that many
+                               targets); else: [0] largest d+ run as a wave task (64,
                                at most 512); [1] largest d+ run by the 2048-entry
                                block kernel, above it the 8192-entry one (2048);
                                [2] schedule: TC_AUTO_WORKLIST (0, default) or
@@ -515,6 +519,9 @@ int tc_count_learned(tc_ctx* ctx, tc_graph* g, tc_model* m, uint64_t* count,
  * an edge never leaves its graph, so neither does a work list) and
  * accumulates per-graph uint64 counts.  The count sequence is captured once
  * in a hipGraph and replayed. */
+/* The work-list form counts over 16-bit lists (as tc_count's AUTO does) when
+ * every graph has at most 65,535 vertices; wave_max_deg, wave_chunk and
+ * filter_min then only shape the per-graph launches. */
 typedef struct tc_batch_sched {
   uint32_t wave_max_deg;  /* vertices with 2 <= d+ <= this run as wave tasks (64) */
   uint32_t wave_chunk;    /* wave tasks fetched per cursor bump (16)              */

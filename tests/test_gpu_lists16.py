@@ -66,3 +66,21 @@ def test_learned_count_and_many_lists(ctx):
     assert g.count_learned(learned.load(ctx)).count == expect
     assert g.count_learned(None).count == expect
     g.close()
+
+
+@pytest.mark.parametrize("n", [65534, 65535, 65536])
+def test_batch_id_border(ctx, n):
+    """Graphs up to 65,535 vertices take 16-bit local ids; one more vertex in
+    any of them sends the batch to the 32-bit tasks."""
+    e = np.zeros(0, np.uint32)
+    s, d = tcamd.gen_er(n, 400_003, 11)
+    last = (np.array([0, n - 1, n - 1], np.uint32), np.array([n - 1, 1, 0], np.uint32), n)
+    graphs = [(*complete(70), 70), (e, e, 3), (s, d, n), (*complete(9), 64), last,
+              (*complete(513), 600), (e, e, 1)]
+    expect = [orc.pipeline_count(a, b, "degree")[0] if len(a) else 0 for a, b, _ in graphs]
+    b = ctx.batch(graphs)
+    for sched in (None, dict(grid=3), dict(form=1)):
+        for _ in range(3):  # replays of the captured launch
+            assert b.count(sched)[0].tolist() == expect
+    assert b.count_pergraph()[0].tolist() == expect
+    b.close()
