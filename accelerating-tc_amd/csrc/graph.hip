@@ -132,28 +132,46 @@ __device__ inline unsigned long long wave_sum_u64(unsigned long long v) {
   return v;
 }
 
-// acc[0] += sum d+^2, acc[1] += sum d- d+, acc[2] = max d+
-__global__ void k_csr_stats(const uint32_t* __restrict__ rowptr, const uint32_t* __restrict__ indeg,
-                            uint32_t n, unsigned long long* acc) {
-  unsigned long long s1 = 0, s2 = 0;
-  uint32_t mx = 0;
+// acc[0] += sum d+^2, acc[1] += sum d- d+ (d+ of every entry's target),
+// acc[2] = max d+.  A few hundred workgroups with one atomic each per figure:
+// an atomic per wave on the same three words serialised at about 14 ns
+// (n = 2^21: 1.16 ms).
+__global__ __launch_bounds__(256) void k_csr_stats(const uint32_t* __restrict__ rowptr,
+                                                   const uint32_t* __restrict__ col, uint32_t n,
+                                                   uint64_t m, unsigned long long* acc) {
+  __shared__ unsigned long long red[3][4];
+  unsigned long long s1 = 0, s2 = 0, mx = 0;
   for (uint64_t v = gtid(); v < n; v += gstride()) {
-    uint64_t d = rowptr[v + 1] - rowptr[v];
+    const uint64_t d = rowptr[v + 1] - rowptr[v];
     s1 += d * d;
-    s2 += d * (uint64_t)indeg[v];
-    mx = d > mx ? (uint32_t)d : mx;
+    mx = d > mx ? d : mx;
+  }
+  for (uint64_t e = gtid(); e < m; e += gstride()) {
+    const uint32_t v = col[e];
+    s2 += rowptr[v + 1] - rowptr[v];
   }
   s1 = wave_sum_u64(s1);
   s2 = wave_sum_u64(s2);
   for (int off = 32; off > 0; off >>= 1) {
-    uint32_t o = __shfl_down(mx, off, 64);
+    const unsigned long long o = __shfl_down(mx, off, 64);
     mx = o > mx ? o : mx;
   }
   if ((threadIdx.x & 63) == 0) {
-    atomicAdd(acc + 0, s1);
-    atomicAdd(acc + 1, s2);
-    atomicMax(acc + 2, (unsigned long long)mx);
+    red[0][threadIdx.x >> 6] = s1;
+    red[1][threadIdx.x >> 6] = s2;
+    red[2][threadIdx.x >> 6] = mx;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicAdd(acc + 0, red[0][0] + red[0][1] + red[0][2] + red[0][3]);
+    atomicAdd(acc + 1, red[1][0] + red[1][1] + red[1][2] + red[1][3]);
+    atomicMax(acc + 2, max(max(red[2][0], red[2][1]), max(red[2][2], red[2][3])));
+  }
+}
+
+__global__ void k_row_degrees(const uint32_t* __restrict__ rp, uint32_t n,
+                              uint32_t* __restrict__ deg) {
+  for (uint64_t v = gtid(); v < n; v += gstride()) deg[v] = rp[v + 1] - rp[v];
 }
 
 // ---- A-direction peel (edge_directing/A-direction-seri.cpp:35-153) --------
@@ -171,37 +189,160 @@ __global__ void k_adir_init(const uint32_t* __restrict__ rp, uint32_t n, int32_t
   }
 }
 
-__global__ void k_adir_scan(uint32_t n, const int32_t* __restrict__ rtd, int32_t* prio, float t,
-                            int32_t label, uint32_t* frontier, uint32_t* fcount) {
-  for (uint64_t v = gtid(); v < n; v += gstride()) {
-    if (prio[v] == -1 && (float)rtd[v] <= t) {
-      prio[v] = label;
-      frontier[atomicAdd(fcount, 1u)] = (uint32_t)v;
-    }
+// Vertices collected by one wave in LDS on their way to a list: the list's
+// counter takes one atomic per 64 of them or more (atomics on one word are
+// serialised, about 14 ns each, and were most of a peel level's time).
+struct Collect {
+  uint32_t* buf;    // 128 words
+  uint32_t* list;
+  uint32_t* count;
+  uint32_t held;    // wave-uniform
+
+  __device__ void flush() {
+    if (!held) return;
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(count, held);
+    at = __shfl(at, 0, 64);
+    dev::wave_sync();
+    for (uint32_t i = lane; i < held; i += 64) list[at + i] = buf[i];
+    dev::wave_sync();
+    held = 0;
   }
+  // every lane of the wave calls it
+  __device__ void add(bool take, uint32_t v) {
+    const uint64_t mask = dev::lanes(take);
+    if (!mask) return;
+    if (take) buf[dev::lanes_below(mask, held)] = v;
+    held = dev::uniform(held + (uint32_t)__popcll(mask));
+    if (held >= 64) flush();
+  }
+};
+
+// frontier = the unpeeled vertices within the threshold, labelled
+__global__ __launch_bounds__(256) void k_adir_scan(uint32_t n, const int32_t* __restrict__ rtd,
+                                                   int32_t* prio, float t, int32_t label,
+                                                   uint32_t* frontier, uint32_t* fcount) {
+  __shared__ uint32_t buf[4][128];
+  Collect out{buf[threadIdx.x >> 6], frontier, fcount, 0u};
+  for (uint64_t v0 = gtid() & ~63ull; v0 < n; v0 += gstride()) {
+    const uint64_t v = v0 + (threadIdx.x & 63);
+    const bool take = v < n && prio[v] == -1 && (float)rtd[v] <= t;
+    if (take) prio[v] = label;
+    out.add(take, (uint32_t)v);
+  }
+  out.flush();
 }
 
-// A peeled neighbour takes 2 from the runtime degree (it is listed twice in
-// allEdges); a vertex is peeled when its degree first reaches the threshold,
-// which makes the labels independent of the order of the frontier.
-__global__ void k_adir_expand(const uint32_t* __restrict__ frontier, uint32_t fsize,
-                              const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
-                              int32_t* rtd, int32_t* prio, float t, int32_t label,
-                              uint32_t* next, uint32_t* ncount) {
-  const uint32_t lane = threadIdx.x & 63;
+// What a peeled vertex does to its neighbours, A-direction: a peeled neighbour
+// takes 2 from the runtime degree (it is listed twice in allEdges); a vertex
+// is peeled when its degree first reaches the threshold, which makes the
+// labels independent of the order of the frontier.
+struct AdirStep {
+  int32_t* rtd;
+  int32_t* prio;
+  float t;
+  int32_t label;
+  __device__ bool live(uint32_t y) const {
+    return __hip_atomic_load(prio + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == -1;
+  }
+  __device__ bool take(uint32_t y) const {
+    const int32_t old = atomicSub(rtd + y, 2);
+    if (!((float)old > t && (float)(old - 2) <= t)) return false;
+    prio[y] = label;
+    return true;
+  }
+};
+
+// One level: step for every unpeeled neighbour y (live) of every frontier
+// vertex; the ones it takes form the next frontier (order free).  A wave takes per
+// (1 .. 64) frontier vertices and walks their neighbours back to back, 64 at a
+// time, each lane finding its vertex by a search over the prefix of the
+// lengths in LDS: with a wave per vertex most lanes idled on the short rows
+// that make up the early levels.  Rows of kLongRow entries or more are set
+// aside in pieces of that length (`big`: bounds) for k_peel_big, so no wave is
+// left with a hub.
+constexpr uint32_t kLongRow = 2048;
+
+// Four neighbours of each lane (kEmpty: none), their loads and atomics in
+// flight together.
+template <class Step>
+__device__ inline void peel4(const uint32_t (&y)[4], const Step& step, Collect& out) {
+  bool live[4], take[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) live[u] = y[u] != dev::kEmpty && step.live(y[u]);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) take[u] = live[u] && step.take(y[u]);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) out.add(take[u], y[u]);
+}
+
+template <class Step>
+__global__ __launch_bounds__(256) void k_peel_expand(const uint32_t* __restrict__ frontier,
+                                                     uint32_t fsize, uint32_t per,
+                                                     const uint32_t* __restrict__ rp,
+                                                     const uint32_t* __restrict__ col, Step step,
+                                                     uint32_t* next, uint32_t* ncount, uint2* big,
+                                                     uint32_t* nbig) {
+  __shared__ uint32_t pre[4][64], at[4][64], buf[4][128];
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint64_t wave = gtid() >> 6, nwaves = gstride() >> 6;
-  for (uint64_t f = wave; f < fsize; f += nwaves) {
-    uint32_t v = frontier[f];
-    for (uint32_t e = rp[v] + lane; e < rp[v + 1]; e += 64) {
-      uint32_t y = col[e];
-      if (__hip_atomic_load(prio + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != -1) continue;
-      int32_t old = atomicSub(rtd + y, 2);
-      if ((float)old > t && (float)(old - 2) <= t) {
-        prio[y] = label;
-        next[atomicAdd(ncount, 1u)] = y;
+  Collect out{buf[wv], next, ncount, 0u};
+  for (uint64_t f = wave * per; f < fsize; f += nwaves * per) {
+    uint32_t b = 0, len = 0;
+    if (lane < per && f + lane < fsize) {
+      const uint32_t v = frontier[f + lane];
+      b = rp[v];
+      len = rp[v + 1] - b;
+    }
+    uint64_t lng = dev::lanes(len >= kLongRow);
+    while (lng) {
+      const uint32_t j = (uint32_t)__builtin_ctzll(lng);
+      lng &= lng - 1;
+      const uint32_t vb = __shfl(b, j, 64), vl = __shfl(len, j, 64);
+      const uint32_t pieces = (vl + kLongRow - 1) / kLongRow;
+      uint32_t p0 = 0;
+      if (lane == 0) p0 = atomicAdd(nbig, pieces);
+      p0 = __shfl(p0, 0, 64);
+      for (uint32_t i = lane; i < pieces; i += 64)
+        big[p0 + i] = make_uint2(vb + i * kLongRow, vb + min(vl, (i + 1) * kLongRow));
+      if (lane == j) len = 0;
+    }
+    const uint32_t incl = dev::wave_incl_scan_dpp(len), total = __shfl(incl, 63, 64);
+    pre[wv][lane] = incl - len;
+    at[wv][lane] = b;
+    dev::wave_sync();
+    for (uint32_t i0 = 0; i0 < total; i0 += 256) {
+      uint32_t y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t i = i0 + 64 * u + lane, j = dev::seg64(pre[wv], i);
+        y[u] = i < total ? col[at[wv][j] + (i - pre[wv][j])] : dev::kEmpty;
       }
+      peel4(y, step, out);
+    }
+    dev::wave_sync();
+  }
+  out.flush();
+}
+
+template <class Step>
+__global__ __launch_bounds__(256) void k_peel_big(const uint2* __restrict__ big, uint32_t nbig,
+                                                  const uint32_t* __restrict__ col, Step step,
+                                                  uint32_t* next, uint32_t* ncount) {
+  __shared__ uint32_t buf[4][128];
+  const uint32_t lane = threadIdx.x & 63;
+  Collect out{buf[threadIdx.x >> 6], next, ncount, 0u};
+  for (uint64_t k = gtid() >> 6; k < nbig; k += gstride() >> 6) {
+    const uint2 r = big[k];
+    for (uint32_t i0 = r.x; i0 < r.y; i0 += 256) {
+      uint32_t y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) y[u] = i0 + 64 * u + lane < r.y ? col[i0 + 64 * u + lane] : dev::kEmpty;
+      peel4(y, step, out);
     }
   }
+  out.flush();
 }
 
 // ---- Bisson/A-direction.cpp degree record ----------------------------------
@@ -308,8 +449,11 @@ __global__ void k_adir_cross(const uint64_t* __restrict__ ev, uint64_t E,
   }
 }
 
-__global__ void k_min_unpeeled(uint32_t n, const int32_t* __restrict__ val,
-                               const int32_t* __restrict__ state, int32_t* out) {
+// One atomic per workgroup (launched with a few hundred).
+__global__ __launch_bounds__(256) void k_min_unpeeled(uint32_t n, const int32_t* __restrict__ val,
+                                                      const int32_t* __restrict__ state,
+                                                      int32_t* out) {
+  __shared__ int32_t red[4];
   int32_t mn = INT32_MAX;
   for (uint64_t v = gtid(); v < n; v += gstride())
     if (state[v] == -1 && val[v] < mn) mn = val[v];
@@ -317,7 +461,12 @@ __global__ void k_min_unpeeled(uint32_t n, const int32_t* __restrict__ val,
     int32_t o = __shfl_down(mn, off, 64);
     mn = o < mn ? o : mn;
   }
-  if ((threadIdx.x & 63) == 0 && mn != INT32_MAX) atomicMin(out, mn);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mn;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    mn = min(min(red[0], red[1]), min(red[2], red[3]));
+    if (mn != INT32_MAX) atomicMin(out, mn);
+  }
 }
 
 // ---- k-core (edge_directing/kcore_direction.cpp:91-126) --------------------
@@ -333,37 +482,39 @@ __global__ void k_core_init(const uint32_t* __restrict__ rp, uint32_t n, int32_t
 
 // `step` (optional) receives the index of the frontier that removes each
 // vertex: every frontier is one step, numbered over the whole peel.
-__global__ void k_core_scan(uint32_t n, const int32_t* __restrict__ deg, int32_t* core, int32_t k,
-                            uint32_t* frontier, uint32_t* fcount, int32_t* step, int32_t t) {
-  for (uint64_t v = gtid(); v < n; v += gstride()) {
-    if (core[v] == -1 && deg[v] <= k) {
+__global__ __launch_bounds__(256) void k_core_scan(uint32_t n, const int32_t* __restrict__ deg,
+                                                   int32_t* core, int32_t k, uint32_t* frontier,
+                                                   uint32_t* fcount, int32_t* step, int32_t t) {
+  __shared__ uint32_t buf[4][128];
+  Collect out{buf[threadIdx.x >> 6], frontier, fcount, 0u};
+  for (uint64_t v0 = gtid() & ~63ull; v0 < n; v0 += gstride()) {
+    const uint64_t v = v0 + (threadIdx.x & 63);
+    const bool take = v < n && core[v] == -1 && deg[v] <= k;
+    if (take) {
       core[v] = k;
       if (step) step[v] = t;
-      frontier[atomicAdd(fcount, 1u)] = (uint32_t)v;
     }
+    out.add(take, (uint32_t)v);
   }
+  out.flush();
 }
 
-__global__ void k_core_expand(const uint32_t* __restrict__ frontier, uint32_t fsize,
-                              const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
-                              int32_t* deg, int32_t* core, int32_t k, uint32_t* next,
-                              uint32_t* ncount, int32_t* step, int32_t t) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint64_t wave = gtid() >> 6, nwaves = gstride() >> 6;
-  for (uint64_t f = wave; f < fsize; f += nwaves) {
-    uint32_t v = frontier[f];
-    for (uint32_t e = rp[v] + lane; e < rp[v + 1]; e += 64) {
-      uint32_t y = col[e];
-      if (__hip_atomic_load(core + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != -1) continue;
-      int32_t old = atomicSub(deg + y, 1);
-      if (old == k + 1) {
-        core[y] = k;
-        if (step) step[y] = t;
-        next[atomicAdd(ncount, 1u)] = y;
-      }
-    }
+struct CoreStep {
+  int32_t* deg;
+  int32_t* core;
+  int32_t k;
+  int32_t* step;
+  int32_t t;
+  __device__ bool live(uint32_t y) const {
+    return __hip_atomic_load(core + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == -1;
   }
-}
+  __device__ bool take(uint32_t y) const {
+    if (atomicSub(deg + y, 1) != k + 1) return false;
+    core[y] = k;
+    if (step) step[y] = t;
+    return true;
+  }
+};
 
 // keep[e] for a sorted symmetric key list: ADIR (mode 2), or KCORE (mode 3)
 // and DEGENERACY (mode 5), whose keys both point up from the lower (key, id).
@@ -537,6 +688,35 @@ int read_u32(tc_ctx* c, const uint32_t* dptr, uint32_t* out) {
   return TC_OK;
 }
 
+// One peel level: *ns vertices of the next frontier N from the frontier F of
+// fs vertices.
+template <class Step>
+int peel_level(tc_ctx* c, const uint32_t* F, uint32_t fs, const uint32_t* rp, const uint32_t* col,
+               Step step, uint32_t* N, uint2* big, uint32_t* ns) {
+  uint32_t* cnt = c->scratch.as<uint32_t>();
+  TCX_HIP(hipMemsetAsync(cnt, 0, 8, c->stream));
+  // one vertex a wave until every wave of the GPU has one
+  uint32_t per = 1;
+  while (per < 64 && fs / (2 * per) >= (uint32_t)c->num_cus * 32u) per *= 2;
+  hipLaunchKernelGGL(k_peel_expand<Step>,
+                     dim3(std::min<unsigned>((unsigned)c->num_cus * 8u,
+                                             grid_for(((uint64_t)fs + per - 1) / per * 64))),
+                     dim3(TB), 0, c->stream, F, fs, per, rp, col, step, N, cnt, big, cnt + 1);
+  TCX_HIP(hipGetLastError());
+  uint32_t h[2];  // next frontier, pieces of long rows
+  TCX_HIP(hipMemcpyAsync(h, cnt, 8, hipMemcpyDeviceToHost, c->stream));
+  TCX_HIP(hipStreamSynchronize(c->stream));
+  if (h[1]) {
+    hipLaunchKernelGGL(k_peel_big<Step>,
+                       dim3(std::min<unsigned>((unsigned)c->num_cus * 8u, grid_for(64ull * h[1]))),
+                       dim3(TB), 0, c->stream, big, h[1], col, step, N, cnt);
+    TCX_HIP(hipGetLastError());
+    TCX_TRY(read_u32(c, cnt, h));
+  }
+  *ns = h[0];
+  return TC_OK;
+}
+
 }  // namespace
 
 // Sort keys (in `keys`, scratch of the same size in `tmp`), drop duplicates
@@ -574,16 +754,14 @@ static int csr_from_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint
 }
 
 int compute_csr_stats(tc_ctx* c, tc_graph* g) {
-  DevBuf& indeg = g->indeg;
-  TCX_TRY(indeg.reserve(sizeof(uint32_t) * ((size_t)g->n + 1)));
   TCX_TRY(c->accum.reserve(64));
   unsigned long long* acc = c->accum.as<unsigned long long>();
   TCX_HIP(hipMemsetAsync(acc, 0, 3 * sizeof(unsigned long long), c->stream));
-  hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(g->n)), dim3(TB), 0, c->stream,
-                     indeg.as<uint32_t>(), 0u, (uint64_t)g->n);
-  TCX_TRY(count_ids(c, g->col.as<uint32_t>(), nullptr, g->m_or, g->n, indeg.as<uint32_t>()));
-  hipLaunchKernelGGL(k_csr_stats, dim3(grid_for(g->n)), dim3(TB), 0, c->stream,
-                     g->rowptr.as<uint32_t>(), indeg.as<uint32_t>(), g->n, acc);
+  hipLaunchKernelGGL(k_csr_stats,
+                     dim3(std::min<unsigned>(grid_for(std::max<uint64_t>(g->n, g->m_or)),
+                                             (unsigned)c->num_cus * 8u)),
+                     dim3(TB), 0, c->stream, g->rowptr.as<uint32_t>(), g->col.as<uint32_t>(), g->n,
+                     g->m_or, acc);
   TCX_HIP(hipGetLastError());
   unsigned long long h[3];
   TCX_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, c->stream));
@@ -684,7 +862,8 @@ static int adir_level_ordered(tc_ctx* c, AdirOrdered& o, const uint32_t* F, uint
 static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, const uint32_t* col,
                      int32_t* prio, int32_t* rec = nullptr, double thre_param = 0) {
   const bool omp = thre_param > 0;
-  DevBuf rtd, fa, fb;
+  DevBuf rtd, fa, fb, big;
+  TCX_TRY(big.reserve(16 * (m2 / kLongRow + 1)));
   TCX_TRY(rtd.reserve(sizeof(int32_t) * ((size_t)n + 1)));
   TCX_TRY(fa.reserve(sizeof(uint32_t) * ((size_t)n + 1)));
   TCX_TRY(fb.reserve(sizeof(uint32_t) * ((size_t)n + 1)));
@@ -719,7 +898,6 @@ static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, con
   uint64_t peeled = 0;
   uint32_t* F = fa.as<uint32_t>();
   uint32_t* N = fb.as<uint32_t>();
-  const unsigned expand_grid = 4096;
   for (;;) {
     uint32_t fs = 0;
     if (rec) {  // ascending ids, as the serial scan appends them
@@ -735,7 +913,7 @@ static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, con
       TCX_HIP(hipGetLastError());
     } else {
       TCX_HIP(hipMemsetAsync(cnt, 0, sizeof(uint32_t), c->stream));
-      hipLaunchKernelGGL(k_adir_scan, dim3(grid_for(n)), dim3(TB), 0, c->stream, n,
+      hipLaunchKernelGGL(k_adir_scan, dim3(std::min(grid_for(n), 1024u)), dim3(TB), 0, c->stream, n,
                          rtd.as<int32_t>(), prio, threshold, label, F, cnt);
       TCX_HIP(hipGetLastError());
       TCX_TRY(read_u32(c, cnt, &fs));
@@ -750,13 +928,9 @@ static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, con
         TCX_TRY(adir_level_ordered(c, ord, F, fs, rp, col, rtd.as<int32_t>(), prio, threshold,
                                    label, rec, N, &ns));
       } else {
-        TCX_HIP(hipMemsetAsync(cnt, 0, sizeof(uint32_t), c->stream));
-        hipLaunchKernelGGL(k_adir_expand,
-                           dim3(std::min<unsigned>(expand_grid, grid_for(fs * 64ull))), dim3(TB),
-                           0, c->stream, F, fs, rp, col, rtd.as<int32_t>(), prio, threshold,
-                           label, N, cnt);
-        TCX_HIP(hipGetLastError());
-        TCX_TRY(read_u32(c, cnt, &ns));
+        TCX_TRY(peel_level(c, F, fs, rp, col,
+                           AdirStep{rtd.as<int32_t>(), prio, threshold, label}, N,
+                           big.as<uint2>(), &ns));
       }
       peeled += ns;
       std::swap(F, N);
@@ -767,7 +941,7 @@ static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, con
     step();
     // Rounds whose scan finds nothing only advance the label and threshold.
     TCX_HIP(hipMemsetAsync(cnt, 0x7f, sizeof(int32_t), c->stream));
-    hipLaunchKernelGGL(k_min_unpeeled, dim3(grid_for(n)), dim3(TB), 0, c->stream, n,
+    hipLaunchKernelGGL(k_min_unpeeled, dim3(std::min(grid_for(n), 512u)), dim3(TB), 0, c->stream, n,
                        rtd.as<int32_t>(), prio, (int32_t*)cnt);
     TCX_HIP(hipGetLastError());
     int32_t minr = 0;
@@ -784,9 +958,10 @@ static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, con
 // every vertex.  A vertex removed at step t has at most core[v] neighbours
 // removed at step t or later (its remaining degree when its frontier formed),
 // so orienting every edge from the lower (step, id) bounds d+(v) by core[v].
-static int kcore_peel(tc_ctx* c, uint32_t n, const uint32_t* rp, const uint32_t* col,
+static int kcore_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, const uint32_t* col,
                       int32_t* core, int32_t* step = nullptr) {
-  DevBuf deg, fa, fb;
+  DevBuf deg, fa, fb, big;
+  TCX_TRY(big.reserve(16 * (m2 / kLongRow + 1)));
   TCX_TRY(deg.reserve(sizeof(int32_t) * ((size_t)n + 1)));
   TCX_TRY(fa.reserve(sizeof(uint32_t) * ((size_t)n + 1)));
   TCX_TRY(fb.reserve(sizeof(uint32_t) * ((size_t)n + 1)));
@@ -801,7 +976,7 @@ static int kcore_peel(tc_ctx* c, uint32_t n, const uint32_t* rp, const uint32_t*
   uint32_t* N = fb.as<uint32_t>();
   while (removed < n) {
     TCX_HIP(hipMemsetAsync(cnt, 0, sizeof(uint32_t), c->stream));
-    hipLaunchKernelGGL(k_core_scan, dim3(grid_for(n)), dim3(TB), 0, c->stream, n,
+    hipLaunchKernelGGL(k_core_scan, dim3(std::min(grid_for(n), 1024u)), dim3(TB), 0, c->stream, n,
                        deg.as<int32_t>(), core, k, F, cnt, step, t);
     TCX_HIP(hipGetLastError());
     uint32_t fs = 0;
@@ -809,13 +984,9 @@ static int kcore_peel(tc_ctx* c, uint32_t n, const uint32_t* rp, const uint32_t*
     removed += fs;
     if (fs) ++t;
     while (fs > 0) {
-      TCX_HIP(hipMemsetAsync(cnt, 0, sizeof(uint32_t), c->stream));
-      hipLaunchKernelGGL(k_core_expand, dim3(std::min<unsigned>(4096, grid_for(fs * 64ull))),
-                         dim3(TB), 0, c->stream, F, fs, rp, col, deg.as<int32_t>(), core, k, N,
-                         cnt, step, t);
-      TCX_HIP(hipGetLastError());
       uint32_t ns = 0;
-      TCX_TRY(read_u32(c, cnt, &ns));
+      TCX_TRY(peel_level(c, F, fs, rp, col, CoreStep{deg.as<int32_t>(), core, k, step, t}, N,
+                         big.as<uint2>(), &ns));
       removed += ns;
       if (ns) ++t;
       std::swap(F, N);
@@ -823,13 +994,23 @@ static int kcore_peel(tc_ctx* c, uint32_t n, const uint32_t* rp, const uint32_t*
     }
     if (removed >= n) break;
     TCX_HIP(hipMemsetAsync(cnt, 0x7f, sizeof(int32_t), c->stream));
-    hipLaunchKernelGGL(k_min_unpeeled, dim3(grid_for(n)), dim3(TB), 0, c->stream, n,
+    hipLaunchKernelGGL(k_min_unpeeled, dim3(std::min(grid_for(n), 512u)), dim3(TB), 0, c->stream, n,
                        deg.as<int32_t>(), core, (int32_t*)cnt);
     TCX_HIP(hipGetLastError());
     int32_t mind = 0;
     TCX_TRY(read_u32(c, cnt, (uint32_t*)&mind));
     k = std::max(k + 1, mind);
   }
+  return TC_OK;
+}
+
+int vertex_degrees(tc_ctx* c, tc_graph* g) {
+  if (g->vdeg_version == g->sched_version) return TC_OK;
+  TCX_TRY(g->vdeg.reserve(4 * ((size_t)g->n + 1)));
+  hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(g->n)), dim3(TB), 0, c->stream,
+                     g->vdeg.as<uint32_t>(), 0u, (uint64_t)g->n);
+  TCX_TRY(count_ids(c, g->col.as<uint32_t>(), nullptr, g->m_or, g->n, g->vdeg.as<uint32_t>()));
+  g->vdeg_version = g->sched_version;
   return TC_OK;
 }
 
@@ -1211,6 +1392,10 @@ static int orient_impl(tc_ctx* c, tc_graph* g, int mode, uint32_t flags, int tie
     TCX_HIP(hipGetLastError());
     TCX_TRY(csr_from_keys(c, g, keys, tmp, m, n_out, false));
     g->orient_mode = mode;
+    if (mode != TC_ORIENT_ID && n_out == n) {  // the raw degrees stay with the graph
+      swap(g->vdeg, deg);
+      g->vdeg_version = g->sched_version;
+    }
     return TC_OK;
   }
   return orient_peeled(c, g, mode, 0, tie);
@@ -1231,11 +1416,11 @@ static int orient_peeled(tc_ctx* c, tc_graph* g, int mode, double thre_param, in
       TCX_TRY(adir_peel(c, n, m2, srp.as<uint32_t>(), scol.as<uint32_t>(), g->vkey.as<int32_t>(),
                         nullptr, mode == TC_ORIENT_ADIR_OMP ? thre_param : 0));
     } else if (mode == TC_ORIENT_KCORE) {
-      TCX_TRY(kcore_peel(c, n, srp.as<uint32_t>(), scol.as<uint32_t>(), g->vkey.as<int32_t>()));
+      TCX_TRY(kcore_peel(c, n, m2, srp.as<uint32_t>(), scol.as<uint32_t>(), g->vkey.as<int32_t>()));
     } else {
       DevBuf core;
       TCX_TRY(core.reserve(4 * ((size_t)n + 1)));
-      TCX_TRY(kcore_peel(c, n, srp.as<uint32_t>(), scol.as<uint32_t>(), core.as<int32_t>(),
+      TCX_TRY(kcore_peel(c, n, m2, srp.as<uint32_t>(), scol.as<uint32_t>(), core.as<int32_t>(),
                          g->vkey.as<int32_t>()));
     }
   }
@@ -1259,6 +1444,11 @@ static int orient_peeled(tc_ctx* c, tc_graph* g, int mode, double thre_param, in
   DevBuf* spare = holder == &keys ? &tmp : &keys;
   TCX_TRY(csr_from_keys(c, g, *holder, *spare, mo, n, true));
   g->orient_mode = mode;
+  TCX_TRY(g->vdeg.reserve(4 * ((size_t)n + 1)));
+  hipLaunchKernelGGL(k_row_degrees, dim3(grid_for(n)), dim3(TB), 0, c->stream, srp.as<uint32_t>(),
+                     n, g->vdeg.as<uint32_t>());
+  TCX_HIP(hipGetLastError());
+  g->vdeg_version = g->sched_version;
   return TC_OK;
 }
 

@@ -153,7 +153,11 @@ struct tc_graph {
   tcx::DevBuf rowptr;       // uint32[n+1]
   tcx::DevBuf col;          // uint32[m_or]
   tcx::DevBuf esrc;         // uint32[m_or]  source of each CSR edge
-  tcx::DevBuf indeg;        // uint32[n]  in-degrees of the oriented CSR
+  // uint32[n] a degree of each vertex (of the raw records, the simple graph or
+  // the CSR's in-edges, whichever the orientation had at hand) and the CSR it
+  // goes with; vertex_degrees() makes it when there is none
+  tcx::DevBuf vdeg;
+  uint64_t vdeg_version = ~0ull;
   tcx::DevBuf vkey;         // int32[n] ADIR priority / KCORE core number
   uint64_t sum_out_sq = 0, sum_in_out = 0;
   // cached schedules (valid for the current CSR)
@@ -192,6 +196,7 @@ int select_flagged_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags,
 int build_csr_from_keys(tc_ctx* c, tc_graph* g, uint64_t* keys, uint64_t nkeys,
                         int end_bit);
 int compute_csr_stats(tc_ctx* c, tc_graph* g);
+int vertex_degrees(tc_ctx* c, tc_graph* g);
 int build_sym(tc_ctx* c, tc_graph* g, DevBuf& rowptr, DevBuf& col, uint64_t* m2);
 // A new graph holding a device copy of g's raw records (not oriented); its
 // vertex count is the records' largest id + 1.  A graph without raw records

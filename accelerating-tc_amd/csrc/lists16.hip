@@ -11,7 +11,7 @@ namespace {
 
 using namespace dev;
 
-constexpr uint32_t kHistBins = 4096;  // in-degree histogram, the last bin open
+constexpr uint32_t kHistBins = 4096;  // degree histogram, the last bin open
 // A graph of more than 65,535 vertices takes the layer when at least this
 // share of its entries gets a 16-bit id; below it, the tail's work lists and
 // tasks cost as much as the layer saves (Barabasi-Albert, 90,000 vertices, 16
@@ -31,8 +31,8 @@ __global__ void k_fill16(uint32_t* p, uint32_t v, uint64_t n) {
   for (uint64_t i = gtid(); i < n; i += gstride()) p[i] = v;
 }
 
-// hist[min(indeg, bins - 1)] += 1, and the in-degree sum of the open bin
-__global__ __launch_bounds__(TB) void k_indeg_hist(const uint32_t* __restrict__ indeg, uint32_t n,
+// hist[min(deg, bins - 1)] += 1, and the degree sum of the open bin
+__global__ __launch_bounds__(TB) void k_deg_hist(const uint32_t* __restrict__ deg, uint32_t n,
                                                    uint32_t* __restrict__ hist,
                                                    unsigned long long* open_sum) {
   __shared__ uint32_t h[kHistBins];
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(TB) void k_indeg_hist(const uint32_t* __restrict__ 
   __syncthreads();
   unsigned long long s = 0;
   for (uint64_t v = gtid(); v < n; v += gstride()) {
-    const uint32_t d = indeg[v];
+    const uint32_t d = deg[v];
     if (d >= kHistBins - 1) s += d;
     atomicAdd(h + min(d, kHistBins - 1), 1u);
   }
@@ -50,15 +50,15 @@ __global__ __launch_bounds__(TB) void k_indeg_hist(const uint32_t* __restrict__ 
   flush_count(s, open_sum);
 }
 
-__global__ void k_hub_flags(const uint32_t* __restrict__ indeg, uint32_t n, uint32_t t,
+__global__ void k_hub_flags(const uint32_t* __restrict__ deg, uint32_t n, uint32_t t,
                             uint32_t* __restrict__ f) {
-  for (uint64_t v = gtid(); v < n; v += gstride()) f[v] = indeg[v] >= t ? 1u : 0u;
+  for (uint64_t v = gtid(); v < n; v += gstride()) f[v] = deg[v] >= t ? 1u : 0u;
 }
 
-__global__ void k_hub_ids(const uint32_t* __restrict__ indeg, const uint32_t* __restrict__ pos,
+__global__ void k_hub_ids(const uint32_t* __restrict__ deg, const uint32_t* __restrict__ pos,
                           uint32_t n, uint32_t t, uint16_t* __restrict__ id) {
   for (uint64_t v = gtid(); v < n; v += gstride())
-    id[v] = indeg[v] >= t ? (uint16_t)pos[v] : (uint16_t)kPad16;
+    id[v] = deg[v] >= t ? (uint16_t)pos[v] : (uint16_t)kPad16;
 }
 
 // f[e] = 1 where the entry has a 16-bit id; f[m] = 0
@@ -249,21 +249,27 @@ int read_back(tc_ctx* c, const void* src, T* out) {
   return TC_OK;
 }
 
-// 16-bit ids by in-degree: the vertices of in-degree t and above for the
-// smallest t that leaves at most kMax16 of them.  *share = the part of the
-// CSR's entries that get one.
-int hub_ids(tc_ctx* c, tc_graph* g, DevBuf& id, double* share) {
+// 16-bit ids by degree (in skewed graphs the in-degree follows it: R-MAT-21 has
+// 0.928 of its entries among the 65,535 vertices of largest degree, 0.929 among
+// those of largest in-degree): the vertices of degree t and above for the
+// smallest t that leaves at most kMax16 of them.  *some: whether they can hold
+// kMinShare of the entries (in-degrees are at most the degrees).
+int hub_ids(tc_ctx* c, tc_graph* g, DevBuf& id, bool* some) {
   const uint32_t n = g->n;
+  *some = false;
+  // just above the limit (65,536 vertices) in-degrees decide: the few that are
+  // zero need no id, so nothing is left to the tail
+  if (n <= kMax16 + 1024) g->vdeg_version = ~0ull;
+  TCX_TRY(vertex_degrees(c, g));
   DevBuf hist;
   TCX_TRY(hist.reserve(4 * kHistBins + 8));
   TCX_HIP(hipMemsetAsync(hist.p, 0, 4 * kHistBins + 8, c->stream));
-  hipLaunchKernelGGL(k_indeg_hist, dim3(std::min<unsigned>(grid_for(n), c->num_cus * 2u)), dim3(TB),
-                     0, c->stream, g->indeg.as<uint32_t>(), n, hist.as<uint32_t>(),
+  hipLaunchKernelGGL(k_deg_hist, dim3(std::min<unsigned>(grid_for(n), c->num_cus * 2u)), dim3(TB),
+                     0, c->stream, g->vdeg.as<uint32_t>(), n, hist.as<uint32_t>(),
                      reinterpret_cast<unsigned long long*>(hist.as<uint32_t>() + kHistBins));
   TCX_HIP(hipGetLastError());
   struct { uint32_t bin[kHistBins]; unsigned long long open; } h;
   TCX_TRY(read_back(c, hist.p, &h));
-  *share = 0;
   uint64_t have = 0, sum = 0;
   uint32_t t = kHistBins;
   while (t > 1 && have + h.bin[t - 1] <= kMax16) {
@@ -271,17 +277,17 @@ int hub_ids(tc_ctx* c, tc_graph* g, DevBuf& id, double* share) {
     have += h.bin[t];
     sum += t == kHistBins - 1 ? h.open : (uint64_t)t * h.bin[t];
   }
-  if (t == kHistBins) return TC_OK;  // too many in the open bin
-  *share = (double)sum / (double)g->m_or;
-  if (*share < kMinShare) return TC_OK;
+  // (t == kHistBins: too many in the open bin)
+  if (t == kHistBins || (double)sum < kMinShare * (double)g->m_or) return TC_OK;
+  *some = true;
   DevBuf flag, pos;
   TCX_TRY(flag.reserve(4 * ((size_t)n + 1)));
   TCX_TRY(pos.reserve(4 * ((size_t)n + 1)));
   TCX_TRY(id.reserve(2 * ((size_t)n + 1)));
-  hipLaunchKernelGGL(k_hub_flags, dim3(grid_for(n)), dim3(TB), 0, c->stream, g->indeg.as<uint32_t>(),
+  hipLaunchKernelGGL(k_hub_flags, dim3(grid_for(n)), dim3(TB), 0, c->stream, g->vdeg.as<uint32_t>(),
                      n, t, flag.as<uint32_t>());
   TCX_TRY(exclusive_scan_u32(c, flag.as<uint32_t>(), pos.as<uint32_t>(), n));
-  hipLaunchKernelGGL(k_hub_ids, dim3(grid_for(n)), dim3(TB), 0, c->stream, g->indeg.as<uint32_t>(),
+  hipLaunchKernelGGL(k_hub_ids, dim3(grid_for(n)), dim3(TB), 0, c->stream, g->vdeg.as<uint32_t>(),
                      pos.as<uint32_t>(), n, t, id.as<uint16_t>());
   TCX_HIP(hipGetLastError());
   return TC_OK;
@@ -379,6 +385,7 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
 
 // Rows, work lists and slices for the ids `id` (null: every vertex id is its
 // own 16-bit id; id_all: every vertex has one, and there is no tail).
+// L.usable is left false when too few entries have an id.
 int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, Lists16& L) {
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
@@ -397,6 +404,7 @@ int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, Lists16& L) {
     TCX_TRY(exclusive_scan_u32(c, flag.as<uint32_t>(), pre_b.as<uint32_t>(), m + 1));
     pre = pre_b.as<uint32_t>();
     TCX_TRY(read_back(c, pre + m, &with_id));
+    if ((double)with_id < kMinShare * (double)m) return TC_OK;
   }
   const bool tail = with_id < m;
   TCX_TRY(cnt.reserve(4 * ((size_t)n + 1)));
@@ -412,6 +420,7 @@ int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, Lists16& L) {
   TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), id, false, L.hub));
   L.tail.tasks = 0;
   if (tail) TCX_TRY(work_lists(c, g, tcnt.as<uint32_t>(), id, true, L.tail));
+  L.usable = true;
   return TC_OK;
 }
 
@@ -422,18 +431,10 @@ int lists16(tc_ctx* c, tc_graph* g) {
   if (L.version == g->sched_version) return TC_OK;
   L.usable = false;
   if (g->n && g->m_or) {
-    if (g->n <= kMax16) {
-      TCX_TRY(build(c, g, nullptr, true, L));
-      L.usable = true;
-    } else {
-      DevBuf id;
-      double share = 0;
-      TCX_TRY(hub_ids(c, g, id, &share));
-      if (share >= kMinShare) {
-        TCX_TRY(build(c, g, id.as<uint16_t>(), false, L));
-        L.usable = true;
-      }
-    }
+    DevBuf id;
+    bool some = true;
+    if (g->n > kMax16) TCX_TRY(hub_ids(c, g, id, &some));
+    if (some) TCX_TRY(build(c, g, id.as<uint16_t>(), g->n <= kMax16, L));
   }
   L.version = g->sched_version;
   return TC_OK;
@@ -454,7 +455,6 @@ int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* v
       hipLaunchKernelGGL(k_graph_of, dim3(grid_for(L.hub.tasks)), dim3(TB), 0, c->stream,
                          L.hub.who.as<uint32_t>(), L.hub.tasks, gid);
     TCX_HIP(hipGetLastError());
-    L.usable = true;
   }
   L.version = g->sched_version;
   return TC_OK;
