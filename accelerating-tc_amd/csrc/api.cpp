@@ -26,27 +26,6 @@ int fail(int status, const char* fmt, ...) {
   return status;
 }
 
-int DevBuf::reserve(size_t want) {
-  if (want <= bytes && p) return TC_OK;
-  release();
-  if (want == 0) want = 64;
-  hipError_t e = hipMalloc(&p, want);
-  if (e != hipSuccess) {
-    p = nullptr;
-    bytes = 0;
-    (void)hipGetLastError();
-    return fail(TC_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", want, hipGetErrorString(e));
-  }
-  bytes = want;
-  return TC_OK;
-}
-
-void DevBuf::release() {
-  if (p) (void)hipFree(p);
-  p = nullptr;
-  bytes = 0;
-}
-
 void parallel_for(uint64_t n, void (*fn)(uint64_t, uint64_t, void*), void* arg,
                   unsigned max_threads) {
   unsigned hw = std::thread::hardware_concurrency();
@@ -118,6 +97,11 @@ int tc_ctx_create(int device, tc_ctx** out) {
     delete c;
     return fail(TC_ERR_HIP, "stream/event creation failed");
   }
+  if (hipHostMalloc(&c->pin, tcx::kPinBytes, hipHostMallocDefault) != hipSuccess) {
+    tc_ctx_destroy(c);
+    return fail(TC_ERR_NOMEM, "pinned host page allocation failed");
+  }
+  c->pool = tcx::pool_create(device, c->total_mem);
   *out = c;
   return TC_OK;
 }
@@ -135,7 +119,10 @@ int tc_ctx_destroy(tc_ctx* c) {
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->stream) (void)hipStreamDestroy(c->stream);
-  delete c;
+  if (c->pin) (void)hipHostFree(c->pin);
+  std::shared_ptr<tcx::Pool> pool = c->pool;
+  delete c;  // its last buffers go to the pool
+  tcx::pool_retire(std::move(pool));
   return TC_OK;
 }
 

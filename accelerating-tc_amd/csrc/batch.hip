@@ -383,6 +383,7 @@ extern "C" {
 
 int tc_batch_create(tc_ctx* c, uint32_t ngraphs, const uint64_t* eoff, const uint32_t* src,
                     const uint32_t* dst, const uint32_t* nverts, tc_batch** out) {
+  PoolScope scope(c);
   if (!c || !out || !eoff || !nverts || ngraphs == 0) return fail(TC_ERR_ARG, "bad arguments");
   *out = nullptr;
   if (eoff[0] != 0) return fail(TC_ERR_ARG, "edge_off[0] must be 0");
@@ -444,6 +445,7 @@ int tc_batch_info_get(const tc_batch* b, tc_graph_info* info) {
 }
 
 int tc_batch_stream_bytes(tc_ctx* c, tc_batch* b, double* bytes) {
+  PoolScope scope(c);
   TCX_TRY(check_batch(c, b));
   if (!bytes) return fail(TC_ERR_ARG, "NULL output");
   return tc_auto_stream_bytes(c, b->g, nullptr, bytes);
@@ -451,6 +453,7 @@ int tc_batch_stream_bytes(tc_ctx* c, tc_batch* b, double* bytes) {
 
 int tc_batch_count(tc_ctx* c, tc_batch* b, const tc_batch_sched* sched, uint64_t* counts,
                    tc_timing* timing) {
+  PoolScope scope(c);
   TCX_TRY(check_batch(c, b));
   if (!counts) return fail(TC_ERR_ARG, "NULL counts");
   const tc_batch_sched s = fill(sched, c);
@@ -507,6 +510,7 @@ int tc_batch_count(tc_ctx* c, tc_batch* b, const tc_batch_sched* sched, uint64_t
 
 int tc_batch_count_pergraph(tc_ctx* c, tc_batch* b, const tc_batch_sched* sched,
                             uint64_t* counts, tc_timing* timing) {
+  PoolScope scope(c);
   TCX_TRY(check_batch(c, b));
   if (!counts) return fail(TC_ERR_ARG, "NULL counts");
   const tc_batch_sched s = fill(sched, c);

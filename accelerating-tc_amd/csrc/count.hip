@@ -5,6 +5,7 @@
 // with uint64 per-lane partials, a wave reduction and one atomic per wave.
 // Integer sums are order-free, so any schedule gives the same exact count.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -900,24 +901,9 @@ using namespace tcx;
 
 namespace {
 
-struct Timer {
-  tc_ctx* c;
-  float ms = 0;
-  explicit Timer(tc_ctx* cc) : c(cc) {}
-  int begin() {
-    TCX_HIP(hipEventRecord(c->ev0, c->stream));
-    return TC_OK;
-  }
-  int end() {
-    TCX_HIP(hipEventRecord(c->ev1, c->stream));
-    TCX_HIP(hipEventSynchronize(c->ev1));
-    TCX_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    return TC_OK;
-  }
-};
-
 // Event marks between consecutive count launches: mark() before each launch,
-// finish() after the last; gives the total and the longest launch.
+// end() after the last; finish(), once the stream has been waited for, gives
+// the total and the longest launch.
 struct LaunchMarks {
   tc_ctx* c;
   int n = 0;
@@ -929,10 +915,12 @@ struct LaunchMarks {
     ++n;
     return TC_OK;
   }
-  int finish(tc_timing* tm) {
+  int end() {
     if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
     TCX_HIP(hipEventRecord(c->lev[n], c->stream));
-    TCX_HIP(hipEventSynchronize(c->lev[n]));
+    return TC_OK;
+  }
+  int finish(tc_timing* tm) {
     tm->ms_count = 0;
     tm->ms_dominant = 0;
     for (int i = 0; i < n; ++i) {
@@ -962,6 +950,7 @@ extern "C" {
 
 int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
              tc_timing* timing) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!count) return fail(TC_ERR_ARG, "NULL count");
   tc_sched s;
@@ -982,11 +971,11 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   }
   const uint32_t* rp = g->rowptr.as<uint32_t>();
   const uint32_t* col = g->col.as<uint32_t>();
-  Timer prep(c);
   LaunchMarks lm(c);
   bool on16 = false;  // AUTO over the 16-bit list layer
-  TCX_TRY(prep.begin());
-  // schedule (cached per graph)
+  // schedule (cached per graph; building one waits for the device, so the host
+  // clock times it, and a cached one costs no event)
+  const auto prep0 = std::chrono::steady_clock::now();
   switch (s.kernel) {
     case TC_KERNEL_HU:
       TCX_TRY(hu_schedule(c, g, s.grid_size ? s.grid_size : 30000u));  // Hu/tc.cu:7
@@ -1028,8 +1017,8 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     default:
       break;
   }
-  TCX_TRY(prep.end());
-  TCX_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long), c->stream));
+  tm.ms_prep = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - prep0).count();
+  if (!on16) TCX_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long), c->stream));
   switch (s.kernel) {
     case TC_KERNEL_HU: {
       TCX_TRY(lm.mark());
@@ -1179,24 +1168,23 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     }
   }
   TCX_HIP(hipGetLastError());
-  TCX_TRY(lm.finish(&tm));
+  TCX_TRY(lm.end());
   unsigned long long h = 0;
   if (on16) {
     unsigned long long part[kAccBytes16 / 8];
-    TCX_HIP(hipMemcpyAsync(part, c->scratch.p, kAccBytes16, hipMemcpyDeviceToHost, c->stream));
-    TCX_HIP(hipStreamSynchronize(c->stream));
+    TCX_TRY(fetch(c, part, c->scratch.p, kAccBytes16));
     h = sum16(part);
   } else {
-    TCX_HIP(hipMemcpyAsync(&h, acc, 8, hipMemcpyDeviceToHost, c->stream));
-    TCX_HIP(hipStreamSynchronize(c->stream));
+    TCX_TRY(fetch(c, &h, acc, 8));
   }
+  TCX_TRY(lm.finish(&tm));
   *count = h;
-  tm.ms_prep = prep.ms;
   if (timing) *timing = tm;
   return TC_OK;
 }
 
 int tc_auto_stream_bytes(tc_ctx* c, tc_graph* g, const tc_sched* sched, double* bytes) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!bytes) return fail(TC_ERR_ARG, "NULL output");
   tc_sched s;
@@ -1223,6 +1211,7 @@ int tc_auto_stream_bytes(tc_ctx* c, tc_graph* g, const tc_sched* sched, double* 
 }
 
 int tc_count_per_vertex(tc_ctx* c, tc_graph* g, uint64_t* tri) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!tri) return fail(TC_ERR_ARG, "NULL output");
   if (g->n == 0) return TC_OK;
@@ -1235,6 +1224,7 @@ int tc_count_per_vertex(tc_ctx* c, tc_graph* g, uint64_t* tri) {
 }
 
 int tc_hu_workload(tc_ctx* c, tc_graph* g, int64_t* w) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!w) return fail(TC_ERR_ARG, "NULL output");
   if (g->n == 0) return TC_OK;
@@ -1249,6 +1239,7 @@ int tc_hu_workload(tc_ctx* c, tc_graph* g, int64_t* w) {
 }
 
 int tc_hu_block_starts(tc_ctx* c, tc_graph* g, uint32_t nblocks, int32_t* start) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!start || nblocks == 0) return fail(TC_ERR_ARG, "bad arguments");
   ensure_version(g);
@@ -1260,6 +1251,7 @@ int tc_hu_block_starts(tc_ctx* c, tc_graph* g, uint32_t nblocks, int32_t* start)
 }
 
 int tc_fox_workload(tc_ctx* c, tc_graph* g, int32_t* w) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!w) return fail(TC_ERR_ARG, "NULL output");
   if (g->m_or == 0) return TC_OK;
@@ -1275,6 +1267,7 @@ int tc_fox_workload(tc_ctx* c, tc_graph* g, int32_t* w) {
 }
 
 int tc_fox_bin_sizes(tc_ctx* c, tc_graph* g, uint32_t max_lanes, uint64_t* count) {
+  PoolScope scope(c);
   TCX_TRY(check_ready(c, g));
   if (!count) return fail(TC_ERR_ARG, "NULL output");
   if (max_lanes == 0 || max_lanes > 64 || (max_lanes & (max_lanes - 1)))

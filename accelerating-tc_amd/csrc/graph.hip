@@ -683,9 +683,7 @@ int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint3
 }
 
 int read_u32(tc_ctx* c, const uint32_t* dptr, uint32_t* out) {
-  TCX_HIP(hipMemcpyAsync(out, dptr, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, out, dptr, sizeof(uint32_t));
 }
 
 // One peel level: *ns vertices of the next frontier N from the frontier F of
@@ -704,8 +702,7 @@ int peel_level(tc_ctx* c, const uint32_t* F, uint32_t fs, const uint32_t* rp, co
                      dim3(TB), 0, c->stream, F, fs, per, rp, col, step, N, cnt, big, cnt + 1);
   TCX_HIP(hipGetLastError());
   uint32_t h[2];  // next frontier, pieces of long rows
-  TCX_HIP(hipMemcpyAsync(h, cnt, 8, hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
+  TCX_TRY(fetch(c, h, cnt, 8));
   if (h[1]) {
     hipLaunchKernelGGL(k_peel_big<Step>,
                        dim3(std::min<unsigned>((unsigned)c->num_cus * 8u, grid_for(64ull * h[1]))),
@@ -734,14 +731,14 @@ static int csr_from_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint
     uniq = other;
     if (nuniq > 0) {
       uint64_t last = 0;
-      TCX_HIP(hipMemcpyAsync(&last, uniq + nuniq - 1, 8, hipMemcpyDeviceToHost, c->stream));
-      TCX_HIP(hipStreamSynchronize(c->stream));
+      TCX_TRY(fetch(c, &last, uniq + nuniq - 1, 8));
       if ((uint32_t)(last >> 32) == n_out) --nuniq;  // sentinel
     }
   }
   if (nuniq > kMaxCsrEntries)
     return fail(TC_ERR_RANGE, "%llu oriented edges exceed the 32-bit CSR offsets",
                 (unsigned long long)nuniq);
+  if (g->exported) TCX_HIP(hipDeviceSynchronize());
   g->n = n_out;
   g->m_or = nuniq;
   TCX_TRY(g->rowptr.reserve(sizeof(uint32_t) * ((size_t)n_out + 1)));
@@ -764,8 +761,7 @@ int compute_csr_stats(tc_ctx* c, tc_graph* g) {
                      g->m_or, acc);
   TCX_HIP(hipGetLastError());
   unsigned long long h[3];
-  TCX_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
+  TCX_TRY(fetch(c, h, acc, sizeof(h)));
   g->sum_out_sq = h[0];
   g->sum_in_out = h[1];
   g->max_out = (uint32_t)h[2];
@@ -790,8 +786,7 @@ static int sym_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint64_t*
   TCX_TRY(unique_u64(c, sorted, other, nk, &nu));
   if (nu > 0) {
     uint64_t last = 0;
-    TCX_HIP(hipMemcpyAsync(&last, other + nu - 1, 8, hipMemcpyDeviceToHost, c->stream));
-    TCX_HIP(hipStreamSynchronize(c->stream));
+    TCX_TRY(fetch(c, &last, other + nu - 1, 8));
     if ((uint32_t)(last >> 32) == g->n_raw) --nu;
   }
   *out = other;
@@ -1064,6 +1059,7 @@ extern "C" {
 
 int tc_graph_create(tc_ctx* c, const uint32_t* src, const uint32_t* dst, uint64_t m,
                     uint32_t n_hint, tc_graph** out) {
+  PoolScope scope(c);
   if (!c || !out) return fail(TC_ERR_ARG, "NULL argument");
   if (m && (!src || !dst)) return fail(TC_ERR_ARG, "NULL edge arrays");
   *out = nullptr;
@@ -1075,14 +1071,10 @@ int tc_graph_create(tc_ctx* c, const uint32_t* src, const uint32_t* dst, uint64_
   if (st == TC_OK) st = g->dst.reserve(4 * std::max<uint64_t>(m, 1));
   if (st != TC_OK) { delete g; return st; }
   if (m) {
-    hipError_t e1 = hipMemcpyAsync(g->src.p, src, 4 * m, hipMemcpyHostToDevice, c->stream);
-    hipError_t e2 = hipMemcpyAsync(g->dst.p, dst, 4 * m, hipMemcpyHostToDevice, c->stream);
-    if (e1 != hipSuccess || e2 != hipSuccess) {
-      delete g;
-      return fail(TC_ERR_HIP, "edge upload failed");
-    }
+    st = upload(c, g->src.p, src, 4 * m);
+    if (st == TC_OK) st = upload(c, g->dst.p, dst, 4 * m);
     uint32_t ms = 0, md = 0;
-    st = max_u32(c, g->src.as<uint32_t>(), m, &ms);
+    if (st == TC_OK) st = max_u32(c, g->src.as<uint32_t>(), m, &ms);
     if (st == TC_OK) st = max_u32(c, g->dst.as<uint32_t>(), m, &md);
     if (st != TC_OK) { delete g; return st; }
     uint32_t mx = std::max(ms, md);
@@ -1108,12 +1100,14 @@ int tc_graph_destroy(tc_graph* g) {
   if (g->ctx) {
     (void)hipSetDevice(g->ctx->device);
     (void)hipStreamSynchronize(g->ctx->stream);
+    if (g->exported) (void)hipDeviceSynchronize();
   }
   delete g;
   return TC_OK;
 }
 
 int tc_graph_simplify(tc_ctx* c, tc_graph* g) {
+  PoolScope scope(c);
   TCX_TRY(check_records(g));
   if (c != g->ctx) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (g->m_raw == 0) return TC_OK;
@@ -1132,8 +1126,7 @@ int tc_graph_simplify(tc_ctx* c, tc_graph* g) {
   TCX_TRY(unique_u64(c, sorted, other, g->m_raw, &nu));
   if (nu > 0) {
     uint64_t last = 0;
-    TCX_HIP(hipMemcpyAsync(&last, other + nu - 1, 8, hipMemcpyDeviceToHost, c->stream));
-    TCX_HIP(hipStreamSynchronize(c->stream));
+    TCX_TRY(fetch(c, &last, other + nu - 1, 8));
     if ((uint32_t)(last >> 32) == g->n_raw) --nu;
   }
   hipLaunchKernelGGL(k_unzip, dim3(grid_for(nu)), dim3(TB), 0, c->stream, other, nu,
@@ -1152,6 +1145,7 @@ int tc_graph_relabel_aorder(tc_ctx* c, tc_graph* g, uint32_t* perm_out) {
 
 int tc_graph_relabel_aorder_model(tc_ctx* c, tc_graph* g, const tc_bw_model* model,
                                   uint32_t* perm_out) {
+  PoolScope scope(c);
   if (!model) return fail(TC_ERR_ARG, "NULL bandwidth model");
   // the bucket heaps need a strict weak order: finite, positive bandwidths
   for (int l = 2; l < 10; ++l)
@@ -1206,6 +1200,7 @@ int tc_graph_relabel_aorder_model(tc_ctx* c, tc_graph* g, const tc_bw_model* mod
 }
 
 int tc_graph_relabel(tc_ctx* c, tc_graph* g, int mode, uint32_t* perm_out) {
+  PoolScope scope(c);
   TCX_TRY(check_records(g));
   if (c != g->ctx) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (mode < TC_RELABEL_COMPACT || mode > TC_RELABEL_ADIR)
@@ -1297,6 +1292,7 @@ static int orient_peeled(tc_ctx* c, tc_graph* g, int mode, double thre_param, in
 static int orient_impl(tc_ctx* c, tc_graph* g, int mode, uint32_t flags, int tie);
 
 int tc_graph_orient(tc_ctx* c, tc_graph* g, int mode, uint32_t flags) {
+  PoolScope scope(c);
   TCX_TRY(check_records(g));
   if (c != g->ctx) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (mode < TC_ORIENT_ID || mode > TC_ORIENT_DEGENERACY)
@@ -1307,6 +1303,7 @@ int tc_graph_orient(tc_ctx* c, tc_graph* g, int mode, uint32_t flags) {
 }
 
 int tc_graph_orient_ties(tc_ctx* c, tc_graph* g, int mode, int tie) {
+  PoolScope scope(c);
   TCX_TRY(check_records(g));
   if (c != g->ctx) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (mode != TC_ORIENT_ADIR && mode != TC_ORIENT_DEGREE)
@@ -1316,6 +1313,7 @@ int tc_graph_orient_ties(tc_ctx* c, tc_graph* g, int mode, int tie) {
 }
 
 int tc_graph_adir_cost(tc_ctx* c, tc_graph* g, double* cost) {
+  PoolScope scope(c);
   if (!c || !g || !cost) return fail(TC_ERR_ARG, "NULL argument");
   if (c != g->ctx) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (g->orient_mode < 0) return fail(TC_ERR_STATE, "graph must be oriented");
@@ -1453,6 +1451,7 @@ static int orient_peeled(tc_ctx* c, tc_graph* g, int mode, double thre_param, in
 }
 
 int tc_graph_orient_adir_omp(tc_ctx* c, tc_graph* g, double thre_param) {
+  PoolScope scope(c);
   TCX_TRY(check_records(g));
   if (c != g->ctx) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (!(thre_param > 0) || !std::isfinite(thre_param))
@@ -1513,6 +1512,7 @@ int tc_graph_save_csr(const tc_graph* g, const char* path) {
 }
 
 int tc_graph_load_csr(tc_ctx* c, const char* path, tc_graph** out) {
+  PoolScope scope(c);
   if (!c || !path || !out) return fail(TC_ERR_ARG, "NULL argument");
   *out = nullptr;
   FILE* f = fopen(path, "rb");
@@ -1642,6 +1642,7 @@ int tc_graph_device_csr(const tc_graph* g, const uint32_t** rowptr, const uint32
   if (g->orient_mode < 0) return fail(TC_ERR_STATE, "graph not oriented");
   *rowptr = g->rowptr.as<uint32_t>();
   *col = g->col.as<uint32_t>();
+  g->exported = true;
   return TC_OK;
 }
 

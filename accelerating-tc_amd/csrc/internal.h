@@ -37,11 +37,40 @@ int fail(int status, const char* fmt, ...);
     if (_s != TC_OK) return _s; \
   } while (0)
 
+// ---- device memory --------------------------------------------------------
+// Freed blocks of one context, kept for its next buffers (alloc.cpp).  All of
+// a context's work is on its one stream, so a block that a freed buffer leaves
+// behind is safe for the next buffer of the same context at once.
+struct Pool;
+// While one lives, this thread's buffers come from the context's pool (NULL,
+// or no scope: from hipMalloc).  Entry points that allocate open one.
+struct PoolScope {
+  explicit PoolScope(const tc_ctx* c);
+  ~PoolScope();
+  PoolScope(const PoolScope&) = delete;
+  PoolScope& operator=(const PoolScope&) = delete;
+ private:
+  Pool* before;
+};
+std::shared_ptr<Pool> pool_create(int device, uint64_t total_mem);
+// The context's stream is idle: its blocks go to the device's other contexts,
+// and back to the system with the last of them.
+void pool_retire(std::shared_ptr<Pool> pool);
+
+// Host-to-device copy of pageable memory on the context's stream; the host
+// memory has been read when it returns.
+int upload(tc_ctx* c, void* dst, const void* src, size_t bytes);
+// Device-to-host copy through the context's pinned page (at most kPinBytes);
+// waits for the stream.
+constexpr size_t kPinBytes = 32768;
+int fetch(tc_ctx* c, void* out, const void* src, size_t bytes);
+
 // ---- device buffer ------------------------------------------------------
-// Owns one hipMalloc'd region; grows on demand (contents are not kept).
+// Owns one region; grows on demand (contents are not kept).
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  std::shared_ptr<Pool> pool;  // where the region goes back to (null: hipFree)
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
@@ -54,6 +83,7 @@ struct DevBuf {
 inline void swap(DevBuf& a, DevBuf& b) {
   std::swap(a.p, b.p);
   std::swap(a.bytes, b.bytes);
+  std::swap(a.pool, b.pool);
 }
 
 }  // namespace tcx
@@ -62,6 +92,8 @@ struct tc_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  std::shared_ptr<tcx::Pool> pool;
+  void* pin = nullptr;      // kPinBytes of pinned host memory
   hipEvent_t lev[17] = {};  // per-launch timing marks (created on first use)
   uint64_t total_mem = 0;
   int num_cus = 256;
@@ -160,6 +192,9 @@ struct tc_graph {
   uint64_t vdeg_version = ~0ull;
   tcx::DevBuf vkey;         // int32[n] ADIR priority / KCORE core number
   uint64_t sum_out_sq = 0, sum_in_out = 0;
+  // tc_graph_device_csr gave the CSR's addresses out: work on any stream may
+  // read it, so its memory is let go only when the device is idle
+  mutable bool exported = false;
   // cached schedules (valid for the current CSR)
   uint64_t sched_version = 0;
   tcx::SchedCache sc;

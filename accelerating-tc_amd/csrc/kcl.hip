@@ -1066,6 +1066,7 @@ int cached_plan(tc_ctx* c, tc_graph* g, uint32_t k, tc_model* m, float* prep_ms)
 extern "C" {
 
 int kcl_root_features(tc_ctx* c, tc_graph* g, uint32_t k, float* X) {
+  PoolScope scope(c);
   TCX_TRY(kcl_check(c, g, k));
   if (!X) return fail(TC_ERR_ARG, "NULL output");
   if (g->n == 0) return TC_OK;
@@ -1078,6 +1079,7 @@ int kcl_root_features(tc_ctx* c, tc_graph* g, uint32_t k, float* X) {
 
 int kcl_measure_costs(tc_ctx* c, tc_graph* g, uint32_t k, int variant, float* cost_us,
                       uint64_t* count) {
+  PoolScope scope(c);
   TCX_TRY(kcl_check(c, g, k));
   if (!cost_us) return fail(TC_ERR_ARG, "NULL output");
   if (variant != KCL_VARIANT_PIVOT && variant != KCL_VARIANT_MERGE)
@@ -1107,6 +1109,7 @@ int kcl_measure_costs(tc_ctx* c, tc_graph* g, uint32_t k, int variant, float* co
 }
 
 int kcl_learned_plan(tc_ctx* c, tc_graph* g, uint32_t k, tc_model* m, uint8_t* path) {
+  PoolScope scope(c);
   TCX_TRY(kcl_check(c, g, k));
   if (!m || !path) return fail(TC_ERR_ARG, "NULL argument");
   const uint32_t n = g->n;
@@ -1119,6 +1122,7 @@ int kcl_learned_plan(tc_ctx* c, tc_graph* g, uint32_t k, tc_model* m, uint8_t* p
 
 int kcl_count_learned(tc_ctx* c, tc_graph* g, uint32_t k, tc_model* m, uint64_t* count,
                       tc_timing* timing) {
+  PoolScope scope(c);
   if (!count) return fail(TC_ERR_ARG, "NULL argument");
   if (!m) return kcl_count(c, g, k, KCL_VARIANT_AUTO, count, timing);
   TCX_TRY(kcl_check(c, g, k));
@@ -1143,6 +1147,7 @@ int kcl_count_learned(tc_ctx* c, tc_graph* g, uint32_t k, tc_model* m, uint64_t*
 
 int kcl_count(tc_ctx* c, tc_graph* g, uint32_t k, int variant, uint64_t* count,
               tc_timing* timing) {
+  PoolScope scope(c);
   if (!c || !g || !count) return fail(TC_ERR_ARG, "NULL argument");
   if (g->ctx != c) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (g->orient_mode < 0) return fail(TC_ERR_STATE, "graph must be oriented before counting");
@@ -1178,6 +1183,7 @@ int kcl_count(tc_ctx* c, tc_graph* g, uint32_t k, int variant, uint64_t* count,
 
 int kcl_count_roots(tc_ctx* c, tc_graph* g, uint32_t k, const uint32_t* roots, uint64_t nroots,
                     uint64_t* count, tc_timing* timing) {
+  PoolScope scope(c);
   TCX_TRY(kcl_check(c, g, k));
   if (!count || (nroots && !roots)) return fail(TC_ERR_ARG, "NULL argument");
   *count = 0;

@@ -244,9 +244,7 @@ __global__ void k_graph_of(uint32_t* __restrict__ who, uint64_t nt,
 
 template <class T>
 int read_back(tc_ctx* c, const void* src, T* out) {
-  TCX_HIP(hipMemcpyAsync(out, src, sizeof(T), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, out, src, sizeof(T));
 }
 
 // 16-bit ids by degree (in skewed graphs the in-degree follows it: R-MAT-21 has

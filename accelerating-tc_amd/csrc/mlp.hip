@@ -838,6 +838,7 @@ extern "C" {
 uint32_t tc_model_num_params(void) { return P; }
 
 int tc_model_create(tc_ctx* c, uint64_t seed, tc_model** out) {
+  PoolScope scope(c);
   if (!c || !out) return fail(TC_ERR_ARG, "NULL argument");
   *out = nullptr;
   TCX_HIP(hipSetDevice(c->device));
@@ -1051,6 +1052,7 @@ int tc_model_set_bw_model(tc_model* md, const tc_bw_model* bw) {
 }
 
 int tc_graph_features(tc_ctx* c, tc_graph* g, const tc_model* md, float* X) {
+  PoolScope scope(c);
   if (!c || !g || !X) return fail(TC_ERR_ARG, "NULL argument");
   if (g->ctx != c) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (g->orient_mode < 0) return fail(TC_ERR_STATE, "graph must be oriented");
@@ -1071,6 +1073,7 @@ int tc_graph_features(tc_ctx* c, tc_graph* g, const tc_model* md, float* X) {
 }
 
 int tc_graph_measure_costs(tc_ctx* c, tc_graph* g, int variant, float* cost_us, uint64_t* count) {
+  PoolScope scope(c);
   if (!c || !g || !cost_us) return fail(TC_ERR_ARG, "NULL argument");
   if (g->ctx != c) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (g->orient_mode < 0) return fail(TC_ERR_STATE, "graph must be oriented");
@@ -1157,6 +1160,7 @@ int check_graph(tc_ctx* c, tc_graph* g, tc_model* md) {
 
 int tc_graph_cell_features(tc_ctx* c, tc_graph* g, const tc_model* md, uint32_t level,
                            float* X) {
+  PoolScope scope(c);
   TCX_TRY(check_graph(c, g, nullptr));
   if (!X) return fail(TC_ERR_ARG, "NULL argument");
   if (md && md->ctx != c) return fail(TC_ERR_ARG, "model belongs to another context");
@@ -1174,6 +1178,7 @@ int tc_graph_cell_features(tc_ctx* c, tc_graph* g, const tc_model* md, uint32_t 
 
 int tc_graph_measure_cells(tc_ctx* c, tc_graph* g, int narrow, uint32_t level, uint32_t reps,
                            float* us, uint64_t* counts) {
+  PoolScope scope(c);
   TCX_TRY(check_graph(c, g, nullptr));
   if (!us) return fail(TC_ERR_ARG, "NULL argument");
   if (level > TC_CELL_MAX_LEVEL) return fail(TC_ERR_ARG, "level %u > %d", level, TC_CELL_MAX_LEVEL);
@@ -1222,6 +1227,7 @@ int tc_graph_measure_cells(tc_ctx* c, tc_graph* g, int narrow, uint32_t level, u
 }
 
 int tc_learned_cells(tc_ctx* c, tc_graph* g, tc_model* md, uint32_t* narrow_cells, float* Y) {
+  PoolScope scope(c);
   TCX_TRY(check_graph(c, g, md));
   if (!narrow_cells) return fail(TC_ERR_ARG, "NULL argument");
   float y[kCells * O] = {};
@@ -1233,6 +1239,7 @@ int tc_learned_cells(tc_ctx* c, tc_graph* g, tc_model* md, uint32_t* narrow_cell
 
 int tc_graph_orient_learned(tc_ctx* c, tc_graph* g, int mode, tc_model* md, int* chosen,
                             double* predicted_us, double* adir_cost) {
+  PoolScope scope(c);
   if (!c || !g) return fail(TC_ERR_ARG, "NULL argument");
   if (g->ctx != c) return fail(TC_ERR_ARG, "graph belongs to another context");
   if (md && md->ctx != c) return fail(TC_ERR_ARG, "model belongs to another context");
@@ -1270,6 +1277,7 @@ int tc_graph_orient_learned(tc_ctx* c, tc_graph* g, int mode, tc_model* md, int*
 }
 
 int tc_learned_assignment(tc_ctx* c, tc_graph* g, tc_model* md, uint8_t* variant) {
+  PoolScope scope(c);
   TCX_TRY(check_graph(c, g, md));
   if (!variant) return fail(TC_ERR_ARG, "NULL argument");
   const uint32_t n = g->n;
@@ -1305,6 +1313,7 @@ int tc_learned_assignment(tc_ctx* c, tc_graph* g, tc_model* md, uint8_t* variant
 }
 
 int tc_count_learned(tc_ctx* c, tc_graph* g, tc_model* md, uint64_t* count, tc_timing* timing) {
+  PoolScope scope(c);
   TCX_TRY(check_graph(c, g, md));
   if (!count) return fail(TC_ERR_ARG, "NULL argument");
   if (!md) {  // the fixed rule: AUTO's 32-bit work-list tasks

@@ -73,9 +73,7 @@ int unique_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n,
     return rocprim::unique(t, b, in, out, d_cnt, (size_t)n, rocprim::equal_to<uint64_t>(),
                            c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(n_out, d_cnt, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, n_out, d_cnt, sizeof(uint64_t));
 }
 
 int exclusive_scan_u32(tc_ctx* c, const uint32_t* in, uint32_t* out, uint64_t n) {
@@ -110,9 +108,7 @@ int max_u32(tc_ctx* c, const uint32_t* in, uint64_t n, uint32_t* result) {
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
     return rocprim::reduce(t, b, in, d, 0u, (size_t)n, rocprim::maximum<uint32_t>(), c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(result, d, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, result, d, sizeof(uint32_t));
 }
 
 int min_i32(tc_ctx* c, const int32_t* in, uint64_t n, int32_t* result) {
@@ -124,9 +120,7 @@ int min_i32(tc_ctx* c, const int32_t* in, uint64_t n, int32_t* result) {
     return rocprim::reduce(t, b, in, d, (int32_t)INT32_MAX, (size_t)n,
                            rocprim::minimum<int32_t>(), c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(result, d, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, result, d, sizeof(int32_t));
 }
 
 int sum_u64(tc_ctx* c, const uint64_t* in, uint64_t n, uint64_t* result) {
@@ -138,9 +132,7 @@ int sum_u64(tc_ctx* c, const uint64_t* in, uint64_t n, uint64_t* result) {
     return rocprim::reduce(t, b, in, d, (uint64_t)0, (size_t)n, rocprim::plus<uint64_t>(),
                            c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(result, d, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, result, d, sizeof(uint64_t));
 }
 
 int select_flagged_u32(tc_ctx* c, const uint32_t* in, const uint8_t* flags,
@@ -151,9 +143,7 @@ int select_flagged_u32(tc_ctx* c, const uint32_t* in, const uint8_t* flags,
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
     return rocprim::select(t, b, in, flags, out, d_cnt, (size_t)n, c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(n_out, d_cnt, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, n_out, d_cnt, sizeof(uint64_t));
 }
 
 int select_flagged_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags,
@@ -164,9 +154,7 @@ int select_flagged_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags,
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
     return rocprim::select(t, b, in, flags, out, d_cnt, (size_t)n, c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(n_out, d_cnt, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, n_out, d_cnt, sizeof(uint64_t));
 }
 
 int select_indices(tc_ctx* c, const uint8_t* flags, uint64_t n, uint32_t* out,
@@ -178,9 +166,7 @@ int select_indices(tc_ctx* c, const uint8_t* flags, uint64_t n, uint32_t* out,
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
     return rocprim::select(t, b, it, flags, out, d_cnt, (size_t)n, c->stream);
   }));
-  TCX_HIP(hipMemcpyAsync(n_out, d_cnt, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
-  return TC_OK;
+  return fetch(c, n_out, d_cnt, sizeof(uint64_t));
 }
 
 }  // namespace tcx
