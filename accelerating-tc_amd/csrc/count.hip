@@ -581,6 +581,13 @@ static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin);
 // and wave tasks (default thresholds) with one output per vertex.
 int per_vertex_counts(tc_ctx* c, tc_graph* g, unsigned long long* tri) {
   if (g->n == 0) return TC_OK;
+  TCX_TRY(lists16(c, g, true));
+  if (g->sc.l16.usable) {
+    TCX_TRY(c->scratch.reserve(kCurBytes16));
+    TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kCurBytes16, c->stream));
+    TCX_HIP(hipMemsetAsync(tri, 0, 8 * (size_t)g->n, c->stream));
+    return count16_vertices(c, g, c->scratch.as<uint32_t>(), tri);
+  }
   TCX_TRY(auto_schedule(c, g, 64u, 2048u));
   const SchedCache& sc = g->sc;
   const uint32_t* rp = g->rowptr.as<uint32_t>();

@@ -113,7 +113,8 @@ struct Rows16 {
   DevBuf row;                      // uint2[n]: first unit of the row, units
   DevBuf col;                      // entries, rows padded to whole units
   DevBuf se;                       // uint2[entries]: row of each work-list entry's list
-  DevBuf who;                      // uint32[tasks]: owner
+  DevBuf who;                      // uint32[tasks]: owner (its graph, in a batch)
+  DevBuf cred;                     // uint32[entries], when built for per-vertex counts
   DevBuf act;                      // uint4[tasks + 1]: entry range, owner's row
   DevBuf slice;                    // uint2[nslice + 1]: first (task, entry) of each slice
   uint64_t units = 0, entries = 0, tasks = 0;
@@ -122,6 +123,7 @@ struct Rows16 {
 struct Lists16 {
   uint64_t version = ~0ull;        // the CSR it was built (or found unsuitable) for
   bool usable = false;
+  bool credit = false;             // built for per-vertex counts too
   Rows16 hub, tail;                // entries with 16-bit ids, the others (32-bit)
 };
 
@@ -245,17 +247,21 @@ int worklists(tc_ctx* c, tc_graph* g);
 
 // ---- the 16-bit list layer (lists16.hip) -----------------------------------
 // Builds (or keeps) g's layer when its lists suit it (g->sc.l16.usable).
-int lists16(tc_ctx* c, tc_graph* g);
+// credit: for per-vertex counts too.
+int lists16(tc_ctx* c, tc_graph* g, bool credit = false);
 // Enqueues the count over a usable layer; acc: kAccBytes16 bytes, cleared;
 // sum16 adds the copied-back accumulators.
 constexpr size_t kAccBytes16 = 8 * 64 * 16;
 int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches);
 unsigned long long sum16(const unsigned long long* acc);
+// tri[u] += the triangles whose first vertex is u, over a layer built with
+// credit; cursor: kCurBytes16 bytes, cleared.
+constexpr size_t kCurBytes16 = 64 * 128;
+int count16_vertices(tc_ctx* c, tc_graph* g, uint32_t* cursor, unsigned long long* tri);
 // The same for a batch's union graph: 16-bit ids are the ids within each
 // graph (vertex v of graph gid[v], which starts at voff[gid[v]]; device
 // arrays), so every graph must have at most 65,535 vertices.  Counts go to
 // counts[graph]; cursor: kCurBytes16 bytes, cleared.
-constexpr size_t kCurBytes16 = 64 * 128;
 int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* voff);
 int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
                    unsigned long long* counts);

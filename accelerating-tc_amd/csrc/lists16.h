@@ -33,6 +33,21 @@ struct Wave16 {
   uint2 ring[kRing16];
 };
 
+// What a per-vertex count adds to the LDS of a wave: whom each list of the ring
+// and each queued entry is credited to (kEmpty: the task's owner).
+struct Credit16 {
+  uint32_t ring[kRing16];
+  uint32_t q[128];
+};
+
+// Sum over each group of four lanes (DPP quad permutations).
+__device__ inline uint32_t group_sum(uint32_t x) {
+  static_assert(kGroup16 == 4, "a group is a DPP quad");
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, false);  // lanes 1 0 3 2
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, false);  // lanes 2 3 0 1
+  return x;
+}
+
 __device__ inline void map16_set(uint32_t* map, uint32_t c) {
   if (c != kPad16) atomicOr(map + ((c & 8191u) >> 2), 1u << ((c >> 13) + 8u * (c & 3u)));
 }
@@ -91,16 +106,6 @@ __device__ inline void map32_clear4(uint32_t* map, const uint4& q) {
     if (d[i] != kEmpty) map[hash24(d[i]) >> 21] = 0u;
 }
 
-// Entries of the wave's queue from position `from` on that are in the row
-// a[lo, hi) (this lane's one).
-__device__ inline uint32_t queue32(const uint32_t* Q, uint32_t from, uint32_t n, uint32_t lane,
-                                   const uint32_t* __restrict__ a, uint32_t lo, uint32_t hi) {
-  wave_sync();
-  const uint32_t x = lane < n ? Q[from + lane] : kEmpty;
-  wave_sync();
-  return x != kEmpty && contains(a, lo, hi, x) ? 1u : 0u;
-}
-
 // Per-wave state of a 32-bit task: its row (entries of col seen as uint32)
 // and the queued entries.
 struct Probe32 {
@@ -109,10 +114,28 @@ struct Probe32 {
   uint32_t* Q;
 };
 
+// The n queued entries from position `from` on that are in the task's row
+// (this lane's one, for the owner).  CRED: those of a list that is credited
+// elsewhere are added there.
+template <bool CRED>
+__device__ inline uint32_t queue32(const Probe32& P, uint32_t from, uint32_t n, uint32_t lane,
+                                   const Credit16* C, unsigned long long* out) {
+  wave_sync();
+  const uint32_t x = lane < n ? P.Q[from + lane] : kEmpty;
+  const uint32_t to = CRED && lane < n ? C->q[from + lane] : kEmpty;
+  wave_sync();
+  if (x == kEmpty || !contains(P.a, P.lo, P.hi, x)) return 0u;
+  if (to == kEmpty) return 1u;
+  atomicAdd(out + to, 1ull);
+  return 0u;
+}
+
 // The four entries of q: those whose bit is set are queued; 64 queued ones
 // are searched at once.
+template <bool CRED>
 __device__ inline uint32_t map32_count4(const uint8_t* map, const uint4& q, Probe32& P,
-                                        uint32_t lane) {
+                                        uint32_t lane, uint32_t to, Credit16* C,
+                                        unsigned long long* out) {
   const uint32_t d[4] = {q.x, q.y, q.z, q.w};
   uint32_t b[4], t[4], c = 0;
 #pragma unroll
@@ -126,11 +149,15 @@ __device__ inline uint32_t map32_count4(const uint8_t* map, const uint4& q, Prob
                      d[i] != kEmpty;
     const uint64_t m = lanes(hit);
     if (m) {
-      if (hit) P.Q[lanes_below(m, P.qn)] = d[i];
+      if (hit) {
+        const uint32_t k = lanes_below(m, P.qn);
+        P.Q[k] = d[i];
+        if (CRED) C->q[k] = to;
+      }
       P.qn = uniform(P.qn + (uint32_t)__popcll(m));
       if (P.qn >= 64) {
         P.qn -= 64;
-        c += queue32(P.Q, P.qn, 64, lane, P.a, P.lo, P.hi);
+        c += queue32<CRED>(P, P.qn, 64, lane, C, out);
       }
     }
   }
@@ -144,10 +171,15 @@ __device__ inline uint32_t map32_count4(const uint8_t* map, const uint4& q, Prob
 // every group are in flight together.  The bounds pass through a ring in
 // LDS, 64 per refill, the next 64 already loaded (nb: this lane's of the
 // first 64).  B16: 16-bit entries (else 32-bit ones, with P).
-template <bool B16, int U>
+// CRED: the members of a list with cred[list] != kEmpty are added to
+// out[cred[list]] instead of being returned, by its group when it goes on to
+// another list.
+template <bool B16, bool CRED, int U>
 __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
                                               const uint2* __restrict__ se, uint32_t total,
-                                              uint2 nb, uint32_t lane, Wave16& W, Probe32& P) {
+                                              uint2 nb, uint32_t lane, Wave16& W, Probe32& P,
+                                              const uint32_t* __restrict__ cred, Credit16* C,
+                                              unsigned long long* out) {
   const uint8_t* map = reinterpret_cast<const uint8_t*>(W.map);
   const uint32_t j = lane & (kGroup16 - 1);
   constexpr uint64_t kLastLanes = 0x8888888888888888ull;
@@ -157,9 +189,13 @@ __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
   uint32_t cur = 0;            // next unit of this group's list
   int32_t rem = 0;             // its units left
   uint32_t cnt = 0, held = 0;  // wave-uniform: lists taken, list bounds in the ring so far
+  uint32_t tag = kEmpty, ctag = kEmpty, cacc = 0;  // CRED: list being read / counted, its members
+  uint32_t ncr = kEmpty;
+  if (CRED && lane < total) ncr = cred[lane];
   for (;;) {
     uint4 w[U];
     uint64_t busy[U];
+    uint32_t tg[U];
 #pragma unroll
     for (int s = 0; s < U; ++s) {
       // one bit per group that needs a list, at its last lane, so that every
@@ -168,8 +204,10 @@ __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
       if (m && cnt < total) {
         if (held - cnt < 64 / kGroup16 && held < total) {
           W.ring[(held + lane) & (kRing16 - 1)] = nb;
+          if (CRED) C->ring[(held + lane) & (kRing16 - 1)] = ncr;
           held = uniform(total - held < 64 ? total : held + 64);
           nb = held + lane < total ? se[held + lane] : make_uint2(0u, 0u);
+          if (CRED) ncr = held + lane < total ? cred[held + lane] : kEmpty;
           wave_sync();
           sum += acc;  // at most 64 lists since the last refill: no overflow
           acc = 0;
@@ -179,18 +217,42 @@ __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
           const uint2 b = W.ring[k & (kRing16 - 1)];
           cur = b.x;
           rem = (int32_t)b.y;
+          if (CRED) tag = C->ring[k & (kRing16 - 1)];
         }
         cnt = uniform(cnt + (uint32_t)__popcll(m));
       }
       busy[s] = lanes(rem > 0);
+      tg[s] = tag;
       w[s] = (int32_t)j < rem ? col[(uint64_t)cur + j] : make_uint4(~0u, ~0u, ~0u, ~0u);
       cur += kGroup16;
       rem -= (int32_t)kGroup16;
     }
 #pragma unroll
-    for (int s = 0; s < U; ++s)
-      if (busy[s]) acc += B16 ? map16_count8(map, w[s]) : map32_count4(map, w[s], P, lane);
+    for (int s = 0; s < U; ++s) {
+      if (!busy[s]) continue;
+      if (!B16) {
+        acc += map32_count4<CRED>(map, w[s], P, lane, tg[s], C, out);
+      } else if (!CRED) {
+        acc += map16_count8(map, w[s]);
+      } else {
+        if (lanes(tg[s] != ctag)) {
+          const uint32_t t = group_sum(cacc);
+          if (tg[s] != ctag) {
+            if (ctag == kEmpty) acc += cacc;
+            else if (j == 0 && t) atomicAdd(out + ctag, (unsigned long long)t);
+            cacc = 0;
+            ctag = tg[s];
+          }
+        }
+        cacc += map16_count8(map, w[s]);
+      }
+    }
     if (cnt >= total && lanes(rem > 0) == 0) break;
+  }
+  if (B16 && CRED) {
+    const uint32_t t = group_sum(cacc);
+    if (ctag == kEmpty) acc += cacc;
+    else if (j == 0 && t) atomicAdd(out + ctag, (unsigned long long)t);
   }
   return sum + acc;
 }
@@ -209,16 +271,18 @@ __device__ inline void map_clear(uint32_t* map, const uint4& q) {
 
 // One task: the owner's row own (first unit, units; q0: its unit `lane`) and
 // the lists se[0, total) (nb: list `lane`).
-template <bool B16, int U>
+template <bool B16, bool CRED, int U>
 __device__ inline unsigned long long task16(const uint4* __restrict__ col, uint2 own, uint4 q0,
                                             const uint2* __restrict__ se, uint32_t total, uint2 nb,
-                                            uint32_t lane, Wave16& W, uint32_t* Q) {
+                                            uint32_t lane, Wave16& W, uint32_t* Q,
+                                            const uint32_t* __restrict__ cred, Credit16* C,
+                                            unsigned long long* out) {
   map_set<B16>(W.map, q0);
   for (uint32_t k = lane + 64; k < own.y; k += 64) map_set<B16>(W.map, col[(uint64_t)own.x + k]);
   wave_sync();
   Probe32 P{reinterpret_cast<const uint32_t*>(col + own.x), 0u, 4 * own.y, 0u, Q};
-  unsigned long long c = stream16<B16, U>(col, se, total, nb, lane, W, P);
-  if (!B16 && P.qn) c += queue32(Q, 0, P.qn, lane, P.a, P.lo, P.hi);
+  unsigned long long c = stream16<B16, CRED, U>(col, se, total, nb, lane, W, P, cred, C, out);
+  if (!B16 && P.qn) c += queue32<CRED>(P, 0, P.qn, lane, C, out);
   wave_sync();
   // (a 16-bit padding entry clears the last word, whose bits all go in this
   // pass)
@@ -228,8 +292,10 @@ __device__ inline unsigned long long task16(const uint4* __restrict__ col, uint2
   return c;
 }
 
-// Where the counts of k_count16 go: one total, or one per vertex (the task's
-// owner) or per graph, by who[task].
+// Where the counts of k_count16 go: one total; one per vertex (who[task], the
+// owner, is the first vertex of the triangles on the lists of its out-edges;
+// cred[entry] names it for the lists of its in-edges); or one per graph
+// (who[task]).
 enum Out16 { kOutTotal = 0, kOutVertex = 1, kOutGraph = 2 };
 
 // Counts over the rows.  act[i] = (first and end entry of the task's work list
@@ -260,11 +326,14 @@ __global__ __launch_bounds__(TB) void k_count16(const uint4* __restrict__ col,
                                                 const uint2* __restrict__ se,
                                                 const uint4* __restrict__ act,
                                                 const uint32_t* __restrict__ who,
+                                                const uint32_t* __restrict__ cred,
                                                 const uint2* __restrict__ slice, uint32_t nslice,
                                                 uint32_t* __restrict__ cursor,
                                                 unsigned long long* __restrict__ total) {
   __shared__ Wave16 S[TB / 64];
   __shared__ uint32_t Q[TB / 64][B16 ? 1 : 128];
+  constexpr bool kCred = OUT == kOutVertex;
+  __shared__ Credit16 C[kCred ? TB / 64 : 1];
   __shared__ unsigned long long red[TB / 64];
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint4 pad = make_uint4(~0u, ~0u, ~0u, ~0u);
@@ -312,7 +381,8 @@ __global__ __launch_bounds__(TB) void k_count16(const uint4* __restrict__ col,
           graph = w;
         }
         const unsigned long long c =
-            task16<B16, U>(col, make_uint2(a.z, a.w), own, se + at, end - at, nb, lane, W, Q[wv]);
+            task16<B16, kCred, U>(col, make_uint2(a.z, a.w), own, se + at, end - at, nb, lane, W,
+                                  Q[wv], kCred ? cred + at : nullptr, C + (kCred ? wv : 0), total);
         if (OUT == kOutVertex) {
           const unsigned long long t = wave_sum(c);
           if (lane == 0 && t) atomicAdd(total + w, t);

@@ -139,6 +139,8 @@ __global__ void k_scatter16(const uint32_t* __restrict__ rp, const uint32_t* __r
   }
 }
 
+constexpr uint32_t kInEdge = 0x80000000u;  // key flag: the owner is the edge's target
+
 // Work-list key (owner << 32 | streamed) of every edge u -> v: the end with
 // the longer row (cnt entries) owns it, u on a tie; no key ((n << 32), sorted
 // last) when either row is empty, or the owner u's only entry is v itself.
@@ -151,18 +153,20 @@ __global__ void k_keys16(const uint32_t* __restrict__ esrc, const uint32_t* __re
     const uint32_t u = esrc[e], v = col[e], cu = cnt[u], cv = cnt[v];
     uint64_t k = (uint64_t)n << 32;
     if (cu && cv) {
-      if (cv > cu) k = ((uint64_t)v << 32) | u;
+      if (cv > cu) k = ((uint64_t)v << 32) | u | kInEdge;
       else if (cu > 1 || (id && id[v] == kPad16) != tail) k = ((uint64_t)u << 32) | v;
     }
     key[e] = k;
   }
 }
 
-// se[i] = row of the streamed list of sorted key i; cost[owner] += its group
+// se[i] = row of the streamed list of sorted key i; cred[i] (optional) = whom a
+// per-vertex count credits it to (lists16.h); cost[owner] += its group
 // steps, summed over each wave's runs of one owner before the atomic.
 __global__ __launch_bounds__(TB) void k_entries16(const uint64_t* __restrict__ key, uint64_t E,
                                                   const uint2* __restrict__ row,
                                                   uint2* __restrict__ se,
+                                                  uint32_t* __restrict__ cred,
                                                   unsigned long long* __restrict__ cost) {
   const uint32_t lane = threadIdx.x & 63;
   for (uint64_t b = gtid() & ~63ull; b < E; b += gstride()) {
@@ -170,8 +174,10 @@ __global__ __launch_bounds__(TB) void k_entries16(const uint64_t* __restrict__ k
     uint32_t o = 0xFFFFFFFFu, st = 0;
     if (i < E) {
       const uint64_t k = key[i];
-      const uint2 r = row[(uint32_t)k];
+      const uint32_t y = (uint32_t)k & ~kInEdge;
+      const uint2 r = row[y];
       se[i] = r;
+      if (cred) cred[i] = (uint32_t)k & kInEdge ? y : kEmpty;
       o = (uint32_t)(k >> 32);
       st = (r.y + kGroup16 - 1) / kGroup16;
     }
@@ -317,7 +323,7 @@ int place_rows(tc_ctx* c, uint32_t n, const uint32_t* cnt, uint32_t per, Rows16&
 // Work lists over the rows R (cnt entries each), grouped by owner, and
 // slices of equal work.
 int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, bool tail,
-               Rows16& R) {
+               bool credit, Rows16& R) {
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   DevBuf keys, tmp, wrp, cost, flags, work, prew;
@@ -342,13 +348,14 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
   R.nslice = 0;
   if (!kept) return TC_OK;
   TCX_TRY(R.se.reserve(8ull * kept));
+  if (credit) TCX_TRY(R.cred.reserve(4ull * kept));
   TCX_TRY(cost.reserve(8 * ((size_t)n + 1)));
   TCX_TRY(flags.reserve((size_t)n + 1));
   TCX_TRY(ids.reserve(4 * ((size_t)n + 1)));
   TCX_HIP(hipMemsetAsync(cost.p, 0, 8 * (size_t)n, c->stream));
   hipLaunchKernelGGL(k_entries16, dim3(grid_for(kept)), dim3(TB), 0, c->stream, sorted,
                      (uint64_t)kept, R.row.as<uint2>(), R.se.as<uint2>(),
-                     cost.as<unsigned long long>());
+                     credit ? R.cred.as<uint32_t>() : nullptr, cost.as<unsigned long long>());
   hipLaunchKernelGGL(k_nonempty, dim3(grid_for(n)), dim3(TB), 0, c->stream, wrp.as<uint32_t>(), n,
                      flags.as<uint8_t>());
   TCX_HIP(hipGetLastError());
@@ -384,7 +391,7 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
 // Rows, work lists and slices for the ids `id` (null: every vertex id is its
 // own 16-bit id; id_all: every vertex has one, and there is no tail).
 // L.usable is left false when too few entries have an id.
-int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, Lists16& L) {
+int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, bool credit, Lists16& L) {
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
@@ -415,24 +422,26 @@ int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, Lists16& L) {
                      pre, L.hub.row.as<uint2>(), L.hub.col.as<uint16_t>(),
                      L.tail.row.as<uint2>(), L.tail.col.as<uint32_t>());
   TCX_HIP(hipGetLastError());
-  TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), id, false, L.hub));
+  TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), id, false, credit, L.hub));
   L.tail.tasks = 0;
-  if (tail) TCX_TRY(work_lists(c, g, tcnt.as<uint32_t>(), id, true, L.tail));
+  if (tail) TCX_TRY(work_lists(c, g, tcnt.as<uint32_t>(), id, true, credit, L.tail));
   L.usable = true;
+  L.credit = credit;
   return TC_OK;
 }
 
 }  // namespace
 
-int lists16(tc_ctx* c, tc_graph* g) {
+int lists16(tc_ctx* c, tc_graph* g, bool credit) {
   Lists16& L = g->sc.l16;
-  if (L.version == g->sched_version) return TC_OK;
+  if (L.version == g->sched_version && (!L.usable || L.credit || !credit)) return TC_OK;
+  L.version = ~0ull;
   L.usable = false;
   if (g->n && g->m_or) {
     DevBuf id;
     bool some = true;
     if (g->n > kMax16) TCX_TRY(hub_ids(c, g, id, &some));
-    if (some) TCX_TRY(build(c, g, id.as<uint16_t>(), g->n <= kMax16, L));
+    if (some) TCX_TRY(build(c, g, id.as<uint16_t>(), g->n <= kMax16, credit, L));
   }
   L.version = g->sched_version;
   return TC_OK;
@@ -448,7 +457,7 @@ int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* v
     hipLaunchKernelGGL(k_local_ids, dim3(grid_for(g->n)), dim3(TB), 0, c->stream, gid, voff, g->n,
                        id.as<uint16_t>());
     TCX_HIP(hipGetLastError());
-    TCX_TRY(build(c, g, id.as<uint16_t>(), true, L));
+    TCX_TRY(build(c, g, id.as<uint16_t>(), true, false, L));
     if (L.hub.tasks)
       hipLaunchKernelGGL(k_graph_of, dim3(grid_for(L.hub.tasks)), dim3(TB), 0, c->stream,
                          L.hub.who.as<uint32_t>(), L.hub.tasks, gid);
@@ -465,7 +474,8 @@ int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
     hipLaunchKernelGGL((k_count16<true, kOutGraph, 4>),
                        dim3(std::min<uint32_t>(grid, (uint32_t)c->num_cus * 4u)), dim3(TB), 0,
                        c->stream, R.col.as<uint4>(), R.se.as<uint2>(), R.act.as<uint4>(),
-                       R.who.as<uint32_t>(), R.slice.as<uint2>(), R.nslice, cursor, counts);
+                       R.who.as<uint32_t>(), (const uint32_t*)nullptr, R.slice.as<uint2>(),
+                       R.nslice, cursor, counts);
   TCX_HIP(hipGetLastError());
   return TC_OK;
 }
@@ -479,11 +489,26 @@ int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint
     if (!R.tasks) return;
     hipLaunchKernelGGL(kernel, dim3(G), dim3(TB), 0, c->stream, R.col.as<uint4>(),
                        R.se.as<uint2>(), R.act.as<uint4>(), R.who.as<uint32_t>(),
-                       R.slice.as<uint2>(), R.nslice, cur, acc);
+                       R.cred.as<uint32_t>(), R.slice.as<uint2>(), R.nslice, cur, acc);
     ++*launches;
   };
   launch(k_count16<true, kOutTotal, 4>, L.hub, reinterpret_cast<uint32_t*>(acc + 8));
   launch(k_count16<false, kOutTotal, 4>, L.tail, reinterpret_cast<uint32_t*>(acc + 9));
+  TCX_HIP(hipGetLastError());
+  return TC_OK;
+}
+
+int count16_vertices(tc_ctx* c, tc_graph* g, uint32_t* cursor, unsigned long long* tri) {
+  const Lists16& L = g->sc.l16;
+  auto launch = [&](auto kernel, const Rows16& R, uint32_t* cur) {
+    if (R.tasks)
+      hipLaunchKernelGGL(kernel, dim3((uint32_t)c->num_cus * 4u), dim3(TB), 0, c->stream,
+                         R.col.as<uint4>(), R.se.as<uint2>(), R.act.as<uint4>(),
+                         R.who.as<uint32_t>(), R.cred.as<uint32_t>(), R.slice.as<uint2>(),
+                         R.nslice, cur, tri);
+  };
+  launch(k_count16<true, kOutVertex, 4>, L.hub, cursor);
+  launch(k_count16<false, kOutVertex, 4>, L.tail, cursor + 1);
   TCX_HIP(hipGetLastError());
   return TC_OK;
 }

@@ -84,3 +84,19 @@ def test_batch_id_border(ctx, n):
             assert b.count(sched)[0].tolist() == expect
     assert b.count_pergraph()[0].tolist() == expect
     b.close()
+
+
+@pytest.mark.parametrize("make,n", [(lambda: complete(130), 0), (lambda: rmat(12, 16, 5), 4096),
+                                    (lambda: rmat(17, 12, 6), 1 << 17)])
+def test_per_vertex(ctx, make, n):
+    """Every entry against the oracle's, before and after a plain count of the
+    same graph (which builds the layer without the credits)."""
+    s, d = make()
+    for o in (tcamd.ORIENT_ID, tcamd.ORIENT_ADIR):
+        g = ctx.graph(s, d, n).orient(o)
+        want = orc.count_per_vertex(*g.csr())
+        assert g.count().count == want.sum()
+        for _ in range(2):
+            np.testing.assert_array_equal(g.count_per_vertex(), want)
+        assert g.count().count == want.sum()
+        g.close()
