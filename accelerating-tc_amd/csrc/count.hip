@@ -32,17 +32,21 @@ __device__ inline uint32_t owner_of(const uint32_t* pre, uint32_t E, uint32_t t)
 
 // Hu/tc.cu:22-35: W(u) = (sum_{v in N+(u)} d+(v)) * (unsigned)log2(d+(u)).
 // floor(log2(d)) for d >= 1 is 31 - clz(d) exactly.
+// 16 lanes a row: a thread per row left the wide rows' gathers in series
+// (R-MAT-19 0.54 ms).
 __global__ void k_hu_work(const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
                           uint32_t n, int64_t* __restrict__ w) {
-  for (uint64_t u = gtid(); u < n; u += gstride()) {
-    uint32_t b = rp[u], e = rp[u + 1];
+  const uint32_t j = threadIdx.x & 15;
+  for (uint64_t u = gtid() >> 4; u < n; u += gstride() >> 4) {
+    const uint32_t b = rp[u], e = rp[u + 1];
     int64_t tot = 0;
-    for (uint32_t k = b; k < e; ++k) {
-      uint32_t v = col[k];
+    for (uint32_t k = b + j; k < e; k += 16) {
+      const uint32_t v = col[k];
       tot += rp[v + 1] - rp[v];
     }
-    uint32_t d = e - b;
-    w[u] = d == 0 ? 0 : tot * (int64_t)(31 - __clz(d));
+    for (int off = 8; off > 0; off >>= 1) tot += __shfl_xor(tot, off, 16);
+    const uint32_t d = e - b;
+    if (j == 0) w[u] = d == 0 ? 0 : tot * (int64_t)(31 - __clz(d));
   }
 }
 
@@ -245,157 +249,6 @@ __global__ void k_row_flags(const uint32_t* __restrict__ rp, uint32_t n, uint32_
     uint32_t d = rp[u + 1] - rp[u];
     f[u] = (d >= min_d && d <= max_d) ? 1 : 0;
   }
-}
-
-// ---- Hu: workgroup per vertex range, N+(u) slices staged in LDS ----------
-//
-// Hu/tc.cu:69-201 re-designed for wave64: the range's adjacency slice is
-// copied into LDS by all lanes (coalesced), the wedges u->v->w of the slice
-// are flattened with an LDS prefix sum so consecutive lanes read consecutive
-// w from HBM, and w is binary-searched in the LDS copy of N+(u).  A vertex
-// whose list exceeds the slice searches N+(u) in global memory instead
-// (the reference's cacheWorked == false path).
-template <int SLICE, int ROWCAP>
-struct HuLds {
-  uint32_t col[SLICE];
-  uint32_t vst[SLICE];
-  uint32_t pre[SLICE + 1];
-  uint16_t row[SLICE];
-  uint32_t rof[ROWCAP + 1];
-  uint32_t wsum[TB / 64];
-  uint32_t u2;
-};
-
-// Stage edges [ebase, ebase+E) into LDS: v, start of N+(v), wedge prefix.
-template <int SLICE, int ROWCAP>
-__device__ inline uint32_t stage_edges(HuLds<SLICE, ROWCAP>& L, const uint32_t* __restrict__ rp,
-                                       const uint32_t* __restrict__ col, uint32_t ebase, uint32_t E,
-                                       bool by_row = false) {
-  const uint32_t tid = threadIdx.x;
-  for (uint32_t e = tid; e < E; e += TB) {
-    uint32_t v = col[ebase + e];
-    uint32_t vs = rp[v];
-    L.col[e] = v;
-    L.vst[e] = vs;
-    uint32_t c = rp[v + 1] - vs;
-    if (by_row) {
-      const uint32_t r = L.row[e];
-      if (L.rof[r + 1] - L.rof[r] < 2) c = 0;
-    }
-    L.pre[e] = c;
-  }
-  __syncthreads();
-  // block exclusive scan, blocked layout: thread t owns [t*K, t*K+K)
-  constexpr int K = SLICE / TB;
-  uint32_t loc[K];
-  uint32_t sum = 0;
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    uint32_t e = tid * K + k;
-    uint32_t x = e < E ? L.pre[e] : 0;
-    loc[k] = sum;
-    sum += x;
-  }
-  // inclusive wave scan of per-thread sums
-  const uint32_t lane = tid & 63, wv = tid >> 6;
-  uint32_t inc = sum;
-  for (int off = 1; off < 64; off <<= 1) {
-    uint32_t o = __shfl_up(inc, off, 64);
-    if (lane >= (uint32_t)off) inc += o;
-  }
-  if (lane == 63) L.wsum[wv] = inc;
-  __syncthreads();
-  uint32_t wbase = 0;
-  for (uint32_t i = 0; i < wv; ++i) wbase += L.wsum[i];
-  uint32_t tbase = wbase + inc - sum;
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    uint32_t e = tid * K + k;
-    if (e < E) L.pre[e] = tbase + loc[k];
-  }
-  uint32_t total = 0;
-  for (uint32_t i = 0; i < TB / 64; ++i) total += L.wsum[i];
-  if (tid == 0) L.pre[E] = total;
-  __syncthreads();
-  return total;
-}
-
-template <int SLICE, int ROWCAP>
-__global__ __launch_bounds__(TB) void k_hu(const uint32_t* __restrict__ rp,
-                                           const uint32_t* __restrict__ col,
-                                           const int32_t* __restrict__ start, int skip_hubs,
-                                           unsigned long long* total) {
-  __shared__ HuLds<SLICE, ROWCAP> L;
-  const uint32_t tid = threadIdx.x;
-  const uint32_t ub = (uint32_t)start[blockIdx.x], ue = (uint32_t)start[blockIdx.x + 1];
-  unsigned long long cnt = 0;
-  uint32_t u = ub;
-  while (u < ue) {
-    if (tid == 0) {
-      uint32_t base = rp[u];
-      if (rp[u + 1] - base > SLICE) {
-        L.u2 = u;  // hub: its list does not fit the slice
-      } else {
-        uint32_t lo = u + 1, hi = min(ue, u + ROWCAP);
-        while (lo < hi) {
-          uint32_t mid = (lo + hi + 1) >> 1;
-          if (rp[mid] - base <= SLICE) lo = mid;
-          else hi = mid - 1;
-        }
-        L.u2 = lo;
-      }
-    }
-    __syncthreads();
-    const uint32_t u2 = L.u2;
-    if (u2 == u && skip_hubs) {
-      // scheduled by the hub kernel
-      __syncthreads();
-      u = u + 1;
-      continue;
-    }
-    if (u2 == u) {
-      // hub path: N+(u) stays in HBM/L2
-      const uint32_t ab = rp[u], du = rp[u + 1] - ab;
-      for (uint32_t k0 = 0; k0 < du; k0 += SLICE) {
-        uint32_t E = min((uint32_t)SLICE, du - k0);
-        uint32_t T = stage_edges(L, rp, col, ab + k0, E);
-        for (uint32_t t = tid; t < T; t += TB) {
-          uint32_t e = owner_of(L.pre, E, t);
-          uint32_t w = col[L.vst[e] + (t - L.pre[e])];
-          cnt += contains(col, ab, ab + du, w);
-        }
-        __syncthreads();
-      }
-      u = u + 1;
-      continue;
-    }
-    const uint32_t base = rp[u];
-    const uint32_t E = rp[u2] - base;
-    const uint32_t R = u2 - u;
-    for (uint32_t r = tid; r <= R; r += TB) L.rof[r] = rp[u + r] - base;
-    __syncthreads();
-    for (uint32_t e = tid; e < E; e += TB) {
-      uint32_t lo = 0, hi = R - 1;  // row r with rof[r] <= e < rof[r+1]
-      while (lo < hi) {
-        uint32_t mid = (lo + hi + 1) >> 1;
-        if (L.rof[mid] <= e) lo = mid;
-        else hi = mid - 1;
-      }
-      L.row[e] = (uint16_t)lo;
-    }
-    // stage_edges begins with a barrier-free pass that writes col/vst/pre,
-    // then synchronises; rows with d+(u) < 2 get no wedges.
-    uint32_t T = stage_edges(L, rp, col, base, E, true);
-    for (uint32_t t = tid; t < T; t += TB) {
-      uint32_t e = owner_of(L.pre, E, t);
-      uint32_t w = col[L.vst[e] + (t - L.pre[e])];
-      uint32_t r = L.row[e];
-      cnt += contains(L.col, L.rof[r], L.rof[r + 1], w);
-    }
-    __syncthreads();
-    u = u2;
-  }
-  flush_count(cnt, total);
 }
 
 // ---- Bisson: wave per row, bitmap of N+(u) for long rows -----------------
@@ -636,7 +489,7 @@ static int hu_schedule(tc_ctx* c, tc_graph* g, uint32_t nblocks) {
   if (sc.hu_nblocks == nblocks) return TC_OK;
   DevBuf w;
   TCX_TRY(w.reserve(8 * ((size_t)g->n + 1)));
-  hipLaunchKernelGGL(k_hu_work, dim3(grid_for(g->n)), dim3(TB), 0, c->stream,
+  hipLaunchKernelGGL(k_hu_work, dim3(grid_for(16ull * g->n)), dim3(TB), 0, c->stream,
                      g->rowptr.as<uint32_t>(), g->col.as<uint32_t>(), g->n, w.as<int64_t>());
   TCX_HIP(hipGetLastError());
   TCX_TRY(block_starts(c, g, w, nblocks, sc.hu_start));
@@ -979,13 +832,15 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   const uint32_t* rp = g->rowptr.as<uint32_t>();
   const uint32_t* col = g->col.as<uint32_t>();
   LaunchMarks lm(c);
-  bool on16 = false;  // AUTO over the 16-bit list layer
+  bool on16 = false;  // counted by the kernels of lists16.h
   // schedule (cached per graph; building one waits for the device, so the host
   // clock times it, and a cached one costs no event)
   const auto prep0 = std::chrono::steady_clock::now();
   switch (s.kernel) {
     case TC_KERNEL_HU:
       TCX_TRY(hu_schedule(c, g, s.grid_size ? s.grid_size : 30000u));  // Hu/tc.cu:7
+      TCX_TRY(hu16(c, g, g->sc.hu_start.as<int32_t>(), g->sc.hu_nblocks));
+      on16 = true;
       break;
     case TC_KERNEL_BISSON:
       TCX_TRY(rows_schedule(c, g));
@@ -1028,10 +883,10 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   if (!on16) TCX_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long), c->stream));
   switch (s.kernel) {
     case TC_KERNEL_HU: {
+      TCX_TRY(c->scratch.reserve(kAccBytes16));
+      TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kAccBytes16, c->stream));
       TCX_TRY(lm.mark());
-      hipLaunchKernelGGL((k_hu<2048, 1024>), dim3(g->sc.hu_nblocks), dim3(TB), 0, c->stream, rp,
-                         col, g->sc.hu_start.as<int32_t>(), 0, acc);
-      tm.launches = 1;
+      TCX_TRY(count_hu16(c, g, c->scratch.as<unsigned long long>(), &tm.launches));
       break;
     }
     case TC_KERNEL_BISSON: {
@@ -1237,7 +1092,7 @@ int tc_hu_workload(tc_ctx* c, tc_graph* g, int64_t* w) {
   if (g->n == 0) return TC_OK;
   DevBuf d;
   TCX_TRY(d.reserve(8 * (size_t)g->n));
-  hipLaunchKernelGGL(k_hu_work, dim3(grid_for(g->n)), dim3(TB), 0, c->stream,
+  hipLaunchKernelGGL(k_hu_work, dim3(grid_for(16ull * g->n)), dim3(TB), 0, c->stream,
                      g->rowptr.as<uint32_t>(), g->col.as<uint32_t>(), g->n, d.as<int64_t>());
   TCX_HIP(hipGetLastError());
   TCX_HIP(hipMemcpyAsync(w, d.p, 8 * (size_t)g->n, hipMemcpyDeviceToHost, c->stream));

@@ -127,6 +127,14 @@ struct Lists16 {
   Rows16 hub, tail;                // entries with 16-bit ids, the others (32-bit)
 };
 
+// Hu's method: push lists over the hub rows of a usable layer (else over
+// 32-bit rows of its own), cut by Hu's vertex partition.
+struct Hu16 {
+  uint64_t version = ~0ull;
+  uint32_t nblocks = 0;
+  Rows16 rows;
+};
+
 // Per-graph schedules, rebuilt when the oriented CSR changes.
 struct SchedCache {
   uint64_t version = ~0ull;
@@ -148,6 +156,7 @@ struct SchedCache {
   uint64_t nw_small = 0, nw_large = 0, nw_huge = 0, nw_lane = 0;
   uint64_t wl_entries = 0;         // edges kept in the work lists
   Lists16 l16;
+  Hu16 hu16;
   double wl_bytes = 0;             // bytes one count streams (see count.hip)
   bool rows_ok = false;
   DevBuf rows;                     // rows with d+ >= 2
@@ -254,6 +263,9 @@ int lists16(tc_ctx* c, tc_graph* g, bool credit = false);
 constexpr size_t kAccBytes16 = 8 * 64 * 16;
 int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches);
 unsigned long long sum16(const unsigned long long* acc);
+// Hu's method for the vertex blocks start[0 .. nblocks] (device array).
+int hu16(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks);
+int count_hu16(tc_ctx* c, tc_graph* g, unsigned long long* acc, uint32_t* launches);
 // tri[u] += the triangles whose first vertex is u, over a layer built with
 // credit; cursor: kCurBytes16 bytes, cleared.
 constexpr size_t kCurBytes16 = 64 * 128;

@@ -27,9 +27,15 @@ constexpr uint32_t kMap16Words = 2048;  // bit map: id c is bit c >> 13 of byte 
 constexpr uint32_t kGroup16 = 4;        // lanes that read one list together (64 bytes a step)
 constexpr uint32_t kRing16 = 128;       // list bounds held in LDS per wave
 
-// LDS of one wave.
+constexpr uint32_t kMap32Words = 512;   // hashed map of a 32-bit row
+
+// LDS of one wave.  The hashed map takes a quarter of the exact one's: twice
+// the waves fit, and its false hits (a row of 100 entries: 0.6 % of the
+// streamed ones) only cost a search.
+template <bool B16>
 struct Wave16 {
-  uint32_t map[kMap16Words];
+  static constexpr uint32_t kWords = B16 ? kMap16Words : kMap32Words;
+  uint32_t map[kWords];
   uint2 ring[kRing16];
 };
 
@@ -86,7 +92,7 @@ __device__ inline uint32_t map16_count8(const uint8_t* map, const uint4& q) {
   return c;
 }
 
-// The hashed map of a 32-bit row: id x sets bit (t >> 16) & 7 of byte t >> 19,
+// The hashed map of a 32-bit row: id x sets bit (t >> 18) & 7 of byte t >> 21,
 // t = x * K (24-bit factors, one full-rate multiply).
 __device__ inline uint32_t hash24(uint32_t x) { return __umul24(x, 0x9E3779u); }
 
@@ -95,7 +101,7 @@ __device__ inline void map32_set4(uint32_t* map, const uint4& q) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t t = hash24(d[i]);
-    if (d[i] != kEmpty) atomicOr(map + (t >> 21), 1u << (((t >> 16) & 7u) + 8u * ((t >> 19) & 3u)));
+    if (d[i] != kEmpty) atomicOr(map + (t >> 23), 1u << (((t >> 18) & 7u) + 8u * ((t >> 21) & 3u)));
   }
 }
 
@@ -103,7 +109,7 @@ __device__ inline void map32_clear4(uint32_t* map, const uint4& q) {
   const uint32_t d[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    if (d[i] != kEmpty) map[hash24(d[i]) >> 21] = 0u;
+    if (d[i] != kEmpty) map[hash24(d[i]) >> 23] = 0u;
 }
 
 // Per-wave state of a 32-bit task: its row (entries of col seen as uint32)
@@ -141,11 +147,11 @@ __device__ inline uint32_t map32_count4(const uint8_t* map, const uint4& q, Prob
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     t[i] = hash24(d[i]);
-    b[i] = map[t[i] >> 19];
+    b[i] = map[t[i] >> 21];
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const bool hit = __builtin_amdgcn_ubfe(b[i], __builtin_amdgcn_ubfe(t[i], 16u, 3u), 1u) != 0u &&
+    const bool hit = __builtin_amdgcn_ubfe(b[i], __builtin_amdgcn_ubfe(t[i], 18u, 3u), 1u) != 0u &&
                      d[i] != kEmpty;
     const uint64_t m = lanes(hit);
     if (m) {
@@ -177,7 +183,8 @@ __device__ inline uint32_t map32_count4(const uint8_t* map, const uint4& q, Prob
 template <bool B16, bool CRED, int U>
 __device__ inline unsigned long long stream16(const uint4* __restrict__ col,
                                               const uint2* __restrict__ se, uint32_t total,
-                                              uint2 nb, uint32_t lane, Wave16& W, Probe32& P,
+                                              uint2 nb, uint32_t lane, Wave16<B16>& W,
+                                              Probe32& P,
                                               const uint32_t* __restrict__ cred, Credit16* C,
                                               unsigned long long* out) {
   const uint8_t* map = reinterpret_cast<const uint8_t*>(W.map);
@@ -274,7 +281,7 @@ __device__ inline void map_clear(uint32_t* map, const uint4& q) {
 template <bool B16, bool CRED, int U>
 __device__ inline unsigned long long task16(const uint4* __restrict__ col, uint2 own, uint4 q0,
                                             const uint2* __restrict__ se, uint32_t total, uint2 nb,
-                                            uint32_t lane, Wave16& W, uint32_t* Q,
+                                            uint32_t lane, Wave16<B16>& W, uint32_t* Q,
                                             const uint32_t* __restrict__ cred, Credit16* C,
                                             unsigned long long* out) {
   map_set<B16>(W.map, q0);
@@ -330,15 +337,15 @@ __global__ __launch_bounds__(TB) void k_count16(const uint4* __restrict__ col,
                                                 const uint2* __restrict__ slice, uint32_t nslice,
                                                 uint32_t* __restrict__ cursor,
                                                 unsigned long long* __restrict__ total) {
-  __shared__ Wave16 S[TB / 64];
+  __shared__ Wave16<B16> S[TB / 64];
   __shared__ uint32_t Q[TB / 64][B16 ? 1 : 128];
   constexpr bool kCred = OUT == kOutVertex;
   __shared__ Credit16 C[kCred ? TB / 64 : 1];
   __shared__ unsigned long long red[TB / 64];
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint4 pad = make_uint4(~0u, ~0u, ~0u, ~0u);
-  Wave16& W = S[wv];
-  for (uint32_t i = lane; i < kMap16Words; i += 64) W.map[i] = 0;
+  Wave16<B16>& W = S[wv];
+  for (uint32_t i = lane; i < W.kWords; i += 64) W.map[i] = 0;
   wave_sync();
   unsigned long long cnt = 0;
   uint32_t graph = 0xFFFFFFFFu;

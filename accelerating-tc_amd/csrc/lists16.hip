@@ -12,14 +12,21 @@ namespace {
 using namespace dev;
 
 constexpr uint32_t kHistBins = 4096;  // degree histogram, the last bin open
-// A graph of more than 65,535 vertices takes the layer when at least this
-// share of its entries gets a 16-bit id; below it, the tail's work lists and
-// tasks cost as much as the layer saves (Barabasi-Albert, 90,000 vertices, 16
-// edges each, share 0.73: 75 us either way; ER of 100,000 vertices and 1.5 M
-// edges, share 0.7: 86 against 106 us; R-MAT graphs are at 0.88-1.0).  Smaller
-// graphs always take it: 14 against 60-120 us at 3,001 vertices, 41 against 90
-// us on ER of 65,536 vertices and 2^20 edges.
-constexpr double kMinShare = 0.7;
+// A graph of more than 65,535 vertices takes the layer when kMinShare of its
+// entries get a 16-bit id; or, where the average pushed list has kLongList
+// entries, when kMinEntries of them do and kMinStream of the entries that the
+// push lists stream (sum over edges of the target's row).  Skewed graphs stream
+// their hubs' entries most (R-MAT-24: 22 against 44 ms).  With short rows, all
+// alike, the tail's work lists and tasks cost more than the layer saves
+// (random geometric, 90,000 vertices, average list 17: 116 against 103 us;
+// Barabasi-Albert, 10^6 vertices, average list 8, by Hu's method: 680 against
+// 323 us over 32-bit rows).  Smaller graphs always take it: 14 against 60-120
+// us at 3,001 vertices, 41 against 90 us on ER of 65,536 vertices and 2^20
+// edges.
+constexpr double kMinShare = 0.85, kMinEntries = 0.4, kMinStream = 0.75;
+constexpr uint64_t kLongList = 32;
+constexpr int kU32 = 2;             // steps in flight over 32-bit rows
+constexpr uint32_t kWg32 = 8;       // workgroups a CU over 32-bit rows
 constexpr uint64_t kTaskCost = 48;  // a task's own row and map, in group steps
 
 unsigned grid_for(uint64_t n, int tb = TB) {
@@ -103,6 +110,16 @@ __global__ void k_counts16(const uint32_t* __restrict__ rp, const uint32_t* __re
     cnt[u] = c;
     if (tcnt) tcnt[u] = e - b - c;
   }
+}
+
+// *sum += the 16-bit entries that the push lists stream
+__global__ __launch_bounds__(TB) void k_streamed(const uint32_t* __restrict__ col, uint64_t m,
+                                                 const uint32_t* __restrict__ cnt,
+                                                 unsigned long long* sum) {
+  __shared__ unsigned long long red[TB / 64];
+  unsigned long long s = 0;
+  for (uint64_t e = gtid(); e < m; e += gstride()) s += cnt[col[e]];
+  flush_block(s, sum, red);
 }
 
 // The rows' class counters (n + 1 entries), per entries to a unit.
@@ -248,6 +265,63 @@ __global__ void k_graph_of(uint32_t* __restrict__ who, uint64_t nt,
   for (uint64_t i = gtid(); i < nt; i += gstride()) who[i] = gid[who[i]];
 }
 
+// The push lists of Hu's method: owner u streams the rows of its out-edges'
+// targets, in CSR order.
+__global__ void k_push16(const uint32_t* __restrict__ col, uint64_t m,
+                         const uint2* __restrict__ row, uint2* __restrict__ se) {
+  for (uint64_t e = gtid(); e < m; e += gstride()) se[e] = row[col[e]];
+}
+
+__global__ void k_push_flags(const uint32_t* __restrict__ rp, const uint2* __restrict__ row,
+                             uint32_t n, uint8_t* __restrict__ f) {
+  for (uint64_t u = gtid(); u < n; u += gstride()) f[u] = rp[u + 1] - rp[u] >= 2 && row[u].y ? 1 : 0;
+}
+
+__global__ void k_push_tasks(const uint32_t* __restrict__ ids, uint32_t nt,
+                             const uint32_t* __restrict__ rp, const uint2* __restrict__ row,
+                             uint32_t m, uint4* __restrict__ act) {
+  for (uint64_t i = gtid(); i <= nt; i += gstride()) {
+    if (i == nt) {
+      act[i] = make_uint4(m, m, 0u, 0u);
+      continue;
+    }
+    const uint32_t u = ids[i];
+    const uint2 r = row[u];
+    act[i] = make_uint4(rp[u], rp[u + 1], r.x, r.y);
+  }
+}
+
+// slice[s]: vertex block s / parts of Hu's partition, its edges cut into
+// `parts`; first task with edges beyond the cut.
+__global__ void k_hu_slices(const int32_t* __restrict__ start, uint32_t nblocks, uint32_t parts,
+                            const uint32_t* __restrict__ rp, const uint4* __restrict__ act,
+                            uint32_t nt, uint32_t m, uint2* __restrict__ slice) {
+  for (uint64_t s = gtid(); s <= (uint64_t)nblocks * parts; s += gstride()) {
+    uint32_t at = m;
+    if (s < (uint64_t)nblocks * parts) {
+      const uint32_t b = rp[start[s / parts]], e = rp[start[s / parts + 1]];
+      at = b + (uint32_t)((uint64_t)(e - b) * (s % parts) / parts);
+    }
+    uint32_t lo = 0, hi = nt;  // first task that ends beyond the cut
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (act[mid].y > at) hi = mid;
+      else lo = mid + 1;
+    }
+    slice[s] = make_uint2(lo, max(at, act[lo].x));
+  }
+}
+
+// Every entry as a 32-bit one (rows of graphs that the 16-bit ids do not suit)
+__global__ void k_scatter32(const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
+                            const uint32_t* __restrict__ esrc, uint64_t m,
+                            const uint2* __restrict__ row, uint32_t* __restrict__ out) {
+  for (uint64_t e = gtid(); e < m; e += gstride()) {
+    const uint32_t u = esrc[e];
+    out[4ull * row[u].x + ((uint32_t)e - rp[u])] = col[e];
+  }
+}
+
 template <class T>
 int read_back(tc_ctx* c, const void* src, T* out) {
   return fetch(c, out, src, sizeof(T));
@@ -257,7 +331,7 @@ int read_back(tc_ctx* c, const void* src, T* out) {
 // 0.928 of its entries among the 65,535 vertices of largest degree, 0.929 among
 // those of largest in-degree): the vertices of degree t and above for the
 // smallest t that leaves at most kMax16 of them.  *some: whether they can hold
-// kMinShare of the entries (in-degrees are at most the degrees).
+// enough of the entries (in-degrees are at most the degrees).
 int hub_ids(tc_ctx* c, tc_graph* g, DevBuf& id, bool* some) {
   const uint32_t n = g->n;
   *some = false;
@@ -282,7 +356,8 @@ int hub_ids(tc_ctx* c, tc_graph* g, DevBuf& id, bool* some) {
     sum += t == kHistBins - 1 ? h.open : (uint64_t)t * h.bin[t];
   }
   // (t == kHistBins: too many in the open bin)
-  if (t == kHistBins || (double)sum < kMinShare * (double)g->m_or) return TC_OK;
+  const double least = g->sum_in_out >= kLongList * g->m_or ? kMinEntries : kMinShare;
+  if (t == kHistBins || (double)sum < least * (double)g->m_or) return TC_OK;
   *some = true;
   DevBuf flag, pos;
   TCX_TRY(flag.reserve(4 * ((size_t)n + 1)));
@@ -384,7 +459,6 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
                      prew.as<uint64_t>(), R.act.as<uint4>(), (uint32_t)nt, R.entries, (uint32_t)ns,
                      R.slice.as<uint2>());
   TCX_HIP(hipGetLastError());
-  TCX_HIP(hipStreamSynchronize(c->stream));  // before the scratch buffers go
   return TC_OK;
 }
 
@@ -409,13 +483,24 @@ int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, bool credit, 
     TCX_TRY(exclusive_scan_u32(c, flag.as<uint32_t>(), pre_b.as<uint32_t>(), m + 1));
     pre = pre_b.as<uint32_t>();
     TCX_TRY(read_back(c, pre + m, &with_id));
-    if ((double)with_id < kMinShare * (double)m) return TC_OK;
+    const double least = g->sum_in_out >= kLongList * m ? kMinEntries : kMinShare;
+    if ((double)with_id < least * (double)m) return TC_OK;
   }
   const bool tail = with_id < m;
   TCX_TRY(cnt.reserve(4 * ((size_t)n + 1)));
   if (tail) TCX_TRY(tcnt.reserve(4 * ((size_t)n + 1)));
   hipLaunchKernelGGL(k_counts16, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp, pre, n,
                      cnt.as<uint32_t>(), tail ? tcnt.as<uint32_t>() : nullptr);
+  if ((double)with_id < kMinShare * (double)m) {
+    TCX_TRY(c->accum.reserve(64));
+    TCX_HIP(hipMemsetAsync(c->accum.p, 0, 8, c->stream));
+    hipLaunchKernelGGL(k_streamed, dim3(std::min<unsigned>(grid_for(m), c->num_cus * 8u)), dim3(TB),
+                       0, c->stream, col, m, cnt.as<uint32_t>(), c->accum.as<unsigned long long>());
+    TCX_HIP(hipGetLastError());
+    unsigned long long hub = 0;
+    TCX_TRY(read_back(c, c->accum.p, &hub));
+    if ((double)hub < kMinStream * (double)g->sum_in_out) return TC_OK;
+  }
   TCX_TRY(place_rows(c, n, cnt.as<uint32_t>(), 8, L.hub));
   if (tail) TCX_TRY(place_rows(c, n, tcnt.as<uint32_t>(), 4, L.tail));
   hipLaunchKernelGGL(k_scatter16, dim3(grid_for(m)), dim3(TB), 0, c->stream, rp, col, esrc, m, id,
@@ -483,32 +568,112 @@ int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
 int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches) {
   const Lists16& L = g->sc.l16;
   const uint32_t G = grid ? grid : (uint32_t)c->num_cus * 4u;
+  const uint32_t G32 = grid ? grid : (uint32_t)c->num_cus * kWg32;
   // the cursors ride between the accumulators, one line each
   static_assert(kCurStride16 * 4 == kAccStride16 * 8, "one line per accumulator");
-  auto launch = [&](auto kernel, const Rows16& R, uint32_t* cur) {
+  auto launch = [&](auto kernel, uint32_t G, const Rows16& R, uint32_t* cur) {
     if (!R.tasks) return;
     hipLaunchKernelGGL(kernel, dim3(G), dim3(TB), 0, c->stream, R.col.as<uint4>(),
                        R.se.as<uint2>(), R.act.as<uint4>(), R.who.as<uint32_t>(),
                        R.cred.as<uint32_t>(), R.slice.as<uint2>(), R.nslice, cur, acc);
     ++*launches;
   };
-  launch(k_count16<true, kOutTotal, 4>, L.hub, reinterpret_cast<uint32_t*>(acc + 8));
-  launch(k_count16<false, kOutTotal, 4>, L.tail, reinterpret_cast<uint32_t*>(acc + 9));
+  launch(k_count16<true, kOutTotal, 4>, G, L.hub, reinterpret_cast<uint32_t*>(acc + 8));
+  launch(k_count16<false, kOutTotal, kU32>, G32, L.tail, reinterpret_cast<uint32_t*>(acc + 9));
   TCX_HIP(hipGetLastError());
   return TC_OK;
 }
 
 int count16_vertices(tc_ctx* c, tc_graph* g, uint32_t* cursor, unsigned long long* tri) {
   const Lists16& L = g->sc.l16;
-  auto launch = [&](auto kernel, const Rows16& R, uint32_t* cur) {
+  auto launch = [&](auto kernel, uint32_t per_cu, const Rows16& R, uint32_t* cur) {
     if (R.tasks)
-      hipLaunchKernelGGL(kernel, dim3((uint32_t)c->num_cus * 4u), dim3(TB), 0, c->stream,
+      hipLaunchKernelGGL(kernel, dim3((uint32_t)c->num_cus * per_cu), dim3(TB), 0, c->stream,
                          R.col.as<uint4>(), R.se.as<uint2>(), R.act.as<uint4>(),
                          R.who.as<uint32_t>(), R.cred.as<uint32_t>(), R.slice.as<uint2>(),
                          R.nslice, cur, tri);
   };
-  launch(k_count16<true, kOutVertex, 4>, L.hub, cursor);
-  launch(k_count16<false, kOutVertex, 4>, L.tail, cursor + 1);
+  launch(k_count16<true, kOutVertex, 4>, 4u, L.hub, cursor);
+  launch(k_count16<false, kOutVertex, kU32>, kWg32, L.tail, cursor + 1);
+  TCX_HIP(hipGetLastError());
+  return TC_OK;
+}
+
+// Hu's method (Hu/tc.cu:69-201): the vertex blocks of its work model, N+(u)
+// held in LDS, every wedge u -> v -> w looked up in it.  Here N+(u) is the bit
+// map of k_count16 and a block's edges are the slices, so a block costs a wave
+// 3.5 vector instructions an entry where a workgroup spent an owner search and
+// a binary search on each wedge: R-MAT-19 11.8 -> 1.3 ms, ER of 10^6 vertices
+// and 8 * 10^6 edges (32-bit rows) 0.40 -> 0.33 ms, random geometric of 300,000
+// vertices and average degree 48 1.59 -> 0.54 ms.
+int hu16(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks) {
+  Hu16& H = g->sc.hu16;
+  TCX_TRY(lists16(c, g));
+  const bool b16 = g->sc.l16.usable;
+  const uint32_t n = g->n;
+  const uint64_t m = g->m_or;
+  const uint32_t* rp = g->rowptr.as<uint32_t>();
+  if (H.version != g->sched_version) {
+    if (!b16) {
+      DevBuf cnt;
+      TCX_TRY(cnt.reserve(4 * ((size_t)n + 1)));
+      hipLaunchKernelGGL(k_counts16, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp,
+                         (const uint32_t*)nullptr, n, cnt.as<uint32_t>(), (uint32_t*)nullptr);
+      TCX_TRY(place_rows(c, n, cnt.as<uint32_t>(), 4, H.rows));
+      hipLaunchKernelGGL(k_scatter32, dim3(grid_for(m)), dim3(TB), 0, c->stream, rp,
+                         g->col.as<uint32_t>(), g->esrc.as<uint32_t>(), m, H.rows.row.as<uint2>(),
+                         H.rows.col.as<uint32_t>());
+    }
+    const uint2* row = (b16 ? g->sc.l16.hub : H.rows).row.as<uint2>();
+    DevBuf flags, ids;
+    TCX_TRY(flags.reserve((size_t)n + 1));
+    TCX_TRY(ids.reserve(4 * ((size_t)n + 1)));
+    TCX_TRY(H.rows.se.reserve(8 * m));
+    hipLaunchKernelGGL(k_push16, dim3(grid_for(m)), dim3(TB), 0, c->stream, g->col.as<uint32_t>(),
+                       m, row, H.rows.se.as<uint2>());
+    hipLaunchKernelGGL(k_push_flags, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp, row, n,
+                       flags.as<uint8_t>());
+    TCX_TRY(select_indices(c, flags.as<uint8_t>(), n, ids.as<uint32_t>(), &H.rows.tasks));
+    TCX_TRY(H.rows.act.reserve(16 * (H.rows.tasks + 1)));
+    hipLaunchKernelGGL(k_push_tasks, dim3(grid_for(H.rows.tasks + 1)), dim3(TB), 0, c->stream,
+                       ids.as<uint32_t>(), (uint32_t)H.rows.tasks, rp, row, (uint32_t)m,
+                       H.rows.act.as<uint4>());
+    TCX_HIP(hipGetLastError());
+    H.version = g->sched_version;
+    H.nblocks = 0;
+  }
+  if (H.nblocks != nblocks) {
+    // few blocks: four waves each, as a workgroup would have
+    const uint32_t parts = nblocks < (uint32_t)c->num_cus * 32u ? 4u : 1u;
+    H.rows.nslice = nblocks * parts;
+    TCX_TRY(H.rows.slice.reserve(8 * ((size_t)H.rows.nslice + 1)));
+    hipLaunchKernelGGL(k_hu_slices, dim3(grid_for((uint64_t)H.rows.nslice + 1)), dim3(TB), 0,
+                       c->stream, start, nblocks, parts, rp, H.rows.act.as<uint4>(),
+                       (uint32_t)H.rows.tasks, (uint32_t)m, H.rows.slice.as<uint2>());
+    TCX_HIP(hipGetLastError());
+    H.nblocks = nblocks;
+  }
+  return TC_OK;
+}
+
+int count_hu16(tc_ctx* c, tc_graph* g, unsigned long long* acc, uint32_t* launches) {
+  const Lists16& L = g->sc.l16;
+  const Rows16& R = g->sc.hu16.rows;
+  auto launch = [&](auto kernel, uint32_t per_cu, const uint4* col, const Rows16& Q,
+                    uint32_t* cur) {
+    if (!Q.tasks) return;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)c->num_cus * per_cu), dim3(TB), 0, c->stream, col,
+                       Q.se.as<uint2>(), Q.act.as<uint4>(), (const uint32_t*)nullptr,
+                       (const uint32_t*)nullptr, Q.slice.as<uint2>(), Q.nslice, cur, acc);
+    ++*launches;
+  };
+  uint32_t* cur = reinterpret_cast<uint32_t*>(acc + 8);
+  if (L.usable) {
+    launch(k_count16<true, kOutTotal, 4>, 4u, L.hub.col.as<uint4>(), R, cur);
+    launch(k_count16<false, kOutTotal, kU32>, kWg32, L.tail.col.as<uint4>(), L.tail, cur + 2);
+  } else {
+    launch(k_count16<false, kOutTotal, kU32>, kWg32, R.col.as<uint4>(), R, cur);
+  }
   TCX_HIP(hipGetLastError());
   return TC_OK;
 }

@@ -41,8 +41,8 @@ HBM_PEAK_GBPS = 8000.0
 METRIC = "TC edges/s + HBM GB/s % peak; learned/batched vs plain HIP, exact counts"
 KERNELS = ["hu", "bisson", "fox", "tricore", "auto", "learned"]
 KERNEL_SYMBOL = {
-    "hu": "k_hu<2048, 1024>", "bisson": "k_bisson", "fox": "k_fox<L>",
-    "tricore": "k_tricore", "auto": "k_auto<2048>", "learned": "k_auto<2048>",
+    "hu": "k_count16", "bisson": "k_bisson", "fox": "k_fox<L>",
+    "tricore": "k_tricore", "auto": "k_count16", "learned": "k_count16",
 }
 
 WORKLOADS = {

@@ -100,3 +100,18 @@ def test_per_vertex(ctx, make, n):
             np.testing.assert_array_equal(g.count_per_vertex(), want)
         assert g.count().count == want.sum()
         g.close()
+
+
+@pytest.mark.parametrize("blocks", [1, 977, 30000])
+@pytest.mark.parametrize("make,n", [(lambda: rmat(17, 8, 3), 1 << 17),        # 16-bit rows and a tail
+                                    (lambda: tcamd.gen_er(70001, 300_007, 5), 0),  # over 65,535 ids
+                                    (lambda: tcamd.gen_er(300_001, 900_001, 5), 0),  # 32-bit rows
+                                    (lambda: complete(1030), 0)])                  # long rows, no tail
+def test_hu(ctx, make, n, blocks):
+    s, d = make()
+    for o in (tcamd.ORIENT_ID, tcamd.ORIENT_DEGREE):
+        g = ctx.graph(s, d, n).orient(o)
+        want = g.count(auto_thresholds=[64, 2048, 0, 8]).count
+        for _ in range(2):
+            assert g.count("hu", grid_size=blocks).count == want
+        g.close()
