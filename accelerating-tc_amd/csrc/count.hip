@@ -251,6 +251,20 @@ __global__ void k_row_flags(const uint32_t* __restrict__ rp, uint32_t n, uint32_
   }
 }
 
+// Bisson's and TriCore's methods run on the kernels of lists16.h where the
+// graph is large enough for a first count, which builds the lists, not to lose
+// by it: at 1.4-1.5 * 10^6 edges (random geometric, average degree 24) a first
+// count takes 0.28 (k_bisson) or 0.46 ms (k_tricore) against 0.36 or 0.53, at
+// 2 * 10^6 (ER, 300,000 vertices) 0.38 or 0.61 against 0.29 or 0.48, on R-MAT-16
+// with 9 * 10^5 edges and 9 * 10^7 wedges 1.5 or 0.40 against 0.52 or 0.42.
+// Later counts are 2 to 20 times as fast: R-MAT-18 with 3.6 * 10^6 edges 7.67 or
+// 1.82 against 0.33 or 0.15 ms.
+constexpr uint64_t kListEdges = 3u << 19, kListWedges = 1u << 26;
+
+static bool on_lists(const tc_graph* g) {
+  return g->m_or >= kListEdges || g->sum_in_out >= kListWedges;
+}
+
 // ---- Bisson: wave per row, bitmap of N+(u) for long rows -----------------
 //
 // Bisson/tc.cu:18-104 re-designed: rows with d+ > min_deg mark N+(u) in a
@@ -833,6 +847,7 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   const uint32_t* col = g->col.as<uint32_t>();
   LaunchMarks lm(c);
   bool on16 = false;  // counted by the kernels of lists16.h
+  const Lists16* lists = &g->sc.l16;
   // schedule (cached per graph; building one waits for the device, so the host
   // clock times it, and a cached one costs no event)
   const auto prep0 = std::chrono::steady_clock::now();
@@ -843,7 +858,12 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
       on16 = true;
       break;
     case TC_KERNEL_BISSON:
-      TCX_TRY(rows_schedule(c, g));
+      on16 = !s.bitmap_min_deg && on_lists(g);  // the caller's bound is k_bisson's
+      TCX_TRY(on16 ? bisson16(c, g) : rows_schedule(c, g));
+      break;
+    case TC_KERNEL_TRICORE:
+      on16 = s.tricore_parts <= 1 && on_lists(g);  // a pass of several spans two ranges
+      if (on16) TCX_TRY(lists16or32(c, g, &lists));
       break;
     case TC_KERNEL_FOX: {
       uint32_t L = s.fox_max_lanes ? s.fox_max_lanes : 64;
@@ -881,14 +901,19 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   }
   tm.ms_prep = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - prep0).count();
   if (!on16) TCX_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long), c->stream));
-  switch (s.kernel) {
-    case TC_KERNEL_HU: {
-      TCX_TRY(c->scratch.reserve(kAccBytes16));
-      TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kAccBytes16, c->stream));
-      TCX_TRY(lm.mark());
-      TCX_TRY(count_hu16(c, g, c->scratch.as<unsigned long long>(), &tm.launches));
-      break;
-    }
+  if (on16) {
+    TCX_TRY(c->scratch.reserve(kAccBytes16));
+    TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kAccBytes16, c->stream));
+    TCX_TRY(lm.mark());
+    unsigned long long* acc16 = c->scratch.as<unsigned long long>();
+    const Push16& P = g->sc.push16;
+    if (s.kernel == TC_KERNEL_HU)
+      TCX_TRY(count_push16(c, g, P.hu_slice, P.hu_nslice, 0, acc16, &tm.launches));
+    else if (s.kernel == TC_KERNEL_BISSON)
+      TCX_TRY(count_push16(c, g, P.slice, P.nslice, s.grid_size, acc16, &tm.launches));
+    else
+      TCX_TRY(count16(c, *lists, s.grid_size, acc16, &tm.launches));
+  } else switch (s.kernel) {
     case TC_KERNEL_BISSON: {
       uint32_t G = s.grid_size ? s.grid_size : (uint32_t)c->num_cus * 8u;
       uint32_t min_deg = s.bitmap_min_deg ? s.bitmap_min_deg : 64;
@@ -965,13 +990,6 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     }
     case TC_KERNEL_AUTO: {
       const SchedCache& sc = g->sc;
-      if (on16) {
-        TCX_TRY(c->scratch.reserve(kAccBytes16));
-        TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kAccBytes16, c->stream));
-        TCX_TRY(lm.mark());
-        TCX_TRY(count16(c, g, s.grid_size, c->scratch.as<unsigned long long>(), &tm.launches));
-        break;
-      }
       TCX_TRY(c->scratch.reserve(64));
       uint32_t* cursor = c->scratch.as<uint32_t>();
       TCX_HIP(hipMemsetAsync(cursor, 0, 8 * sizeof(uint32_t), c->stream));

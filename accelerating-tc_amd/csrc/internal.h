@@ -127,12 +127,15 @@ struct Lists16 {
   Rows16 hub, tail;                // entries with 16-bit ids, the others (32-bit)
 };
 
-// Hu's method: push lists over the hub rows of a usable layer (else over
-// 32-bit rows of its own), cut by Hu's vertex partition.
-struct Hu16 {
+// Push lists (a task streams the rows of all its out-neighbours) over the hub
+// rows of a usable layer, else over the rows of l32, with Hu's and Bisson's
+// slices of them.
+struct Push16 {
   uint64_t version = ~0ull;
-  uint32_t nblocks = 0;
-  Rows16 rows;
+  DevBuf se, act;                  // as in Rows16
+  uint64_t tasks = 0;
+  DevBuf hu_slice, slice;
+  uint32_t hu_blocks = 0, hu_nslice = 0, nslice = 0;
 };
 
 // Per-graph schedules, rebuilt when the oriented CSR changes.
@@ -156,7 +159,8 @@ struct SchedCache {
   uint64_t nw_small = 0, nw_large = 0, nw_huge = 0, nw_lane = 0;
   uint64_t wl_entries = 0;         // edges kept in the work lists
   Lists16 l16;
-  Hu16 hu16;
+  Lists16 l32;                     // all entries 32-bit (in tail); usable: with work lists
+  Push16 push16;
   double wl_bytes = 0;             // bytes one count streams (see count.hip)
   bool rows_ok = false;
   DevBuf rows;                     // rows with d+ >= 2
@@ -258,14 +262,20 @@ int worklists(tc_ctx* c, tc_graph* g);
 // Builds (or keeps) g's layer when its lists suit it (g->sc.l16.usable).
 // credit: for per-vertex counts too.
 int lists16(tc_ctx* c, tc_graph* g, bool credit = false);
-// Enqueues the count over a usable layer; acc: kAccBytes16 bytes, cleared;
-// sum16 adds the copied-back accumulators.
+// The layer where usable, else (l32) the same over 32-bit rows of all entries.
+int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use);
+// Enqueues the count over them; acc: kAccBytes16 bytes, cleared; sum16 adds the
+// copied-back accumulators.
 constexpr size_t kAccBytes16 = 8 * 64 * 16;
-int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches);
+int count16(tc_ctx* c, const Lists16& L, uint32_t grid, unsigned long long* acc,
+            uint32_t* launches);
 unsigned long long sum16(const unsigned long long* acc);
-// Hu's method for the vertex blocks start[0 .. nblocks] (device array).
+// Push lists with slices for Hu's vertex blocks start[0 .. nblocks] (device
+// array), or of equally many edges each (Bisson's method).
 int hu16(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks);
-int count_hu16(tc_ctx* c, tc_graph* g, unsigned long long* acc, uint32_t* launches);
+int bisson16(tc_ctx* c, tc_graph* g);
+int count_push16(tc_ctx* c, tc_graph* g, const DevBuf& slice, uint32_t nslice, uint32_t grid,
+                 unsigned long long* acc, uint32_t* launches);
 // tri[u] += the triangles whose first vertex is u, over a layer built with
 // credit; cursor: kCurBytes16 bytes, cleared.
 constexpr size_t kCurBytes16 = 64 * 128;

@@ -291,15 +291,17 @@ __global__ void k_push_tasks(const uint32_t* __restrict__ ids, uint32_t nt,
   }
 }
 
-// slice[s]: vertex block s / parts of Hu's partition, its edges cut into
-// `parts`; first task with edges beyond the cut.
-__global__ void k_hu_slices(const int32_t* __restrict__ start, uint32_t nblocks, uint32_t parts,
-                            const uint32_t* __restrict__ rp, const uint4* __restrict__ act,
-                            uint32_t nt, uint32_t m, uint2* __restrict__ slice) {
+// slice[s]: vertex block s / parts (start; null: one block of all n vertices),
+// its edges cut into `parts`; first task with edges beyond the cut.
+__global__ void k_edge_slices(const int32_t* __restrict__ start, uint32_t nblocks, uint32_t parts,
+                              uint32_t n, const uint32_t* __restrict__ rp,
+                              const uint4* __restrict__ act, uint32_t nt, uint32_t m,
+                              uint2* __restrict__ slice) {
   for (uint64_t s = gtid(); s <= (uint64_t)nblocks * parts; s += gstride()) {
     uint32_t at = m;
     if (s < (uint64_t)nblocks * parts) {
-      const uint32_t b = rp[start[s / parts]], e = rp[start[s / parts + 1]];
+      const uint32_t b = start ? rp[start[s / parts]] : 0u;
+      const uint32_t e = start ? rp[start[s / parts + 1]] : rp[n];
       at = b + (uint32_t)((uint64_t)(e - b) * (s % parts) / parts);
     }
     uint32_t lo = 0, hi = nt;  // first task that ends beyond the cut
@@ -565,8 +567,8 @@ int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
   return TC_OK;
 }
 
-int count16(tc_ctx* c, tc_graph* g, uint32_t grid, unsigned long long* acc, uint32_t* launches) {
-  const Lists16& L = g->sc.l16;
+int count16(tc_ctx* c, const Lists16& L, uint32_t grid, unsigned long long* acc,
+            uint32_t* launches) {
   const uint32_t G = grid ? grid : (uint32_t)c->num_cus * 4u;
   const uint32_t G32 = grid ? grid : (uint32_t)c->num_cus * kWg32;
   // the cursors ride between the accumulators, one line each
@@ -599,6 +601,47 @@ int count16_vertices(tc_ctx* c, tc_graph* g, uint32_t* cursor, unsigned long lon
   return TC_OK;
 }
 
+// The rows of l32: every entry a 32-bit one (graphs that the 16-bit ids do not
+// suit).  cnt: row lengths.
+static int rows32(tc_ctx* c, tc_graph* g, DevBuf& cnt) {
+  Lists16& L = g->sc.l32;
+  const uint32_t n = g->n;
+  const uint64_t m = g->m_or;
+  const uint32_t* rp = g->rowptr.as<uint32_t>();
+  TCX_TRY(cnt.reserve(4 * ((size_t)n + 1)));
+  hipLaunchKernelGGL(k_counts16, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp,
+                     (const uint32_t*)nullptr, n, cnt.as<uint32_t>(), (uint32_t*)nullptr);
+  if (L.version == g->sched_version) return TC_OK;
+  L.version = ~0ull;
+  L.usable = false;  // until the work lists are there
+  TCX_TRY(place_rows(c, n, cnt.as<uint32_t>(), 4, L.tail));
+  hipLaunchKernelGGL(k_scatter32, dim3(grid_for(m)), dim3(TB), 0, c->stream, rp,
+                     g->col.as<uint32_t>(), g->esrc.as<uint32_t>(), m, L.tail.row.as<uint2>(),
+                     L.tail.col.as<uint32_t>());
+  TCX_HIP(hipGetLastError());
+  L.version = g->sched_version;
+  return TC_OK;
+}
+
+// TriCore's rule (tricore/src/tricount_gpu.cu:215-290): every edge's shorter
+// list is looked up in its longer one.  Grouped by the owner of the longer list,
+// the edges share one bit map of it, where a wave spent six searches in sampled
+// pivots and about three in the list (one line each) on every entry: R-MAT-19
+// 4.9 -> 0.32 ms, random geometric of 300,000 vertices 2.08 -> 0.67 ms.
+int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use) {
+  TCX_TRY(lists16(c, g));
+  *use = &g->sc.l16;
+  if (g->sc.l16.usable) return TC_OK;
+  Lists16& L = g->sc.l32;
+  *use = &L;
+  if (L.version == g->sched_version && L.usable) return TC_OK;
+  DevBuf cnt;
+  TCX_TRY(rows32(c, g, cnt));
+  TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), nullptr, false, false, L.tail));
+  L.usable = true;
+  return TC_OK;
+}
+
 // Hu's method (Hu/tc.cu:69-201): the vertex blocks of its work model, N+(u)
 // held in LDS, every wedge u -> v -> w looked up in it.  Here N+(u) is the bit
 // map of k_count16 and a block's edges are the slices, so a block costs a wave
@@ -606,73 +649,99 @@ int count16_vertices(tc_ctx* c, tc_graph* g, uint32_t* cursor, unsigned long lon
 // a binary search on each wedge: R-MAT-19 11.8 -> 1.3 ms, ER of 10^6 vertices
 // and 8 * 10^6 edges (32-bit rows) 0.40 -> 0.33 ms, random geometric of 300,000
 // vertices and average degree 48 1.59 -> 0.54 ms.
-int hu16(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks) {
-  Hu16& H = g->sc.hu16;
+int push16(tc_ctx* c, tc_graph* g) {
+  Push16& H = g->sc.push16;
   TCX_TRY(lists16(c, g));
+  if (H.version == g->sched_version) return TC_OK;
   const bool b16 = g->sc.l16.usable;
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
-  if (H.version != g->sched_version) {
-    if (!b16) {
-      DevBuf cnt;
-      TCX_TRY(cnt.reserve(4 * ((size_t)n + 1)));
-      hipLaunchKernelGGL(k_counts16, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp,
-                         (const uint32_t*)nullptr, n, cnt.as<uint32_t>(), (uint32_t*)nullptr);
-      TCX_TRY(place_rows(c, n, cnt.as<uint32_t>(), 4, H.rows));
-      hipLaunchKernelGGL(k_scatter32, dim3(grid_for(m)), dim3(TB), 0, c->stream, rp,
-                         g->col.as<uint32_t>(), g->esrc.as<uint32_t>(), m, H.rows.row.as<uint2>(),
-                         H.rows.col.as<uint32_t>());
-    }
-    const uint2* row = (b16 ? g->sc.l16.hub : H.rows).row.as<uint2>();
-    DevBuf flags, ids;
-    TCX_TRY(flags.reserve((size_t)n + 1));
-    TCX_TRY(ids.reserve(4 * ((size_t)n + 1)));
-    TCX_TRY(H.rows.se.reserve(8 * m));
-    hipLaunchKernelGGL(k_push16, dim3(grid_for(m)), dim3(TB), 0, c->stream, g->col.as<uint32_t>(),
-                       m, row, H.rows.se.as<uint2>());
-    hipLaunchKernelGGL(k_push_flags, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp, row, n,
-                       flags.as<uint8_t>());
-    TCX_TRY(select_indices(c, flags.as<uint8_t>(), n, ids.as<uint32_t>(), &H.rows.tasks));
-    TCX_TRY(H.rows.act.reserve(16 * (H.rows.tasks + 1)));
-    hipLaunchKernelGGL(k_push_tasks, dim3(grid_for(H.rows.tasks + 1)), dim3(TB), 0, c->stream,
-                       ids.as<uint32_t>(), (uint32_t)H.rows.tasks, rp, row, (uint32_t)m,
-                       H.rows.act.as<uint4>());
-    TCX_HIP(hipGetLastError());
-    H.version = g->sched_version;
-    H.nblocks = 0;
-  }
-  if (H.nblocks != nblocks) {
-    // few blocks: four waves each, as a workgroup would have
-    const uint32_t parts = nblocks < (uint32_t)c->num_cus * 32u ? 4u : 1u;
-    H.rows.nslice = nblocks * parts;
-    TCX_TRY(H.rows.slice.reserve(8 * ((size_t)H.rows.nslice + 1)));
-    hipLaunchKernelGGL(k_hu_slices, dim3(grid_for((uint64_t)H.rows.nslice + 1)), dim3(TB), 0,
-                       c->stream, start, nblocks, parts, rp, H.rows.act.as<uint4>(),
-                       (uint32_t)H.rows.tasks, (uint32_t)m, H.rows.slice.as<uint2>());
-    TCX_HIP(hipGetLastError());
-    H.nblocks = nblocks;
-  }
+  DevBuf cnt, flags, ids;
+  if (!b16) TCX_TRY(rows32(c, g, cnt));
+  const uint2* row = (b16 ? g->sc.l16.hub : g->sc.l32.tail).row.as<uint2>();
+  TCX_TRY(flags.reserve((size_t)n + 1));
+  TCX_TRY(ids.reserve(4 * ((size_t)n + 1)));
+  TCX_TRY(H.se.reserve(8 * m));
+  hipLaunchKernelGGL(k_push16, dim3(grid_for(m)), dim3(TB), 0, c->stream, g->col.as<uint32_t>(),
+                     m, row, H.se.as<uint2>());
+  hipLaunchKernelGGL(k_push_flags, dim3(grid_for(n)), dim3(TB), 0, c->stream, rp, row, n,
+                     flags.as<uint8_t>());
+  TCX_TRY(select_indices(c, flags.as<uint8_t>(), n, ids.as<uint32_t>(), &H.tasks));
+  TCX_TRY(H.act.reserve(16 * (H.tasks + 1)));
+  hipLaunchKernelGGL(k_push_tasks, dim3(grid_for(H.tasks + 1)), dim3(TB), 0, c->stream,
+                     ids.as<uint32_t>(), (uint32_t)H.tasks, rp, row, (uint32_t)m,
+                     H.act.as<uint4>());
+  TCX_HIP(hipGetLastError());
+  H.version = g->sched_version;
+  H.hu_blocks = 0;
+  H.nslice = 0;
   return TC_OK;
 }
 
-int count_hu16(tc_ctx* c, tc_graph* g, unsigned long long* acc, uint32_t* launches) {
+static int edge_slices(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks,
+                       uint32_t parts, DevBuf& slice, uint32_t* nslice) {
+  const Push16& H = g->sc.push16;
+  const uint32_t ns = nblocks * parts;
+  *nslice = 0;
+  TCX_TRY(slice.reserve(8 * ((size_t)ns + 1)));
+  hipLaunchKernelGGL(k_edge_slices, dim3(grid_for((uint64_t)ns + 1)), dim3(TB), 0, c->stream, start,
+                     nblocks, parts, g->n, g->rowptr.as<uint32_t>(), H.act.as<uint4>(),
+                     (uint32_t)H.tasks, (uint32_t)g->m_or, slice.as<uint2>());
+  TCX_HIP(hipGetLastError());
+  *nslice = ns;
+  return TC_OK;
+}
+
+int hu16(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks) {
+  TCX_TRY(push16(c, g));
+  Push16& H = g->sc.push16;
+  if (H.hu_blocks == nblocks) return TC_OK;
+  H.hu_blocks = 0;
+  // few blocks: four waves each, as a workgroup would have
+  const uint32_t parts = nblocks < (uint32_t)c->num_cus * 32u ? 4u : 1u;
+  TCX_TRY(edge_slices(c, g, start, nblocks, parts, H.hu_slice, &H.hu_nslice));
+  H.hu_blocks = nblocks;
+  return TC_OK;
+}
+
+// Bisson's method (Bisson/tc.cu:18-104): a bit map of N+(u) in which the lists
+// of u's out-neighbours are looked up.  The map is k_count16's, in LDS and
+// exact, where a workgroup had n bits in memory behind a hashed filter; the
+// slices have equally many edges, 16 a wave.  R-MAT-19 19.4 -> 0.75 ms, ER of
+// 10^6 vertices 1.25 -> 0.30 ms (8 * 10^6 edges, 32-bit rows).
+int bisson16(tc_ctx* c, tc_graph* g) {
+  TCX_TRY(push16(c, g));
+  Push16& H = g->sc.push16;
+  if (H.nslice) return TC_OK;
+  return edge_slices(c, g, nullptr, 1u, (uint32_t)c->num_cus * 256u, H.slice, &H.nslice);
+}
+
+int count_push16(tc_ctx* c, tc_graph* g, const DevBuf& slice, uint32_t nslice, uint32_t grid,
+                 unsigned long long* acc, uint32_t* launches) {
   const Lists16& L = g->sc.l16;
-  const Rows16& R = g->sc.hu16.rows;
-  auto launch = [&](auto kernel, uint32_t per_cu, const uint4* col, const Rows16& Q,
+  const Push16& H = g->sc.push16;
+  auto launch = [&](auto kernel, uint32_t per_cu, const uint4* col, const uint2* se,
+                    const uint4* act, uint64_t tasks, const DevBuf& slice, uint32_t nslice,
                     uint32_t* cur) {
-    if (!Q.tasks) return;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)c->num_cus * per_cu), dim3(TB), 0, c->stream, col,
-                       Q.se.as<uint2>(), Q.act.as<uint4>(), (const uint32_t*)nullptr,
-                       (const uint32_t*)nullptr, Q.slice.as<uint2>(), Q.nslice, cur, acc);
+    if (!tasks) return;
+    hipLaunchKernelGGL(kernel, dim3(grid ? grid : (uint32_t)c->num_cus * per_cu), dim3(TB), 0,
+                       c->stream, col, se, act, (const uint32_t*)nullptr, (const uint32_t*)nullptr,
+                       slice.as<uint2>(), nslice, cur, acc);
     ++*launches;
   };
   uint32_t* cur = reinterpret_cast<uint32_t*>(acc + 8);
+  const uint2* se = H.se.as<uint2>();
+  const uint4* act = H.act.as<uint4>();
   if (L.usable) {
-    launch(k_count16<true, kOutTotal, 4>, 4u, L.hub.col.as<uint4>(), R, cur);
-    launch(k_count16<false, kOutTotal, kU32>, kWg32, L.tail.col.as<uint4>(), L.tail, cur + 2);
+    launch(k_count16<true, kOutTotal, 4>, 4u, L.hub.col.as<uint4>(), se, act, H.tasks, slice,
+           nslice, cur);
+    const Rows16& T = L.tail;
+    launch(k_count16<false, kOutTotal, kU32>, kWg32, T.col.as<uint4>(), T.se.as<uint2>(),
+           T.act.as<uint4>(), T.tasks, T.slice, T.nslice, cur + 2);
   } else {
-    launch(k_count16<false, kOutTotal, kU32>, kWg32, R.col.as<uint4>(), R, cur);
+    launch(k_count16<false, kOutTotal, kU32>, kWg32, g->sc.l32.tail.col.as<uint4>(), se, act,
+           H.tasks, slice, nslice, cur);
   }
   TCX_HIP(hipGetLastError());
   return TC_OK;

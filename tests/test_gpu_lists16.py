@@ -115,3 +115,18 @@ def test_hu(ctx, make, n, blocks):
         for _ in range(2):
             assert g.count("hu", grid_size=blocks).count == want
         g.close()
+
+
+@pytest.mark.parametrize("kernel", ["bisson", "tricore"])
+@pytest.mark.parametrize("make,n", [(lambda: rmat(17, 16, 3), 1 << 17),               # 16-bit rows, tail
+                                    (lambda: tcamd.gen_er(400_001, 1_600_003, 5), 0),  # 32-bit rows
+                                    (lambda: complete(1800), 0)])                  # no tail, long rows
+def test_bisson_and_tricore(ctx, kernel, make, n):
+    s, d = make()
+    for o in (tcamd.ORIENT_ID, tcamd.ORIENT_DEGREE):
+        g = ctx.graph(s, d, n).orient(o)
+        want = g.count(auto_thresholds=[64, 2048, 0, 8]).count
+        other = {"bisson": {"bitmap_min_deg": 64}, "tricore": {"tricore_parts": 2}}[kernel]
+        for args in ({}, {"grid_size": 3}, other):
+            assert g.count(kernel, **args).count == want
+        g.close()
