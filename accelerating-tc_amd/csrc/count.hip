@@ -775,41 +775,6 @@ using namespace tcx;
 
 namespace {
 
-// Event marks between consecutive count launches: mark() before each launch,
-// end() after the last; finish(), once the stream has been waited for, gives
-// the total and the longest launch.
-struct LaunchMarks {
-  tc_ctx* c;
-  int n = 0;
-  explicit LaunchMarks(tc_ctx* cc) : c(cc) {}
-  int mark() {
-    if (n >= 16) return TC_OK;  // later launches fold into the last interval
-    if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
-    TCX_HIP(hipEventRecord(c->lev[n], c->stream));
-    ++n;
-    return TC_OK;
-  }
-  int end() {
-    if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
-    TCX_HIP(hipEventRecord(c->lev[n], c->stream));
-    return TC_OK;
-  }
-  int finish(tc_timing* tm) {
-    tm->ms_count = 0;
-    tm->ms_dominant = 0;
-    for (int i = 0; i < n; ++i) {
-      float ms = 0;
-      TCX_HIP(hipEventElapsedTime(&ms, c->lev[i], c->lev[i + 1]));
-      tm->ms_count += ms;
-      if (ms > tm->ms_dominant) {
-        tm->ms_dominant = ms;
-        tm->dominant_kernel = (uint32_t)i;
-      }
-    }
-    return TC_OK;
-  }
-};
-
 int check_ready(tc_ctx* c, tc_graph* g) {
   if (!c || !g) return fail(TC_ERR_ARG, "NULL argument");
   if (g->ctx != c) return fail(TC_ERR_ARG, "graph belongs to another context");

@@ -179,6 +179,10 @@ struct SchedCache {
   uint64_t kcl_version = ~0ull, kcl_model = ~0ull;
   uint32_t kcl_k = 0;
   DevBuf kcl_path, kcl_key;
+  // k-clique roots, widest first, and how many have d+ > i (see kcl_order)
+  uint64_t kcl_order_version = ~0ull;
+  DevBuf kcl_order;
+  std::vector<uint32_t> kcl_wider;
   // degeneracy-oriented copy of the graph for k-clique counting when the
   // caller's orientation leaves roots wider than the LDS bit matrix
   uint64_t kcl_degen_version = ~0ull;
@@ -287,6 +291,41 @@ int count16_vertices(tc_ctx* c, tc_graph* g, uint32_t* cursor, unsigned long lon
 int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* voff);
 int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
                    unsigned long long* counts);
+
+// Event marks between consecutive count launches: mark() before each launch,
+// end() after the last; finish(), once the stream has been waited for, gives
+// the total and the longest launch.
+struct LaunchMarks {
+  tc_ctx* c;
+  int n = 0;
+  explicit LaunchMarks(tc_ctx* cc) : c(cc) {}
+  int mark() {
+    if (n >= 16) return TC_OK;  // later launches fold into the last interval
+    if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
+    TCX_HIP(hipEventRecord(c->lev[n], c->stream));
+    ++n;
+    return TC_OK;
+  }
+  int end() {
+    if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
+    TCX_HIP(hipEventRecord(c->lev[n], c->stream));
+    return TC_OK;
+  }
+  int finish(tc_timing* tm) {
+    tm->ms_count = 0;
+    tm->ms_dominant = 0;
+    for (int i = 0; i < n; ++i) {
+      float ms = 0;
+      TCX_HIP(hipEventElapsedTime(&ms, c->lev[i], c->lev[i + 1]));
+      tm->ms_count += ms;
+      if (ms > tm->ms_dominant) {
+        tm->ms_dominant = ms;
+        tm->dominant_kernel = (uint32_t)i;
+      }
+    }
+    return TC_OK;
+  }
+};
 
 // ---- cost model and per-vertex counts (mlp.hip, count.hip) ---------------
 // Predicted log2 costs Y[n][2] for device features X[n][8]; fails when the

@@ -8,6 +8,10 @@
 //  * MERGE path (any d+(u)): a wave walks the clique tree depth-first;
 //    candidate lists live in per-wave HBM scratch and each intersection is
 //    a wave-wide binary-search + ballot compaction.
+//  * PIVOT path (d+(u) <= 1024): the bit matrix in LDS, counted by pivoting.
+//  * DIRECT path (k <= 5, d+(u) <= 512; kcl_direct.h): the bit matrix in
+//    registers, common neighbours of vertex pairs in scalar registers.  The
+//    default for those k, pivoting beyond.
 // Every k-clique has a unique source in the DAG and a unique chain order,
 // so it is counted exactly once on either path.
 #include <algorithm>
@@ -22,6 +26,8 @@ namespace {
 constexpr int kMaxK = 12;
 constexpr int kKclFeatures = TC_MODEL_FEATURES;
 constexpr uint32_t kPivotMax = 1024;  // widest bit matrix in LDS (16 words per row)
+constexpr uint32_t kDirectMaxK = 5;   // largest k of the direct path
+constexpr int kDirectWords = 8;       // its widest matrix (words per row)
 constexpr int kCompactWords = 4;      // pivot matrices this wide pack C's members per pass
 
 __device__ inline uint64_t gtid() { return (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; }
@@ -55,16 +61,28 @@ __device__ inline bool contains(const uint32_t* a, uint32_t lo, uint32_t hi, uin
   return false;
 }
 
-// keys[i] = hi - d+(roots[i]): an ascending sort puts the widest roots first.
-__global__ void k_root_keys(const uint32_t* __restrict__ rp, const uint32_t* __restrict__ roots,
-                            uint64_t nr, uint32_t hi, uint32_t* __restrict__ keys) {
-  for (uint64_t i = gtid(); i < nr; i += gstride()) {
-    const uint32_t u = roots[i];
-    keys[i] = hi - (rp[u + 1] - rp[u]);
+constexpr uint32_t kOrderBins = kPivotMax + 2;  // d+ 0 .. kPivotMax, and beyond
+
+// key[u] puts the widest roots first in an ascending sort (those beyond
+// kPivotMax in id order); bin[d] counts the roots of out-degree d.
+__global__ __launch_bounds__(256) void k_root_order(const uint32_t* __restrict__ rp, uint32_t n,
+                                                    uint32_t* __restrict__ key,
+                                                    uint32_t* __restrict__ id,
+                                                    uint32_t* __restrict__ bin) {
+  __shared__ uint32_t s_bin[kOrderBins];
+  for (uint32_t i = threadIdx.x; i < kOrderBins; i += 256) s_bin[i] = 0;
+  __syncthreads();
+  for (uint64_t u = gtid(); u < n; u += gstride()) {
+    const uint32_t d = min(rp[u + 1] - rp[u], kPivotMax + 1);
+    key[u] = kPivotMax + 1 - d;
+    id[u] = (uint32_t)u;
+    atomicAdd(s_bin + d, 1u);
   }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < kOrderBins; i += 256)
+    if (s_bin[i]) atomicAdd(bin + i, s_bin[i]);
 }
 
-// f[u] = lo <= d+(u) <= hi, and (with a plan) the plan sends u to `want`
 __global__ void k_deg_flags(const uint32_t* __restrict__ rp, uint32_t n, uint32_t lo, uint32_t hi,
                             const uint8_t* __restrict__ path, uint8_t want,
                             uint8_t* __restrict__ f) {
@@ -777,6 +795,8 @@ __global__ __launch_bounds__(64 * NW) void k_kcl_pivot(const uint32_t* __restric
 }  // namespace
 }  // namespace tcx
 
+#include "kcl_direct.h"
+
 using namespace tcx;
 
 static unsigned grid_for(uint64_t n, int tb = 256) {
@@ -804,6 +824,35 @@ __global__ void k_fixed_plan(const uint32_t* __restrict__ rp, uint32_t n, uint32
     path[u] = (d >= need && d <= hi) ? want : 255;
     key[u] = 0xFFFFFFFFu - d;
   }
+}
+
+// The roots in sc.kcl_order, widest first, kept until the CSR changes.
+int kcl_order(tc_ctx* c, tc_graph* g) {
+  SchedCache& sc = g->sc;
+  if (sc.kcl_order_version == g->sched_version) return TC_OK;
+  sc.kcl_order_version = ~0ull;
+  const uint32_t n = g->n;
+  DevBuf buf, bin;
+  TCX_TRY(buf.reserve(12 * ((size_t)n + 1)));
+  TCX_TRY(sc.kcl_order.reserve(4 * ((size_t)n + 1)));
+  TCX_TRY(bin.reserve(4 * kOrderBins));
+  uint32_t* key = buf.as<uint32_t>();
+  uint32_t *ktmp = key + n + 1, *vtmp = ktmp + n + 1;
+  TCX_HIP(hipMemsetAsync(bin.p, 0, 4 * kOrderBins, c->stream));
+  hipLaunchKernelGGL(k_root_order, dim3(std::min(grid_for(n), (unsigned)c->num_cus * 4u)),
+                     dim3(256), 0, c->stream, g->rowptr.as<uint32_t>(), n, key,
+                     sc.kcl_order.as<uint32_t>(), bin.as<uint32_t>());
+  TCX_HIP(hipGetLastError());
+  uint32_t *sk = nullptr, *sv = nullptr;
+  TCX_TRY(sort_pairs_u32_u32(c, key, ktmp, sc.kcl_order.as<uint32_t>(), vtmp, n, 11, &sk, &sv));
+  if (sv != sc.kcl_order.as<uint32_t>())
+    TCX_HIP(hipMemcpyAsync(sc.kcl_order.p, sv, 4ull * n, hipMemcpyDeviceToDevice, c->stream));
+  uint32_t h[kOrderBins];
+  TCX_TRY(fetch(c, h, bin.p, sizeof(h)));
+  sc.kcl_wider.assign(kOrderBins, 0);
+  for (uint32_t i = kOrderBins - 1; i > 0; --i) sc.kcl_wider[i - 1] = sc.kcl_wider[i] + h[i];
+  sc.kcl_order_version = g->sched_version;
+  return TC_OK;
 }
 
 // Counts k-cliques over the roots with d+ >= k-1 (k >= 3, m+ > 0).  plan
@@ -847,39 +896,49 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
   }
   DevBuf flags, roots, scratch, sortbuf, claimbuf;
   const float us_per_tick = 1000.f / (float)c->wall_clock_khz;
-  TCX_TRY(flags.reserve((size_t)g->n + 1));
-  TCX_TRY(roots.reserve(4 * ((size_t)g->n + 1)));
-  TCX_TRY(claimbuf.reserve(64));
-  TCX_TRY(c->accum.reserve(64));
-  unsigned long long* acc = c->accum.as<unsigned long long>();
-  TCX_HIP(hipMemsetAsync(acc, 0, 8, c->stream));
-  float total_ms = 0;
+  // the default variant's k <= 5 take the direct path up to kDirectWords
+  const bool direct = k <= kDirectMaxK && (plan || variant == KCL_VARIANT_AUTO);
+  // a bucket's roots are a range of the kept order, unless a plan selects them
+  const bool ordered = !plan && (variant == KCL_VARIANT_AUTO || variant == KCL_VARIANT_PIVOT);
+  if (ordered) {
+    TCX_TRY(kcl_order(c, g));
+  } else {
+    TCX_TRY(flags.reserve((size_t)g->n + 1));
+    TCX_TRY(roots.reserve(4 * ((size_t)g->n + 1)));
+  }
+  // the count, a claim counter per bucket and, for the direct path, its groups'
+  constexpr size_t kClaimBytes = 4 * kClaimGroups * kClaimStride;
+  const size_t claim_bytes = 128 + (direct ? 4 * kClaimBytes : 0);
+  TCX_TRY(claimbuf.reserve(claim_bytes));
+  unsigned long long* acc = claimbuf.as<unsigned long long>();
+  TCX_HIP(hipMemsetAsync(acc, 0, claim_bytes, c->stream));
+  uint32_t* groups = reinterpret_cast<uint32_t*>(acc + 16);
+  LaunchMarks lm(c);
+  int widths[17];
   for (const Bucket& b : buckets) {
     uint32_t lo = std::max(b.lo, need);
     if (lo > b.hi) continue;
-    const uint8_t* path = plan ? plan->path : nullptr;
-    const uint8_t want = b.w == 0 ? 1 : 0;
-    hipLaunchKernelGGL(k_deg_flags, dim3(grid_for(g->n)), dim3(256), 0, c->stream, rp, g->n, lo,
-                       b.hi, path, want, flags.as<uint8_t>());
-    TCX_HIP(hipGetLastError());
     uint64_t nr = 0;
-    TCX_TRY(select_indices(c, flags.as<uint8_t>(), g->n, roots.as<uint32_t>(), &nr));
-    if (nr == 0) continue;
-    // each launch takes its roots in the plan's order, or (pivot launches
-    // without a plan) widest first; sorted before the timed region
-    const uint32_t* order = roots.as<uint32_t>();
-    if (!plan && b.pivot) {
-      TCX_TRY(sortbuf.reserve(12 * (nr + 1)));
-      uint32_t* keys = sortbuf.as<uint32_t>();
-      uint32_t* ktmp = keys + nr + 1;
-      uint32_t* vtmp = ktmp + nr + 1;
-      hipLaunchKernelGGL(k_root_keys, dim3(grid_for(nr)), dim3(256), 0, c->stream, rp,
-                         roots.as<uint32_t>(), nr, b.hi, keys);
+    const uint32_t* order = nullptr;
+    if (ordered) {
+      // roots with lo <= d+ <= hi: those wider than lo - 1 but not than hi
+      const std::vector<uint32_t>& wider = g->sc.kcl_wider;
+      const uint32_t past = b.hi < kOrderBins - 1 ? wider[b.hi] : 0u;
+      nr = (lo - 1 < kOrderBins - 1 ? wider[lo - 1] : 0u) - past;
+      if (nr == 0) continue;
+      order = g->sc.kcl_order.as<uint32_t>() + past;
+    } else {
+      const uint8_t* path = plan ? plan->path : nullptr;
+      const uint8_t want = b.w == 0 ? 1 : 0;
+      hipLaunchKernelGGL(k_deg_flags, dim3(grid_for(g->n)), dim3(256), 0, c->stream, rp, g->n, lo,
+                         b.hi, path, want, flags.as<uint8_t>());
       TCX_HIP(hipGetLastError());
-      uint32_t *sk = nullptr, *sv = nullptr;
-      TCX_TRY(sort_pairs_u32_u32(c, keys, ktmp, roots.as<uint32_t>(), vtmp, nr, 11, &sk, &sv));
-      order = sv;
-    } else if (plan) {
+      TCX_TRY(select_indices(c, flags.as<uint8_t>(), g->n, roots.as<uint32_t>(), &nr));
+      if (nr == 0) continue;
+      order = roots.as<uint32_t>();
+    }
+    if (plan) {
+      // each launch takes its roots in the plan's order
       TCX_TRY(sortbuf.reserve(12 * (nr + 1)));
       uint32_t* keys = sortbuf.as<uint32_t>();
       uint32_t* ktmp = keys + nr + 1;
@@ -891,15 +950,38 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       TCX_TRY(sort_pairs_u32_u32(c, keys, ktmp, roots.as<uint32_t>(), vtmp, nr, 32, &sk, &sv));
       order = sv;
     }
-    TCX_HIP(hipEventRecord(c->ev0, c->stream));
+    unsigned long long* claim = acc + 1 + tm.launches;
+    widths[lm.n] = b.w;
     if (b.w == 0) {
       uint32_t G = (uint32_t)std::min<uint64_t>(nr, (uint64_t)c->num_cus * 8);
       uint32_t maxd = std::max<uint32_t>(g->max_out, 1);
       uint32_t slots = k > 3 ? k - 3 : 1;
       TCX_TRY(scratch.reserve(4ull * G * slots * maxd));
+      TCX_TRY(lm.mark());
       // cost: CU-microseconds (one wave of the num_cus * 8 holds 1/8 of a CU)
       hipLaunchKernelGGL(k_kcl_merge, dim3(G), dim3(64), 0, c->stream, rp, col, order, nr, k,
                          maxd, slots, scratch.as<uint32_t>(), acc, cost, us_per_tick / 8.f);
+    } else if (b.pivot && direct && b.w <= kDirectWords) {
+      // workgroups of b.w waves: 32 waves a CU, 16 with 8-word rows (registers)
+      const uint64_t per_cu = b.w == 8 ? 2 : 32 / b.w, slots = (uint64_t)c->num_cus * per_cu;
+      // k = 5 repeats the wider roots where they leave workgroups idle; building
+      // the matrix again costs more next to counting in a 4-word one (R-MAT-16:
+      // 1,955 roots, 2,048 slots, 1.68 against 1.79 ms with two copies; 439
+      // roots of 8 words, 512 slots, 1.44 against 1.33)
+      uint32_t copies = 1;
+      while (k == 5 && b.w > 1 && copies < 8 && nr * copies * (b.w == 8 ? 1 : 2) < slots) copies *= 2;
+      const uint32_t G = (uint32_t)std::min<uint64_t>(nr * copies, slots);
+      const uint32_t chunk =
+          (uint32_t)std::min<uint64_t>(8 / b.w, (nr * copies + slots - 1) / slots);
+      const float cs = us_per_tick / (float)per_cu;
+      TCX_TRY(lm.mark());
+      switch (b.w) {
+        case 1: hipLaunchKernelGGL((k_kcl_direct<1, 1>), dim3(G), dim3(64), 0, c->stream, rp, col, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
+        case 2: hipLaunchKernelGGL((k_kcl_direct<2, 2>), dim3(G), dim3(128), 0, c->stream, rp, col, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
+        case 4: hipLaunchKernelGGL((k_kcl_direct<4, 4>), dim3(G), dim3(256), 0, c->stream, rp, col, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
+        default: hipLaunchKernelGGL((k_kcl_direct<8, 8>), dim3(G), dim3(512), 0, c->stream, rp, col, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
+      }
+      groups += kClaimBytes / 4;
     } else if (b.pivot) {
       // workgroups resident per CU (LDS- and register-bound for the wide
       // matrices); the wide ones run 8 or 16 walkers per root, and a root
@@ -914,11 +996,10 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       const uint64_t D = 64ull * b.w;
       TCX_TRY(scratch.reserve(8ull * G * nw * (D + 1) * (2ull * b.w + 1)));
       uint64_t* stk = scratch.as<uint64_t>();
-      const uint32_t* rts = order;  // widest first (stable: ties in id order)
+      const uint32_t* rts = order;
       // cost: CU-microseconds (a workgroup holds 1/per_cu of a CU)
       const float cs = us_per_tick / (float)per_cu;
-      unsigned long long* claim = claimbuf.as<unsigned long long>();
-      TCX_HIP(hipMemsetAsync(claim, 0, 8, c->stream));
+      TCX_TRY(lm.mark());
       // narrow roots are cheap: claim several per atomic
       const uint32_t chunk = b.w == 1 ? 16 : (b.w == 2 ? 8 : (b.w == 4 ? 4 : 1));
       switch (b.w) {
@@ -930,6 +1011,7 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       }
     } else {
       uint32_t G = (uint32_t)std::min<uint64_t>(nr, (uint64_t)c->num_cus * 16);
+      TCX_TRY(lm.mark());
       switch (b.w) {
         case 1: hipLaunchKernelGGL(k_kcl_bitmap<1>, dim3(G), dim3(64), 0, c->stream, rp, col, roots.as<uint32_t>(), nr, k, acc); break;
         case 2: hipLaunchKernelGGL(k_kcl_bitmap<2>, dim3(G), dim3(64), 0, c->stream, rp, col, roots.as<uint32_t>(), nr, k, acc); break;
@@ -938,22 +1020,14 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       }
     }
     TCX_HIP(hipGetLastError());
-    TCX_HIP(hipEventRecord(c->ev1, c->stream));
-    TCX_HIP(hipEventSynchronize(c->ev1));
-    float ms = 0;
-    TCX_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    total_ms += ms;
-    if (ms > tm.ms_dominant) {
-      tm.ms_dominant = ms;
-      tm.dominant_kernel = (uint32_t)b.w;
-    }
     tm.launches++;
   }
+  TCX_TRY(lm.end());
   unsigned long long h = 0;
-  TCX_HIP(hipMemcpyAsync(&h, acc, 8, hipMemcpyDeviceToHost, c->stream));
-  TCX_HIP(hipStreamSynchronize(c->stream));
+  TCX_TRY(fetch(c, &h, acc, 8));
+  TCX_TRY(lm.finish(&tm));
+  if (lm.n) tm.dominant_kernel = (uint32_t)widths[tm.dominant_kernel];
   *count = h;
-  tm.ms_count = total_ms;
   if (timing) *timing = tm;
   return TC_OK;
 }

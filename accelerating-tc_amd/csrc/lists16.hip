@@ -646,9 +646,9 @@ int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use) {
 // held in LDS, every wedge u -> v -> w looked up in it.  Here N+(u) is the bit
 // map of k_count16 and a block's edges are the slices, so a block costs a wave
 // 3.5 vector instructions an entry where a workgroup spent an owner search and
-// a binary search on each wedge: R-MAT-19 11.8 -> 1.3 ms, ER of 10^6 vertices
-// and 8 * 10^6 edges (32-bit rows) 0.40 -> 0.33 ms, random geometric of 300,000
-// vertices and average degree 48 1.59 -> 0.54 ms.
+// a binary search on each wedge: R-MAT-19 11.8 -> 0.98 ms, ER of 10^6 vertices
+// and 8 * 10^6 edges (32-bit rows) 0.40 -> 0.31 ms, random geometric of 300,000
+// vertices and average degree 48 1.59 -> 0.53 ms.
 int push16(tc_ctx* c, tc_graph* g) {
   Push16& H = g->sc.push16;
   TCX_TRY(lists16(c, g));
@@ -698,8 +698,13 @@ int hu16(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks) {
   Push16& H = g->sc.push16;
   if (H.hu_blocks == nblocks) return TC_OK;
   H.hu_blocks = 0;
-  // few blocks: four waves each, as a workgroup would have
-  const uint32_t parts = nblocks < (uint32_t)c->num_cus * 32u ? 4u : 1u;
+  // few blocks: four waves each, as a workgroup would have; two where a block
+  // has some 200 edges (R-MAT-19: 258 of them, 0.98 against 1.27 ms with one
+  // and 0.86 with four, which costs ER, 65,536 vertices, 35 of them, 101
+  // against 51 us)
+  const uint32_t parts = nblocks < (uint32_t)c->num_cus * 32u ? 4u
+                         : g->m_or >= 200ull * nblocks        ? 2u
+                                                              : 1u;
   TCX_TRY(edge_slices(c, g, start, nblocks, parts, H.hu_slice, &H.hu_nslice));
   H.hu_blocks = nblocks;
   return TC_OK;
