@@ -72,11 +72,8 @@ int raw_counts(tc_ctx* c, tc_graph* g, RawCounts& rc) {
   hipLaunchKernelGGL(k_zero, dim3(grid_for(5ull * nodes)), dim3(256), 0, c->stream, deg,
                      5ull * nodes);
   if (m) {
-    const unsigned G = (unsigned)std::min<uint64_t>(grid_for(m), (uint64_t)c->num_cus * 4u);
-    hipLaunchKernelGGL(dev::k_count_ids<8192>, dim3(G), dim3(256), 0, c->stream, s, d, m, nodes,
-                       deg);
-    hipLaunchKernelGGL(dev::k_count_ids<8192>, dim3(G), dim3(256), 0, c->stream, s,
-                       (const uint32_t*)nullptr, m, nodes, lp);
+    TCX_TRY(count_ids(c, s, d, m, nodes, deg));
+    TCX_TRY(count_ids(c, s, nullptr, m, nodes, lp));
     hipLaunchKernelGGL(k_rule_counts, dim3(grid_for(m)), dim3(256), 0, c->stream, s, d, m, deg,
                        idb, degb, rtd);
   }

@@ -671,17 +671,6 @@ int csr_launch(tc_ctx* c, const uint64_t* keys, uint64_t m, uint32_t n, uint32_t
   return TC_OK;
 }
 
-// h[x] += occurrences of x in a[0, m) (and b[0, m) when b is not null); h
-// must be zeroed.
-int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint32_t n,
-              uint32_t* h) {
-  if (m == 0) return TC_OK;
-  const unsigned G = (unsigned)std::min<uint64_t>(grid_for(m), (uint64_t)c->num_cus * 4u);
-  hipLaunchKernelGGL(dev::k_count_ids<8192>, dim3(G), dim3(256), 0, c->stream, a, b, m, n, h);
-  TCX_HIP(hipGetLastError());
-  return TC_OK;
-}
-
 int read_u32(tc_ctx* c, const uint32_t* dptr, uint32_t* out) {
   return fetch(c, out, dptr, sizeof(uint32_t));
 }

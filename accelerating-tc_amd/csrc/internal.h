@@ -246,6 +246,15 @@ int select_indices(tc_ctx* c, const uint8_t* flags, uint64_t n, uint32_t* out,
 int select_flagged_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags,
                        uint64_t* out, uint64_t n, uint64_t* n_out);
 
+// ---- passes over long arrays (passes.hip) ----------------------------------
+// h[x] += occurrences of x < n in a[0, m) (and b[0, m) when b is not null).
+int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint32_t n,
+              uint32_t* h);
+// The keys with flags[i] set, or (flags null) the first of each run of equal
+// keys, in order; out must not be in.
+int compact_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags, uint64_t n, uint64_t* out,
+                uint64_t* n_out);
+
 // ---- graph helpers (graph.hip) -------------------------------------------
 int build_csr_from_keys(tc_ctx* c, tc_graph* g, uint64_t* keys, uint64_t nkeys,
                         int end_bit);
