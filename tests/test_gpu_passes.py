@@ -1,6 +1,6 @@
-"""The binned id histogram and the two-pass key compaction: degree and
-A-direction orientations of inputs around the sizes where they take over and
-where the bins end, against the oracle."""
+"""The binned id histogram, the two-pass key compaction and the peel's small
+levels: orientations of inputs around the sizes where they take over and where
+the bins end, against the oracle."""
 import numpy as np
 import pytest
 
@@ -37,3 +37,31 @@ def test_skewed(ctx):
     s, d = rmat(17, 16, 5)
     check(ctx, s, d, "degree", tcamd.ORIENT_DEGREE)
     check(ctx, s, d, "adir", tcamd.ORIENT_ADIR)
+
+
+def path(n):
+    v = np.arange(n - 1, dtype=np.uint32)
+    return v, v + 1
+
+
+def star(leaves, hubs=1):
+    """Leaves on hubs that form a clique: one level takes all leaves."""
+    u, v = np.triu_indices(hubs + 4, 1)
+    leaf = np.arange(leaves) + hubs + 4
+    return (np.concatenate([u, leaf]).astype(np.uint32),
+            np.concatenate([v, np.arange(leaves) % hubs]).astype(np.uint32))
+
+
+def ring_of(n, reach):
+    """Every vertex joined to the next `reach`: whole levels of one row length."""
+    u = np.repeat(np.arange(n), reach)
+    return u.astype(np.uint32), ((u + np.tile(np.arange(1, reach + 1), n)) % n).astype(np.uint32)
+
+
+@pytest.mark.parametrize("make", [lambda: path(2), lambda: path(5001), lambda: star(1023), lambda: star(1024),
+                                  lambda: star(1025), lambda: star(3000, 40), lambda: star(20000, 3),
+                                  lambda: ring_of(1024, 4), lambda: ring_of(1023, 5), lambda: rmat(10, 12, 3)])
+def test_small_levels(ctx, make):
+    s, d = make()
+    for mode, o in (("adir", tcamd.ORIENT_ADIR), ("kcore", tcamd.ORIENT_KCORE)):
+        check(ctx, s, d, mode, o)
