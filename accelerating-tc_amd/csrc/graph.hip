@@ -50,8 +50,9 @@ __global__ void k_low_degree_flag(const uint32_t* deg, uint32_t n, uint32_t* fla
 __global__ void k_orient_keys(const uint32_t* __restrict__ s, const uint32_t* __restrict__ d,
                               uint64_t m, const uint32_t* __restrict__ deg, int mode,
                               const uint32_t* __restrict__ pruned_before, uint32_t n_out,
-                              const uint32_t* __restrict__ tie, uint64_t* __restrict__ keys) {
-  const uint64_t sentinel = (uint64_t)n_out << 32;
+                              const uint32_t* __restrict__ tie, int shift,
+                              uint64_t* __restrict__ keys) {
+  const uint64_t sentinel = (uint64_t)n_out << shift;
   for (uint64_t i = gtid(); i < m; i += gstride()) {
     uint32_t a = s[i], b = d[i];
     bool swap;
@@ -71,9 +72,9 @@ __global__ void k_orient_keys(const uint32_t* __restrict__ s, const uint32_t* __
       key = sentinel;
     } else if (pruned_before) {
       if (deg[os] <= 1 || deg[od] <= 1) key = sentinel;  // Hu/preTC.cu:151-160
-      else key = ((uint64_t)(os - pruned_before[os]) << 32) | (od - pruned_before[od]);
+      else key = ((uint64_t)(os - pruned_before[os]) << shift) | (od - pruned_before[od]);
     } else {
-      key = ((uint64_t)os << 32) | od;
+      key = ((uint64_t)os << shift) | od;
     }
     keys[i] = key;
   }
@@ -91,15 +92,15 @@ __global__ void k_simple_keys(const uint32_t* __restrict__ s, const uint32_t* __
 
 // Both directions of every non-loop record (A-direction-seri.cpp:215-221).
 __global__ void k_sym_keys(const uint32_t* __restrict__ s, const uint32_t* __restrict__ d,
-                           uint64_t m, uint32_t n, uint64_t* __restrict__ keys) {
+                           uint64_t m, uint32_t n, int shift, uint64_t* __restrict__ keys) {
   for (uint64_t i = gtid(); i < m; i += gstride()) {
     uint32_t a = s[i], b = d[i];
     if (a == b) {
-      keys[2 * i] = (uint64_t)n << 32;
-      keys[2 * i + 1] = (uint64_t)n << 32;
+      keys[2 * i] = (uint64_t)n << shift;
+      keys[2 * i + 1] = (uint64_t)n << shift;
     } else {
-      keys[2 * i] = ((uint64_t)a << 32) | b;
-      keys[2 * i + 1] = ((uint64_t)b << 32) | a;
+      keys[2 * i] = ((uint64_t)a << shift) | b;
+      keys[2 * i + 1] = ((uint64_t)b << shift) | a;
     }
   }
 }
@@ -133,22 +134,29 @@ __device__ inline unsigned long long wave_sum_u64(unsigned long long v) {
 }
 
 // acc[0] += sum d+^2, acc[1] += sum d- d+ (d+ of every entry's target),
-// acc[2] = max d+.  A few hundred workgroups with one atomic each per figure:
-// an atomic per wave on the same three words serialised at about 14 ns
-// (n = 2^21: 1.16 ms).
-__global__ __launch_bounds__(256) void k_csr_stats(const uint32_t* __restrict__ rowptr,
-                                                   const uint32_t* __restrict__ col, uint32_t n,
-                                                   uint64_t m, unsigned long long* acc) {
-  __shared__ unsigned long long red[3][4];
+// acc[2] = max d+.  One workgroup a CU with one atomic per figure: atomics on
+// three words of a line serialise at about 14 ns, and were all of the time with
+// one per wave (n = 2^21: 1.16 ms) or eight workgroups a CU (n = 2^18, 3.8 * 10^6
+// entries: 84 us).
+constexpr uint32_t kStatThreads = 1024, kStatWaves = kStatThreads / 64;
+
+__global__ __launch_bounds__(kStatThreads) void k_csr_stats(const uint32_t* __restrict__ rowptr,
+                                                            const uint32_t* __restrict__ col,
+                                                            uint32_t n, uint64_t m,
+                                                            unsigned long long* acc) {
+  __shared__ unsigned long long red[3][kStatWaves];
   unsigned long long s1 = 0, s2 = 0, mx = 0;
   for (uint64_t v = gtid(); v < n; v += gstride()) {
     const uint64_t d = rowptr[v + 1] - rowptr[v];
     s1 += d * d;
     mx = d > mx ? d : mx;
   }
-  for (uint64_t e = gtid(); e < m; e += gstride()) {
-    const uint32_t v = col[e];
-    s2 += rowptr[v + 1] - rowptr[v];
+  for (uint64_t e0 = gtid(); e0 < m; e0 += 4 * gstride()) {
+    uint32_t v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = e0 + i * gstride() < m ? col[e0 + i * gstride()] : dev::kEmpty;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s2 += v[i] != dev::kEmpty ? rowptr[v[i] + 1] - rowptr[v[i]] : 0u;
   }
   s1 = wave_sum_u64(s1);
   s2 = wave_sum_u64(s2);
@@ -163,9 +171,14 @@ __global__ __launch_bounds__(256) void k_csr_stats(const uint32_t* __restrict__ 
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    atomicAdd(acc + 0, red[0][0] + red[0][1] + red[0][2] + red[0][3]);
-    atomicAdd(acc + 1, red[1][0] + red[1][1] + red[1][2] + red[1][3]);
-    atomicMax(acc + 2, max(max(red[2][0], red[2][1]), max(red[2][2], red[2][3])));
+    for (uint32_t w = 1; w < kStatWaves; ++w) {
+      s1 += red[0][w];
+      s2 += red[1][w];
+      mx = max(mx, red[2][w]);
+    }
+    atomicAdd(acc + 0, s1);
+    atomicAdd(acc + 1, s2);
+    atomicMax(acc + 2, mx);
   }
 }
 
@@ -803,18 +816,26 @@ int peel_small(tc_ctx* c, uint32_t*& F, uint32_t*& N, uint32_t& fs, const uint32
 
 }  // namespace
 
+// Keys a << shift | b of ids up to n (the sentinel's source) that unique_u64 turns
+// into a << 32 | b: without the unused bits between, sorting takes two passes
+// fewer at n = 2^18 (37 us each for 4.2 * 10^6 keys) and one at 2^21 (0.36 ms, 6.7 *
+// 10^7 keys).
+static int key_shift(uint64_t nkeys, uint32_t n) {
+  return nkeys >= kMinCompact ? std::max(1, (int)bit_width_u32(n)) : 32;
+}
+
 // Sort keys (in `keys`, scratch of the same size in `tmp`), drop duplicates
 // and the sentinel, build the graph's oriented CSR.
 static int csr_from_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint64_t nkeys,
-                         uint32_t n_out, bool already_sorted_unique) {
+                         uint32_t n_out, bool already_sorted_unique, int shift = 32) {
   uint64_t* sorted = keys.as<uint64_t>();
   uint64_t nuniq = nkeys;
   uint64_t* uniq = sorted;
   if (!already_sorted_unique) {
-    int end_bit = 32 + bit_width_u32(n_out);
+    int end_bit = shift + bit_width_u32(n_out);
     TCX_TRY(sort_u64(c, keys.as<uint64_t>(), tmp.as<uint64_t>(), nkeys, end_bit, &sorted));
     uint64_t* other = sorted == keys.as<uint64_t>() ? tmp.as<uint64_t>() : keys.as<uint64_t>();
-    TCX_TRY(unique_u64(c, sorted, other, nkeys, &nuniq));
+    TCX_TRY(unique_u64(c, sorted, other, nkeys, &nuniq, shift));
     uniq = other;
     if (nuniq > 0) {
       uint64_t last = 0;
@@ -841,10 +862,11 @@ int compute_csr_stats(tc_ctx* c, tc_graph* g) {
   TCX_TRY(c->accum.reserve(64));
   unsigned long long* acc = c->accum.as<unsigned long long>();
   TCX_HIP(hipMemsetAsync(acc, 0, 3 * sizeof(unsigned long long), c->stream));
+  const uint64_t blocks = (std::max<uint64_t>(g->n, g->m_or) + kStatThreads - 1) / kStatThreads;
   hipLaunchKernelGGL(k_csr_stats,
-                     dim3(std::min<unsigned>(grid_for(std::max<uint64_t>(g->n, g->m_or)),
-                                             (unsigned)c->num_cus * 8u)),
-                     dim3(TB), 0, c->stream, g->rowptr.as<uint32_t>(), g->col.as<uint32_t>(), g->n,
+                     dim3((unsigned)std::min<uint64_t>(std::max<uint64_t>(blocks, 1),
+                                                       (uint64_t)c->num_cus)),
+                     dim3(kStatThreads), 0, c->stream, g->rowptr.as<uint32_t>(), g->col.as<uint32_t>(), g->n,
                      g->m_or, acc);
   TCX_HIP(hipGetLastError());
   unsigned long long h[3];
@@ -859,18 +881,19 @@ int compute_csr_stats(tc_ctx* c, tc_graph* g) {
 static int sym_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint64_t** out,
                     uint64_t* m2) {
   uint64_t nk = 2 * g->m_raw;
+  const int shift = key_shift(nk, g->n_raw);
   TCX_TRY(keys.reserve(8 * std::max<uint64_t>(nk, 1)));
   TCX_TRY(tmp.reserve(8 * std::max<uint64_t>(nk, 1)));
   hipLaunchKernelGGL(k_sym_keys, dim3(grid_for(g->m_raw)), dim3(TB), 0, c->stream,
-                     g->src.as<uint32_t>(), g->dst.as<uint32_t>(), g->m_raw, g->n_raw,
+                     g->src.as<uint32_t>(), g->dst.as<uint32_t>(), g->m_raw, g->n_raw, shift,
                      keys.as<uint64_t>());
   TCX_HIP(hipGetLastError());
   uint64_t* sorted;
   TCX_TRY(sort_u64(c, keys.as<uint64_t>(), tmp.as<uint64_t>(), nk,
-                   32 + bit_width_u32(g->n_raw), &sorted));
+                   shift + bit_width_u32(g->n_raw), &sorted));
   uint64_t* other = sorted == keys.as<uint64_t>() ? tmp.as<uint64_t>() : keys.as<uint64_t>();
   uint64_t nu = 0;
-  TCX_TRY(unique_u64(c, sorted, other, nk, &nu));
+  TCX_TRY(unique_u64(c, sorted, other, nk, &nu, shift));
   if (nu > 0) {
     uint64_t last = 0;
     TCX_TRY(fetch(c, &last, other + nu - 1, 8));
@@ -1498,9 +1521,9 @@ static int orient_impl(tc_ctx* c, tc_graph* g, int mode, uint32_t flags, int tie
     hipLaunchKernelGGL(k_orient_keys, dim3(grid_for(m)), dim3(TB), 0, c->stream,
                        g->src.as<uint32_t>(), g->dst.as<uint32_t>(), m, deg.as<uint32_t>(), mode,
                        pruned_before, n_out, tie != TC_TIE_ID ? tkey.as<uint32_t>() : nullptr,
-                       keys.as<uint64_t>());
+                       key_shift(m, n_out), keys.as<uint64_t>());
     TCX_HIP(hipGetLastError());
-    TCX_TRY(csr_from_keys(c, g, keys, tmp, m, n_out, false));
+    TCX_TRY(csr_from_keys(c, g, keys, tmp, m, n_out, false, key_shift(m, n_out)));
     g->orient_mode = mode;
     if (mode != TC_ORIENT_ID && n_out == n) {  // the raw degrees stay with the graph
       swap(g->vdeg, deg);

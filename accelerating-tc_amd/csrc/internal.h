@@ -231,8 +231,9 @@ int sort_pairs_u64_u32(tc_ctx* c, uint64_t* keys, uint64_t* ktmp, uint32_t* vals
 int sort_pairs_u32_u32(tc_ctx* c, uint32_t* keys, uint32_t* ktmp, uint32_t* vals,
                        uint32_t* vtmp, uint64_t n, int end_bit, uint32_t** skeys,
                        uint32_t** svals);
+// (shift: as for compact_u64; 32 below kMinCompact keys)
 int unique_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n,
-               uint64_t* n_out);
+               uint64_t* n_out, int shift = 32);
 int exclusive_scan_u32(tc_ctx* c, const uint32_t* in, uint32_t* out, uint64_t n);
 int exclusive_scan_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n);
 int inclusive_scan_i64(tc_ctx* c, const int64_t* in, int64_t* out, uint64_t n);
@@ -251,9 +252,13 @@ int select_flagged_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags,
 int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint32_t n,
               uint32_t* h);
 // The keys with flags[i] set, or (flags null) the first of each run of equal
-// keys, in order; out must not be in.
+// keys, in order; out must not be in.  Keys a << shift | b come out as
+// a << 32 | b.
 int compact_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags, uint64_t n, uint64_t* out,
-                uint64_t* n_out);
+                uint64_t* n_out, int shift = 32);
+// Keys from which on compact_u64 takes over from the single pass (two more
+// launches, so small inputs keep it).
+constexpr uint64_t kMinCompact = 1u << 20;
 
 // ---- graph helpers (graph.hip) -------------------------------------------
 int build_csr_from_keys(tc_ctx* c, tc_graph* g, uint64_t* keys, uint64_t nkeys,

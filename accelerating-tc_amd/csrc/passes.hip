@@ -84,26 +84,27 @@ __global__ __launch_bounds__(kTileThreads) void k_bin_ids(const uint32_t* __rest
   for (uint32_t i = tid; i <= nb; i += kTileThreads) b[i] = (uint16_t)off[i];  // <= 8192
 }
 
-// Workgroup (bin, s): part[s][ids of the bin].  A wave takes 64 tiles' borders
-// at a time and keeps four tiles' ids in flight.
+// Workgroup (bin, s): part[s][ids of the bin].  A wave takes the borders of
+// `per` (a multiple of 4, at most 64) tiles at a time and keeps four tiles' ids
+// in flight.
 __global__ __launch_bounds__(1024) void k_bin_hist(const uint16_t* __restrict__ ids,
                                                    const uint16_t* __restrict__ border,
                                                    uint32_t ntile, uint32_t nb, uint32_t S,
-                                                   uint32_t* __restrict__ part) {
+                                                   uint32_t per, uint32_t* __restrict__ part) {
   __shared__ uint32_t hist[kBinIds];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const uint32_t bin = blockIdx.x % nb, s = blockIdx.x / nb;
   for (uint32_t i = tid; i < kBinIds; i += 1024) hist[i] = 0;
   __syncthreads();
-  // tiles s + S * j, j = wv * 64 + lane, and on by 16 waves
-  for (uint64_t j0 = (uint64_t)wv * 64; s + S * j0 < ntile; j0 += 16 * 64) {
+  // tiles s + S * j, j = wv * per + lane, and on by 16 waves
+  for (uint64_t j0 = (uint64_t)wv * per; s + S * j0 < ntile; j0 += 16 * per) {
     const uint64_t t = s + S * (j0 + lane);
     uint32_t lo = 0, hi = 0;
-    if (t < ntile) {
+    if (lane < per && t < ntile) {
       lo = border[t * (nb + 1) + bin];
       hi = border[t * (nb + 1) + bin + 1];
     }
-    for (uint32_t q = 0; q < 64; q += 4) {
+    for (uint32_t q = 0; q < per; q += 4) {
       uint32_t l[4], h[4], v[4];
       const uint16_t* p[4];
 #pragma unroll
@@ -170,7 +171,8 @@ __global__ __launch_bounds__(TB) void k_keep_count(const uint64_t* __restrict__ 
 __global__ __launch_bounds__(TB) void k_keep_write(const uint64_t* __restrict__ key,
                                                    const uint8_t* __restrict__ flags, uint64_t n,
                                                    uint64_t nw, const uint64_t* __restrict__ at,
-                                                   uint64_t* __restrict__ out) {
+                                                   uint32_t shift, uint64_t* __restrict__ out) {
+  const uint64_t low = (1ull << shift) - 1;
   const uint32_t lane = threadIdx.x & 63;
   for (uint64_t w = gtid() >> 6; w < nw; w += gstride() >> 6) {
     uint64_t to = at[w];
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(TB) void k_keep_write(const uint64_t* __restrict__ 
       const uint64_t k = i < n ? key[i] : 0;
       const bool take = i < n && kept(key, flags, i, k);
       const uint64_t mask = dev::lanes(take);
-      if (take) out[to + dev::lanes_below(mask, 0u)] = k;
+      if (take) out[to + dev::lanes_below(mask, 0u)] = (k >> shift) << 32 | (k & low);
       to += (uint32_t)__popcll(mask);
     }
   }
@@ -206,8 +208,11 @@ int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint3
       hipLaunchKernelGGL(k_bin_ids, dim3((unsigned)tiles), dim3(kTileThreads), 0, c->stream,
                          i ? b : a, m, n, bits, nb, bin.as<uint16_t>() + i * tiles * kTileIds,
                          border.as<uint16_t>() + i * tiles * (nb + 1));
+    // tiles a wave of a workgroup has
+    const uint32_t share = (uint32_t)((nt / S + 16) / 16);
     hipLaunchKernelGGL(k_bin_hist, dim3(nb * S), dim3(1024), 0, c->stream, bin.as<uint16_t>(),
-                       border.as<uint16_t>(), (uint32_t)nt, nb, S, part.as<uint32_t>());
+                       border.as<uint16_t>(), (uint32_t)nt, nb, S,
+                       std::min<uint32_t>(64, (share + 3) / 4 * 4), part.as<uint32_t>());
     hipLaunchKernelGGL(k_bin_sum, dim3(grid_for(1ull << bits)), dim3(TB), 0, c->stream,
                        part.as<uint32_t>(), bits, S, n, h);
     TCX_HIP(hipGetLastError());
@@ -220,7 +225,7 @@ int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint3
 }
 
 int compact_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags, uint64_t n, uint64_t* out,
-                uint64_t* n_out) {
+                uint64_t* n_out, int shift) {
   const uint64_t nw = (n + kWaveKeys - 1) / kWaveKeys;
   DevBuf cnt, at;
   TCX_TRY(cnt.reserve(8 * (nw + 1)));
@@ -230,7 +235,7 @@ int compact_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags, uint64_t n,
   TCX_HIP(hipGetLastError());
   TCX_TRY(exclusive_scan_u64(c, cnt.as<uint64_t>(), at.as<uint64_t>(), nw + 1));
   hipLaunchKernelGGL(k_keep_write, dim3(grid_for(64 * nw)), dim3(TB), 0, c->stream, in, flags, n,
-                     nw, at.as<uint64_t>(), out);
+                     nw, at.as<uint64_t>(), (uint32_t)shift, out);
   TCX_HIP(hipGetLastError());
   return fetch(c, n_out, at.as<uint64_t>() + nw, 8);
 }

@@ -9,10 +9,6 @@
 namespace tcx {
 
 namespace {
-// Keys from which on compact_u64 takes over (two more launches, so small inputs
-// keep the single pass).
-constexpr uint64_t kMinCompact = 1u << 20;
-
 template <class F>
 int run_prim(tc_ctx* c, F&& f) {
   size_t bytes = 0;
@@ -69,9 +65,9 @@ int sort_pairs_u32_u32(tc_ctx* c, uint32_t* keys, uint32_t* ktmp, uint32_t* vals
 }
 
 int unique_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n,
-               uint64_t* n_out) {
+               uint64_t* n_out, int shift) {
   if (n == 0) { *n_out = 0; return TC_OK; }
-  if (n >= kMinCompact) return compact_u64(c, in, nullptr, n, out, n_out);
+  if (n >= kMinCompact) return compact_u64(c, in, nullptr, n, out, n_out, shift);
   TCX_TRY(c->prim_out.reserve(64));
   uint64_t* d_cnt = c->prim_out.as<uint64_t>();
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {

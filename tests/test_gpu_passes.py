@@ -65,3 +65,15 @@ def test_small_levels(ctx, make):
     s, d = make()
     for mode, o in (("adir", tcamd.ORIENT_ADIR), ("kcore", tcamd.ORIENT_KCORE)):
         check(ctx, s, d, mode, o)
+
+
+@pytest.mark.parametrize("n,m", [(300_000, (1 << 20) - 1), (300_000, 1 << 20), (1_500_000, 1 << 20)])
+def test_pruned(ctx, n, m):
+    # keys over fewer rows than ids, packed from 2^20 records on
+    s, d = tcamd.gen_er(n, m, 11)
+    g = ctx.graph(s, d).orient(tcamd.ORIENT_DEGREE)
+    want = g.count().count
+    g.orient(tcamd.ORIENT_DEGREE, prune_deg1=True)
+    assert g.info().n < n
+    assert g.count().count == want
+    g.close()
