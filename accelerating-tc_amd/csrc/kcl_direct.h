@@ -10,15 +10,19 @@
 // scalar registers (v_readlane, s_and); one v_and and one v_bcnt per 32 bits add
 // up the edges inside A, with A itself as the execution mask.  No LDS and no
 // divergence in the inner loop; words below y are left out at compile time.
+// For k = 5 the out-neighbours are numbered by ascending degree: most pairs then
+// have their y, and their few words, at the end (4-word rows: 2.7 words a pair
+// against 4.0 in the order of ids; R-MAT-16 3.9 -> 3.2 ms in all).
 // One-word rows (d+ <= 64) would leave most lanes idle and run at the scalar
 // unit's rate; there a lane takes an edge of the sub-graph, from a list
 // written while the matrix is built (k = 5, random geometric, 250,000 vertices,
 // degree 48: 0.52 against 1.23 ms; k = 4: 0.39 against 0.47).
 //
 // Measured with the pivot kernels before, R-MAT-16 of 1.7 * 10^6 edges, k = 5:
-// 8 words 4.4 -> 1.34 ms, 4 words 12.2 -> 1.60, 2 words 5.5 -> 0.62, 1 word 3.5 ->
-// 0.26; k = 4: 7.3 -> 0.85 ms in all.  Vector-ALU issue is 80 % busy in the 4-word
-// kernel (26 * 10^6 pairs, 10^9 instructions), a third of it building the matrix.
+// 8 words 4.4 -> 1.07 ms, 4 words 12.2 -> 1.30, 2 words 5.5 -> 0.53, 1 word 3.5 ->
+// 0.26; k = 4: 7.3 -> 0.85 ms in all.  Vector-ALU issue was 80 % busy in the 4-word
+// kernel with the order of ids (26 * 10^6 pairs, 10^9 instructions, a third of
+// them building the matrix).
 #pragma once
 
 #include "internal.h"
@@ -137,10 +141,11 @@ template <int W, int NW>
 __global__ __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : W == 4 ? 6 : 8))) void k_kcl_direct(
     const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
-    const uint32_t* __restrict__ roots, uint64_t nroots, uint32_t copies, uint32_t chunk,
-    uint32_t k, unsigned long long* total, uint32_t* claim, float* __restrict__ cost,
+    const uint32_t* __restrict__ deg, const uint32_t* __restrict__ roots, uint64_t nroots,
+    uint32_t copies, uint32_t chunk, uint32_t k, unsigned long long* total, uint32_t* claim, float* __restrict__ cost,
     float cost_scale) {
   constexpr uint32_t D = 64 * W, T = 64 * NW;
+  constexpr bool kPairs = W == 1;
   constexpr uint32_t kG = 8;  // lanes that read one out-list together
   constexpr uint32_t kU = 4;  // entries a lane takes of it at once
   constexpr uint64_t kLast = 0x8080808080808080ull;  // the groups' last lanes
@@ -149,12 +154,15 @@ __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : W == 4 ? 6 : 8))) void k_kcl_dir
   __shared__ uint2 s_be[D];
   __shared__ __align__(16) uint64_t s_M[D * W];  // bit (a, b), a < b
   __shared__ uint64_t s_C0[NW][W];
+  // wider rows: the place of each out-neighbour in ascending order of degree
+  __shared__ __align__(16) uint32_t s_key[kPairs ? 4 : D];
+  __shared__ uint16_t s_pos[kPairs ? 1 : D];
   __shared__ uint32_t s_ti;
   // one-word rows: the edges a | b << 8 of the sub-graph, each the work of a lane
-  constexpr bool kPairs = W == 1;
   __shared__ uint16_t s_pair[kPairs ? 64 * 63 / 2 : 1];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = uniform32(tid >> 6);
   const uint32_t Q = copies * NW;
+  const bool by_degree = !kPairs && k == 5;
   const uint64_t ntask = nroots * copies;
   unsigned long long cnt = 0;
   const uint32_t ng = min(kClaimGroups, gridDim.x), cq = blockIdx.x % ng;
@@ -190,10 +198,23 @@ __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : W == 4 ? 6 : 8))) void k_kcl_dir
         }
         s_list[i] = x;
         s_be[i] = be;
+        if (by_degree) s_key[i] = i < d ? min(deg[x], (1u << 22) - 1) << 10 | i : 0xFFFFFFFFu;
       }
       for (uint32_t i = tid; i < D * W / 2; i += T)
         reinterpret_cast<uint4*>(s_M)[i] = make_uint4(0u, 0u, 0u, 0u);
       __syncthreads();
+      if (by_degree) {
+        for (uint32_t i = tid; i < d; i += T) {
+          const uint32_t key = s_key[i];
+          uint32_t r = 0;
+          for (uint32_t j = 0; j < d; j += 4) {
+            const uint4 o = *reinterpret_cast<const uint4*>(s_key + j);
+            r += (o.x < key) + (o.y < key) + (o.z < key) + (o.w < key);
+          }
+          s_pos[i] = (uint16_t)r;
+        }
+        __syncthreads();
+      }
       if (kPairs) {
         px = 0xFFFFFFFFu;
         pbe = make_uint2(0u, 0u);
@@ -257,7 +278,12 @@ __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : W == 4 ? 6 : 8))) void k_kcl_dir
 #pragma unroll
           for (uint32_t s = 0; s < kU; ++s) {
             const bool hit = x[s] != 0xFFFFFFFFu && s_list[lo[s]] == x[s];
-            const uint32_t a = min(xi, lo[s]), b = max(xi, lo[s]);
+            uint32_t pa = xi, pb = lo[s];
+            if (by_degree && hit) {
+              pa = s_pos[pa];
+              pb = s_pos[pb];
+            }
+            const uint32_t a = min(pa, pb), b = max(pa, pb);
             if (hit)
               atomicOr(reinterpret_cast<uint32_t*>(s_M) + 2 * W * a + (b >> 5), 1u << (b & 31));
             if (kPairs) {
