@@ -41,9 +41,12 @@ HBM_PEAK_GBPS = 8000.0
 METRIC = "TC edges/s + HBM GB/s % peak; learned/batched vs plain HIP, exact counts"
 KERNELS = ["hu", "bisson", "fox", "tricore", "auto", "learned"]
 KERNEL_SYMBOL = {
-    "hu": "k_count16", "bisson": "k_bisson", "fox": "k_fox<L>",
-    "tricore": "k_tricore", "auto": "k_count16", "learned": "k_count16",
+    "hu": "k_count16", "bisson": "k_count16", "fox": "k_fox<L>",
+    "tricore": "k_count16", "auto": "k_count16", "learned": "k_count16",
 }
+# Bytes per streamed list entry of the head kernel: 2 where the graph is counted
+# over 16-bit rows (k_count16), 4 over the 32-bit work lists (k_auto_wl).
+ENTRY_BYTES = {"ba24": 4}
 
 WORKLOADS = {
     "rmat22": dict(kind="rmat", scale=22, ef=16, seed=22, aorder=True, orient="adir"),
@@ -234,6 +237,10 @@ def run_batched(args, w, steps, warmup, with_cpu):
     sched = b.autotune()
     t_tune = time.perf_counter() - t0
     stream = b.stream_bytes(sched.form)  # the bytes of the chosen form
+    # k_count16 counts batches of graphs of at most 65,535 vertices: 2 bytes an entry
+    on16 = max(max(int(g[0].max()), int(g[1].max())) for g in graphs if len(g[0])) < 65535
+    if on16:
+        stream /= 2
     log(f"[bench] autotune {sched.as_dict()} in {t_tune:.1f}s; the chosen form streams "
         f"{stream/1e9:.2f} GB")
 
@@ -263,7 +270,7 @@ def run_batched(args, w, steps, warmup, with_cpu):
         log(f"[bench] cpu baseline {cpu['value']:.3e} edges/s ({cpu['sample']})")
     b.close()
     ctx.close()
-    return dict(info=info, m=m, graphs=len(graphs), counts=cb, sched=sched.as_dict(), stream=stream,
+    return dict(info=info, m=m, graphs=len(graphs), counts=cb, on16=on16, sched=sched.as_dict(), stream=stream,
                 wall_b=wall_b, ev_b=ev_b, wall_p=wall_p, ev_p=ev_p, launches_p=launches_p,
                 cpu=cpu, t_gen=t_gen, t_prep=t_prep, t_tune=t_tune)
 
@@ -277,7 +284,7 @@ def batched_desc(w):
 def main_batched(args, w):
     r = run_batched(args, w, args.steps, args.warmup, not args.no_cpu)
     info, m = r["info"], r["m"]
-    kb = r["stream"]  # the bytes k_batch streams under the chosen form
+    kb = r["stream"]  # the bytes streamed under the chosen form
     achieved = kb / (r["ev_b"] * 1e-3) / 1e9
     line = {
         "metric": METRIC,
@@ -295,10 +302,10 @@ def main_batched(args, w):
         "roofline": {
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBPS, "traffic": load_traffic("batched", "batched"),
-            "kernel": "k_batch<2048>", "bytes_per_count": kb,
+            "kernel": "k_count16" if r["on16"] else "k_batch<2048>", "bytes_per_count": kb,
             "bytes_rule": "work-list form: tc_batch_stream_bytes (per task 20 + 4 d+(x), per "
                           "work-list entry 8 + 4 d+(y)); push form: 4(n+1) + 12 m+ + "
-                          "4 sum d- d+",
+                          "4 sum d- d+; half of it over 16-bit rows",
             "bytes_push_form": kernel_bytes(info),
             "bytes_alg_edge_model": info.bytes_alg,
         },
@@ -473,7 +480,7 @@ def valu_peak():
 
 
 def kclique_roofline(workload, per_k):
-    """The pivot kernels are bound by VALU issue, not HBM: the wave
+    """The k-clique kernels are bound by VALU issue, not HBM: the wave
     instructions a count issues (SQ_INSTS_VALU summed over the launch's
     kernels, profiles/valu_<workload>.json) over its hipEvent time, against
     the issue peak.  The largest k with a profile is reported."""
@@ -490,7 +497,7 @@ def kclique_roofline(workload, per_k):
     achieved = insts[str(k)] / (per_k[k]["ms_kernels"] * 1e-3)
     return {"bound": "valu", "achieved": achieved, "peak": peak,
             "unit": "wave-instructions/s", "frac": achieved / peak, "peak_source": source,
-            "traffic": None, "kernel": "k_kcl_pivot (all widths)", "k": k,
+            "traffic": None, "kernel": "k_kcl_direct, k_kcl_pivot<16, 16>", "k": k,
             "valu_insts_per_count": insts[str(k)]}
 
 
@@ -578,20 +585,27 @@ def run_triangles(args, w, kernels, with_cpu):
     g.close()
     ctx.close()
     return dict(info=info, m=m, head=head, results=results, cpu=cpu, cpu_par=cpu_par,
-                t_gen=t_gen, t_prep=t_prep, stream=stream)
+                t_gen=t_gen, t_prep=t_prep, stream=stream,
+                entry_bytes=ENTRY_BYTES.get(name_of(w), 2))
 
 
-def triangle_roofline(info, hr, traffic, stream):
-    """The head kernel (k_auto_wl, AUTO and the learned schedule) streams the
-    work-list bytes of tc_auto_stream_bytes whatever variant runs each task."""
+def name_of(w):
+    return next(k for k, v in WORKLOADS.items() if v is w)
+
+
+def triangle_roofline(info, hr, traffic, stream, entry_bytes):
+    """The head kernel (AUTO and the learned schedule) streams its work lists:
+    tc_auto_stream_bytes counts them at 4 bytes an entry, k_count16 reads 2."""
+    stream = stream * entry_bytes / 4
     achieved = stream / (hr["ms_kernels"] * 1e-3) / 1e9
     return {
         "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-        "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic, "kernel": "k_auto_wl<2048>",
+        "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic, "kernel": "k_count16" if entry_bytes == 2 else "k_auto_wl<2048>",
         "bytes_per_count": stream,
-        "bytes_rule": "tc_auto_stream_bytes: per task x, 20 + 4 d+(x) (task id, row bounds in "
-                      "both CSRs, N+(x)); per work-list entry y, 8 + 4 d+(y) (its row bounds, "
-                      "stored with the entry, and N+(y))",
+        "bytes_rule": "tc_auto_stream_bytes x entry bytes / 4: per task x, 20 + 4 d+(x) (task id, "
+                      "row bounds in both CSRs, N+(x)); per work-list entry y, 8 + 4 d+(y) (its "
+                      "row bounds, stored with the entry, and N+(y)); half of it over 16-bit rows",
+        "entry_bytes": entry_bytes,
         "bytes_push_form": kernel_bytes(info),
         "bytes_alg_edge_model": info.bytes_alg,
     }
@@ -611,7 +625,8 @@ def leg_summary(name, w, r, traffic=None):
     hr = r["results"][r["head"]]
     return {"workload": describe(w), "n": r["info"].n, "m": r["m"], "count": hr["count"],
             "engine": r["head"], "edges_per_s": hr["edges_per_s"], "ms_per_step": hr["ms_wall"],
-            "roofline": triangle_roofline(r["info"], hr, traffic, r["stream"]),
+            "roofline": triangle_roofline(r["info"], hr, traffic, r["stream"],
+                                          r["entry_bytes"]),
             "learned_vs_plain": vs_plain(r["results"], r["head"], traffic),
             "kernels": {k: {kk: (round(v, 4) if isinstance(v, float) else v)
                             for kk, v in x.items()} for k, x in r["results"].items()}}
@@ -714,7 +729,7 @@ def main():
             "n": info.n, "m": m, "count": hr["count"], "engine": head,
             "parallelism": "single GPU",
         },
-        "roofline": triangle_roofline(info, hr, traffic, r["stream"]),
+        "roofline": triangle_roofline(info, hr, traffic, r["stream"], r["entry_bytes"]),
         "cpu_baseline": r["cpu"],
         "cpu_baseline_parallel": r["cpu_par"],
         "learned_vs_plain": vs_plain(r["results"], head, traffic),

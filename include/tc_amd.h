@@ -110,7 +110,8 @@ typedef struct tc_sched {
   uint32_t grid_size;       /* Hu: work-balanced blocks (default 30000);
                                Bisson/TriCore/AUTO: resident workgroups          */
   uint32_t lds_slice;       /* reserved                                          */
-  uint32_t bitmap_min_deg;  /* Bisson: d+ above which the bitmap path runs (64)  */
+  uint32_t bitmap_min_deg;  /* Bisson: d+ above which the bitmap path runs (64);
+                               given, large graphs keep that kernel too          */
   uint32_t fox_max_lanes;   /* Fox: widest lanes-per-edge bin, 1..64 (64)        */
   uint32_t tricore_parts;   /* TriCore: node-range partitions (1)                */
   uint32_t auto_bins;       /* reserved                                          */
