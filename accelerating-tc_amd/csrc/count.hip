@@ -260,6 +260,9 @@ __global__ void k_row_flags(const uint32_t* __restrict__ rp, uint32_t n, uint32_
 // Later counts are 2 to 20 times as fast: R-MAT-18 with 3.6 * 10^6 edges 7.67 or
 // 1.82 against 0.33 or 0.15 ms.
 constexpr uint64_t kListEdges = 3u << 19, kListWedges = 1u << 26;
+// Fox's method: its bins take as long to build as the lists (first count, ER of 2 *
+// 10^4 edges 0.24 against 0.30 ms, R-MAT-14 of 5.5 * 10^4 0.50 against 0.25).
+constexpr uint64_t kFoxListEdges = 1u << 15;
 
 static bool on_lists(const tc_graph* g) {
   return g->m_or >= kListEdges || g->sum_in_out >= kListWedges;
@@ -835,6 +838,12 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
       if (L != 1 && L != 2 && L != 4 && L != 8 && L != 16 && L != 32 && L != 64)
         return fail(TC_ERR_ARG, "fox_max_lanes must be a power of two <= 64");
       if (s.fox_rearrange > 1) return fail(TC_ERR_ARG, "fox_rearrange must be 0 or 1");
+      // (the caller's bins are k_fox's)
+      on16 = !s.fox_max_lanes && !s.fox_rearrange && g->m_or >= kFoxListEdges;
+      if (on16) {
+        TCX_TRY(lists16or32(c, g, &lists));
+        break;
+      }
       TCX_TRY(fox_schedule(c, g, L, s.fox_rearrange == 1));
       break;
     }

@@ -633,11 +633,15 @@ static int rows32(tc_ctx* c, tc_graph* g, DevBuf& cnt) {
   return TC_OK;
 }
 
-// TriCore's rule (tricore/src/tricount_gpu.cu:215-290): every edge's shorter
-// list is looked up in its longer one.  Grouped by the owner of the longer list,
-// the edges share one bit map of it, where a wave spent six searches in sampled
-// pivots and about three in the list (one line each) on every entry: R-MAT-19
-// 4.9 -> 0.32 ms, random geometric of 300,000 vertices 2.08 -> 0.67 ms.
+// TriCore's rule (tricore/src/tricount_gpu.cu:215-290), and Fox's
+// (Fox/tc.cu:18-125): every edge's shorter list is looked up in its longer one.
+// Grouped by the owner of the longer list, the edges share one bit map of it,
+// where a wave spent six searches in sampled pivots and about three in the list
+// (one line each) on every entry (TriCore), or log2 of the list's length of
+// them (Fox); slices of equal work take the place of Fox's bins by work.
+// TriCore: R-MAT-19 4.9 -> 0.32 ms, random geometric of 300,000 vertices 2.08 ->
+// 0.67 ms; Fox: 7.6 -> 0.32 and 2.9 -> 0.66 ms, ER of 65,536 vertices and 2^20
+// edges 0.18 -> 0.041 ms.
 int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use) {
   TCX_TRY(lists16(c, g));
   *use = &g->sc.l16;

@@ -41,7 +41,7 @@ HBM_PEAK_GBPS = 8000.0
 METRIC = "TC edges/s + HBM GB/s % peak; learned/batched vs plain HIP, exact counts"
 KERNELS = ["hu", "bisson", "fox", "tricore", "auto", "learned"]
 KERNEL_SYMBOL = {
-    "hu": "k_count16", "bisson": "k_count16", "fox": "k_fox<L>",
+    "hu": "k_count16", "bisson": "k_count16", "fox": "k_count16",
     "tricore": "k_count16", "auto": "k_count16", "learned": "k_count16",
 }
 # Bytes per streamed list entry of the head kernel: 2 where the graph is counted

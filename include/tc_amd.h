@@ -112,7 +112,8 @@ typedef struct tc_sched {
   uint32_t lds_slice;       /* reserved                                          */
   uint32_t bitmap_min_deg;  /* Bisson: d+ above which the bitmap path runs (64);
                                given, large graphs keep that kernel too          */
-  uint32_t fox_max_lanes;   /* Fox: widest lanes-per-edge bin, 1..64 (64)        */
+  uint32_t fox_max_lanes;   /* Fox: widest lanes-per-edge bin, 1..64 (64); given
+                               (or fox_rearrange), the binned kernels run        */
   uint32_t tricore_parts;   /* TriCore: node-range partitions (1)                */
   uint32_t auto_bins;       /* reserved                                          */
   uint32_t auto_thresholds[4]; /* AUTO: with [0], [1] and [3] all 0 the WORKLIST

@@ -117,16 +117,16 @@ def test_hu(ctx, make, n, blocks):
         g.close()
 
 
-@pytest.mark.parametrize("kernel", ["bisson", "tricore"])
+@pytest.mark.parametrize("kernel", ["bisson", "tricore", "fox"])
 @pytest.mark.parametrize("make,n", [(lambda: rmat(17, 16, 3), 1 << 17),               # 16-bit rows, tail
                                     (lambda: tcamd.gen_er(400_001, 1_600_003, 5), 0),  # 32-bit rows
                                     (lambda: complete(1800), 0)])                  # no tail, long rows
-def test_bisson_and_tricore(ctx, kernel, make, n):
+def test_bisson_tricore_fox(ctx, kernel, make, n):
     s, d = make()
     for o in (tcamd.ORIENT_ID, tcamd.ORIENT_DEGREE):
         g = ctx.graph(s, d, n).orient(o)
         want = g.count(auto_thresholds=[64, 2048, 0, 8]).count
-        other = {"bisson": {"bitmap_min_deg": 64}, "tricore": {"tricore_parts": 2}}[kernel]
+        other = {"bisson": {"bitmap_min_deg": 64}, "tricore": {"tricore_parts": 2}, "fox": {"fox_max_lanes": 64}}[kernel]
         for args in ({}, {"grid_size": 3}, other):
             assert g.count(kernel, **args).count == want
         g.close()
