@@ -215,6 +215,16 @@ int fetch(tc_ctx* c, void* out, const void* src, size_t bytes) {
   return TC_OK;
 }
 
+int fetch2(tc_ctx* c, uint64_t* out, const uint64_t* src, uint64_t* out2, const uint64_t* src2) {
+  uint64_t* pin = static_cast<uint64_t*>(c->pin);
+  TCX_HIP(hipMemcpyAsync(pin, src, 8, hipMemcpyDeviceToHost, c->stream));
+  if (out2) TCX_HIP(hipMemcpyAsync(pin + 1, src2, 8, hipMemcpyDeviceToHost, c->stream));
+  TCX_HIP(hipStreamSynchronize(c->stream));
+  *out = pin[0];
+  if (out2) *out2 = pin[1];
+  return TC_OK;
+}
+
 // Pageable memory goes to the device at the speed of one host thread's copy
 // into the runtime's pinned buffer (25 GB/s); four threads filling pinned
 // slots of our own keep the link busy.

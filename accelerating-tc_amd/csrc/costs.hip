@@ -54,12 +54,7 @@ int raw_counts(tc_ctx* c, tc_graph* g, RawCounts& rc) {
   const uint32_t* s = g->src.as<uint32_t>();
   const uint32_t* d = g->dst.as<uint32_t>();
   uint32_t mx = 0;
-  if (m) {
-    uint32_t ms = 0, md = 0;
-    TCX_TRY(max_u32(c, s, m, &ms));
-    TCX_TRY(max_u32(c, d, m, &md));
-    mx = std::max(ms, md);
-  }
+  if (m) TCX_TRY(max_ids(c, s, d, m, &mx));
   const uint32_t nodes = mx + 1;
   rc.nodes = nodes;
   DevBuf buf;

@@ -558,7 +558,7 @@ static int fox_schedule(tc_ctx* c, tc_graph* g, uint32_t max_lanes, bool rearran
                      w.as<int32_t>());
   TCX_HIP(hipGetLastError());
   uint32_t mx = 0;
-  TCX_TRY(max_u32(c, w.as<uint32_t>(), m, &mx));
+  TCX_TRY(max_ids(c, w.as<uint32_t>(), nullptr, m, &mx));
   std::vector<int32_t> thr;
   fox_thresholds((int)mx, max_lanes, thr);
   int nthr = (int)thr.size();

@@ -835,13 +835,10 @@ static int csr_from_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint
     int end_bit = shift + bit_width_u32(n_out);
     TCX_TRY(sort_u64(c, keys.as<uint64_t>(), tmp.as<uint64_t>(), nkeys, end_bit, &sorted));
     uint64_t* other = sorted == keys.as<uint64_t>() ? tmp.as<uint64_t>() : keys.as<uint64_t>();
-    TCX_TRY(unique_u64(c, sorted, other, nkeys, &nuniq, shift));
+    uint64_t last = 0;
+    TCX_TRY(unique_u64(c, sorted, other, nkeys, &nuniq, shift, &last));
     uniq = other;
-    if (nuniq > 0) {
-      uint64_t last = 0;
-      TCX_TRY(fetch(c, &last, uniq + nuniq - 1, 8));
-      if ((uint32_t)(last >> 32) == n_out) --nuniq;  // sentinel
-    }
+    if (nuniq > 0 && last >> shift == n_out) --nuniq;  // sentinel
   }
   if (nuniq > kMaxCsrEntries)
     return fail(TC_ERR_RANGE, "%llu oriented edges exceed the 32-bit CSR offsets",
@@ -893,12 +890,9 @@ static int sym_keys(tc_ctx* c, tc_graph* g, DevBuf& keys, DevBuf& tmp, uint64_t*
                    shift + bit_width_u32(g->n_raw), &sorted));
   uint64_t* other = sorted == keys.as<uint64_t>() ? tmp.as<uint64_t>() : keys.as<uint64_t>();
   uint64_t nu = 0;
-  TCX_TRY(unique_u64(c, sorted, other, nk, &nu, shift));
-  if (nu > 0) {
-    uint64_t last = 0;
-    TCX_TRY(fetch(c, &last, other + nu - 1, 8));
-    if ((uint32_t)(last >> 32) == g->n_raw) --nu;
-  }
+  uint64_t last = 0;
+  TCX_TRY(unique_u64(c, sorted, other, nk, &nu, shift, &last));
+  if (nu > 0 && last >> shift == g->n_raw) --nu;
   *out = other;
   *m2 = nu;
   return TC_OK;
@@ -1159,14 +1153,13 @@ int graph_clone_records(tc_ctx* c, const tc_graph* g, tc_graph** out) {
       (hipMemcpyAsync(h->src.p, ps, 4 * m, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
        hipMemcpyAsync(h->dst.p, pd, 4 * m, hipMemcpyDeviceToDevice, c->stream) != hipSuccess))
     st = fail(TC_ERR_HIP, "record copy failed");
-  uint32_t ms = 0, md = 0;
-  if (st == TC_OK && m) st = max_u32(c, h->src.as<uint32_t>(), m, &ms);
-  if (st == TC_OK && m) st = max_u32(c, h->dst.as<uint32_t>(), m, &md);
+  uint32_t mx = 0;
+  if (st == TC_OK && m) st = max_ids(c, h->src.as<uint32_t>(), h->dst.as<uint32_t>(), m, &mx);
   if (st != TC_OK) {
     delete h;
     return st;
   }
-  h->n = m ? std::max(ms, md) + 1 : 0;
+  h->n = m ? mx + 1 : 0;
   h->n_raw = h->n;
   *out = h;
   return TC_OK;
@@ -1208,11 +1201,9 @@ int tc_graph_create(tc_ctx* c, const uint32_t* src, const uint32_t* dst, uint64_
   if (m) {
     st = upload(c, g->src.p, src, 4 * m);
     if (st == TC_OK) st = upload(c, g->dst.p, dst, 4 * m);
-    uint32_t ms = 0, md = 0;
-    if (st == TC_OK) st = max_u32(c, g->src.as<uint32_t>(), m, &ms);
-    if (st == TC_OK) st = max_u32(c, g->dst.as<uint32_t>(), m, &md);
+    uint32_t mx = 0;
+    if (st == TC_OK) st = max_ids(c, g->src.as<uint32_t>(), g->dst.as<uint32_t>(), m, &mx);
     if (st != TC_OK) { delete g; return st; }
-    uint32_t mx = std::max(ms, md);
     if (mx >= 0x7FFFFFFFu) {
       delete g;
       return fail(TC_ERR_RANGE, "vertex id %u exceeds 2^31-2", mx);
@@ -1322,10 +1313,9 @@ int tc_graph_relabel_aorder_model(tc_ctx* c, tc_graph* g, const tc_bw_model* mod
   // as the largest id + 1 (A-direction-seri.cpp:187-193), not the old n.
   uint32_t new_n = 0;
   if (g->m_raw) {
-    uint32_t ms = 0, md = 0;
-    TCX_TRY(max_u32(c, g->src.as<uint32_t>(), g->m_raw, &ms));
-    TCX_TRY(max_u32(c, g->dst.as<uint32_t>(), g->m_raw, &md));
-    new_n = std::max(ms, md) + 1;
+    uint32_t mx = 0;
+    TCX_TRY(max_ids(c, g->src.as<uint32_t>(), g->dst.as<uint32_t>(), g->m_raw, &mx));
+    new_n = mx + 1;
   }
   TCX_HIP(hipStreamSynchronize(c->stream));
   if (perm_out) std::copy(h_perm.begin(), h_perm.end(), perm_out);
@@ -1345,10 +1335,9 @@ int tc_graph_relabel(tc_ctx* c, tc_graph* g, int mode, uint32_t* perm_out) {
   uint32_t* d = g->dst.as<uint32_t>();
   uint32_t n = 1;  // max id + 1 over the records, as the tools compute it
   if (m) {
-    uint32_t ms = 0, md = 0;
-    TCX_TRY(max_u32(c, s, m, &ms));
-    TCX_TRY(max_u32(c, d, m, &md));
-    n = std::max(ms, md) + 1;
+    uint32_t mx = 0;
+    TCX_TRY(max_ids(c, s, d, m, &mx));
+    n = mx + 1;
   }
   DevBuf deg, perm, key, ktmp, ids, itmp;
   TCX_TRY(perm.reserve(4ull * n));

@@ -64,6 +64,8 @@ int upload(tc_ctx* c, void* dst, const void* src, size_t bytes);
 // waits for the stream.
 constexpr size_t kPinBytes = 32768;
 int fetch(tc_ctx* c, void* out, const void* src, size_t bytes);
+// Two words with one wait (out2 may be null: one).
+int fetch2(tc_ctx* c, uint64_t* out, const uint64_t* src, uint64_t* out2, const uint64_t* src2);
 
 // ---- device buffer ------------------------------------------------------
 // Owns one region; grows on demand (contents are not kept).
@@ -231,13 +233,12 @@ int sort_pairs_u64_u32(tc_ctx* c, uint64_t* keys, uint64_t* ktmp, uint32_t* vals
 int sort_pairs_u32_u32(tc_ctx* c, uint32_t* keys, uint32_t* ktmp, uint32_t* vals,
                        uint32_t* vtmp, uint64_t n, int end_bit, uint32_t** skeys,
                        uint32_t** svals);
-// (shift: as for compact_u64; 32 below kMinCompact keys)
+// (shift, last: as for compact_u64; shift 32 below kMinCompact keys)
 int unique_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n,
-               uint64_t* n_out, int shift = 32);
+               uint64_t* n_out, int shift = 32, uint64_t* last = nullptr);
 int exclusive_scan_u32(tc_ctx* c, const uint32_t* in, uint32_t* out, uint64_t n);
 int exclusive_scan_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n);
 int inclusive_scan_i64(tc_ctx* c, const int64_t* in, int64_t* out, uint64_t n);
-int max_u32(tc_ctx* c, const uint32_t* in, uint64_t n, uint32_t* result);
 int sum_u64(tc_ctx* c, const uint64_t* in, uint64_t n, uint64_t* result);
 int min_i32(tc_ctx* c, const int32_t* in, uint64_t n, int32_t* result);
 int select_flagged_u32(tc_ctx* c, const uint32_t* in, const uint8_t* flags,
@@ -253,9 +254,11 @@ int count_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint3
               uint32_t* h);
 // The keys with flags[i] set, or (flags null) the first of each run of equal
 // keys, in order; out must not be in.  Keys a << shift | b come out as
-// a << 32 | b.
+// a << 32 | b.  last (optional) receives the last key of in.
 int compact_u64(tc_ctx* c, const uint64_t* in, const uint8_t* flags, uint64_t n, uint64_t* out,
-                uint64_t* n_out, int shift = 32);
+                uint64_t* n_out, int shift = 32, uint64_t* last = nullptr);
+// The largest of a[0, m) (and b[0, m) when b is not null), 0 for m = 0.
+int max_ids(tc_ctx* c, const uint32_t* a, const uint32_t* b, uint64_t m, uint32_t* result);
 // Keys from which on compact_u64 takes over from the single pass (two more
 // launches, so small inputs keep it).
 constexpr uint64_t kMinCompact = 1u << 20;

@@ -385,8 +385,7 @@ int place_rows(tc_ctx* c, uint32_t n, const uint32_t* cnt, uint32_t per, Rows16&
   TCX_TRY(exclusive_scan_u64(c, pa.as<uint64_t>(), sa.as<uint64_t>(), (uint64_t)n + 1));
   TCX_TRY(exclusive_scan_u64(c, pb.as<uint64_t>(), sb.as<uint64_t>(), (uint64_t)n + 1));
   uint64_t ta = 0, tb = 0;
-  TCX_TRY(read_back(c, sa.as<uint64_t>() + n, &ta));
-  TCX_TRY(read_back(c, sb.as<uint64_t>() + n, &tb));
+  TCX_TRY(fetch2(c, &ta, sa.as<uint64_t>() + n, &tb, sb.as<uint64_t>() + n));
   R.units = 8 * (ta >> 32) + 4 * (ta & 0xFFFFFFFFu) + 2 * (tb >> 32) + (tb & 0xFFFFFFFFu);
   if (R.units > 0xFFFFFFFFull) return fail(TC_ERR_RANGE, "list rows exceed 2^32 16-byte units");
   TCX_TRY(R.row.reserve(8 * ((size_t)n + 1)));

@@ -65,16 +65,16 @@ int sort_pairs_u32_u32(tc_ctx* c, uint32_t* keys, uint32_t* ktmp, uint32_t* vals
 }
 
 int unique_u64(tc_ctx* c, const uint64_t* in, uint64_t* out, uint64_t n,
-               uint64_t* n_out, int shift) {
+               uint64_t* n_out, int shift, uint64_t* last) {
   if (n == 0) { *n_out = 0; return TC_OK; }
-  if (n >= kMinCompact) return compact_u64(c, in, nullptr, n, out, n_out, shift);
+  if (n >= kMinCompact) return compact_u64(c, in, nullptr, n, out, n_out, shift, last);
   TCX_TRY(c->prim_out.reserve(64));
   uint64_t* d_cnt = c->prim_out.as<uint64_t>();
   TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
     return rocprim::unique(t, b, in, out, d_cnt, (size_t)n, rocprim::equal_to<uint64_t>(),
                            c->stream);
   }));
-  return fetch(c, n_out, d_cnt, sizeof(uint64_t));
+  return fetch2(c, n_out, d_cnt, last, in + n - 1);
 }
 
 int exclusive_scan_u32(tc_ctx* c, const uint32_t* in, uint32_t* out, uint64_t n) {
@@ -99,17 +99,6 @@ int inclusive_scan_i64(tc_ctx* c, const int64_t* in, int64_t* out, uint64_t n) {
     return rocprim::inclusive_scan(t, b, in, out, (size_t)n, rocprim::plus<int64_t>(),
                                    c->stream);
   });
-}
-
-int max_u32(tc_ctx* c, const uint32_t* in, uint64_t n, uint32_t* result) {
-  *result = 0;
-  if (n == 0) return TC_OK;
-  TCX_TRY(c->prim_out.reserve(64));
-  uint32_t* d = c->prim_out.as<uint32_t>();
-  TCX_TRY(run_prim(c, [&](void* t, size_t& b) {
-    return rocprim::reduce(t, b, in, d, 0u, (size_t)n, rocprim::maximum<uint32_t>(), c->stream);
-  }));
-  return fetch(c, result, d, sizeof(uint32_t));
 }
 
 int min_i32(tc_ctx* c, const int32_t* in, uint64_t n, int32_t* result) {

@@ -77,3 +77,14 @@ def test_pruned(ctx, n, m):
     assert g.info().n < n
     assert g.count().count == want
     g.close()
+
+
+@pytest.mark.parametrize("m", [1, 63, 1023, 1024, 1025, 4097, 300_001, 2_100_003])
+def test_largest_id(ctx, m):
+    rng = np.random.default_rng(m)
+    for where, side in ((0, 0), (m - 1, 0), (m // 2, 1), (m - 1, 1)):
+        ends = [rng.integers(0, 5000, m).astype(np.uint32) for _ in range(2)]
+        ends[side][where] = 7654
+        g = ctx.graph(*ends)
+        assert g.info().n == 7655
+        g.close()
