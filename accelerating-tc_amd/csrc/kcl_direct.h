@@ -228,7 +228,8 @@ __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : W == 4 ? 6 : 8))) void k_kcl_dir
       // Every entry of the out-lists is searched in N+(u).  Each group of kG
       // lanes takes kU * kG entries a step, and the wave's next list when its own
       // is used up; the next step's entries are loaded before this one's are
-      // searched.
+      // searched.  8 lanes and 4 entries each: R-MAT-16, k = 4, 886 us against 954
+      // with 4 lanes (one-word rows) and 992 with 4 lanes and 8 entries.
       {
         const uint32_t j = lane & (kG - 1);
         const uint32_t nl = d > wv ? (d - wv + NW - 1) / NW : 0;  // this wave's lists
