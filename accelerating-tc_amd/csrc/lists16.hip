@@ -428,8 +428,8 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
   hipLaunchKernelGGL(k_rowptr_search<uint64_t>, dim3(grid_for((uint64_t)n + 1)), dim3(TB), 0,
                      c->stream, sorted, nk, n, wrp.as<uint32_t>());
   TCX_HIP(hipGetLastError());
-  uint32_t kept = 0;
-  TCX_TRY(read_back(c, wrp.as<uint32_t>() + n, &kept));
+  uint32_t kept = (uint32_t)nk;
+  if (!tail) TCX_TRY(read_back(c, wrp.as<uint32_t>() + n, &kept));
   R.entries = kept;
   R.tasks = 0;
   R.nslice = 0;
