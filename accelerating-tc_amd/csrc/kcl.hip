@@ -981,7 +981,7 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       const float cs = us_per_tick / (float)per_cu;
       TCX_TRY(lm.mark());
       switch (b.w) {
-        case 1: hipLaunchKernelGGL((k_kcl_direct<1, 1>), dim3(G), dim3(64), 0, c->stream, rp, col, deg, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
+        case 1: hipLaunchKernelGGL((g->csr_only ? k_kcl_direct<1, 1, true> : k_kcl_direct<1, 1>), dim3(G), dim3(64), 0, c->stream, rp, col, deg, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
         case 2: hipLaunchKernelGGL((k_kcl_direct<2, 2>), dim3(G), dim3(128), 0, c->stream, rp, col, deg, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
         case 4: hipLaunchKernelGGL((k_kcl_direct<4, 4>), dim3(G), dim3(256), 0, c->stream, rp, col, deg, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
         default: hipLaunchKernelGGL((k_kcl_direct<8, 8>), dim3(G), dim3(512), 0, c->stream, rp, col, deg, order, nr, copies, chunk, k, acc, groups, cost, cs); break;
