@@ -365,8 +365,11 @@ __global__ __launch_bounds__(256) void k_peel_big(const uint2* __restrict__ big,
 // copy and a wait for each cost about 20 us; at most kSmallArcs neighbours keep a
 // level here shorter than that.  k-core of R-MAT-14, 16, 20 (2^18, 2^19, 2^24
 // records): 6.5 -> 4.8, 8.4 -> 6.1, 30.7 -> 25.5 ms, A-direction 1.35 -> 1.08,
-// 2.09 -> 1.88, 7.76 -> 7.61.
+// 2.09 -> 1.88, 7.76 -> 7.61.  kSmallLevels bounds a launch, a level of which takes
+// 2 to 10 us, to some 20 ms at most (a path has a level for every two vertices);
+// the host goes on from the frontier that it leaves.
 constexpr uint32_t kSmallThreads = 1024, kSmallFrontier = 1024, kSmallArcs = 8192;
+constexpr uint32_t kSmallLevels = 2048;
 
 template <class Step>
 __global__ __launch_bounds__(kSmallThreads) void k_peel_small(uint32_t* __restrict__ a,
@@ -381,7 +384,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_peel_small(uint32_t* __restri
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   uint32_t fs = fsize, taken = 0, levels = 0;  // the same in every thread
   uint32_t *F = a, *N = b;
-  while (fs && fs <= kSmallFrontier) {
+  while (fs && fs <= kSmallFrontier && levels < kSmallLevels) {
     // row bounds and the prefix of the lengths
     uint32_t len = 0;
     if (tid < fs) {
@@ -796,8 +799,8 @@ int peel_level(tc_ctx* c, const uint32_t* F, uint32_t fs, const uint32_t* rp, co
 }
 
 // Levels from the frontier F (fs vertices) on in one workgroup: *taken vertices
-// in *levels levels (0: the first is too large), after which F and fs are the frontier
-// to go on with.
+// in *levels levels (0: the first is too large; at most kSmallLevels), after which F
+// and fs are the frontier to go on with.
 template <class Step>
 int peel_small(tc_ctx* c, uint32_t*& F, uint32_t*& N, uint32_t& fs, const uint32_t* rp,
                const uint32_t* col, Step step, uint32_t* taken, uint32_t* levels) {
@@ -1030,7 +1033,7 @@ static int adir_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, con
                            AdirStep{rtd.as<int32_t>(), prio, threshold, label}, &taken, &levels));
         peeled += taken;
         label += (int32_t)levels;
-        small = false;  // what is left, if any, is too large
+        small = levels == kSmallLevels;  // else what is left, if any, is too large
         continue;
       }
       small = !omp && !rec;
@@ -1104,7 +1107,7 @@ static int kcore_peel(tc_ctx* c, uint32_t n, uint64_t m2, const uint32_t* rp, co
         removed += taken;
         t += (int32_t)levels;
         if (levels && fs == 0) --t;  // the last level took nothing
-        small = false;
+        small = levels == kSmallLevels;
         continue;
       }
       small = true;
