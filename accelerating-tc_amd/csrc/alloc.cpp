@@ -3,10 +3,12 @@
 // hipMalloc and hipFree cost 20-300 us apiece at the sizes of a graph's
 // buffers (hipFree also waits for the device): more than half of a one-shot
 // count of a small or mid-sized graph.  A context keeps the blocks its buffers
-// give back, up to 1/16 of the device's memory, and gives them to its next
-// buffers; a destroyed context leaves them, under the same bound, to the
-// device's other contexts, and the last one gives them back to the system.
-// When hipMalloc fails, every kept block is freed and it is tried once more.
+// give back and gives them to its next buffers; a destroyed context leaves them
+// to the device's other contexts, and the last one gives them back to the
+// system.  All contexts of a device together keep at most 1/16 of its memory.
+// tc_ctx_release_memory gives it back, and so does every context when hipMalloc
+// fails, which is then tried once more.
+#include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -17,44 +19,19 @@
 
 namespace tcx {
 
+struct Device;
+
 struct Pool {
   std::mutex mu;
   std::multimap<size_t, void*> blocks;
-  size_t held = 0, cap = 0;
-  int device = 0;
+  Device* dev = nullptr;  // null: nothing is kept
   bool closed = false;
 
   // Smallest kept block of at least `want` bytes that wastes little.
-  void* take(size_t want, size_t* got) {
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = blocks.lower_bound(want);
-    if (it == blocks.end() || it->first > (want < (1u << 20) ? 2 * want : want + want / 4))
-      return nullptr;
-    void* p = it->second;
-    *got = it->first;
-    held -= it->first;
-    blocks.erase(it);
-    return p;
-  }
+  void* take(size_t want, size_t* got);
   // Keeps the block, or returns false when it is not to be kept.
-  bool give(void* p, size_t bytes) {
-    std::lock_guard<std::mutex> lk(mu);
-    if (closed || held + bytes > cap) return false;
-    try {
-      blocks.emplace(bytes, p);
-    } catch (const std::bad_alloc&) {
-      return false;  // a destructor may be giving it back
-    }
-    held += bytes;
-    return true;
-  }
-  std::multimap<size_t, void*> drain() {
-    std::lock_guard<std::mutex> lk(mu);
-    held = 0;
-    std::multimap<size_t, void*> out;
-    out.swap(blocks);
-    return out;
-  }
+  bool give(void* p, size_t bytes);
+  std::multimap<size_t, void*> drain();
 };
 
 namespace {
@@ -71,11 +48,51 @@ struct Staging {
   hipEvent_t free_at[2 * kCopyThreads] = {};
 };
 
+}  // namespace
+
 struct Device {
+  std::atomic<size_t> held{0}, cap{0};  // bytes kept by all pools, and how many may be
   Pool shared;       // blocks of destroyed contexts: no work is pending on them
   int contexts = 0;
   Staging staging;
 };
+
+void* Pool::take(size_t want, size_t* got) {
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = blocks.lower_bound(want);
+  if (it == blocks.end() || it->first > (want < (1u << 20) ? 2 * want : want + want / 4))
+    return nullptr;
+  void* p = it->second;
+  *got = it->first;
+  dev->held -= it->first;
+  blocks.erase(it);
+  return p;
+}
+
+bool Pool::give(void* p, size_t bytes) {
+  if (!dev) return false;
+  std::lock_guard<std::mutex> lk(mu);
+  if (closed) return false;
+  if (dev->held.fetch_add(bytes) + bytes <= dev->cap) {
+    try {
+      blocks.emplace(bytes, p);
+      return true;
+    } catch (const std::bad_alloc&) {  // a destructor may be giving it back
+    }
+  }
+  dev->held -= bytes;
+  return false;
+}
+
+std::multimap<size_t, void*> Pool::drain() {
+  std::lock_guard<std::mutex> lk(mu);
+  std::multimap<size_t, void*> out;
+  out.swap(blocks);
+  for (auto& x : out) dev->held -= x.first;
+  return out;
+}
+
+namespace {
 
 std::mutex g_mu;                              // registry
 std::vector<std::weak_ptr<Pool>> g_pools;
@@ -100,13 +117,9 @@ void free_staging(Staging& s) {
 
 // Every kept block of every pool back to the system.
 void trim_all() {
-  std::vector<std::shared_ptr<Pool>> ps;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    for (auto& w : g_pools)
-      if (auto p = w.lock()) ps.push_back(p);
-  }
-  for (auto& p : ps) free_blocks(p->drain());
+  std::lock_guard<std::mutex> lk(g_mu);
+  for (auto& w : g_pools)
+    if (auto p = w.lock()) free_blocks(p->drain());
   for (Device& d : g_dev) free_blocks(d.shared.drain());
 }
 
@@ -130,36 +143,45 @@ PoolScope::~PoolScope() {
 }
 
 std::shared_ptr<Pool> pool_create(int device, uint64_t total_mem) {
-  auto p = std::make_shared<Pool>();
-  p->device = device;
-  p->cap = (size_t)(total_mem / 16);
-  std::lock_guard<std::mutex> lk(g_mu);
-  if (device >= 0 && device < kMaxDevices) {
-    g_dev[device].contexts++;
-    g_dev[device].shared.cap = p->cap;
+  std::shared_ptr<Pool> p;
+  try {
+    p = std::make_shared<Pool>();
+    std::lock_guard<std::mutex> lk(g_mu);
+    for (size_t i = 0; i < g_pools.size();)
+      if (g_pools[i].expired()) g_pools.erase(g_pools.begin() + (long)i);
+      else ++i;
+    g_pools.push_back(p);
+    if (device >= 0 && device < kMaxDevices) {
+      Device& d = g_dev[device];
+      d.contexts++;
+      d.cap = (size_t)(total_mem / 16);
+      if (!d.shared.dev) d.shared.dev = &d;
+      p->dev = &d;
+    }
+  } catch (const std::bad_alloc&) {
+    return nullptr;
   }
-  for (size_t i = 0; i < g_pools.size();)
-    if (g_pools[i].expired()) g_pools.erase(g_pools.begin() + (long)i);
-    else ++i;
-  g_pools.push_back(p);
   return p;
 }
 
+void pool_release(tc_ctx* c) {
+  if (!c->pool || !c->pool->dev) return;
+  free_blocks(c->pool->drain());
+  free_blocks(c->pool->dev->shared.drain());
+}
+
 void pool_retire(std::shared_ptr<Pool> pool) {
-  if (!pool) return;
+  if (!pool || !pool->dev) return;
   {
     std::lock_guard<std::mutex> lk(pool->mu);
     pool->closed = true;
   }
+  Device& d = *pool->dev;
+  // under the registry's lock a new context neither uploads through the slots
+  // nor finds blocks while the last one frees them
+  std::lock_guard<std::mutex> lk(g_mu);
   std::multimap<size_t, void*> b = pool->drain();
-  if (pool->device < 0 || pool->device >= kMaxDevices) return free_blocks(std::move(b));
-  Device& d = g_dev[pool->device];
-  bool last;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    last = --d.contexts == 0;
-  }
-  if (last) {
+  if (--d.contexts == 0) {
     free_blocks(std::move(b));
     free_blocks(d.shared.drain());
     free_staging(d.staging);
@@ -173,30 +195,33 @@ int DevBuf::reserve(size_t want) {
   if (want <= bytes && p) return TC_OK;
   release();
   if (want == 0) want = 64;
-  if (t_pool) {
-    pool = t_owner && t_owner.get() == t_pool ? t_owner : nullptr;
-    if (pool) {
-      want = rounded(want);
-      p = pool->take(want, &bytes);
-      if (!p && pool->device >= 0 && pool->device < kMaxDevices)
-        p = g_dev[pool->device].shared.take(want, &bytes);
-      if (p) return TC_OK;
-    }
+  size_t size = want;
+  if (t_pool && t_owner.get() == t_pool && t_owner->dev) {
+    pool = t_owner;
+    size = rounded(want);
+    p = pool->take(size, &bytes);
+    if (!p) p = pool->dev->shared.take(size, &bytes);
+    if (p) return TC_OK;
   }
-  hipError_t e = hipMalloc(&p, want);
+  hipError_t e = hipMalloc(&p, size);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     trim_all();
-    e = hipMalloc(&p, want);
+    e = hipMalloc(&p, size);
+    if (e == hipErrorOutOfMemory && size > want) {  // without the rounding
+      (void)hipGetLastError();
+      size = want;
+      e = hipMalloc(&p, size);
+    }
   }
   if (e != hipSuccess) {
     p = nullptr;
     bytes = 0;
     pool.reset();
     (void)hipGetLastError();
-    return fail(TC_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", want, hipGetErrorString(e));
+    return fail(TC_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", size, hipGetErrorString(e));
   }
-  bytes = want;
+  bytes = size;
   return TC_OK;
 }
 

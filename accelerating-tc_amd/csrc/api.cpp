@@ -102,6 +102,10 @@ int tc_ctx_create(int device, tc_ctx** out) {
     return fail(TC_ERR_NOMEM, "pinned host page allocation failed");
   }
   c->pool = tcx::pool_create(device, c->total_mem);
+  if (!c->pool) {
+    tc_ctx_destroy(c);
+    return fail(TC_ERR_NOMEM, "out of host memory");
+  }
   *out = c;
   return TC_OK;
 }
@@ -129,6 +133,13 @@ int tc_ctx_destroy(tc_ctx* c) {
 int tc_ctx_device_memory(const tc_ctx* c, uint64_t* bytes) {
   if (!c || !bytes) return fail(TC_ERR_ARG, "NULL argument");
   *bytes = c->total_mem;
+  return TC_OK;
+}
+
+int tc_ctx_release_memory(tc_ctx* c) {
+  if (!c) return fail(TC_ERR_ARG, "NULL argument");
+  TCX_HIP(hipSetDevice(c->device));
+  tcx::pool_release(c);
   return TC_OK;
 }
 

@@ -52,7 +52,11 @@ struct PoolScope {
  private:
   Pool* before;
 };
+// (null: out of host memory)
 std::shared_ptr<Pool> pool_create(int device, uint64_t total_mem);
+// The blocks that the context keeps, and those of destroyed ones, back to the
+// system.
+void pool_release(tc_ctx* c);
 // The context's stream is idle: its blocks go to the device's other contexts,
 // and back to the system with the last of them.
 void pool_retire(std::shared_ptr<Pool> pool);

@@ -94,6 +94,7 @@ _sig("tc_last_error", C.c_char_p, [])
 _sig("tc_ctx_create", C.c_int, [C.c_int, C.POINTER(_vp)])
 _sig("tc_ctx_destroy", C.c_int, [_vp])
 _sig("tc_ctx_device_memory", C.c_int, [_vp, C.POINTER(C.c_uint64)])
+_sig("tc_ctx_release_memory", C.c_int, [_vp])
 _sig("tc_file_edge_count", C.c_int, [C.c_char_p, C.POINTER(C.c_uint64)])
 _sig("tc_read_edges", C.c_int, [C.c_char_p, _u32p, _u32p, C.c_uint64, C.POINTER(C.c_uint64)])
 _sig("tc_write_edges", C.c_int, [C.c_char_p, _u32p, _u32p, C.c_uint64])
@@ -233,6 +234,7 @@ _sig("tc_batch_count_pergraph", C.c_int, [_vp, _vp, C.POINTER(BatchSched), _u64p
 
 EXPORTED = [
     "tc_status_str", "tc_last_error", "tc_ctx_create", "tc_ctx_destroy", "tc_ctx_device_memory",
+    "tc_ctx_release_memory",
     "tc_file_edge_count", "tc_read_edges", "tc_write_edges", "tc_list2bin", "tc_bin2list", "tc_read_gr",
     "tc_gen_er", "tc_gen_rmat", "tc_gen_ba", "tc_gen_rgg", "tc_graph_create", "tc_graph_destroy",
     "tc_graph_simplify", "tc_graph_relabel_aorder", "tc_graph_relabel", "tc_graph_orient", "tc_graph_info_get",
@@ -470,6 +472,11 @@ class Context:
         b = C.c_uint64()
         _check(_lib.tc_ctx_device_memory(self._h, C.byref(b)), "tc_ctx_device_memory")
         return b.value
+
+    def release_memory(self):
+        """Gives the device memory that is kept for reuse back to the system
+        (tc_ctx_release_memory)."""
+        _check(_lib.tc_ctx_release_memory(self._h), "tc_ctx_release_memory")
 
     def close(self):
         if getattr(self, "_h", None):

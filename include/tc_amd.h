@@ -154,6 +154,12 @@ int tc_ctx_create(int device, tc_ctx** out);
 int tc_ctx_destroy(tc_ctx* ctx);
 /* Total device memory in bytes (tricore init_gpu(), tricount_gpu.cu:29-35). */
 int tc_ctx_device_memory(const tc_ctx* ctx, uint64_t* bytes);
+/* Device memory that a context's graphs and calls no longer use is kept for
+ * the next ones: by all contexts of a device together at most 1/16 of its
+ * memory, until the last of them is destroyed or an allocation of the library
+ * fails.  This call gives what ctx (and destroyed contexts of its device) keep
+ * back to the system, for other allocators of the process or the machine. */
+int tc_ctx_release_memory(tc_ctx* ctx);
 
 /* ---- L0: edge files (tools/list2bin.cpp, tools/bin2list.cpp) ---------- */
 /* Record count = size/8; a size that is not a multiple of 8 is TC_ERR_FORMAT
