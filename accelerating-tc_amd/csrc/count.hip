@@ -451,6 +451,7 @@ static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin);
 // and wave tasks (default thresholds) with one output per vertex.
 int per_vertex_counts(tc_ctx* c, tc_graph* g, unsigned long long* tri) {
   if (g->n == 0) return TC_OK;
+  ensure_version(g);  // the task lists are those of the present CSR
   TCX_TRY(lists16(c, g, true));
   if (g->sc.l16.usable) {
     TCX_TRY(c->scratch.reserve(kCurBytes16));
