@@ -130,6 +130,8 @@ struct Lists16 {
   uint64_t version = ~0ull;        // the CSR it was built (or found unsuitable) for
   bool usable = false;
   bool credit = false;             // built for per-vertex counts too
+  bool listed = false;             // with the hub's work lists (else id and cnt to build them)
+  DevBuf id, cnt;                  // uint16[n] 16-bit ids (none: all are their own), uint32[n]
   Rows16 hub, tail;                // entries with 16-bit ids, the others (32-bit)
 };
 

@@ -473,10 +473,21 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
   return TC_OK;
 }
 
+// The hub's work lists of a layer built without them.
+int hub_lists(tc_ctx* c, tc_graph* g, Lists16& L) {
+  TCX_TRY(work_lists(c, g, L.cnt.as<uint32_t>(), L.id.as<uint16_t>(), false, L.credit, L.hub));
+  L.id.release();
+  L.cnt.release();
+  L.listed = true;
+  return TC_OK;
+}
+
 // Rows, work lists and slices for the ids `id` (null: every vertex id is its
 // own 16-bit id; id_all: every vertex has one, and there is no tail).
-// L.usable is left false when too few entries have an id.
-int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, bool credit, Lists16& L) {
+// lists: with the hub's work lists; without them, id and the row lengths stay
+// with L for hub_lists().  L.usable is left false when too few entries have an id.
+int build(tc_ctx* c, tc_graph* g, DevBuf& idbuf, bool id_all, bool credit, bool lists, Lists16& L) {
+  const uint16_t* id = idbuf.as<uint16_t>();
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
@@ -518,30 +529,39 @@ int build(tc_ctx* c, tc_graph* g, const uint16_t* id, bool id_all, bool credit, 
                      pre, L.hub.row.as<uint2>(), L.hub.col.as<uint16_t>(),
                      L.tail.row.as<uint2>(), L.tail.col.as<uint32_t>());
   TCX_HIP(hipGetLastError());
-  TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), id, false, credit, L.hub));
   L.tail.tasks = 0;
   if (tail) TCX_TRY(work_lists(c, g, tcnt.as<uint32_t>(), id, true, credit, L.tail));
-  L.usable = true;
+  swap(L.id, idbuf);
+  swap(L.cnt, cnt);
   L.credit = credit;
+  L.listed = false;
+  if (lists) TCX_TRY(hub_lists(c, g, L));
+  L.usable = true;
   return TC_OK;
 }
 
 }  // namespace
 
-int lists16(tc_ctx* c, tc_graph* g, bool credit) {
+// The rows, and (lists) the hub's work lists, which the push methods do without.
+static int layer16(tc_ctx* c, tc_graph* g, bool credit, bool lists) {
   Lists16& L = g->sc.l16;
-  if (L.version == g->sched_version && (!L.usable || L.credit || !credit)) return TC_OK;
+  if (L.version == g->sched_version && (!L.usable || L.credit || !credit)) {
+    if (L.usable && lists && !L.listed) TCX_TRY(hub_lists(c, g, L));
+    return TC_OK;
+  }
   L.version = ~0ull;
   L.usable = false;
   if (g->n && g->m_or) {
     DevBuf id;
     bool some = true;
     if (g->n > kMax16) TCX_TRY(hub_ids(c, g, id, &some));
-    if (some) TCX_TRY(build(c, g, id.as<uint16_t>(), g->n <= kMax16, credit, L));
+    if (some) TCX_TRY(build(c, g, id, g->n <= kMax16, credit, lists, L));
   }
   L.version = g->sched_version;
   return TC_OK;
 }
+
+int lists16(tc_ctx* c, tc_graph* g, bool credit) { return layer16(c, g, credit, true); }
 
 int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* voff) {
   Lists16& L = g->sc.l16;
@@ -553,7 +573,7 @@ int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* v
     hipLaunchKernelGGL(k_local_ids, dim3(grid_for(g->n)), dim3(TB), 0, c->stream, gid, voff, g->n,
                        id.as<uint16_t>());
     TCX_HIP(hipGetLastError());
-    TCX_TRY(build(c, g, id.as<uint16_t>(), true, false, L));
+    TCX_TRY(build(c, g, id, true, false, true, L));
     if (L.hub.tasks)
       hipLaunchKernelGGL(k_graph_of, dim3(grid_for(L.hub.tasks)), dim3(TB), 0, c->stream,
                          L.hub.who.as<uint32_t>(), L.hub.tasks, gid);
@@ -664,7 +684,7 @@ int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use) {
 // vertices and average degree 48 1.59 -> 0.53 ms.
 int push16(tc_ctx* c, tc_graph* g) {
   Push16& H = g->sc.push16;
-  TCX_TRY(lists16(c, g));
+  TCX_TRY(layer16(c, g, false, false));
   if (H.version == g->sched_version) return TC_OK;
   const bool b16 = g->sc.l16.usable;
   const uint32_t n = g->n;
