@@ -251,6 +251,161 @@ __global__ void k_row_flags(const uint32_t* __restrict__ rp, uint32_t n, uint32_
   }
 }
 
+// ---- Hu: workgroup per vertex range, N+(u) slices staged in LDS ----------
+//
+// Hu/tc.cu:69-201 re-designed for wave64: the range's adjacency slice is
+// copied into LDS by all lanes (coalesced), the wedges u->v->w of the slice
+// are flattened with an LDS prefix sum so consecutive lanes read consecutive
+// w from HBM, and w is binary-searched in the LDS copy of N+(u).  A vertex
+// whose list exceeds the slice searches N+(u) in global memory instead
+// (the reference's cacheWorked == false path).
+//
+// The first counts of a CSR run here; later ones stream the list rows (hu_rows).
+// `total` holds kHuAcc accumulators kHuAccStride words apart: with one for
+// all, and an atomic per wave, the 120,000 of them were most of the time where
+// every block has triangles (random geometric, 60,000 vertices, average degree
+// 24: 1,256 -> 153 us; ER of 65,536 vertices and 2^20 edges 202 -> 187).
+constexpr uint32_t kHuAcc = 64, kHuAccStride = 16;
+static_assert(8 * kHuAcc * kHuAccStride == kAccBytes16, "added up by sum16");
+
+template <int SLICE, int ROWCAP>
+struct HuLds {
+  uint32_t col[SLICE];
+  uint32_t vst[SLICE];
+  uint32_t pre[SLICE + 1];
+  uint16_t row[SLICE];
+  uint32_t rof[ROWCAP + 1];
+  uint32_t wsum[TB / 64];
+  uint32_t u2;
+};
+
+// Stage edges [ebase, ebase+E) into LDS: v, start of N+(v), wedge prefix.
+template <int SLICE, int ROWCAP>
+__device__ inline uint32_t stage_edges(HuLds<SLICE, ROWCAP>& L, const uint32_t* __restrict__ rp,
+                                       const uint32_t* __restrict__ col, uint32_t ebase, uint32_t E,
+                                       bool by_row = false) {
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t e = tid; e < E; e += TB) {
+    uint32_t v = col[ebase + e];
+    uint32_t vs = rp[v];
+    L.col[e] = v;
+    L.vst[e] = vs;
+    uint32_t c = rp[v + 1] - vs;
+    if (by_row) {
+      const uint32_t r = L.row[e];
+      if (L.rof[r + 1] - L.rof[r] < 2) c = 0;
+    }
+    L.pre[e] = c;
+  }
+  __syncthreads();
+  // block exclusive scan, blocked layout: thread t owns [t*K, t*K+K)
+  constexpr int K = SLICE / TB;
+  uint32_t loc[K];
+  uint32_t sum = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    uint32_t e = tid * K + k;
+    uint32_t x = e < E ? L.pre[e] : 0;
+    loc[k] = sum;
+    sum += x;
+  }
+  // inclusive wave scan of per-thread sums
+  const uint32_t lane = tid & 63, wv = tid >> 6;
+  uint32_t inc = sum;
+  for (int off = 1; off < 64; off <<= 1) {
+    uint32_t o = __shfl_up(inc, off, 64);
+    if (lane >= (uint32_t)off) inc += o;
+  }
+  if (lane == 63) L.wsum[wv] = inc;
+  __syncthreads();
+  uint32_t wbase = 0;
+  for (uint32_t i = 0; i < wv; ++i) wbase += L.wsum[i];
+  uint32_t tbase = wbase + inc - sum;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    uint32_t e = tid * K + k;
+    if (e < E) L.pre[e] = tbase + loc[k];
+  }
+  uint32_t total = 0;
+  for (uint32_t i = 0; i < TB / 64; ++i) total += L.wsum[i];
+  if (tid == 0) L.pre[E] = total;
+  __syncthreads();
+  return total;
+}
+
+template <int SLICE, int ROWCAP>
+__global__ __launch_bounds__(TB) void k_hu(const uint32_t* __restrict__ rp,
+                                           const uint32_t* __restrict__ col,
+                                           const int32_t* __restrict__ start,
+                                           unsigned long long* total) {
+  __shared__ HuLds<SLICE, ROWCAP> L;
+  __shared__ unsigned long long red[TB / 64];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t ub = (uint32_t)start[blockIdx.x], ue = (uint32_t)start[blockIdx.x + 1];
+  unsigned long long cnt = 0;
+  uint32_t u = ub;
+  while (u < ue) {
+    if (tid == 0) {
+      uint32_t base = rp[u];
+      if (rp[u + 1] - base > SLICE) {
+        L.u2 = u;  // hub: its list does not fit the slice
+      } else {
+        uint32_t lo = u + 1, hi = min(ue, u + ROWCAP);
+        while (lo < hi) {
+          uint32_t mid = (lo + hi + 1) >> 1;
+          if (rp[mid] - base <= SLICE) lo = mid;
+          else hi = mid - 1;
+        }
+        L.u2 = lo;
+      }
+    }
+    __syncthreads();
+    const uint32_t u2 = L.u2;
+    if (u2 == u) {
+      // hub path: N+(u) stays in HBM/L2
+      const uint32_t ab = rp[u], du = rp[u + 1] - ab;
+      for (uint32_t k0 = 0; k0 < du; k0 += SLICE) {
+        uint32_t E = min((uint32_t)SLICE, du - k0);
+        uint32_t T = stage_edges(L, rp, col, ab + k0, E);
+        for (uint32_t t = tid; t < T; t += TB) {
+          uint32_t e = owner_of(L.pre, E, t);
+          uint32_t w = col[L.vst[e] + (t - L.pre[e])];
+          cnt += contains(col, ab, ab + du, w);
+        }
+        __syncthreads();
+      }
+      u = u + 1;
+      continue;
+    }
+    const uint32_t base = rp[u];
+    const uint32_t E = rp[u2] - base;
+    const uint32_t R = u2 - u;
+    for (uint32_t r = tid; r <= R; r += TB) L.rof[r] = rp[u + r] - base;
+    __syncthreads();
+    for (uint32_t e = tid; e < E; e += TB) {
+      uint32_t lo = 0, hi = R - 1;  // row r with rof[r] <= e < rof[r+1]
+      while (lo < hi) {
+        uint32_t mid = (lo + hi + 1) >> 1;
+        if (L.rof[mid] <= e) lo = mid;
+        else hi = mid - 1;
+      }
+      L.row[e] = (uint16_t)lo;
+    }
+    // stage_edges begins with a barrier-free pass that writes col/vst/pre,
+    // then synchronises; rows with d+(u) < 2 get no wedges.
+    uint32_t T = stage_edges(L, rp, col, base, E, true);
+    for (uint32_t t = tid; t < T; t += TB) {
+      uint32_t e = owner_of(L.pre, E, t);
+      uint32_t w = col[L.vst[e] + (t - L.pre[e])];
+      uint32_t r = L.row[e];
+      cnt += contains(L.col, L.rof[r], L.rof[r + 1], w);
+    }
+    __syncthreads();
+    u = u2;
+  }
+  flush_block(cnt, total + (blockIdx.x % kHuAcc) * kHuAccStride, red);
+}
+
 // Bisson's and TriCore's methods run on the kernels of lists16.h where the
 // graph is large enough for a first count, which builds the lists, not to lose
 // by it: at 1.4-1.5 * 10^6 edges (random geometric, average degree 24) a first
@@ -263,9 +418,47 @@ constexpr uint64_t kListEdges = 3u << 19, kListWedges = 1u << 26;
 // Fox's method: its bins take as long to build as the lists (first count, ER of 2 *
 // 10^4 edges 0.24 against 0.30 ms, R-MAT-14 of 5.5 * 10^4 0.50 against 0.25).
 constexpr uint64_t kFoxListEdges = 1u << 15;
+// Of more than kOnePart vertices, whose lists have two parts, from kFoxTailEdges on
+// (ER of 72,000 vertices and 4 * 10^5 edges, first count: 293 us over the bins, 624
+// over the lists; Barabasi-Albert, 99,354 and 6 * 10^5: 1,151 and 619).
+constexpr uint64_t kFoxTailEdges = 1u << 19;
+constexpr uint32_t kOnePart = 65535;
 
 static bool on_lists(const tc_graph* g) {
   return g->m_or >= kListEdges || g->sum_in_out >= kListWedges;
+}
+
+// Hu's and Fox's methods and the per-vertex counts keep their kernel over the CSR for
+// the first kFirstCounts counts of a smaller graph, whose lists cost as much as
+// about three of those counts: a graph that is counted once does not pay for
+// them, and one that is counted often pays no more than twice the better choice.
+// ER of 100,000 vertices and 8 * 10^5 edges, Hu: 138 us a count, 96 over the rows,
+// 601 with building them; per vertex 343, 143, 800.  ER of 20,000 and 1.6 * 10^5
+// edges, Hu: 96, 46, 228.  Rows that are there already are used at once.
+constexpr uint32_t kFirstCounts = 3;
+
+static bool often(uint32_t& counts) {
+  if (counts >= kFirstCounts) return true;
+  ++counts;
+  return false;
+}
+
+static bool rows_built(const tc_graph* g) {
+  return g->sc.l16.version == g->sched_version && g->sc.l16.usable;
+}
+
+static bool hu_rows(tc_graph* g) {
+  return on_lists(g) || rows_built(g) || often(g->sc.hu_counts);
+}
+
+static bool fox_rows(tc_graph* g) {
+  if (g->m_or < kFoxListEdges) return false;
+  return g->m_or >= kFoxTailEdges || g->n <= kOnePart || rows_built(g) || often(g->sc.fox_counts);
+}
+
+static bool vertex_rows(tc_graph* g) {
+  return g->n <= kOnePart || on_lists(g) || (rows_built(g) && g->sc.l16.credit) ||
+         often(g->sc.vertex_counts);
 }
 
 // ---- Bisson: wave per row, bitmap of N+(u) for long rows -----------------
@@ -433,6 +626,7 @@ static int ensure_version(tc_graph* g) {
     sc.wl_ok = false;
     sc.rows_ok = false;
     sc.fox_lanes = 0;
+    sc.hu_counts = sc.fox_counts = sc.vertex_counts = 0;
     sc.version = g->sched_version;
   }
   return TC_OK;
@@ -452,8 +646,9 @@ static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin);
 int per_vertex_counts(tc_ctx* c, tc_graph* g, unsigned long long* tri) {
   if (g->n == 0) return TC_OK;
   ensure_version(g);  // the task lists are those of the present CSR
-  TCX_TRY(lists16(c, g, true));
-  if (g->sc.l16.usable) {
+  const bool rows = vertex_rows(g);
+  if (rows) TCX_TRY(lists16(c, g, true));
+  if (rows && g->sc.l16.usable) {
     TCX_TRY(c->scratch.reserve(kCurBytes16));
     TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kCurBytes16, c->stream));
     TCX_HIP(hipMemsetAsync(tri, 0, 8 * (size_t)g->n, c->stream));
@@ -823,8 +1018,8 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   switch (s.kernel) {
     case TC_KERNEL_HU:
       TCX_TRY(hu_schedule(c, g, s.grid_size ? s.grid_size : 30000u));  // Hu/tc.cu:7
-      TCX_TRY(hu16(c, g, g->sc.hu_start.as<int32_t>(), g->sc.hu_nblocks));
-      on16 = true;
+      on16 = hu_rows(g);
+      if (on16) TCX_TRY(hu16(c, g, g->sc.hu_start.as<int32_t>(), g->sc.hu_nblocks));
       break;
     case TC_KERNEL_BISSON:
       on16 = !s.bitmap_min_deg && on_lists(g);  // the caller's bound is k_bisson's
@@ -840,7 +1035,7 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
         return fail(TC_ERR_ARG, "fox_max_lanes must be a power of two <= 64");
       if (s.fox_rearrange > 1) return fail(TC_ERR_ARG, "fox_rearrange must be 0 or 1");
       // (the caller's bins are k_fox's)
-      on16 = !s.fox_max_lanes && !s.fox_rearrange && g->m_or >= kFoxListEdges;
+      on16 = !s.fox_max_lanes && !s.fox_rearrange && fox_rows(g);
       if (on16) {
         TCX_TRY(lists16or32(c, g, &lists));
         break;
@@ -875,12 +1070,16 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
       break;
   }
   tm.ms_prep = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - prep0).count();
-  if (!on16) TCX_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long), c->stream));
-  if (on16) {
+  const bool spread = on16 || s.kernel == TC_KERNEL_HU;  // many accumulators (sum16)
+  if (spread) {
     TCX_TRY(c->scratch.reserve(kAccBytes16));
     TCX_HIP(hipMemsetAsync(c->scratch.p, 0, kAccBytes16, c->stream));
+  } else {
+    TCX_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long), c->stream));
+  }
+  unsigned long long* acc16 = c->scratch.as<unsigned long long>();
+  if (on16) {
     TCX_TRY(lm.mark());
-    unsigned long long* acc16 = c->scratch.as<unsigned long long>();
     const Push16& P = g->sc.push16;
     if (s.kernel == TC_KERNEL_HU)
       TCX_TRY(count_push16(c, g, P.hu_slice, P.hu_nslice, 0, acc16, &tm.launches));
@@ -889,6 +1088,13 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     else
       TCX_TRY(count16(c, *lists, s.grid_size, acc16, &tm.launches));
   } else switch (s.kernel) {
+    case TC_KERNEL_HU: {
+      TCX_TRY(lm.mark());
+      hipLaunchKernelGGL((k_hu<2048, 1024>), dim3(g->sc.hu_nblocks), dim3(TB), 0, c->stream, rp,
+                         col, g->sc.hu_start.as<int32_t>(), acc16);
+      tm.launches = 1;
+      break;
+    }
     case TC_KERNEL_BISSON: {
       uint32_t G = s.grid_size ? s.grid_size : (uint32_t)c->num_cus * 8u;
       uint32_t min_deg = s.bitmap_min_deg ? s.bitmap_min_deg : 64;
@@ -1025,7 +1231,7 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   TCX_HIP(hipGetLastError());
   TCX_TRY(lm.end());
   unsigned long long h = 0;
-  if (on16) {
+  if (spread) {
     unsigned long long part[kAccBytes16 / 8];
     TCX_TRY(fetch(c, part, c->scratch.p, kAccBytes16));
     h = sum16(part);

@@ -169,6 +169,8 @@ struct SchedCache {
   Lists16 l16;
   Lists16 l32;                     // all entries 32-bit (in tail); usable: with work lists
   Push16 push16;
+  // counts of this CSR so far that did without list rows (up to a bound)
+  uint32_t hu_counts = 0, fox_counts = 0, vertex_counts = 0;
   double wl_bytes = 0;             // bytes one count streams (see count.hip)
   bool rows_ok = false;
   DevBuf rows;                     // rows with d+ >= 2
