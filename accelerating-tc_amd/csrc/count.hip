@@ -447,6 +447,8 @@ static bool rows_built(const tc_graph* g) {
   return g->sc.l16.version == g->sched_version && g->sc.l16.usable;
 }
 
+static bool room(const tc_graph* g) { return g->sc.no_rows_version != g->sched_version; }
+
 static bool hu_rows(tc_graph* g) {
   return on_lists(g) || rows_built(g) || often(g->sc.hu_counts);
 }
@@ -700,6 +702,7 @@ static int block_starts(tc_ctx* c, tc_graph* g, DevBuf& w, uint32_t nblocks, Dev
 static int hu_schedule(tc_ctx* c, tc_graph* g, uint32_t nblocks) {
   SchedCache& sc = g->sc;
   if (sc.hu_nblocks == nblocks) return TC_OK;
+  sc.hu_nblocks = 0;  // (a build that fails leaves none)
   DevBuf w;
   TCX_TRY(w.reserve(8 * ((size_t)g->n + 1)));
   hipLaunchKernelGGL(k_hu_work, dim3(grid_for(16ull * g->n)), dim3(TB), 0, c->stream,
@@ -742,6 +745,7 @@ static void fox_thresholds(int max_work, uint32_t max_lanes, std::vector<int32_t
 static int fox_schedule(tc_ctx* c, tc_graph* g, uint32_t max_lanes, bool rearrange) {
   SchedCache& sc = g->sc;
   if (sc.fox_lanes == max_lanes && sc.fox_rearr == rearrange) return TC_OK;
+  sc.fox_lanes = 0;
   const uint64_t m = g->m_or;
   DevBuf w, bin, btmp, ids, itmp;
   TCX_TRY(w.reserve(4 * std::max<uint64_t>(m, 1)));
@@ -821,6 +825,7 @@ static int gather_flags(tc_ctx* c, const uint8_t* in, const uint32_t* idx, uint3
 static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin) {
   SchedCache& sc = g->sc;
   if (sc.auto_ok && sc.auto_wmax == wmax && sc.auto_hmin == hmin) return TC_OK;
+  sc.auto_ok = false;
   const uint32_t n = g->n;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
   DevBuf flags, key, ktmp, ids, itmp;
@@ -871,6 +876,7 @@ static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin) {
 static int wl_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin, uint32_t lmax) {
   SchedCache& sc = g->sc;
   if (sc.wl_ok && sc.wl_wmax == wmax && sc.wl_hmin == hmin && sc.wl_lmax == lmax) return TC_OK;
+  sc.wl_ok = false;
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
@@ -1015,19 +1021,25 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   // schedule (cached per graph; building one waits for the device, so the host
   // clock times it, and a cached one costs no event)
   const auto prep0 = std::chrono::steady_clock::now();
+  auto rows_or = [&](int st) {  // without room for the rows the method's own kernel counts
+    if (st == TC_OK) return st;
+    on16 = false;
+    return without_rows(g, st);
+  };
   switch (s.kernel) {
     case TC_KERNEL_HU:
       TCX_TRY(hu_schedule(c, g, s.grid_size ? s.grid_size : 30000u));  // Hu/tc.cu:7
-      on16 = hu_rows(g);
-      if (on16) TCX_TRY(hu16(c, g, g->sc.hu_start.as<int32_t>(), g->sc.hu_nblocks));
+      on16 = room(g) && hu_rows(g);
+      if (on16) TCX_TRY(rows_or(hu16(c, g, g->sc.hu_start.as<int32_t>(), g->sc.hu_nblocks)));
       break;
     case TC_KERNEL_BISSON:
-      on16 = !s.bitmap_min_deg && on_lists(g);  // the caller's bound is k_bisson's
-      TCX_TRY(on16 ? bisson16(c, g) : rows_schedule(c, g));
+      on16 = room(g) && !s.bitmap_min_deg && on_lists(g);  // the caller's bound is k_bisson's
+      if (on16) TCX_TRY(rows_or(bisson16(c, g)));
+      if (!on16) TCX_TRY(rows_schedule(c, g));
       break;
     case TC_KERNEL_TRICORE:
-      on16 = s.tricore_parts <= 1 && on_lists(g);  // a pass of several spans two ranges
-      if (on16) TCX_TRY(lists16or32(c, g, &lists));
+      on16 = room(g) && s.tricore_parts <= 1 && on_lists(g);  // a pass of several spans two ranges
+      if (on16) TCX_TRY(rows_or(lists16or32(c, g, &lists)));
       break;
     case TC_KERNEL_FOX: {
       uint32_t L = s.fox_max_lanes ? s.fox_max_lanes : 64;
@@ -1035,12 +1047,9 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
         return fail(TC_ERR_ARG, "fox_max_lanes must be a power of two <= 64");
       if (s.fox_rearrange > 1) return fail(TC_ERR_ARG, "fox_rearrange must be 0 or 1");
       // (the caller's bins are k_fox's)
-      on16 = !s.fox_max_lanes && !s.fox_rearrange && fox_rows(g);
-      if (on16) {
-        TCX_TRY(lists16or32(c, g, &lists));
-        break;
-      }
-      TCX_TRY(fox_schedule(c, g, L, s.fox_rearrange == 1));
+      on16 = room(g) && !s.fox_max_lanes && !s.fox_rearrange && fox_rows(g);
+      if (on16) TCX_TRY(rows_or(lists16or32(c, g, &lists)));
+      if (!on16) TCX_TRY(fox_schedule(c, g, L, s.fox_rearrange == 1));
       break;
     }
     case TC_KERNEL_AUTO: {

@@ -125,6 +125,9 @@ struct Rows16 {
   DevBuf slice;                    // uint2[nslice + 1]: first (task, entry) of each slice
   uint64_t units = 0, entries = 0, tasks = 0;
   uint32_t nslice = 0;
+  void release() {
+    for (DevBuf* b : {&row, &col, &se, &who, &cred, &act, &slice}) b->release();
+  }
 };
 struct Lists16 {
   uint64_t version = ~0ull;        // the CSR it was built (or found unsuitable) for
@@ -133,6 +136,12 @@ struct Lists16 {
   bool listed = false;             // with the hub's work lists (else id and cnt to build them)
   DevBuf id, cnt;                  // uint16[n] 16-bit ids (none: all are their own), uint32[n]
   Rows16 hub, tail;                // entries with 16-bit ids, the others (32-bit)
+  void release() {
+    usable = false;
+    for (DevBuf* b : {&id, &cnt}) b->release();
+    hub.release();
+    tail.release();
+  }
 };
 
 // Push lists (a task streams the rows of all its out-neighbours) over the hub
@@ -144,6 +153,10 @@ struct Push16 {
   uint64_t tasks = 0;
   DevBuf hu_slice, slice;
   uint32_t hu_blocks = 0, hu_nslice = 0, nslice = 0;
+  void release() {
+    version = ~0ull;
+    for (DevBuf* b : {&se, &act, &hu_slice, &slice}) b->release();
+  }
 };
 
 // Per-graph schedules, rebuilt when the oriented CSR changes.
@@ -169,6 +182,7 @@ struct SchedCache {
   Lists16 l16;
   Lists16 l32;                     // all entries 32-bit (in tail); usable: with work lists
   Push16 push16;
+  uint64_t no_rows_version = ~0ull;  // the CSR that l32 or push16 found no room for
   // counts of this CSR so far that did without list rows (up to a bound)
   uint32_t hu_counts = 0, fox_counts = 0, vertex_counts = 0;
   double wl_bytes = 0;             // bytes one count streams (see count.hip)
@@ -288,11 +302,15 @@ int graph_clone_records(tc_ctx* c, const tc_graph* g, tc_graph** out);
 int worklists(tc_ctx* c, tc_graph* g);
 
 // ---- the 16-bit list layer (lists16.hip) -----------------------------------
-// Builds (or keeps) g's layer when its lists suit it (g->sc.l16.usable).
-// credit: for per-vertex counts too.
+// Builds (or keeps) g's layer when its lists suit it and there is memory for it
+// (g->sc.l16.usable).  credit: for per-vertex counts too.
 int lists16(tc_ctx* c, tc_graph* g, bool credit = false);
 // The layer where usable, else (l32) the same over 32-bit rows of all entries.
 int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use);
+// After a failure of lists16or32, hu16 or bisson16: where the rows have no room
+// (memory, or 2^32 units) they are let go, the CSR is counted without them
+// from now on, and the status is TC_OK.
+int without_rows(tc_graph* g, int status);
 // Enqueues the count over them; acc: kAccBytes16 bytes, cleared; sum16 adds the
 // copied-back accumulators.
 constexpr size_t kAccBytes16 = 8 * 64 * 16;

@@ -542,8 +542,10 @@ int build(tc_ctx* c, tc_graph* g, DevBuf& idbuf, bool id_all, bool credit, bool 
 
 }  // namespace
 
+static bool no_room(int status) { return status == TC_ERR_NOMEM || status == TC_ERR_RANGE; }
+
 // The rows, and (lists) the hub's work lists, which the push methods do without.
-static int layer16(tc_ctx* c, tc_graph* g, bool credit, bool lists) {
+static int build_layer16(tc_ctx* c, tc_graph* g, bool credit, bool lists) {
   Lists16& L = g->sc.l16;
   if (L.version == g->sched_version && (!L.usable || L.credit || !credit)) {
     if (L.usable && lists && !L.listed) TCX_TRY(hub_lists(c, g, L));
@@ -561,7 +563,27 @@ static int layer16(tc_ctx* c, tc_graph* g, bool credit, bool lists) {
   return TC_OK;
 }
 
+// A layer that there is no room for does not suit the graph: every count has a
+// kernel that needs less.
+static int layer16(tc_ctx* c, tc_graph* g, bool credit, bool lists) {
+  const int st = build_layer16(c, g, credit, lists);
+  if (!no_room(st)) return st;
+  g->sc.l16.release();
+  g->sc.push16.release();  // (over its rows)
+  g->sc.l16.version = g->sched_version;
+  return TC_OK;
+}
+
 int lists16(tc_ctx* c, tc_graph* g, bool credit) { return layer16(c, g, credit, true); }
+
+int without_rows(tc_graph* g, int status) {
+  if (!no_room(status)) return status;
+  g->sc.push16.release();
+  g->sc.l32.release();
+  g->sc.l32.version = ~0ull;
+  g->sc.no_rows_version = g->sched_version;
+  return TC_OK;
+}
 
 int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* voff) {
   Lists16& L = g->sc.l16;
@@ -569,12 +591,16 @@ int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* v
   L.usable = false;
   if (g->n && g->m_or) {
     DevBuf id;
-    TCX_TRY(id.reserve(2 * (size_t)g->n));
-    hipLaunchKernelGGL(k_local_ids, dim3(grid_for(g->n)), dim3(TB), 0, c->stream, gid, voff, g->n,
-                       id.as<uint16_t>());
-    TCX_HIP(hipGetLastError());
-    TCX_TRY(build(c, g, id, true, false, true, L));
-    if (L.hub.tasks)
+    int st = id.reserve(2 * (size_t)g->n);
+    if (st == TC_OK) {
+      hipLaunchKernelGGL(k_local_ids, dim3(grid_for(g->n)), dim3(TB), 0, c->stream, gid, voff, g->n,
+                         id.as<uint16_t>());
+      TCX_HIP(hipGetLastError());
+      st = build(c, g, id, true, false, true, L);
+    }
+    if (no_room(st)) L.release();
+    else TCX_TRY(st);
+    if (L.usable && L.hub.tasks)
       hipLaunchKernelGGL(k_graph_of, dim3(grid_for(L.hub.tasks)), dim3(TB), 0, c->stream,
                          L.hub.who.as<uint32_t>(), L.hub.tasks, gid);
     TCX_HIP(hipGetLastError());
