@@ -703,6 +703,7 @@ static int hu_schedule(tc_ctx* c, tc_graph* g, uint32_t nblocks) {
   SchedCache& sc = g->sc;
   if (sc.hu_nblocks == nblocks) return TC_OK;
   sc.hu_nblocks = 0;  // (a build that fails leaves none)
+  ++sc.builds;
   DevBuf w;
   TCX_TRY(w.reserve(8 * ((size_t)g->n + 1)));
   hipLaunchKernelGGL(k_hu_work, dim3(grid_for(16ull * g->n)), dim3(TB), 0, c->stream,
@@ -716,6 +717,7 @@ static int hu_schedule(tc_ctx* c, tc_graph* g, uint32_t nblocks) {
 static int rows_schedule(tc_ctx* c, tc_graph* g) {
   SchedCache& sc = g->sc;
   if (sc.rows_ok) return TC_OK;
+  ++sc.builds;
   DevBuf flags;
   TCX_TRY(flags.reserve((size_t)g->n + 1));
   TCX_TRY(sc.rows.reserve(4 * ((size_t)g->n + 1)));
@@ -746,6 +748,7 @@ static int fox_schedule(tc_ctx* c, tc_graph* g, uint32_t max_lanes, bool rearran
   SchedCache& sc = g->sc;
   if (sc.fox_lanes == max_lanes && sc.fox_rearr == rearrange) return TC_OK;
   sc.fox_lanes = 0;
+  ++sc.builds;
   const uint64_t m = g->m_or;
   DevBuf w, bin, btmp, ids, itmp;
   TCX_TRY(w.reserve(4 * std::max<uint64_t>(m, 1)));
@@ -826,6 +829,7 @@ static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin) {
   SchedCache& sc = g->sc;
   if (sc.auto_ok && sc.auto_wmax == wmax && sc.auto_hmin == hmin) return TC_OK;
   sc.auto_ok = false;
+  ++sc.builds;
   const uint32_t n = g->n;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
   DevBuf flags, key, ktmp, ids, itmp;
@@ -877,6 +881,7 @@ static int wl_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin, uin
   SchedCache& sc = g->sc;
   if (sc.wl_ok && sc.wl_wmax == wmax && sc.wl_hmin == hmin && sc.wl_lmax == lmax) return TC_OK;
   sc.wl_ok = false;
+  ++sc.builds;
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
   const uint32_t* rp = g->rowptr.as<uint32_t>();
@@ -1018,9 +1023,11 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
   LaunchMarks lm(c);
   bool on16 = false;  // counted by the kernels of lists16.h
   const Lists16* lists = &g->sc.l16;
-  // schedule (cached per graph; building one waits for the device, so the host
-  // clock times it, and a cached one costs no event)
+  // schedule (cached per graph, and a cached one costs no event: the host clock
+  // times the call, and what a call that builds one does not spend in the count
+  // is its preparation)
   const auto prep0 = std::chrono::steady_clock::now();
+  const uint64_t builds0 = g->sc.builds;
   auto rows_or = [&](int st) {  // without room for the rows the method's own kernel counts
     if (st == TC_OK) return st;
     on16 = false;
@@ -1078,7 +1085,8 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     default:
       break;
   }
-  tm.ms_prep = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - prep0).count();
+  const bool built = g->sc.builds != builds0;
+  if (!built) tm.ms_prep = ms_since(prep0);
   const bool spread = on16 || s.kernel == TC_KERNEL_HU;  // many accumulators (sum16)
   if (spread) {
     TCX_TRY(c->scratch.reserve(kAccBytes16));
@@ -1248,6 +1256,7 @@ int tc_count(tc_ctx* c, tc_graph* g, const tc_sched* sched_in, uint64_t* count,
     TCX_TRY(fetch(c, &h, acc, 8));
   }
   TCX_TRY(lm.finish(&tm));
+  if (built) tm.ms_prep = ms_since(prep0) - tm.ms_count;
   *count = h;
   if (timing) *timing = tm;
   return TC_OK;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <memory>
@@ -193,7 +194,7 @@ struct SchedCache {
   bool fox_rearr = false;
   DevBuf fox_eids;                 // edge ids grouped by lanes-per-edge bin
   std::vector<uint64_t> fox_off;   // bin offsets (bins+1)
-  float ms_prep = 0;
+  uint64_t builds = 0;             // schedules built so far (each waits for the device)
   // learned schedule (per model id)
   uint64_t learned_version = ~0ull, learned_model = ~0ull;
   DevBuf l_blk, l_wav, l_huge, l_lan;
@@ -335,23 +336,46 @@ int lists16_batch(tc_ctx* c, tc_graph* g, const uint32_t* gid, const uint32_t* v
 int count16_graphs(tc_ctx* c, tc_graph* g, uint32_t grid, uint32_t* cursor,
                    unsigned long long* counts);
 
-// Event marks between consecutive count launches: mark() before each launch,
-// end() after the last; finish(), once the stream has been waited for, gives
-// the total and the longest launch.
+inline float ms_since(std::chrono::steady_clock::time_point t0) {
+  return std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
+}
+
+// Event marks around count launches: mark() before each launch, stop() where
+// other work follows one (else the next mark ends its interval), end() after
+// the last; finish(), once the stream has been waited for, gives the total and
+// the longest launch.
 struct LaunchMarks {
   tc_ctx* c;
-  int n = 0;
+  int n = 0;                // intervals
+  int ev = 0;               // events recorded
+  int first[16], last[16];  // an interval's events
+  bool open = false;
   explicit LaunchMarks(tc_ctx* cc) : c(cc) {}
+  int record() {
+    if (!c->lev[ev]) TCX_HIP(hipEventCreate(&c->lev[ev]));
+    TCX_HIP(hipEventRecord(c->lev[ev], c->stream));
+    return TC_OK;
+  }
   int mark() {
-    if (n >= 16) return TC_OK;  // later launches fold into the last interval
-    if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
-    TCX_HIP(hipEventRecord(c->lev[n], c->stream));
-    ++n;
+    if (ev >= 16) return TC_OK;  // later launches fold into the last interval
+    TCX_TRY(record());
+    if (open) last[n - 1] = ev;
+    first[n++] = ev++;
+    open = true;
+    return TC_OK;
+  }
+  int stop() {
+    if (!open || ev >= 16) return TC_OK;
+    TCX_TRY(record());
+    last[n - 1] = ev++;
+    open = false;
     return TC_OK;
   }
   int end() {
-    if (!c->lev[n]) TCX_HIP(hipEventCreate(&c->lev[n]));
-    TCX_HIP(hipEventRecord(c->lev[n], c->stream));
+    if (!open) return TC_OK;
+    TCX_TRY(record());
+    last[n - 1] = ev;
+    open = false;
     return TC_OK;
   }
   int finish(tc_timing* tm) {
@@ -359,7 +383,7 @@ struct LaunchMarks {
     tm->ms_dominant = 0;
     for (int i = 0; i < n; ++i) {
       float ms = 0;
-      TCX_HIP(hipEventElapsedTime(&ms, c->lev[i], c->lev[i + 1]));
+      TCX_HIP(hipEventElapsedTime(&ms, c->lev[first[i]], c->lev[last[i]]));
       tm->ms_count += ms;
       if (ms > tm->ms_dominant) {
         tm->ms_dominant = ms;

@@ -919,7 +919,7 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
   TCX_HIP(hipMemsetAsync(acc, 0, claim_bytes, c->stream));
   uint32_t* groups = reinterpret_cast<uint32_t*>(acc + 16);
   LaunchMarks lm(c);
-  int widths[17];
+  int widths[16];
   for (const Bucket& b : buckets) {
     uint32_t lo = std::max(b.lo, need);
     if (lo > b.hi) continue;
@@ -956,11 +956,11 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       order = sv;
     }
     unsigned long long* claim = acc + 1 + tm.launches;
-    widths[lm.n] = b.w;
     if (b.w == 0) {
       uint32_t G = (uint32_t)std::min<uint64_t>(nr, (uint64_t)c->num_cus * 8);
       uint32_t maxd = std::max<uint32_t>(g->max_out, 1);
       uint32_t slots = k > 3 ? k - 3 : 1;
+      TCX_TRY(lm.stop());
       TCX_TRY(scratch.reserve(4ull * G * slots * maxd));
       TCX_TRY(lm.mark());
       // cost: CU-microseconds (one wave of the num_cus * 8 holds 1/8 of a CU)
@@ -999,6 +999,7 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
           (uint32_t)std::min<uint64_t>(max_copies, std::max<uint64_t>(1, (4 * slots + nr - 1) / nr));
       const uint32_t G = (uint32_t)std::min<uint64_t>(nr * copies, slots);
       const uint64_t D = 64ull * b.w;
+      TCX_TRY(lm.stop());
       TCX_TRY(scratch.reserve(8ull * G * nw * (D + 1) * (2ull * b.w + 1)));
       uint64_t* stk = scratch.as<uint64_t>();
       const uint32_t* rts = order;
@@ -1025,6 +1026,8 @@ int kcl_run(tc_ctx* c, tc_graph* g, uint32_t k, int variant, const KclPlan* plan
       }
     }
     TCX_HIP(hipGetLastError());
+    widths[lm.n - 1] = b.w;
+    if (!ordered) TCX_TRY(lm.stop());  // the next bucket's roots are selected in between
     tm.launches++;
   }
   TCX_TRY(lm.end());

@@ -475,6 +475,7 @@ int work_lists(tc_ctx* c, tc_graph* g, const uint32_t* cnt, const uint16_t* id, 
 
 // The hub's work lists of a layer built without them.
 int hub_lists(tc_ctx* c, tc_graph* g, Lists16& L) {
+  ++g->sc.builds;
   TCX_TRY(work_lists(c, g, L.cnt.as<uint32_t>(), L.id.as<uint16_t>(), false, L.credit, L.hub));
   L.id.release();
   L.cnt.release();
@@ -551,6 +552,7 @@ static int build_layer16(tc_ctx* c, tc_graph* g, bool credit, bool lists) {
     if (L.usable && lists && !L.listed) TCX_TRY(hub_lists(c, g, L));
     return TC_OK;
   }
+  ++g->sc.builds;
   L.version = ~0ull;
   L.usable = false;
   if (g->n && g->m_or) {
@@ -694,6 +696,7 @@ int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use) {
   Lists16& L = g->sc.l32;
   *use = &L;
   if (L.version == g->sched_version && L.usable) return TC_OK;
+  ++g->sc.builds;
   DevBuf cnt;
   TCX_TRY(rows32(c, g, cnt));
   TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), nullptr, false, false, L.tail));
@@ -712,6 +715,7 @@ int push16(tc_ctx* c, tc_graph* g) {
   Push16& H = g->sc.push16;
   TCX_TRY(layer16(c, g, false, false));
   if (H.version == g->sched_version) return TC_OK;
+  ++g->sc.builds;
   const bool b16 = g->sc.l16.usable;
   const uint32_t n = g->n;
   const uint64_t m = g->m_or;
@@ -740,6 +744,7 @@ int push16(tc_ctx* c, tc_graph* g) {
 
 static int edge_slices(tc_ctx* c, tc_graph* g, const int32_t* start, uint32_t nblocks,
                        uint32_t parts, DevBuf& slice, uint32_t* nslice) {
+  ++g->sc.builds;
   const Push16& H = g->sc.push16;
   const uint32_t ns = nblocks * parts;
   *nslice = 0;

@@ -138,7 +138,8 @@ typedef struct tc_sched {
 
 typedef struct tc_timing {
   float ms_count;           /* hipEvent time of the count kernels only           */
-  float ms_prep;            /* schedule building (work model, bins) on device    */
+  float ms_prep;            /* building schedules and lists: what the first call
+                               on a CSR does not spend in the count; ~0 once kept */
   uint32_t launches;        /* count-kernel launches                             */
   uint32_t dominant_kernel; /* index of the kernel with the most time            */
   float ms_dominant;        /* its hipEvent time                                 */
