@@ -513,11 +513,17 @@ int tc_graph_orient_learned(tc_ctx* ctx, tc_graph* g, int mode, tc_model* m, int
                             double* predicted_us, double* adir_cost);
 /* Variant chosen for each vertex's task (TC_VARIANT_*, 255 = no task): the
  * cell's choice within the task's limits (above).  model NULL gives the
- * fixed rule's variants (tc_count's AUTO work-list schedule). */
+ * fixed rule's variants (tc_count's AUTO 32-bit work-list schedule). */
 int tc_learned_assignment(tc_ctx* ctx, tc_graph* g, tc_model* m, uint8_t* variant);
-/* Exact count with the learned schedule (block tasks by descending work, as
- * the fixed rule orders them; wave and lane tasks in id order); model NULL
- * counts with the fixed rule (tc_count, TC_KERNEL_AUTO). */
+/* Exact count with the learned schedule.  A graph that AUTO counts over 16-bit
+ * list rows (at most 65,535 vertices, or most entries in that many targets) is
+ * counted over them whatever the model predicts: they have one split of the
+ * work, into equal slices.  The model schedules the 32-bit work-list tasks of
+ * the other graphs (block tasks by descending work, as the fixed rule orders
+ * them; wave and lane tasks in id order).  Its predictions (tc_learned_cells,
+ * tc_graph_orient_learned) are of those tasks on every graph.  model NULL counts
+ * with those tasks under the fixed rule, also where AUTO uses the rows
+ * (tc_count, TC_KERNEL_AUTO with auto_thresholds[0] = 64). */
 int tc_count_learned(tc_ctx* ctx, tc_graph* g, tc_model* m, uint64_t* count,
                      tc_timing* timing);
 
@@ -602,7 +608,7 @@ int kcl_gpu_solver(const char* path, uint32_t k, uint64_t* total, size_t n_chunk
  * No counterpart in the reference (k-clique/kcl.cu runs one path for every
  * root).  The cost model of tc_model_* (8 features -> 2 log2 costs) is
  * trained on per-root costs measured by the kernels themselves and picks,
- * per root, the LDS bit-matrix pivot path or the merge path.  The count is
+ * per root, the bit-matrix path or the merge path.  The count is
  * exact whatever the model predicts. */
 /* Per-root features X[n][8] for k (zero for roots with d+ < k-1):
  * log2(1+d+), log2(1+m) with m the edges of the sub-graph of N+(u),
@@ -613,13 +619,14 @@ int kcl_gpu_solver(const char* path, uint32_t k, uint64_t* total, size_t n_chunk
 int kcl_root_features(tc_ctx* ctx, tc_graph* g, uint32_t k, float* X);
 /* Measured cost of every root on one path, in CU-microseconds (the root's
  * time times the share of a CU its workgroup holds); 0 where not measured.
- * KCL_VARIANT_PIVOT measures the roots with k-1 <= d+ <= 1024,
- * KCL_VARIANT_MERGE every root with d+ >= k-1; count (optional) receives
- * the k-cliques of the measured roots. */
+ * KCL_VARIANT_PIVOT measures the roots with k-1 <= d+ <= 1024 on the kernel over
+ * bit matrices that a plan runs them on (for k <= 5 and d+ <= 512 the direct one,
+ * else pivoting), KCL_VARIANT_MERGE every root with d+ >= k-1; count (optional)
+ * receives the k-cliques of the measured roots. */
 int kcl_measure_costs(tc_ctx* ctx, tc_graph* g, uint32_t k, int variant, float* cost_us,
                       uint64_t* count);
-/* Path per root (0 pivot, 1 merge, 255 none: d+ < k-1).  The fixed rule
- * (pivot iff d+ <= 1024) is the prior: a root moves to the merge path only
+/* Path per root (0 bit matrix, 1 merge, 255 none: d+ < k-1).  The fixed rule
+ * (bit matrix iff d+ <= 1024) is the prior: a root moves to the merge path only
  * for a predicted saving above 25 %. */
 int kcl_learned_plan(tc_ctx* ctx, tc_graph* g, uint32_t k, tc_model* m, uint8_t* path);
 /* Exact k-clique count (3 <= k <= 12) with the learned plan; each launch
