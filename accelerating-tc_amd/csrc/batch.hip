@@ -449,6 +449,10 @@ int tc_batch_stream_bytes(tc_ctx* c, tc_batch* b, double* bytes) {
   PoolScope scope(c);
   TCX_TRY(check_batch(c, b));
   if (!bytes) return fail(TC_ERR_ARG, "NULL output");
+  if (b->ids16) {
+    TCX_TRY(lists16_batch(c, b->g, b->gid.as<uint32_t>(), b->d_voff.as<uint32_t>()));
+    if (b->g->sc.l16.usable) return rows_bytes(c, b->g->sc.l16, bytes);
+  }
   return tc_auto_stream_bytes(c, b->g, nullptr, bytes);
 }
 

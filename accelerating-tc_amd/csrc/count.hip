@@ -1289,6 +1289,20 @@ int tc_auto_stream_bytes(tc_ctx* c, tc_graph* g, const tc_sched* sched, double* 
   return TC_OK;
 }
 
+int tc_count_stream_bytes(tc_ctx* c, tc_graph* g, double* bytes, int* rows) {
+  PoolScope scope(c);
+  TCX_TRY(check_ready(c, g));
+  if (!bytes) return fail(TC_ERR_ARG, "NULL output");
+  *bytes = 0;
+  if (rows) *rows = 0;
+  if (g->m_or == 0 || g->n == 0) return TC_OK;
+  ensure_version(g);
+  TCX_TRY(lists16(c, g));
+  if (!g->sc.l16.usable) return tc_auto_stream_bytes(c, g, nullptr, bytes);
+  if (rows) *rows = 1;
+  return rows_bytes(c, g->sc.l16, bytes);
+}
+
 int tc_count_per_vertex(tc_ctx* c, tc_graph* g, uint64_t* tri) {
   PoolScope scope(c);
   TCX_TRY(check_ready(c, g));

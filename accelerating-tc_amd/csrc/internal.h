@@ -308,6 +308,8 @@ int worklists(tc_ctx* c, tc_graph* g);
 int lists16(tc_ctx* c, tc_graph* g, bool credit = false);
 // The layer where usable, else (l32) the same over 32-bit rows of all entries.
 int lists16or32(tc_ctx* c, tc_graph* g, const Lists16** use);
+// Bytes that one count over a layer with work lists streams.
+int rows_bytes(tc_ctx* c, const Lists16& L, double* bytes);
 // After a failure of lists16or32, hu16 or bisson16: where the rows have no room
 // (memory, or 2^32 units) they are let go, the CSR is counted without them
 // from now on, and the status is TC_OK.

@@ -543,6 +543,34 @@ int build(tc_ctx* c, tc_graph* g, DevBuf& idbuf, bool id_all, bool credit, bool 
 
 }  // namespace
 
+// Bytes that one count over R streams: *sum += 16 per unit of every task's own row
+// and of every list, 8 per work-list entry, 16 per task.
+static __global__ __launch_bounds__(TB) void k_rows_bytes(const uint2* __restrict__ se,
+                                                          uint64_t entries,
+                                                          const uint4* __restrict__ act,
+                                                          uint64_t tasks, unsigned long long* sum) {
+  __shared__ unsigned long long red[TB / 64];
+  unsigned long long s = 0;
+  for (uint64_t i = gtid(); i < entries; i += gstride()) s += 8ull + 16ull * se[i].y;
+  for (uint64_t i = gtid(); i < tasks; i += gstride()) s += 16ull + 16ull * act[i].w;
+  flush_block(s, sum, red);
+}
+
+int rows_bytes(tc_ctx* c, const Lists16& L, double* bytes) {
+  TCX_TRY(c->accum.reserve(64));
+  TCX_HIP(hipMemsetAsync(c->accum.p, 0, 8, c->stream));
+  for (const Rows16* R : {&L.hub, &L.tail})
+    if (R->tasks)
+      hipLaunchKernelGGL(k_rows_bytes, dim3(std::min<unsigned>(grid_for(R->entries), c->num_cus * 8u)),
+                         dim3(TB), 0, c->stream, R->se.as<uint2>(), R->entries, R->act.as<uint4>(),
+                         R->tasks, c->accum.as<unsigned long long>());
+  TCX_HIP(hipGetLastError());
+  unsigned long long h = 0;
+  TCX_TRY(read_back(c, c->accum.p, &h));
+  *bytes = (double)h;
+  return TC_OK;
+}
+
 static bool no_room(int status) { return status == TC_ERR_NOMEM || status == TC_ERR_RANGE; }
 
 // The rows, and (lists) the hub's work lists, which the push methods do without.

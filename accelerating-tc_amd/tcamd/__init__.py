@@ -158,6 +158,7 @@ _sig("tc_count_per_vertex", C.c_int, [_vp, _vp, _u64p])
 _sig("tc_batch_stream_bytes", C.c_int, [_vp, _vp, C.POINTER(C.c_double)])
 _sig("tc_graph_save_csr", C.c_int, [_vp, C.c_char_p])
 _sig("tc_graph_load_csr", C.c_int, [_vp, C.c_char_p, C.POINTER(_vp)])
+_sig("tc_count_stream_bytes", C.c_int, [_vp, _vp, C.POINTER(C.c_double), C.POINTER(C.c_int)])
 _sig("tc_auto_stream_bytes", C.c_int, [_vp, _vp, C.c_void_p, C.POINTER(C.c_double)])
 _sig("tc_count_csr_noalloc", C.c_int, [_vp, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32,
                                        C.c_void_p])
@@ -242,7 +243,7 @@ EXPORTED = [
     "tc_measure_valu_rate", "tc_bw_model_fit",
     "tc_graph_get_csr", "tc_graph_get_edges", "tc_graph_get_vertex_key", "tc_graph_device_csr",
     "tc_hu_workload", "tc_hu_block_starts", "tc_fox_workload", "tc_fox_bin_sizes", "tc_count",
-    "tc_count_per_vertex", "tc_auto_stream_bytes", "tc_cost_functions", "tc_approx_ratio", "kcl_count", "kcl_gpu_solver",
+    "tc_count_per_vertex", "tc_count_stream_bytes", "tc_auto_stream_bytes", "tc_cost_functions", "tc_approx_ratio", "kcl_count", "kcl_gpu_solver",
     "kcl_root_features", "kcl_measure_costs", "kcl_learned_plan", "kcl_count_learned",
     "kcl_count_roots",
     "tc_tricore_init_gpu",
@@ -685,8 +686,17 @@ class Graph:
                 setattr(s, k, v)
         return s
 
+    def count_stream_bytes(self):
+        """(bytes that a default AUTO or learned count streams, whether it runs
+        over 16-bit list rows) (tc_count_stream_bytes)."""
+        out, rows = C.c_double(), C.c_int()
+        _check(_lib.tc_count_stream_bytes(self.ctx.handle, self._h, C.byref(out), C.byref(rows)),
+               "tc_count_stream_bytes")
+        return out.value, bool(rows.value)
+
     def auto_stream_bytes(self, **sched) -> float:
-        """Bytes one AUTO count streams under the schedule (tc_auto_stream_bytes)."""
+        """Bytes one AUTO count streams over the 32-bit lists under the schedule
+        (tc_auto_stream_bytes)."""
         s = self._sched(KERNEL_AUTO, sched)
         out = C.c_double()
         _check(_lib.tc_auto_stream_bytes(self.ctx.handle, self._h, C.byref(s), C.byref(out)),

@@ -16,11 +16,11 @@ same configuration set on the same line: Barabasi-Albert n = 2^24, m = 8
 
 Prints ONE JSON line.  `value` = TC edges/s of the head engine (the learned
 schedule when a trained cost model is present, else AUTO): oriented edges /
-count time, wall clock over K steps (the plain methods, 5-20x slower, are
-timed over min(K, 5) steps after one warm-up).  `roofline.achieved` = the
-head kernel's own streamed bytes per count, 4(n+1) + 12m+ + 4 sum_v d-(v) d+(v)
-(row offsets, each out-list once, and for every edge u->v the bounds and the
-list of v), over the hipEvent time of the count launch.  The `batched` workload counts 4,096
+count time, wall clock over K steps (the plain methods are timed over min(K, 5)
+steps after one warm-up; on large graphs they too run over 16-bit list rows, Fox's
+and TriCore's over AUTO's own lists).  `roofline.achieved` = the bytes that the
+head engine's count streams (tc_count_stream_bytes) over the hipEvent time of
+the count launches.  The `batched` workload counts 4,096
 small graphs (vertex counts log-uniform in [64, 65536], average degree
 uniform in [4, 64], 1/3 each Erdos-Renyi / R-MAT / random geometric, seed 5)
 with one hipGraph replay per step and reports the one-launch-per-graph
@@ -40,13 +40,6 @@ sys.path.insert(0, os.path.join(ROOT, "accelerating-tc_amd"))
 HBM_PEAK_GBPS = 8000.0
 METRIC = "TC edges/s + HBM GB/s % peak; learned/batched vs plain HIP, exact counts"
 KERNELS = ["hu", "bisson", "fox", "tricore", "auto", "learned"]
-KERNEL_SYMBOL = {
-    "hu": "k_count16", "bisson": "k_count16", "fox": "k_count16",
-    "tricore": "k_count16", "auto": "k_count16", "learned": "k_count16",
-}
-# Bytes per streamed list entry of the head kernel: 2 where the graph is counted
-# over 16-bit rows (k_count16), 4 over the 32-bit work lists (k_auto_wl).
-ENTRY_BYTES = {"ba24": 4}
 
 WORKLOADS = {
     "rmat22": dict(kind="rmat", scale=22, ef=16, seed=22, aorder=True, orient="adir"),
@@ -232,15 +225,13 @@ def run_batched(args, w, steps, warmup, with_cpu):
     m = info.m_oriented
     stream = b.stream_bytes()
     log(f"[bench] union n={info.n} m={m} max_out={info.max_out_degree} "
-        f"B_alg={info.bytes_alg/1e9:.2f} GB work-list stream {stream/1e9:.2f} GB prep {t_prep:.1f}s")
+        f"B_alg={info.bytes_alg/1e9:.2f} GB streams {stream/1e9:.2f} GB a count, prep {t_prep:.1f}s")
     t0 = time.perf_counter()
     sched = b.autotune()
     t_tune = time.perf_counter() - t0
     stream = b.stream_bytes(sched.form)  # the bytes of the chosen form
-    # k_count16 counts batches of graphs of at most 65,535 vertices: 2 bytes an entry
-    on16 = max(max(int(g[0].max()), int(g[1].max())) for g in graphs if len(g[0])) < 65535
-    if on16:
-        stream /= 2
+    # k_count16 counts batches of graphs of at most 65,535 vertices
+    on16 = sched.form == tcamd.BATCH_WORKLIST and max(g[2] for g in graphs) <= 65535
     log(f"[bench] autotune {sched.as_dict()} in {t_tune:.1f}s; the chosen form streams "
         f"{stream/1e9:.2f} GB")
 
@@ -303,9 +294,10 @@ def main_batched(args, w):
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBPS, "traffic": load_traffic("batched", "batched"),
             "kernel": "k_count16" if r["on16"] else "k_batch<2048>", "bytes_per_count": kb,
-            "bytes_rule": "work-list form: tc_batch_stream_bytes (per task 20 + 4 d+(x), per "
-                          "work-list entry 8 + 4 d+(y)); push form: 4(n+1) + 12 m+ + "
-                          "4 sum d- d+; half of it over 16-bit rows",
+            "bytes_rule": "work-list form: tc_batch_stream_bytes (over 16-bit rows 16 per unit "
+                          "of every own and streamed row, 8 per entry, 16 per task; else per "
+                          "task 20 + 4 d+(x), per work-list entry 8 + 4 d+(y)); push form: "
+                          "4(n+1) + 12 m+ + 4 sum d- d+",
             "bytes_push_form": kernel_bytes(info),
             "bytes_alg_edge_model": info.bytes_alg,
         },
@@ -525,9 +517,9 @@ def run_triangles(args, w, kernels, with_cpu):
     t_prep = time.perf_counter() - t0
     info = g.info()
     m = info.m_oriented
-    stream = g.auto_stream_bytes()  # the work-list schedule's bytes per count
+    stream, on16 = g.count_stream_bytes()  # the head engine's bytes per count
     log(f"[bench] n={info.n} m={m} max_out={info.max_out_degree} B_alg={info.bytes_alg/1e9:.2f} GB "
-        f"work-list stream {stream/1e9:.2f} GB (push form {kernel_bytes(info)/1e9:.2f} GB) "
+        f"streams {stream/1e9:.2f} GB a count (push form {kernel_bytes(info)/1e9:.2f} GB) "
         f"prep {t_prep:.2f}s (simplify {t_simpl:.2f}s, aorder {t_aorder:.2f}s)")
 
     model = None
@@ -585,27 +577,20 @@ def run_triangles(args, w, kernels, with_cpu):
     g.close()
     ctx.close()
     return dict(info=info, m=m, head=head, results=results, cpu=cpu, cpu_par=cpu_par,
-                t_gen=t_gen, t_prep=t_prep, stream=stream,
-                entry_bytes=ENTRY_BYTES.get(name_of(w), 2))
+                t_gen=t_gen, t_prep=t_prep, stream=stream, on16=on16)
 
 
-def name_of(w):
-    return next(k for k, v in WORKLOADS.items() if v is w)
-
-
-def triangle_roofline(info, hr, traffic, stream, entry_bytes):
-    """The head kernel (AUTO and the learned schedule) streams its work lists:
-    tc_auto_stream_bytes counts them at 4 bytes an entry, k_count16 reads 2."""
-    stream = stream * entry_bytes / 4
+def triangle_roofline(info, hr, traffic, stream, on16):
+    """The head engine (AUTO or the learned schedule): the bytes it streams,
+    over 16-bit rows (on16) or the 32-bit work lists, by its kernels' time."""
     achieved = stream / (hr["ms_kernels"] * 1e-3) / 1e9
     return {
         "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-        "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic, "kernel": "k_count16" if entry_bytes == 2 else "k_auto_wl<2048>",
+        "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic, "kernel": "k_count16" if on16 else "k_auto_wl<2048>",
         "bytes_per_count": stream,
-        "bytes_rule": "tc_auto_stream_bytes x entry bytes / 4: per task x, 20 + 4 d+(x) (task id, "
-                      "row bounds in both CSRs, N+(x)); per work-list entry y, 8 + 4 d+(y) (its "
-                      "row bounds, stored with the entry, and N+(y)); half of it over 16-bit rows",
-        "entry_bytes": entry_bytes,
+        "bytes_rule": "tc_count_stream_bytes: over 16-bit rows 16 per 16-byte unit of every own "
+                      "and streamed row, 8 per work-list entry, 16 per task; else per task x, "
+                      "20 + 4 d+(x), and per work-list entry y, 8 + 4 d+(y)",
         "bytes_push_form": kernel_bytes(info),
         "bytes_alg_edge_model": info.bytes_alg,
     }
@@ -626,7 +611,7 @@ def leg_summary(name, w, r, traffic=None):
     return {"workload": describe(w), "n": r["info"].n, "m": r["m"], "count": hr["count"],
             "engine": r["head"], "edges_per_s": hr["edges_per_s"], "ms_per_step": hr["ms_wall"],
             "roofline": triangle_roofline(r["info"], hr, traffic, r["stream"],
-                                          r["entry_bytes"]),
+                                          r["on16"]),
             "learned_vs_plain": vs_plain(r["results"], r["head"], traffic),
             "kernels": {k: {kk: (round(v, 4) if isinstance(v, float) else v)
                             for kk, v in x.items()} for k, x in r["results"].items()}}
@@ -729,7 +714,7 @@ def main():
             "n": info.n, "m": m, "count": hr["count"], "engine": head,
             "parallelism": "single GPU",
         },
-        "roofline": triangle_roofline(info, hr, traffic, r["stream"], r["entry_bytes"]),
+        "roofline": triangle_roofline(info, hr, traffic, r["stream"], r["on16"]),
         "cpu_baseline": r["cpu"],
         "cpu_baseline_parallel": r["cpu_par"],
         "learned_vs_plain": vs_plain(r["results"], head, traffic),

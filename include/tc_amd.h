@@ -360,7 +360,15 @@ int tc_approx_ratio(tc_ctx* ctx, tc_graph* g, double* ratio);
  * NULL (AUTO with defaults).  timing may be NULL. */
 int tc_count(tc_ctx* ctx, tc_graph* g, const tc_sched* sched, uint64_t* count,
              tc_timing* timing);
-/* Bytes one AUTO count streams under sched (NULL: defaults): for
+/* Bytes that a count by AUTO's default schedule (NULL sched), or by
+ * tc_count_learned with a model, streams.  Where it runs over 16-bit list rows
+ * (*rows, optional, is 1) these are 16 per 16-byte unit of every task's own row
+ * and of every streamed row, padding included, 8 per work-list entry and 16 per
+ * task, over both parts; else tc_auto_stream_bytes' (*rows is 0).  Builds the
+ * lists when needed. */
+int tc_count_stream_bytes(tc_ctx* ctx, tc_graph* g, double* bytes, int* rows);
+/* Bytes one AUTO count streams under sched (NULL: defaults) over the 32-bit lists,
+ * also of a graph that the default schedule counts over 16-bit rows: for
  * TC_AUTO_WORKLIST the sum over tasks x of 20 + 4 d+(x) (task id, row bounds
  * in both CSRs, N+(x)) and over the work list of x of 8 + 4 d+(y) (the row
  * bounds of y, stored with the entry, and N+(y)); for TC_AUTO_PUSH 4(n+1) + 12 m+ + 4 sum_v d-(v) d+(v).
@@ -562,8 +570,9 @@ int tc_batch_create(tc_ctx* ctx, uint32_t ngraphs, const uint64_t* edge_off,
 int tc_batch_destroy(tc_batch* b);
 /* Sizes of the batch's union CSR (n, m+, algorithmic bytes of one count). */
 int tc_batch_info_get(const tc_batch* b, tc_graph_info* info);
-/* Bytes one batched count streams in the work-list form: the work-list
- * bytes of the union CSR (tc_auto_stream_bytes), whatever the task split.
+/* Bytes one batched count streams in the work-list form: as
+ * tc_count_stream_bytes over 16-bit rows, where they are used, else the 32-bit
+ * work-list bytes of the union CSR (tc_auto_stream_bytes), whatever the task split.
  * The push form streams 4(n+1) + 12 m+ + 4 sum d- d+ (tc_batch_info_get). */
 int tc_batch_stream_bytes(tc_ctx* ctx, tc_batch* b, double* bytes);
 /* For each form, tries the wave_max_deg candidates, then filter_min, then
