@@ -104,6 +104,7 @@ using namespace tcx;
 extern "C" {
 
 int tc_cost_functions(tc_ctx* c, tc_graph* g, int k, float* out) {
+  PoolScope scope(c);
   TCX_TRY(check(c, g));
   if (!out) return fail(TC_ERR_ARG, "NULL output");
   RawCounts rc;
@@ -135,6 +136,7 @@ int tc_cost_functions(tc_ctx* c, tc_graph* g, int k, float* out) {
 }
 
 int tc_approx_ratio(tc_ctx* c, tc_graph* g, double* ratio) {
+  PoolScope scope(c);
   TCX_TRY(check(c, g));
   if (!ratio) return fail(TC_ERR_ARG, "NULL output");
   RawCounts rc;

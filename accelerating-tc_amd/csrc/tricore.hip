@@ -153,6 +153,7 @@ void tc_tricore_split(uint64_t* edges, uint64_t m, uint64_t part_num, uint32_t**
     set_error("split: bad arguments");
     return;
   }
+  PoolScope scope(c);
   DevBuf de, keys, tmp, idx, adj;
   if (de.reserve(8 * std::max<uint64_t>(m, 1)) || keys.reserve(8 * std::max<uint64_t>(m, 1)) ||
       tmp.reserve(8 * std::max<uint64_t>(m, 1)) || adj.reserve(4 * std::max<uint64_t>(m, 1)))

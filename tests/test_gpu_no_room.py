@@ -1,7 +1,8 @@
-"""Counts when the memory for list rows is not there.  In a process whose
-hipMalloc refuses one request after the other, every count either gives the
-oracle's value, by a kernel that needs less, or says that memory ran out, and the
-same call afterwards gives the value."""
+"""Device memory from the outside, in a process of its own whose hipMalloc is the
+test's.  Repeated calls ask for none.  And counts when the memory for list rows
+is not there: where one request after the other is refused, every count either
+gives the oracle's value, by a kernel that needs less, or says that memory ran
+out, and the same call afterwards gives the value."""
 import json
 import os
 import subprocess
@@ -95,16 +96,56 @@ print(json.dumps(out))
 """
 
 
-def test_counts_without_room_for_rows(tmp_path):
-    shim = str(tmp_path / "failing_malloc.so")
-    b = subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", shim,
+REPEATED = r"""
+import ctypes as C, json, os, sys
+shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+shim.mallocs.restype = C.c_long
+sys.path.insert(0, os.path.join(sys.argv[2], "accelerating-tc_amd"))
+import tcamd
+ctx = tcamd.Context(0)
+s, d = tcamd.gen_er(300_000, 1_500_000, 1)
+g = ctx.graph(s, d).orient(tcamd.ORIENT_DEGREE)
+ops = {"costs": lambda: g.cost_functions(2), "ratio": g.approx_ratio, "count": g.count,
+       "vertex": g.count_per_vertex, "hu": lambda: g.count("hu"),
+       "orient": lambda: g.orient(tcamd.ORIENT_ADIR),
+       "graph": lambda: ctx.graph(s, d).close()}
+out = {}
+for name, op in ops.items():
+    for _ in range(5):
+        op()
+    before = shim.mallocs()
+    for _ in range(3):
+        op()
+    out[name] = shim.mallocs() - before
+assert before > 0
+ctx.close()
+print(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("shim") / "failing_malloc.so")
+    b = subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", so,
                         os.path.join(TESTS, "failing_malloc.cpp"), "-ldl"],
                        capture_output=True, text=True)
     assert b.returncode == 0, b.stderr[-2000:]
-    r = subprocess.run([sys.executable, "-c", SCRIPT, shim, os.path.dirname(TESTS)],
+    return so
+
+
+def child(script, shim):
+    r = subprocess.run([sys.executable, "-c", script, shim, os.path.dirname(TESTS)],
                        capture_output=True, text=True, timeout=110)
     assert r.returncode == 0, r.stderr[-3000:]
-    out = json.loads(r.stdout)
+    return json.loads(r.stdout)
+
+
+def test_repeated_calls_allocate_nothing(shim):
+    assert set(child(REPEATED, shim).values()) == {0}
+
+
+def test_counts_without_room_for_rows(shim):
+    out = child(SCRIPT, shim)
     # none but what a count cannot do without: the results, and Hu's block starts.  (AUTO,
     # learned and per-vertex counts of the graph that the 16-bit rows do not suit
     # need their task lists.)
