@@ -643,8 +643,8 @@ static unsigned grid_for(uint64_t n, int tb = TB) {
 
 static int auto_schedule(tc_ctx* c, tc_graph* g, uint32_t wmax, uint32_t hmin);
 
-// tri[u] = the triangles whose first vertex is u: the AUTO kernel's block
-// and wave tasks (default thresholds) with one output per vertex.
+// tri[u] = the triangles whose first vertex is u: over the 16-bit rows, or the AUTO
+// kernel's block and wave tasks (default thresholds) with one output per vertex.
 int per_vertex_counts(tc_ctx* c, tc_graph* g, unsigned long long* tri) {
   if (g->n == 0) return TC_OK;
   ensure_version(g);  // the task lists are those of the present CSR

@@ -60,7 +60,17 @@ extern "C" {
 /* Orientation flags. */
 #define TC_FLAG_PRUNE_DEG1 1u   /* Hu/preTC.cu:135-169: drop degree<=1 vertices, compact ids */
 
-/* Counting method. */
+/* Counting method.  All give the same count.  Over 16-bit list rows (or 32-bit ones of
+ * all entries where those do not suit the graph) Fox and TriCore run AUTO's kernel
+ * over AUTO's lists, Hu and Bisson run it over push lists in their own slices;
+ * below, and where there is no memory for rows, each has its own kernel:
+ *   Hu       own kernel for a CSR's first three counts, below 1.5e6 edges and
+ *            6.7e7 wedges;
+ *   Bisson,  own kernel below those sizes, or with bitmap_min_deg /
+ *   TriCore  tricore_parts > 1;
+ *   Fox      own kernel below 32,768 edges, for the first three counts of a CSR
+ *            of more than 65,535 vertices and fewer than 524,288 edges, or with
+ *            fox_max_lanes / fox_rearrange. */
 #define TC_KERNEL_HU 0          /* Hu/tc.cu:69-201      */
 #define TC_KERNEL_BISSON 1      /* Bisson/tc.cu:18-104  */
 #define TC_KERNEL_FOX 2         /* Fox/tc.cu:64-125     */
@@ -375,8 +385,10 @@ int tc_count_stream_bytes(tc_ctx* ctx, tc_graph* g, double* bytes, int* rows);
  * Builds the schedule when needed.  No counterpart in the reference. */
 int tc_auto_stream_bytes(tc_ctx* ctx, tc_graph* g, const tc_sched* sched, double* bytes);
 /* Per-vertex forward counts tri[u] (n entries): the triangles whose first
- * vertex (the tail of the two other arcs) is u, from the AUTO kernel's block
- * and wave tasks with default thresholds.  They sum to tc_count's total. */
+ * vertex (the tail of the two other arcs) is u, over 16-bit list rows where they
+ * suit the graph (not for the first three calls on a CSR of more than 65,535
+ * vertices, fewer than 1.5e6 edges and 6.7e7 wedges), else by AUTO's block and
+ * wave tasks with default thresholds.  They sum to tc_count's total. */
 int tc_count_per_vertex(tc_ctx* ctx, tc_graph* g, uint64_t* tri);
 
 /* ---- counting without device allocation --------------------------------
