@@ -1667,7 +1667,8 @@ int tc_graph_load_csr(tc_ctx* c, const char* path, tc_graph** out) {
   if (rp[0] != 0 || rp[n] != m) return fail(TC_ERR_FORMAT, "%s: row offsets do not span m", path);
   std::vector<uint32_t> esrc(std::max<uint64_t>(m, 1));
   for (uint32_t v = 0; v < n; ++v) {
-    if (rp[v + 1] < rp[v]) return fail(TC_ERR_FORMAT, "%s: row offsets decrease at %u", path, v);
+    if (rp[v + 1] < rp[v] || rp[v + 1] > m)
+      return fail(TC_ERR_FORMAT, "%s: row offsets decrease at or after %u", path, v);
     for (uint32_t e = rp[v]; e < rp[v + 1]; ++e) {
       if (col[e] >= n || col[e] == v || (e > rp[v] && col[e] <= col[e - 1]))
         return fail(TC_ERR_FORMAT, "%s: row %u is not ascending, loop-free and in range", path, v);
