@@ -530,13 +530,15 @@ int build(tc_ctx* c, tc_graph* g, DevBuf& idbuf, bool id_all, bool credit, bool 
                      pre, L.hub.row.as<uint2>(), L.hub.col.as<uint16_t>(),
                      L.tail.row.as<uint2>(), L.tail.col.as<uint32_t>());
   TCX_HIP(hipGetLastError());
+  L.credit = credit;
+  L.listed = lists;
+  if (lists) TCX_TRY(work_lists(c, g, cnt.as<uint32_t>(), id, false, credit, L.hub));
   L.tail.tasks = 0;
   if (tail) TCX_TRY(work_lists(c, g, tcnt.as<uint32_t>(), id, true, credit, L.tail));
-  swap(L.id, idbuf);
-  swap(L.cnt, cnt);
-  L.credit = credit;
-  L.listed = false;
-  if (lists) TCX_TRY(hub_lists(c, g, L));
+  if (!lists) {
+    swap(L.id, idbuf);
+    swap(L.cnt, cnt);
+  }
   L.usable = true;
   return TC_OK;
 }
