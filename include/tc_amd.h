@@ -166,8 +166,8 @@ int tc_ctx_destroy(tc_ctx* ctx);
 /* Total device memory in bytes (tricore init_gpu(), tricount_gpu.cu:29-35). */
 int tc_ctx_device_memory(const tc_ctx* ctx, uint64_t* bytes);
 /* Device memory that a context's graphs and calls no longer use is kept for
- * the next ones: by all contexts of a device together at most 1/16 of its
- * memory, until the last of them is destroyed or an allocation of the library
+ * the next ones: by a context at most 1/16 of the device's memory, by all of its
+ * contexts together 1/8, until the last of them is destroyed or an allocation of the library
  * fails.  This call gives what ctx (and destroyed contexts of its device) keep
  * back to the system, for other allocators of the process or the machine. */
 int tc_ctx_release_memory(tc_ctx* ctx);

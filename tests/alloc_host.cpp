@@ -99,16 +99,23 @@ static void use(tc_ctx* c, size_t bytes, int count) {
 }
 
 int main() {
-  // all contexts together keep 1/16 of the card
+  // a context keeps 1/16 of the card, all of them together 1/8
+  {
+    tc_ctx* c = open_ctx();
+    use(c, kCard / 64, 8);
+    CHECK(used() > 0 && used() <= kCard / 16);
+    close_ctx(c);
+    CHECK(used() == 0);
+  }
   std::vector<tc_ctx*> cs;
   for (int i = 0; i < 16; ++i) cs.push_back(open_ctx());
   for (tc_ctx* c : cs) use(c, kCard / 64, 4);
-  CHECK(used() > 0 && used() <= kCard / 16);
+  CHECK(used() > 0 && used() <= kCard / 8);
   // a destroyed context's blocks count too
   for (int i = 8; i < 16; ++i) close_ctx(cs[i]);
   cs.resize(8);
   for (tc_ctx* c : cs) use(c, kCard / 64, 4);
-  CHECK(used() > 0 && used() <= kCard / 16);
+  CHECK(used() > 0 && used() <= kCard / 8);
 
   // kept blocks are used again
   size_t before = g_mallocs;
@@ -175,7 +182,7 @@ int main() {
           CHECK(memcmp(dst.data(), src.data(), src.size()) == 0);
         }
         if (i % 3 == 0) tcx::pool_release(c);
-        CHECK(used() <= kCard / 16 + 8 * 3 * (kCard / 256) * 9 / 8);
+        CHECK(used() <= kCard / 8 + 8 * 3 * (kCard / 256) * 9 / 8);
         close_ctx(c);
       }
     });
