@@ -1,6 +1,7 @@
 // The device memory of contexts (alloc.cpp) over a HIP runtime of this file: a
 // card of kCard bytes whose blocks are host addresses.  Prints "ok", or what
 // went wrong.
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
@@ -19,6 +20,7 @@ static std::mutex g_card;
 static std::map<void*, size_t> g_live;
 static size_t g_used = 0, g_mallocs = 0;
 static std::atomic<int> g_pinned{0}, g_events{0};
+static std::atomic<long> g_copies_left{-1};  // copies until one fails (-1: none does)
 
 static size_t used() {
   std::lock_guard<std::mutex> lk(g_card);
@@ -60,6 +62,7 @@ hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "out of memory"; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  if (g_copies_left >= 0 && g_copies_left-- == 0) return hipErrorUnknown;
   return memcpy(d, s, n), hipSuccess;
 }
 }
@@ -167,6 +170,21 @@ int main() {
   CHECK(used() == 0);
   for (tc_ctx* c : cs) close_ctx(c);
   CHECK(used() == 0);
+
+  // a staged upload, any copy of which fails, says so, and the next one is whole
+  {
+    std::vector<char> src((9u << 20) + 5), dst(src.size());
+    for (size_t i = 0; i < src.size(); ++i) src[i] = (char)(i * 7 + i / 4096);
+    tc_ctx* c = open_ctx();
+    for (long k = 0; k < 3; ++k) {
+      g_copies_left = k;
+      CHECK(tcx::upload(c, dst.data(), src.data(), src.size()) == TC_ERR_HIP);
+      g_copies_left = -1;
+      std::fill(dst.begin(), dst.end(), 0);
+      CHECK(tcx::upload(c, dst.data(), src.data(), src.size()) == TC_OK && dst == src);
+    }
+    close_ctx(c);
+  }
 
   // contexts that come and go on threads, with uploads through the shared slots
   std::vector<std::thread> th;
